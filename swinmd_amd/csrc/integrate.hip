@@ -13,8 +13,7 @@
 // whole-system sums are block-reduced FP64 atomics.  The step is a fixed
 // sequence of kernels whose list rebuild is gated on a device flag, so it can
 // be captured once into a hipGraph and replayed.
-#include <type_traits>
-
+#include "shake.h"
 #include "smd_internal.h"
 
 namespace smd {
@@ -104,145 +103,146 @@ __global__ __launch_bounds__(256) void k_step_head(IntegArgs a) {
     block_store<4>(v, a.part_vom, a.nb_vom);
 }
 
-// SHAKE of one water (a.mol_start[m], three sites).  Stores the new
-// positions, displacements, unwrapped positions, velocities and vtMinus, adds
-// its constraint virial to v, and leaves the new positions and velocities,
-// the forces it used and the masses in pn, vel, F and ms.
+// What SHAKE reads of one water (sites 3m, 3m + 1, 3m + 2: SHAKE takes 3-site
+// molecules only), loaded in one go before anything waits.
+struct ShakeIn {
+    double ro[3][3], vt[3][3], F[3][3], disp[3][3], real[3][3], ms[3], P[3], bl[3], fnh;
+};
+
+__device__ __forceinline__ void shake_load(const IntegArgs& a, int m, ShakeIn& in) {
+    const int a0 = 3 * m;
+    in.fnh = a.fnh_on_device ? a.scalars[0] : a.fnh_host;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) { in.P[d] = a.mom[3 * m + d]; in.bl[d] = a.bond2[3 * m + d]; }
+    load9(a.pos + 3 * a0, in.ro);
+    load9(a.vtm + 3 * a0, in.vt);
+    load9(a.force + 3 * a0, in.F);
+    if (a.frecip) {   // the sum the reference forms: short-range terms, then k-space
+        double fk[3][3];
+        load9(a.frecip + 3 * a0, fk);
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) in.F[s][d] += fk[s][d];
+    }
+    load9(a.disp + 3 * a0, in.disp);
+    load9(a.real + 3 * a0, in.real);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) in.ms[s] = a.mass[a0 + s];
+}
+
+// SHAKE of one water.  Stores the new positions, displacements, unwrapped
+// positions, velocities and vtMinus, adds its constraint virial to v, and
+// leaves the new positions and velocities in pn and vel.
 // vcm: the MD step's drift velocity (LFIntegrator::run :354-379), removed
 // from vtMinus (the velocity is rewritten below from vtMinus, so only vtMinus
 // needs it); zero outside the MD step.
-__device__ __forceinline__ void shake_mol(const IntegArgs& a, int m, const double (&vcm)[3], double (&v)[9],
-                                          double (&pn)[3][3], double (&vel)[3][3], double (&F)[3][3],
-                                          double (&ms)[3]) {
-    {
-        const int a0 = a.mol_start[m];
-        const double fnh = a.fnh_on_device ? a.scalars[0] : a.fnh_host;
-        const double Px = a.mom[3 * m], Py = a.mom[3 * m + 1], Pz = a.mom[3 * m + 2];
-        const double tol_2 = 2 * a.tol;
-        double ro[3][3], rn[3][3], mr[3], vt[3][3];
+__device__ __forceinline__ void shake_mol(const IntegArgs& a, int m, const ShakeIn& in, const double (&vcm)[3],
+                                          double (&v)[9], double (&pn)[3][3], double (&vel)[3][3]) {
+    const int a0 = 3 * m;
+    double rn[3][3], mr[3], vt[3][3];
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-            const int id = a0 + s;
-            ms[s] = a.mass[id];
-            mr[s] = 1.0 / ms[s];
-            const double h = a.dt * mr[s];
-            for (int d = 0; d < 3; ++d) {
-                ro[s][d] = a.pos[3 * id + d];
-                vt[s][d] = a.vtm[3 * id + d] - vcm[d];
-                double Fd = a.force[3 * id + d];
-                if (a.frecip) {   // the sum the reference forms: short-range terms, then k-space
-                    Fd += a.frecip[3 * id + d];
-                    a.force[3 * id + d] = Fd;
-                }
-                F[s][d] = Fd;
-                double vp;
-                if (a.nose_hoover) {
-                    const double P = d == 0 ? Px : (d == 1 ? Py : Pz);
-                    vp = vt[s][d] + h * (Fd - (fnh * P) / 3.0);
-                } else {
-                    vp = vt[s][d] + h * Fd;
-                }
-                rn[s][d] = ro[s][d] + a.dt * vp;
-            }
-        }
-        // Squared lengths and old-bond vectors are loop invariants; the three
-        // constraints are unrolled so every array index is a constant and the
-        // per-molecule state stays in registers.
-        double bl[3], od[3][3], msum[3];
+    for (int s = 0; s < 3; ++s) {
+        mr[s] = 1.0 / in.ms[s];
+        const double h = a.dt * mr[s];
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const int nx = b == 2 ? 0 : b + 1;
-            bl[b] = a.bond2[3 * m + b];
-            od[b][0] = ro[b][0] - ro[nx][0];
-            od[b][1] = ro[b][1] - ro[nx][1];
-            od[b][2] = ro[b][2] - ro[nx][2];
-            pbc(od[b][0], od[b][1], od[b][2], a.box);
-            msum[b] = mr[b] + mr[nx];
-        }
-        // Minimum image inside the sweeps only for a molecule that spans a
-        // quarter box; otherwise apply_pbc is the identity on its bonds.
-        bool wrap = false;
-#pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const int nx = b == 2 ? 0 : b + 1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                wrap = wrap || fabs(od[b][d]) > 0.25 * a.box.L[d] || fabs(rn[b][d] - rn[nx][d]) > 0.25 * a.box.L[d];
-        }
-        // Gauss-Seidel sweeps (LFIntegrator.cpp:1499-1540).  The update is
-        // predicated instead of branched: an inactive constraint moves its
-        // atoms by exactly 0.0, and its quotient is discarded by a select.
-        // The sweep loop is compiled twice, with and without the minimum
-        // image, and a wave takes the plain one unless one of its molecules
-        // needs wrapping.  The constraint virial sum_s f_s n_s (x) o is kept
-        // as sum_s f_s n_s per constraint and multiplied by o once.
-        int count = 0;
-        bool done = false, failed = false;
-        double wv[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-        auto sweeps = [&](auto wrap_tag) {
-            constexpr bool WRAP = decltype(wrap_tag)::value;
-            while (!done && count < a.max_count && !failed) {
-                done = true;
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const int nx = b == 2 ? 0 : b + 1;
-                    double nX = rn[b][0] - rn[nx][0], nY = rn[b][1] - rn[nx][1], nZ = rn[b][2] - rn[nx][2];
-                    if (WRAP && wrap) pbc(nX, nY, nZ, a.box);
-                    const double diff = bl[b] - len2_exact(nX, nY, nZ);
-                    const double oX = od[b][0], oY = od[b][1], oZ = od[b][2];
-                    const double rno = oX * nX + oY * nY + oZ * nZ;
-                    const bool act = fabs(diff) > bl[b] * tol_2;
-                    failed = failed || (act && rno < bl[b] * a.tol);
-                    const double q = diff / (2 * rno * msum[b]);
-                    const double factor = act ? q : 0.0;
-                    wv[b][0] += factor * nX; wv[b][1] += factor * nY; wv[b][2] += factor * nZ;
-                    const double fX = factor * oX, fY = factor * oY, fZ = factor * oZ;
-                    rn[b][0] += mr[b] * fX; rn[b][1] += mr[b] * fY; rn[b][2] += mr[b] * fZ;
-                    rn[nx][0] -= mr[nx] * fX; rn[nx][1] -= mr[nx] * fY; rn[nx][2] -= mr[nx] * fZ;
-                    done = done && !act;
-                }
-                count++;
-            }
-        };
-        if (__any(wrap)) sweeps(std::true_type{});
-        else sweeps(std::false_type{});
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int x = 0; x < 3; ++x)
-#pragma unroll
-                for (int y = 0; y < 3; ++y) v[3 * x + y] += wv[b][x] * od[b][y];
-        if (a.md_step && m == 0) a.flag[0] = 0;   // every consumer of the rebuild flag has run
-        if (failed) atomicOr(a.status, ST_SHAKE_FAIL);
-        else if (!done) atomicOr(a.status, ST_SHAKE_NOCONV);
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-            const int id = a0 + s;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const double p0 = a.pos[3 * id + d];
-                const double dr = rn[s][d] - p0;
-                pn[s][d] = p0 + dr;
-                a.pos[3 * id + d] = pn[s][d];
-                a.disp[3 * id + d] += dr;
-                a.real[3 * id + d] += dr;
-                const double vp = dr / a.dt;
-                vel[s][d] = (vp + vt[s][d]) * 0.5;
-                a.vel[3 * id + d] = vel[s][d];
-                a.vtm[3 * id + d] = vp;
-            }
+        for (int d = 0; d < 3; ++d) {
+            vt[s][d] = in.vt[s][d] - vcm[d];
+            const double Fd = in.F[s][d];
+            const double vp = a.nose_hoover ? vt[s][d] + h * (Fd - (in.fnh * in.P[d]) / 3.0) : vt[s][d] + h * Fd;
+            rn[s][d] = in.ro[s][d] + a.dt * vp;
         }
     }
+    double od[3][3], nd[3][3];
+    // Minimum image inside the sweeps only for a molecule that spans a
+    // quarter box; otherwise apply_pbc is the identity on its bonds.
+    bool wrap = false;
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const int nx = b == 2 ? 0 : b + 1;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            od[b][d] = in.ro[b][d] - in.ro[nx][d];
+            nd[b][d] = rn[b][d] - rn[nx][d];
+        }
+        pbc(od[b][0], od[b][1], od[b][2], a.box);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            wrap = wrap || fabs(od[b][d]) > 0.25 * a.box.L[d] || fabs(nd[b][d]) > 0.25 * a.box.L[d];
+    }
+    bool done = false, failed = false;
+    double wv[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+    if (!__any(wrap)) {
+        shake_sweeps(od, nd, mr, in.bl, a.tol, a.max_count, rn, wv, done, failed);
+    } else {
+        // Coordinate form of the same sweeps with the minimum image of each
+        // bond.  The update is predicated instead of branched: an inactive
+        // constraint moves its atoms by exactly 0.0.
+        const double tol_2 = 2 * a.tol;
+        int count = 0;
+        while (!done && count < a.max_count && !failed) {
+            done = true;
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                const int nx = b == 2 ? 0 : b + 1;
+                double nX = rn[b][0] - rn[nx][0], nY = rn[b][1] - rn[nx][1], nZ = rn[b][2] - rn[nx][2];
+                if (wrap) pbc(nX, nY, nZ, a.box);
+                const double diff = in.bl[b] - len2_exact(nX, nY, nZ);
+                const double oX = od[b][0], oY = od[b][1], oZ = od[b][2];
+                const double rno = oX * nX + oY * nY + oZ * nZ;
+                const bool act = fabs(diff) > in.bl[b] * tol_2;
+                failed = failed || (act && rno < in.bl[b] * a.tol);
+                const double q = diff / (2 * rno * (mr[b] + mr[nx]));
+                const double factor = act ? q : 0.0;
+                wv[b][0] += factor * nX; wv[b][1] += factor * nY; wv[b][2] += factor * nZ;
+                const double fX = factor * oX, fY = factor * oY, fZ = factor * oZ;
+                rn[b][0] += mr[b] * fX; rn[b][1] += mr[b] * fY; rn[b][2] += mr[b] * fZ;
+                rn[nx][0] -= mr[nx] * fX; rn[nx][1] -= mr[nx] * fY; rn[nx][2] -= mr[nx] * fZ;
+                done = done && !act;
+            }
+            count++;
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+            for (int y = 0; y < 3; ++y) v[3 * x + y] += wv[b][x] * od[b][y];
+    if (a.md_step && m == 0) a.flag[0] = 0;   // every consumer of the rebuild flag has run
+    if (failed) atomicOr(a.status, ST_SHAKE_FAIL);
+    else if (!done) atomicOr(a.status, ST_SHAKE_NOCONV);
+    const double rdt = 1.0 / a.dt;
+    double disp[3][3], real[3][3], vp[3][3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double dr = rn[s][d] - in.ro[s][d];
+            pn[s][d] = in.ro[s][d] + dr;
+            disp[s][d] = in.disp[s][d] + dr;
+            real[s][d] = in.real[s][d] + dr;
+            vp[s][d] = dr * rdt;
+            vel[s][d] = (vp[s][d] + vt[s][d]) * 0.5;
+        }
+    store9(a.pos + 3 * a0, pn);
+    store9(a.disp + 3 * a0, disp);
+    store9(a.real + 3 * a0, real);
+    store9(a.vel + 3 * a0, vel);
+    store9(a.vtm + 3 * a0, vp);
+    if (a.frecip) store9(a.force + 3 * a0, in.F);
 }
 
 __global__ __launch_bounds__(256) void k_shake(IntegArgs a) {
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     double vcm[3] = {0.0, 0.0, 0.0};
-    if (a.md_step) drift_velocity(a, vcm);
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    ShakeIn in;
+    if (m < a.nmol) shake_load(a, m, in);
+    if (a.md_step) drift_velocity(a, vcm);
     if (m < a.nmol) {
-        double pn[3][3], vel[3][3], F[3][3], ms[3];
-        shake_mol(a, m, vcm, v, pn, vel, F, ms);
+        double pn[3][3], vel[3][3];
+        shake_mol(a, m, in, vcm, v, pn, vel);
     }
     // the constraint virial: block partials, added in block order by
     // k_rows_finish
@@ -475,17 +475,22 @@ __global__ __launch_bounds__(KIN_THREADS) void k_kinetics(IntegArgs a, int rewra
 // arithmetic of k_kinetics), then the step's epilogue in the last block.
 __global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int rewrap) {
     double sv[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double v[2] = {0.0, 0.0};
-    double pr[21];
+    double sum[KIN_PARTS];   // rows of part_kin
 #pragma unroll
-    for (int k = 0; k < 21; ++k) pr[k] = 0.0;
+    for (int k = 0; k < KIN_PARTS; ++k) sum[k] = 0.0;
+    double* v = sum + KP_KE;
+    double* pr = sum + KP_PR;
     double vcm[3];
-    drift_velocity(a, vcm);
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    ShakeIn in;
+    if (m < a.nmol) shake_load(a, m, in);
+    drift_velocity(a, vcm);
     if (m < a.nmol) {
-        double pn[3][3], vel[3][3], F[3][3], ms[3];
-        shake_mol(a, m, vcm, sv, pn, vel, F, ms);
-        const int s0 = a.mol_start[m];
+        double pn[3][3], vel[3][3];
+        const double (&F)[3][3] = in.F;
+        const double (&ms)[3] = in.ms;
+        shake_mol(a, m, in, vcm, sv, pn, vel);
+        const int s0 = 3 * m;
         const double M = (0.0 + ms[0] + ms[1]) + ms[2];
         double P[3] = {0, 0, 0}, C[3] = {0, 0, 0};
 #pragma unroll
@@ -522,15 +527,18 @@ __global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int
             double cx = C[0], cy = C[1], cz = C[2];
             pbc(cx, cy, cz, a.box);
             const double dx = cx - C[0], dy = cy - C[1], dz = cz - C[2];
-            for (int i = s0; i < s0 + 3; ++i) { a.pos[3 * i] += dx; a.pos[3 * i + 1] += dy; a.pos[3 * i + 2] += dz; }
+            if (dx != 0.0 || dy != 0.0 || dz != 0.0) {
+#pragma unroll
+                for (int s = 0; s < 3; ++s) { pn[s][0] += dx; pn[s][1] += dy; pn[s][2] += dz; }
+                store9(a.pos + 3 * s0, pn);
+            }
             C[0] = cx; C[1] = cy; C[2] = cz;
         }
         for (int d = 0; d < 3; ++d) a.com[3 * m + d] = C[d];
     }
-    const int nb = gridDim.x;
-    block_store<9>(sv, a.part_kin + (size_t)KP_SH * nb, nb);
-    block_store<2>(v, a.part_kin + (size_t)KP_KE * nb, nb);
-    block_store<21>(pr, a.part_kin + (size_t)KP_PR * nb, nb);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) sum[KP_SH + k] = sv[k];
+    wave_store<KIN_PARTS>(sum, a.part_kin, gridDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_mol_centers(int nmol, const int32_t* __restrict__ ms,

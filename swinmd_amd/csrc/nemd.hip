@@ -40,6 +40,7 @@
 #include <string>
 #include <vector>
 
+#include "shake.h"
 #include "smd_internal.h"
 
 namespace smd {
@@ -600,18 +601,19 @@ __global__ __launch_bounds__(KIN_BLOCK) void k_shake(Args a) {
         double M = 0.0;
 #pragma unroll
         for (int s = 0; s < 3; ++s) M += a.p.mass[s];
-        double ro[3][3], rn[3][3], vt[3][3], F[3][3], mr[3];
+        double ro[3][3], rn[3][3], vt[3][3], F[3][3], Fk[3][3], mr[3], dsp[3][3];
+        load9(a.pos + 3 * a0, ro);
+        load9(a.vtm + 3 * a0, vt);
+        load9(a.fpair + 3 * a0, F);
+        load9(a.frec + 3 * a0, Fk);
+        load9(a.disp + 3 * a0, dsp);   // read ahead of the sweeps
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
-            const int id = a0 + s;
             mr[s] = 1.0 / a.p.mass[s];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                ro[s][d] = a.pos[3 * id + d];
-                double vm = a.vtm[3 * id + d];
-                if (st.apply_drift) vm -= st.drift[d];
-                vt[s][d] = vm;
-                F[s][d] = a.fpair[3 * id + d] + a.frec[3 * id + d];
+                if (st.apply_drift) vt[s][d] -= st.drift[d];
+                F[s][d] += Fk[s][d];
             }
             double vp[3];
 #pragma unroll
@@ -641,77 +643,47 @@ __global__ __launch_bounds__(KIN_BLOCK) void k_shake(Args a) {
         // Gauss-Seidel sweeps (LFIntegrator.cpp:1499-1540) over the cyclic
         // constraints H1-O, O-H2, H2-H1; the bond vectors are short, so the
         // reference's minimum image leaves them as they are.
-        double od[3][3], msum[3];
+        double od[3][3];
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
             const int nx = b == 2 ? 0 : b + 1;
 #pragma unroll
             for (int d = 0; d < 3; ++d) od[b][d] = ro[b][d] - ro[nx][d];
-            msum[b] = mr[b] + mr[nx];
         }
-        const double tol = a.p.shake_tol, tol_2 = 2.0 * tol;
-        double sv[9];
+        double nd[3][3], wv[3][3];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) sv[q] = 0.0;
-        int count = 0;
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) nd[b][d] = rn[b][d] - rn[b == 2 ? 0 : b + 1][d];
         bool done = false, failed = false;
-        while (!done && count < a.p.max_count && !failed) {
-            done = true;
-#pragma unroll
-            for (int b = 0; b < 3; ++b) {
-                const int nx = b == 2 ? 0 : b + 1;
-                const double nX = rn[b][0] - rn[nx][0], nY = rn[b][1] - rn[nx][1], nZ = rn[b][2] - rn[nx][2];
-                const double diff = a.p.b2[b] - (nX * nX + nY * nY + nZ * nZ);
-                if (fabs(diff) > a.p.b2[b] * tol_2) {
-                    const double rno = od[b][0] * nX + od[b][1] * nY + od[b][2] * nZ;
-                    if (rno < a.p.b2[b] * tol) {
-                        failed = true;
-                        break;
-                    }
-                    const double factor = diff / (2 * rno * msum[b]);
-                    const double nn[3] = {nX, nY, nZ};
-#pragma unroll
-                    for (int p = 0; p < 3; ++p)
-#pragma unroll
-                        for (int q = 0; q < 3; ++q) sv[3 * p + q] += factor * nn[p] * od[b][q];
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        const double fo = factor * od[b][d];
-                        rn[b][d] += mr[b] * fo;
-                        rn[nx][d] -= mr[nx] * fo;
-                    }
-                    done = false;
-                }
-            }
-            count++;
-        }
+        shake_sweeps(od, nd, mr, a.p.b2, a.p.shake_tol, a.p.max_count, rn, wv, done, failed);
         if (failed) atomicOr(a.err, E_SHAKE_FAIL);
         else if (!done) atomicOr(a.err, E_SHAKE_NOCONV);
 #pragma unroll
-        for (int q = 0; q < 9; ++q) v[SH_SV + q] = sv[q];
+        for (int q = 0; q < 9; ++q)
+            v[SH_SV + q] = wv[0][q / 3] * od[0][q % 3] + wv[1][q / 3] * od[1][q % 3] + wv[2][q / 3] * od[2][q % 3];
         // new positions, displacement, velocities (:1810-1826)
-        double P[3] = {0.0, 0.0, 0.0}, Cm[3] = {0.0, 0.0, 0.0};
+        const double rdt = 1.0 / dt;
+        double P[3] = {0.0, 0.0, 0.0}, Cm[3] = {0.0, 0.0, 0.0}, pnew[3][3], vnew[3][3];
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
-            const int id = a0 + s;
             double vv = 0.0, dd = 0.0;
-            const double dy_old = a.disp[3 * id + 1];
+            const double dy_old = dsp[s][1];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 const double p0 = ro[s][d];
                 const double dr = rn[s][d] - p0;
                 const double pn = p0 + dr;
-                a.pos[3 * id + d] = pn;
+                pnew[s][d] = pn;
                 double dn = dr;
                 if (d == 0) dn -= dt * gamma * (ro[s][1] - dy_old);
-                const double dsp = a.disp[3 * id + d] + dn;
-                a.disp[3 * id + d] = dsp;
-                dd += dsp * dsp;
-                double vp = dr / dt;
+                dsp[s][d] += dn;
+                dd += dsp[s][d] * dsp[s][d];
+                double vp = dr * rdt;
                 if (d == 0) vp -= gamma * Y;
                 const double vel = 0.5 * (vp + vt[s][d]);
-                a.vel[3 * id + d] = vel;
-                a.vtm[3 * id + d] = vp;
+                vnew[s][d] = vel;
+                vt[s][d] = vp;
                 vv += vel * vel;
                 P[d] += a.p.mass[s] * vel;
                 Cm[d] += a.p.mass[s] * pn;
@@ -741,13 +713,12 @@ __global__ __launch_bounds__(KIN_BLOCK) void k_shake(Args a) {
         double cx = Cm[0], cy = Cm[1], cz = Cm[2];
         le_wrap_point(cx, cy, cz, rp.L, tilt1);
         const double sx = cx - Cm[0], sy = cy - Cm[1], sz = cz - Cm[2];
-        if (sx != 0.0 || sy != 0.0 || sz != 0.0) {
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {
-                const int id = a0 + s;
-                a.pos[3 * id] += sx; a.pos[3 * id + 1] += sy; a.pos[3 * id + 2] += sz;
-            }
-        }
+        for (int s = 0; s < 3; ++s) { pnew[s][0] += sx; pnew[s][1] += sy; pnew[s][2] += sz; }
+        store9(a.pos + 3 * a0, pnew);
+        store9(a.disp + 3 * a0, dsp);
+        store9(a.vel + 3 * a0, vnew);
+        store9(a.vtm + 3 * a0, vt);
         a.com[3 * m] = cx; a.com[3 * m + 1] = cy; a.com[3 * m + 2] = cz;
         a.mom[3 * m] = P[0]; a.mom[3 * m + 1] = P[1]; a.mom[3 * m + 2] = P[2];
     }
@@ -757,7 +728,7 @@ __global__ __launch_bounds__(KIN_BLOCK) void k_shake(Args a) {
         for (int o = WAVE / 2; o > 0; o >>= 1) d2 = fmax(d2, __shfl_xor(d2, o, WAVE));
         if (threadIdx.x % WAVE == 0 && d2 > 0.0) atomicMax(&st.maxd2, (unsigned long long)__double_as_longlong(d2));
     }
-    block_store<NSH>(v, a.sh_part, a.n_sh_blk);
+    wave_store<NSH>(v, a.sh_part, a.n_sh_blk);
 }
 
 // The replica's epilogue, one block of FINISH_THREADS per replica after
@@ -882,7 +853,7 @@ __global__ __launch_bounds__(KIN_BLOCK) void k_start(Args a) {
             v[SH_INTRA] -= a.p.q[s0] * a.p.q[s1] * erf(a.p.alpha * rr) / rr;
         }
     }
-    block_store<NSH>(v, a.sh_part, a.n_sh_blk);
+    wave_store<NSH>(v, a.sh_part, a.n_sh_blk);
 }
 
 }  // namespace nemd

@@ -480,6 +480,52 @@ __device__ __forceinline__ void block_store(double (&v)[NV], double* part, int s
     __syncthreads();   // red may be reused by the next call
 }
 
+// block_store for blocks of one wave: the sums are taken across a transposed
+// copy in LDS, WAVE / S entries in order by each of S lanes per value, instead
+// of a shuffle tree per value.  A shuffle of a double is two LDS permutes, so
+// the tree costs 12 LDS instructions per value against this form's two, and
+// the SHAKE kernels reduce 32 and 41 values per molecule at the end of a
+// serial chain (see k_shake_kinetics for the times).
+template <int NV>
+__device__ __forceinline__ void wave_store(const double (&v)[NV], double* part, int stride) {
+    constexpr int S = NV <= 16 ? 4 : (NV <= 32 ? 2 : 1), LEN = WAVE / S;
+    static_assert(NV <= WAVE, "wave_store: more values than lanes");
+    __shared__ double buf[NV][WAVE + 1];
+    const int lane = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) buf[k][lane] = v[k];
+    __syncthreads();
+    const int k = min(lane / S, NV - 1);
+    const double* row = buf[k] + (lane % S) * LEN;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+    for (int e = 0; e < LEN; e += 4) { s0 += row[e]; s1 += row[e + 1]; s2 += row[e + 2]; s3 += row[e + 3]; }
+    double s = (s0 + s1) + (s2 + s3);
+#pragma unroll
+    for (int o = 1; o < S; o <<= 1) s += __shfl_xor(s, o, WAVE);
+    if (lane % S == 0 && lane / S < NV) part[(size_t)k * stride + blockIdx.x] = s;
+}
+
+// Nine consecutive doubles (a water's three sites) at an 8-byte aligned
+// address in five instructions: global accesses need no more than dword
+// alignment, and a lane's 72 bytes span few lines either way.
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void load9(const double* __restrict__ p, double (&o)[3][3]) {
+    const double2u* q = reinterpret_cast<const double2u*>(p);
+    const double2u a = q[0], b = q[1], c = q[2], d = q[3];
+    o[0][0] = a.x; o[0][1] = a.y; o[0][2] = b.x;
+    o[1][0] = b.y; o[1][1] = c.x; o[1][2] = c.y;
+    o[2][0] = d.x; o[2][1] = d.y; o[2][2] = p[8];
+}
+__device__ __forceinline__ void store9(double* __restrict__ p, const double (&o)[3][3]) {
+    double2u* q = reinterpret_cast<double2u*>(p);
+    q[0] = double2u{o[0][0], o[0][1]};
+    q[1] = double2u{o[0][2], o[1][0]};
+    q[2] = double2u{o[1][1], o[1][2]};
+    q[3] = double2u{o[2][0], o[2][1]};
+    p[8] = o[2][2];
+}
+
 // Fixed-order sum of p[0..n) by one wave: lane l adds p[l], p[l + 64], ...
 // in order, then a shuffle tree; every lane gets the same bits.
 __device__ __forceinline__ double wave_fixed_sum(const volatile double* p, int n) {

@@ -5,49 +5,35 @@
 //   surfDipoleCorrect         :816-937   two passes over atoms
 //   reciprocal_term           :529-698   structure factors, then forces
 //
-// Reciprocal space.  exp(i k.r) with k = 2 pi (nx/Lx, ny/Ly, nz/Lz) factors
-// into X^nx Y^ny Z^nz with X = exp(i 2 pi x / Lx), ...; the k-vectors of the
-// reference's list come in (nx, ny) rows of consecutive nz, so along a row each
-// term is the previous one times Z.  Rows are cut into groups of at most GK
-// consecutive nz.
-//   pass 0 (k_recip_phase): exp(i 2 pi r_p / L_p) per atom and axis.
-//   pass 1 (k_recip_sfac): a block of SF_WAVES waves owns 64 k-groups (one
-//     per lane) and a chunk of atoms.  Per 64-atom tile the block writes each
-//     atom's powers X^0..X^nmax, Y^0.., Z^0.. to LDS (negative powers are
-//     conjugates); a lane then starts its group at q X^nx Y^ny Z^nz0 and walks
-//     the row with one complex product per k.  Per k it sums q sin, q cos and,
-//     for the volume derivatives, q cos d, q sin d (d = r - R_mol) and
-//     q cos |d|^2, q sin |d|^2.  The waves of a block split the tile's atoms
-//     and are added in LDS, so one partial per (chunk, k) reaches memory.
-//   pass 1b (k_recip_reduce): partials summed over chunks in a fixed order,
-//     then per k: energy, volume derivatives and virial (:596-607); the
-//     reference's per-atom Lustig sums of the force loop (:609-658) are sums
-//     over atoms of products with the per-k sums above, so they are formed
-//     here per k; and (b C, b S) for the force pass.
-//   pass 2 (k_recip_force): a block of RF_WAVES waves owns 64 atoms (one per
-//     lane); wave w takes the w-th range of k-groups, with the groups and
-//     (b C, b S) staged in LDS, walks the rows as pass 1 does, and the waves'
-//     partial forces are added in LDS in wave order.
+// Reciprocal space: kspace.h.  Three launches:
+//   k_recip_sfac: structure factors of an atom chunk, phases exp(i 2 pi r_p /
+//     L_p) evaluated on the way and kept for the forces.  With Lustig terms
+//     also the sums weighted by d = r - R_mol and |d|^2.
+//   k_recip_reduce: partials summed over chunks in a fixed order, then per k:
+//     energy, volume derivatives and virial (:596-607) and the force pass's
+//     coefficients; the reference's per-atom Lustig sums of the force loop
+//     (:609-658) are sums over atoms of products with the per-k sums, so they
+//     are formed here per k.
+//   k_recip_force: forces of 64 atoms per block.  Without Lustig sums (the MD
+//     steps, which report no second derivative) it also forms the first
+//     derivative's molecular part, sum_k sum_i f_ik (k.d_i) = sum_i F_i . d_i,
+//     so the d-weighted structure factors are not needed there.
 // Every sum is taken in a fixed order: results do not depend on scheduling.
 #include <algorithm>
-#include <climits>
-
+#include <cstdlib>
 #include <mutex>
 
+#include "kspace.h"
 #include "smd_internal.h"
 
 namespace smd {
 
-constexpr int GK = 8;          // k-vectors per group: consecutive nz within one (nx, ny) row
-constexpr int SF_TILE = 64;    // atoms per LDS tile in the structure-factor pass
-constexpr int SF_WAVES = 8;    // waves per structure-factor block (same groups, different atoms)
-constexpr int RF_WAVES = 16;   // waves per force block (same atoms, different k ranges)
-constexpr int NSUM = 10;       // per-k sums of the structure-factor pass
 constexpr size_t LDS_MAX = 65536;
-
-// d_e1 holds the phases [n][3] (complex) and then, 32-byte aligned, the
-// per-atom (q, d) of the structure-factor pass.
-static inline size_t e1_am_offset(int n) { return (6 * (size_t)n + 3) & ~(size_t)3; }
+constexpr int NSUM = 5;        // weights of the structure factors with Lustig terms: 1, d, |d|^2
+constexpr int SF_CHUNKS = 256; // atom chunks of the structure-factor pass, at most: one block per CU
+// With Lustig terms a chunk's partials are 211 KB (1,535 k): at 192 chunks
+// writing and summing them took 28.8 + 16.6 us, the products 7.
+constexpr int SF_CHUNKS_LUSTIG = 64;
 
 // ---- host setup -----------------------------------------------------------
 
@@ -61,8 +47,8 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     int nmax[3];
     for (int d = 0; d < 3; ++d) nmax[d] = (int)(p->kcut * c->box.L[d] / (2 * PI));
     const double vx = 2.0 * PI / c->box.L[0], vy = 2.0 * PI / c->box.L[1], vz = 2.0 * PI / c->box.L[2];
-    std::vector<double> kv, k2v, ek;
     std::vector<int32_t> kn;
+    std::vector<double> ek;
     for (int nx = 0; nx <= nmax[0]; nx++) {
         const double kx = nx * vx;
         for (int ny = (nx == 0 ? 0 : -nmax[1]); ny <= nmax[1]; ny++) {
@@ -71,15 +57,13 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
                 const double kz = nz * vz;
                 const double k2 = kx * kx + ky * ky + kz * kz;
                 if (k2 < kCut2) {
-                    kv.push_back(kx); kv.push_back(ky); kv.push_back(kz);
-                    k2v.push_back(k2);
                     ek.push_back(exp(-k2 * alphaR4) / k2);
                     kn.push_back(nx); kn.push_back(ny); kn.push_back(nz);
                 }
             }
         }
     }
-    const int K = (int)k2v.size();
+    const int K = (int)ek.size();
     if (K == 0) return fail(c, SMD_EINVAL, "no k-vectors below kcut");
     for (int d = 0; d < 3; ++d) c->nmax[d] = nmax[d];
     auto realloc = [&](auto*& ptr, size_t bytes) -> int {
@@ -88,67 +72,47 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
         if (hipMalloc(&ptr, bytes) != hipSuccess) return fail(c, SMD_ENOMEM, "Ewald allocation of %zu bytes", bytes);
         return SMD_OK;
     };
-    int rc;
-    if ((rc = realloc(c->d_kvec, sizeof(double) * 3 * K))) return rc;
-    if ((rc = realloc(c->d_kmod2, sizeof(double) * K))) return rc;
-    if ((rc = realloc(c->d_expk, sizeof(double) * K))) return rc;
-    if ((rc = realloc(c->d_kn, sizeof(int32_t) * 3 * K))) return rc;
-    // k-groups: runs of at most GK consecutive nz inside one (nx, ny) row,
-    // stored as (first k, count, nx << 16 | (ny & 0xffff), nz of the first k)
-    std::vector<int4> grp;
-    for (int k = 0; k < K;) {
-        int e = k + 1;
-        while (e < K && e - k < GK && kn[3 * e] == kn[3 * k] && kn[3 * e + 1] == kn[3 * k + 1] &&
-               kn[3 * e + 2] == kn[3 * (e - 1) + 2] + 1)
-            ++e;
-        grp.push_back(make_int4(k, e - k, (kn[3 * k] << 16) | (kn[3 * k + 1] & 0xffff), kn[3 * k + 2]));
-        k = e;
-    }
-    const int ng = (int)grp.size();
-    // force-pass ranges: RF_WAVES contiguous group ranges of similar k count
-    std::vector<int32_t> split(RF_WAVES + 1, ng);
-    split[0] = 0;
-    {
-        int r = 1;
-        int64_t acc = 0;
-        for (int g = 0; g < ng && r < RF_WAVES; ++g) {
-            acc += grp[g].y;
-            if (acc >= (int64_t)K * r / RF_WAVES) split[r++] = g + 1;
+    // rows (nx, ny) of the set, in its order, and per (row, |nz|) the factor
+    // exp(-k^2 / 4 alpha^2) / k^2, 0 where the set has no such k
+    KsRows kr{};
+    kr.n1 = nmax[2] + 1;
+    kr.nx1 = nmax[0] + 1;
+    kr.ny1 = nmax[1] + 1;
+    kr.ts = ks_stride(kr.powers());
+    std::vector<int32_t> xy;
+    std::vector<double> rexp;
+    int ng = 0, run = 0;   // runs of at most eight consecutive nz in a row
+    for (int k = 0; k < K; ++k) {
+        const int v = (kn[3 * k] << 16) | (kn[3 * k + 1] & 0xffff);
+        const bool same = !xy.empty() && xy.back() == v;
+        run = same && kn[3 * k + 2] == kn[3 * k - 1] + 1 && run < 8 ? run + 1 : 1;
+        ng += run == 1 ? 1 : 0;
+        if (!same) {
+            xy.push_back(v);
+            rexp.resize(rexp.size() + kr.n1, 0.0);
         }
-        for (; r < RF_WAVES; ++r) split[r] = ng;
+        rexp[rexp.size() - kr.n1 + std::abs(kn[3 * k + 2])] = ek[k];
     }
-    // LDS of the two passes (FP64 and FP32 forms)
-    const int ne = nmax[0] + nmax[1] + nmax[2] + 3;
-    for (int f = 0; f < 2; ++f) {
-        const size_t rsz = f ? sizeof(float) : sizeof(double);
-        const size_t tables = (size_t)ne * (SF_TILE + 1) * 2 * rsz + 5 * SF_TILE * rsz;
-        const size_t red = (size_t)(SF_WAVES - 1) * WAVE * NSUM * sizeof(double);
-        c->sfac_lds[f] = std::max(tables, red);
-        const size_t kdat = ((size_t)K * 2 * rsz + 15) / 16 * 16 + (size_t)ng * sizeof(int4);
-        c->force_lds[f] = std::max(kdat, (size_t)(RF_WAVES - 1) * WAVE * 3 * sizeof(double));
-        if (c->sfac_lds[f] > LDS_MAX || c->force_lds[f] > LDS_MAX)
-            return fail(c, SMD_ENOTSUP, "reciprocal space too large for the LDS-resident passes (%d k-vectors, nmax %d %d %d)",
-                        K, nmax[0], nmax[1], nmax[2]);
-    }
-    c->n_kgrp = ng;
-    if ((rc = realloc(c->d_kgrp, sizeof(int4) * grp.size()))) return rc;
-    if ((rc = realloc(c->d_ksplit, sizeof(int32_t) * (RF_WAVES + 1)))) return rc;
-    if ((rc = realloc(c->d_kf, sizeof(double) * 2 * (size_t)K))) return rc;
-    // structure-factor pass: about one block per CU over (group tile, atom chunk)
-    const int gt = (ng + WAVE - 1) / WAVE;
-    int chunks = std::max(1, 256 / gt);   // at most one block per CU: a single round
-    int per = (c->n + chunks - 1) / chunks;
-    if (per < 32) per = 32;
-    chunks = (c->n + per - 1) / per;
-    c->sfac_chunks = chunks;
-    if ((rc = realloc(c->d_sfac_part, sizeof(double) * NSUM * (size_t)K * chunks))) return rc;
-    if ((rc = realloc(c->d_e1, sizeof(double) * (e1_am_offset(c->n) + 4 * (size_t)c->n)))) return rc;
-    SMD_HIP(c, hipMemcpy(c->d_kgrp, grp.data(), sizeof(int4) * grp.size(), hipMemcpyHostToDevice));
-    SMD_HIP(c, hipMemcpy(c->d_ksplit, split.data(), sizeof(int32_t) * (RF_WAVES + 1), hipMemcpyHostToDevice));
-    SMD_HIP(c, hipMemcpy(c->d_kvec, kv.data(), sizeof(double) * 3 * K, hipMemcpyHostToDevice));
-    SMD_HIP(c, hipMemcpy(c->d_kmod2, k2v.data(), sizeof(double) * K, hipMemcpyHostToDevice));
-    SMD_HIP(c, hipMemcpy(c->d_expk, ek.data(), sizeof(double) * K, hipMemcpyHostToDevice));
-    SMD_HIP(c, hipMemcpy(c->d_kn, kn.data(), sizeof(int32_t) * 3 * K, hipMemcpyHostToDevice));
+    kr.nrows = (int)xy.size();
+    // The sets this path takes: the powers of 64 atoms, and 16 bytes per k
+    // and per run of eight, within 64 KiB.
+    const size_t ne = (size_t)nmax[0] + nmax[1] + nmax[2] + 3;
+    if (ne * KS_TS_NARROW * 16 + 5 * KS_TILE * 8 > LDS_MAX || (size_t)(K + ng) * 16 > LDS_MAX)
+        return fail(c, SMD_ENOTSUP, "reciprocal space too large for the LDS-resident passes (%d k-vectors, nmax %d %d %d)",
+                    K, nmax[0], nmax[1], nmax[2]);
+    int rc;
+    if ((rc = realloc(c->d_kxy, sizeof(int32_t) * xy.size()))) return rc;
+    if ((rc = realloc(c->d_expk, sizeof(double) * rexp.size()))) return rc;
+    if ((rc = realloc(c->d_kf, sizeof(double) * kr.coef_entries()))) return rc;
+    const int nt = (c->n + KS_TILE - 1) / KS_TILE;
+    c->sfac_chunks = std::max(1, std::min(nt, SF_CHUNKS));
+    c->k_part = (size_t)kr.nrows * NSUM * 4 * kr.n1;
+    if ((rc = realloc(c->d_sfac_part, sizeof(double) * c->k_part * c->sfac_chunks))) return rc;
+    if ((rc = realloc(c->d_e1, sizeof(double) * 6 * (size_t)c->n))) return rc;
+    SMD_HIP(c, hipMemcpy(c->d_kxy, xy.data(), sizeof(int32_t) * xy.size(), hipMemcpyHostToDevice));
+    SMD_HIP(c, hipMemcpy(c->d_expk, rexp.data(), sizeof(double) * rexp.size(), hipMemcpyHostToDevice));
+    c->n_krows = kr.nrows;
+    c->n_kruns = ng;
     c->K = K;
     // self and charged-system energies (ctor :69-79)
     double qSum = 0.0, q2Sum = 0.0;
@@ -293,370 +257,237 @@ int ewald_surface(Ctx* c) {
 // ---- reciprocal space ---------------------------------------------------------
 
 struct RecipArgs {
-    int n, K, ng, chunks, per;
-    int nmax[3];
+    int n, K, chunks, per;     // atoms per chunk, a multiple of KS_TILE
+    int vpw;                   // tiles per wave of the structure factors at a time
+    KsRows kr;
     double vk[3];              // 2 pi / L per axis
     const double* pos;
     const double* q;
     const int32_t* mol;
     const double* com;
-    const double* kvec;
-    const double* kmod2;
-    const double* expk;
-    const int4* grp;           // [ng] (first k, count, nx << 16 | ny, nz0)
-    const int32_t* split;      // [RF_WAVES+1] group ranges of the force pass
-    double* part;              // [chunk][K][NSUM]
-    void* kf;                  // [K] (b C, b S) as R pairs
-    double2* e1;               // [n][3] exp(i 2 pi r_p / L_p) per atom (pass 0)
-    double4* am;               // [n] (q, d) per atom, d = r - R_mol (pass 0)
+    const double* expk;        // [nrows][n1]
+    double* part;              // [chunk][nrows][weights][4][n1]
+    void* kf;                  // force-pass coefficients, R
+    double2* e1;               // [n][3] exp(i 2 pi r_p / L_p) per atom
     double* force;
     int store;                 // 1: the force pass stores (separate array), 0: adds
-    double* terms;
     Red red;
     double alphaR4, pi4V, pi8V;
 };
 
-template <typename R>
-struct cplx { R re, im; };
-
-template <typename R>
-__device__ __forceinline__ cplx<R> cmul(cplx<R> a, cplx<R> b) {
-    return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-
-// b^n for |n| <= 2^15 by binary powering; negative n through the conjugate
-// (|b| = 1).
-__device__ __forceinline__ cplx<double> cpow(cplx<double> b, int n) {
-    if (n < 0) { b.im = -b.im; n = -n; }
-    cplx<double> r{1.0, 0.0};
-    for (int it = 0; it < 16 && n; ++it) {
-        if (n & 1) r = cmul(r, b);
-        b = cmul(b, b);
-        n >>= 1;
+struct RecipAtoms {
+    const RecipArgs& a;
+    bool keep;                 // this block's phases go to e1 for the force pass
+    __device__ __forceinline__ double2 phase(int i, int p) const {
+        double s, c;
+        sincos(a.vk[p] * a.pos[3 * i + p], &s, &c);
+        const double2 e = make_double2(c, s);
+        if (keep) a.e1[3 * i + p] = e;
+        return e;
     }
-    return r;
-}
-
-__device__ __forceinline__ int grp_nx(int v) { return v >> 16; }
-__device__ __forceinline__ int grp_ny(int v) { return (int)(short)(v & 0xffff); }
-
-// Pass 0: exp(i 2 pi r_p / L_p) per atom and axis, used by both passes, and
-// each atom's charge and offset from its molecule's centre, read by pass 1.
-__global__ __launch_bounds__(256) void k_recip_phase(int n, const double* __restrict__ pos, double vx, double vy,
-                                                     double vz, double2* __restrict__ e1, const double* __restrict__ q,
-                                                     const int32_t* __restrict__ mol, const double* __restrict__ com,
-                                                     double4* __restrict__ am) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) {
-        const int m = mol[k];
-        am[k] = make_double4(q[k], pos[3 * k] - com[3 * m], pos[3 * k + 1] - com[3 * m + 1],
-                             pos[3 * k + 2] - com[3 * m + 2]);
+    __device__ __forceinline__ double charge(int i) const { return a.q[i]; }
+    __device__ __forceinline__ void offset(int i, double (&d)[3]) const {
+        const int m = a.mol[i];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) d[k] = a.pos[3 * i + k] - a.com[3 * m + k];
     }
-    if (k >= 3 * n) return;
-    const int p = k % 3;
-    const double v = p == 0 ? vx : (p == 1 ? vy : vz);
-    double s, c;
-    sincos(v * pos[k], &s, &c);
-    e1[k] = make_double2(c, s);
-}
+};
 
-// Pass 1.  Sums per k (layout of part): 0 q sin, 1 q cos,
-// 2-4 q cos d, 5-7 q sin d, 8 q cos |d|^2, 9 q sin |d|^2 (reciprocal_term
-// :568-594 and the moments its force loop needs).
-template <typename R, bool LUSTIG>
-__global__ __launch_bounds__(SF_WAVES * WAVE) void k_recip_sfac(RecipArgs a) {
+struct RecipPhases {
+    const double2* e1;
+    __device__ __forceinline__ double2 phase(int i, int p) const { return e1[3 * i + p]; }
+};
+
+// Few atoms wait for the table fill (loads, sincos, powers: about 6 us with
+// the launch), many for the matrix cores.  64 atoms a block until 256 blocks
+// are reached.  The three kernels alone, mixed, 12,288 atoms, 1,535 k: factors
+// 10.0, sums 8.9, forces 9.5 us; a walk along nz on the vector units took
+// 3.8 (phases) + 23.0, 6.2 and 20.9.  3,063 atoms in FP64: 11, 7.3, 11.9
+// against 3.0 + 17.4, 6.0 and 23.7; 48,000 atoms beside the pair kernel: the
+// step 383 -> 316 us.
+template <typename R, int NW>
+__global__ __launch_bounds__(KS_THREADS) void k_recip_sfac(RecipArgs a) {
     extern __shared__ double lds[];
-    constexpr int TS = SF_TILE + 1;   // padded table stride: lanes reading different powers spread over banks
-    cplx<R>* tab = reinterpret_cast<cplx<R>*>(lds);
-    const int ey0 = a.nmax[0] + 1, ez0 = ey0 + a.nmax[1] + 1, ne = ez0 + a.nmax[2] + 1;
-    R* misc = reinterpret_cast<R*>(tab + ne * TS);   // [5][SF_TILE]: q, dx, dy, dz, |d|^2
-    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
-    const int g = blockIdx.x * WAVE + lane;
-    const int ch = blockIdx.y;
-    const int i0 = ch * a.per, i1 = min(a.n, i0 + a.per);
-    int4 gg = make_int4(0, 0, 0, 0);
-    if (g < a.ng) gg = a.grp[g];
-    const int gnx = grp_nx(gg.z), gny = grp_ny(gg.z);
-    const int ix = gnx, iy = ey0 + abs(gny), iz = ez0 + abs(gg.w);
-    const R sy = gny < 0 ? R(-1) : R(1), sz = gg.w < 0 ? R(-1) : R(1);
-    // Sums of this lane's k-group over the wave's atoms of the chunk (a few
-    // dozen), in the pass's precision; they enter FP64 at the cross-wave sum,
-    // and chunks are added in FP64 by k_recip_reduce.
-    R acc[GK][NSUM];
-#pragma unroll
-    for (int t = 0; t < GK; ++t)
-#pragma unroll
-        for (int u = 0; u < NSUM; ++u) acc[t][u] = R(0);
-
-    // Tile fill: thread fu + SF_TILE fp writes atom fu's powers along axis fp
-    // (fp < 3) or its moments (fp == 3).  Its inputs for the next tile are
-    // loaded before the current tile is evaluated.
-    static_assert(SF_WAVES * WAVE >= 4 * SF_TILE, "one fill task per thread");
-    const int fu = threadIdx.x % SF_TILE, fp = threadIdx.x / SF_TILE;
-    const bool filler = fp < 4;
-    double2 pe = make_double2(1.0, 0.0);
-    double4 pm = make_double4(0.0, 0.0, 0.0, 0.0);
-    auto fetch = [&](int t0) {
-        const int ia = t0 + fu;
-        if (filler && ia < i1) {
-            if (fp < 3) pe = a.e1[3 * ia + fp];
-            else pm = a.am[ia];
-        }
-    };
-    fetch(i0);
-    for (int t0 = i0; t0 < i1; t0 += SF_TILE) {
-        const int na = min(SF_TILE, i1 - t0);
-        __syncthreads();
-        if (filler && fu < na) {
-            const int u = fu;
-            if (fp < 3) {
-                // powers 0..nmax of exp(i 2 pi r_p / L_p), by recurrence in FP64
-                const int base = fp == 0 ? 0 : (fp == 1 ? ey0 : ez0);
-                const double c1 = pe.x, s1 = pe.y;
-                double er = 1.0, ei = 0.0;
-                tab[base * TS + u] = {R(1), R(0)};
-                for (int k = 1; k <= a.nmax[fp]; ++k) {
-                    const double nr = er * c1 - ei * s1, ni = er * s1 + ei * c1;
-                    er = nr; ei = ni;
-                    tab[(base + k) * TS + u] = {(R)er, (R)ei};
-                }
-            } else {
-                misc[u] = (R)pm.x;
-                misc[SF_TILE + u] = (R)pm.y;
-                misc[2 * SF_TILE + u] = (R)pm.z;
-                misc[3 * SF_TILE + u] = (R)pm.w;
-                misc[4 * SF_TILE + u] = (R)(pm.y * pm.y + pm.z * pm.z + pm.w * pm.w);
-            }
-        }
-        __syncthreads();
-        fetch(t0 + SF_TILE);
-        if (g < a.ng) {
-            for (int u = w; u < na; u += SF_WAVES) {
-                const R q = misc[u];
-                cplx<R> X = tab[ix * TS + u], Y = tab[iy * TS + u], Z = tab[iz * TS + u];
-                Y.im *= sy;
-                Z.im *= sz;
-                cplx<R> e = cmul(cmul(X, Y), Z);
-                e.re *= q;
-                e.im *= q;
-                const cplx<R> z1 = tab[(ez0 + 1) * TS + u];
-                const R dx = misc[SF_TILE + u], dy = misc[2 * SF_TILE + u], dz = misc[3 * SF_TILE + u];
-                const R d2 = misc[4 * SF_TILE + u];
-                // all GK sums are formed (uniform control flow); those past
-                // the group's count are never stored
-#pragma unroll
-                for (int t = 0; t < GK; ++t) {
-                    acc[t][0] += e.im;
-                    acc[t][1] += e.re;
-                    if constexpr (LUSTIG) {
-                        acc[t][2] += e.re * dx; acc[t][3] += e.re * dy; acc[t][4] += e.re * dz;
-                        acc[t][5] += e.im * dx; acc[t][6] += e.im * dy; acc[t][7] += e.im * dz;
-                        acc[t][8] += e.re * d2; acc[t][9] += e.im * d2;
-                    }
-                    e = cmul(e, z1);
-                }
-            }
-        }
-    }
-    // add the waves' sums (wave order) and store one partial per (chunk, k)
-    double* red = lds;   // [(SF_WAVES-1) * WAVE][NSUM]
-    constexpr int NU = LUSTIG ? NSUM : 2;
-#pragma unroll
-    for (int t = 0; t < GK; ++t) {
-        __syncthreads();
-        if (w > 0)
-#pragma unroll
-            for (int u = 0; u < NU; ++u) red[((w - 1) * WAVE + lane) * NSUM + u] = (double)acc[t][u];
-        __syncthreads();
-        if (w == 0 && g < a.ng && t < gg.y) {
-            double* p = a.part + ((size_t)ch * a.K + gg.x + t) * NSUM;
-#pragma unroll
-            for (int u = 0; u < NSUM; ++u) {
-                double s = (double)acc[t][u];
-                if (u < NU)
-                    for (int v = 0; v < SF_WAVES - 1; ++v) s += red[(v * WAVE + lane) * NSUM + u];
-                p[u] = s;
-            }
-        }
-    }
+    const int i0 = blockIdx.x * a.per, i1 = min(a.n, i0 + a.per);
+    const RecipAtoms at{a, blockIdx.y == 0};
+    ks_sfac<R, NW>(a.kr, at, i0, i1, blockIdx.y, gridDim.y, a.vpw,
+                   ks_tables<R>(a.kr, NW, a.per / KS_TILE), lds,
+                   a.part + (size_t)blockIdx.x * a.kr.nrows * NW * 4 * a.kr.n1);
 }
 
-// Pass 1b: per block, RK_PER_BLOCK k-vectors.  Their chunk partials are
-// summed in chunk order (four chunk quarters added in quarter order), then
-// per k: energy, volume derivatives and virial (:596-607), the force loop's
-// Lustig sums (:609-658) in per-k form, and (b C, b S) for the force pass.
-constexpr int RK_PER_BLOCK = WAVE / NSUM;   // 6 k-vectors: 60 of the 64 lanes
-
-template <typename R, bool LUSTIG>
-__global__ __launch_bounds__(256) void k_recip_reduce(RecipArgs a) {
-    __shared__ double red[3][WAVE];
-    __shared__ double sums[WAVE];
+// One block per row (and per padding row of the last tile, which only clears
+// its coefficients).  The waves sum an equal share of the chunks each, in
+// order, and their shares are added in order; then thread n takes the row's k
+// with nz = +-n.  Bound by the latency of the chunk loads, so a block is as
+// many waves as the sums' LDS allows.
+template <typename R, int NW>
+__global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
+    extern __shared__ double lds[];
+    constexpr bool LUSTIG = NW > 1;
+    const int row = blockIdx.x, nv = NW * 4 * a.kr.n1;
     const int lane = threadIdx.x % WAVE, qt = threadIdx.x / WAVE;
-    const int nv = a.K * NSUM;
-    const int k0 = blockIdx.x * RK_PER_BLOCK;
-    const int v = k0 * NSUM + lane;
-    const bool live = lane < RK_PER_BLOCK * NSUM && v < nv;
-    const int c0 = (a.chunks * qt) / 4, c1 = (a.chunks * (qt + 1)) / 4;
-    double s = 0.0;
-    if (live) {
-#pragma unroll 4
-        for (int ch = c0; ch < c1; ++ch) s += a.part[(size_t)ch * nv + v];
-    }
-    if (qt > 0) red[qt - 1][lane] = s;
-    __syncthreads();
-    if (qt == 0) sums[lane] = live ? ((s + red[0][lane]) + red[1][lane]) + red[2][lane] : 0.0;
-    __syncthreads();
-
+    R* kf = static_cast<R*>(a.kf);
+    ks_coef_pad<R>(a.kr, kf, row, threadIdx.x, blockDim.x);
     double o[3 + 9 + 4] = {0};   // energy, longDeriv, long2ndDeriv, virial[9], Ff, Ffk2, d2UV1, d2UrR
-    const int k = k0 + (int)threadIdx.x;
-    if (threadIdx.x < RK_PER_BLOCK && k < a.K) {
-        const double* sk = sums + threadIdx.x * NSUM;
-        const double kx = a.kvec[3 * k], ky = a.kvec[3 * k + 1], kz = a.kvec[3 * k + 2];
-        const double k2 = a.kmod2[k];
-        const double sinSum = sk[0], cosSum = sk[1];
-        const double te = a.pi4V * a.expk[k] * (sinSum * sinSum + cosSum * cosSum);
-        const double coeff = 2.0 * (a.alphaR4 + 1.0 / k2);
-        const double kk = (te * kx) * kx + (te * ky) * ky + (te * kz) * kz;
-        o[0] = te;
-        o[1] = -te + kk * 2.0 * a.alphaR4;
-        const double t7 = ((7.0 * te * kx) * kx + (7.0 * te * ky) * ky + (7.0 * te * kz) * kz) * 2.0 * a.alphaR4;
-        const double dd = kk * 2.0 * a.alphaR4;
-        const double t2 = ((dd * kx) * kx + (dd * ky) * ky + (dd * kz) * kz) * 2.0 * a.alphaR4;
-        o[2] = 4.0 * te - t7 + t2;
-        o[3 + 0] = te - te * coeff * kx * kx;
-        o[3 + 4] = te - te * coeff * ky * ky;
-        o[3 + 8] = te - te * coeff * kz * kz;
-        o[3 + 1] = -te * coeff * kx * ky;
-        o[3 + 2] = -te * coeff * kx * kz;
-        o[3 + 5] = -te * coeff * ky * kz;
+    if (row < a.kr.nrows) {
+        const int nq = blockDim.x / WAVE;
+        const int c0 = (a.chunks * qt) / nq, c1 = (a.chunks * (qt + 1)) / nq;
+        const size_t stride = (size_t)a.kr.nrows * nv;
+        for (int v = lane; v < nv; v += WAVE) {
+            const double* p = a.part + (size_t)row * nv + v;
+            double s = 0.0;
+#pragma unroll 8
+            for (int ch = c0; ch < c1; ++ch) s += p[(size_t)ch * stride];
+            lds[qt * nv + v] = s;
+        }
+        __syncthreads();
+        for (int v = threadIdx.x; v < nv; v += blockDim.x) {
+            double s = lds[v];
+            for (int q = 1; q < nq; ++q) s += lds[q * nv + v];
+            lds[v] = s;
+        }
+        __syncthreads();
+        const int n = threadIdx.x;   // n1 is at most 58: the set's limit on nmax
+        if (n < a.kr.n1) {
+            const int v = a.kr.xy[row];
+            const int nx = ks_nx(v), ny = ks_ny(v);
+            const double ek = a.expk[(size_t)row * a.kr.n1 + n];
+            const double kx = nx * a.vk[0], ky = ny * a.vk[1];
+            double sum[NW][4];
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) sum[w][p] = lds[(w * 4 + p) * a.kr.n1 + n];
+            const double b = a.pi8V * ek;
+            double G[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+            // +nz, and -nz where the half space has it
+            const int signs = ek == 0.0 ? 0 : (n == 0 || (nx == 0 && ny == 0) ? 1 : 2);
+            for (int s = 0; s < signs; ++s) {
+                const double sg = s ? -1.0 : 1.0;
+                const double kz = sg * n * a.vk[2];
+                const double k2 = kx * kx + ky * ky + kz * kz;
+                const double cosSum = sum[0][0] - sg * sum[0][3], sinSum = sum[0][2] + sg * sum[0][1];
+                const double te = a.pi4V * ek * (sinSum * sinSum + cosSum * cosSum);
+                const double coeff = 2.0 * (a.alphaR4 + 1.0 / k2);
+                const double kk = (te * kx) * kx + (te * ky) * ky + (te * kz) * kz;
+                o[0] += te;
+                o[1] += -te + kk * 2.0 * a.alphaR4;
+                const double t7 = ((7.0 * te * kx) * kx + (7.0 * te * ky) * ky + (7.0 * te * kz) * kz) * 2.0 * a.alphaR4;
+                const double dd = kk * 2.0 * a.alphaR4;
+                const double t2 = ((dd * kx) * kx + (dd * ky) * ky + (dd * kz) * kz) * 2.0 * a.alphaR4;
+                o[2] += 4.0 * te - t7 + t2;
+                o[3 + 0] += te - te * coeff * kx * kx;
+                o[3 + 4] += te - te * coeff * ky * ky;
+                o[3 + 8] += te - te * coeff * kz * kz;
+                o[3 + 1] += -te * coeff * kx * ky;
+                o[3 + 2] += -te * coeff * kx * kz;
+                o[3 + 5] += -te * coeff * ky * kz;
+                if constexpr (LUSTIG) {
+                    double cd[4], sd[4];   // weights d, |d|^2
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        cd[w] = sum[w + 1][0] - sg * sum[w + 1][3];
+                        sd[w] = sum[w + 1][2] + sg * sum[w + 1][1];
+                    }
+                    // sum_i val_i (k.d_i) with val_i = b (q_i sin_i C - q_i cos_i S)
+                    const double kSD = kx * sd[0] + ky * sd[1] + kz * sd[2];
+                    const double kCD = kx * cd[0] + ky * cd[1] + kz * cd[2];
+                    const double ff = b * (cosSum * kSD - sinSum * kCD);
+                    o[12] += ff;
+                    o[13] += ff * (4.0 * a.alphaR4 * k2);
+                    const double bkk = (b * kx) * kx + (b * ky) * ky + (b * kz) * kz;
+                    o[14] += bkk * (cosSum * cd[3] + sinSum * sd[3]);
+                    o[15] += bkk * ((cd[0] * cd[0] + cd[1] * cd[1] + cd[2] * cd[2]) +
+                                    (sd[0] * sd[0] + sd[1] * sd[1] + sd[2] * sd[2]));
+                }
+                G[s][0] = b * cosSum;
+                G[s][1] = b * sinSum;
+            }
+            ks_coef<R>(a.kr, kf, row, n, G[0][0], G[0][1], G[1][0], G[1][1]);
+        }
         o[3 + 3] = o[3 + 1];
         o[3 + 6] = o[3 + 2];
         o[3 + 7] = o[3 + 5];
-        const double b = a.pi8V * a.expk[k];
-        if constexpr (LUSTIG) {
-            // sum_i val_i (k.d_i) with val_i = b (q_i sin_i C - q_i cos_i S)
-            const double kSD = kx * sk[5] + ky * sk[6] + kz * sk[7];
-            const double kCD = kx * sk[2] + ky * sk[3] + kz * sk[4];
-            const double ff = b * (cosSum * kSD - sinSum * kCD);
-            o[12] = ff;
-            o[13] = ff * (4.0 * a.alphaR4 * k2);
-            const double bkk = (b * kx) * kx + (b * ky) * ky + (b * kz) * kz;
-            o[14] = bkk * (cosSum * sk[8] + sinSum * sk[9]);
-            o[15] = bkk * ((sk[2] * sk[2] + sk[3] * sk[3] + sk[4] * sk[4]) + (sk[5] * sk[5] + sk[6] * sk[6] + sk[7] * sk[7]));
-        }
-        R* kf = reinterpret_cast<R*>(a.kf);
-        kf[2 * k] = (R)(b * cosSum);
-        kf[2 * k + 1] = (R)(b * sinSum);
     }
-    __syncthreads();
-    block_part<16>(o, a.red, RS_RECIP);
-}
-
-// Bytes of the (b C, b S) table in the force pass's LDS, rounded up so the
-// k-groups that follow it are 16-byte aligned.
-template <typename R>
-__host__ __device__ constexpr size_t kf_bytes(int K) { return ((size_t)K * 2 * sizeof(R) + 15) / 16 * 16; }
-
-// Pass 2: force on atom i, sum_k (b C q sin - b S q cos) k (:609-658).
-template <typename R>
-__global__ __launch_bounds__(RF_WAVES * WAVE) void k_recip_force(RecipArgs a) {
-    extern __shared__ double lds[];
-    R* kf = reinterpret_cast<R*>(lds);                                   // [K][2]
-    int4* grp = reinterpret_cast<int4*>(reinterpret_cast<char*>(lds) + kf_bytes<R>(a.K));   // [ng]
-    {
-        const R* src = reinterpret_cast<const R*>(a.kf);
-        for (int idx = threadIdx.x; idx < 2 * a.K; idx += blockDim.x) kf[idx] = src[idx];
-        for (int idx = threadIdx.x; idx < a.ng; idx += blockDim.x) grp[idx] = a.grp[idx];
-    }
-    __syncthreads();
-    const int lane = threadIdx.x % WAVE;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int i = blockIdx.x * WAVE + lane;
-    const int ic = min(i, a.n - 1);   // idle lanes repeat the last atom and store nothing
-    double F[3] = {0.0, 0.0, 0.0};
-    {
-        const double q = a.q[ic];
-        const double vx = a.vk[0], vy = a.vk[1], vz = a.vk[2];
-        const double2 ex = a.e1[3 * ic], ey = a.e1[3 * ic + 1], ez = a.e1[3 * ic + 2];
-        const cplx<double> X1{ex.x, ex.y}, Y1{ey.x, ey.y}, Z1{ez.x, ez.y};
-        const cplx<double> Z1c{Z1.re, -Z1.im};
-        const cplx<R> z1{(R)Z1.re, (R)Z1.im};
-        cplx<double> XY{1.0, 0.0}, Zp{1.0, 0.0};
-        cplx<R> e{R(0), R(0)};
-        int cnx = INT_MIN, cny = 0, zp = 0, next_nz = INT_MIN;
-        const int gs = a.split[w], ge = a.split[w + 1];
-        for (int gi = gs; gi < ge; ++gi) {
-            const int4 gg = grp[gi];
-            const int nx = grp_nx(gg.z), ny = grp_ny(gg.z), nz0 = gg.w;
-            if (!(nx == cnx && ny == cny && nz0 == next_nz)) {
-                // a new row: X^nx Y^ny Z^nz0 q
-                if (nx != cnx) {
-                    XY = cmul(cpow(X1, nx), cpow(Y1, ny));
-                    Zp = cpow(Z1, nz0);
-                    cnx = nx; cny = ny; zp = nz0;
-                } else {
-                    for (; cny < ny; ++cny) XY = cmul(XY, Y1);
-                    for (; zp < nz0; ++zp) Zp = cmul(Zp, Z1);
-                    for (; zp > nz0; --zp) Zp = cmul(Zp, Z1c);
-                }
-                const cplx<double> e0 = cmul(XY, Zp);
-                e = {(R)(q * e0.re), (R)(q * e0.im)};
-            }
-            next_nz = nz0 + GK;   // a following group continues this row only after a full group
-            R sv = R(0), szv = R(0);
-            R nzf = (R)nz0;
-            const R* kd = kf + 2 * gg.x;
+    // the sums are in the first wave; the rest of the block has none
+    if (threadIdx.x < WAVE && (int)gridDim.x <= a.red.cap) {
+        double* part = red_part(a.red, RS_RECIP) + blockIdx.x;
 #pragma unroll
-            for (int t = 0; t < GK; ++t) {
-                if (t < gg.y) {
-                    const R val = e.im * kd[2 * t] - e.re * kd[2 * t + 1];
-                    sv += val;
-                    szv += val * nzf;
-                }
-                nzf += R(1);
-                e = cmul(e, z1);
-            }
-            if (gg.y < GK) next_nz = INT_MIN;
-            F[0] += (double)sv * (nx * vx);
-            F[1] += (double)sv * (ny * vy);
-            F[2] += (double)szv * vz;
-        }
-    }
-    // add the waves' forces in wave order
-    __syncthreads();
-    double* red = lds;   // [(RF_WAVES-1) * WAVE][3]
-    if (w > 0) {
-        red[((w - 1) * WAVE + lane) * 3] = F[0];
-        red[((w - 1) * WAVE + lane) * 3 + 1] = F[1];
-        red[((w - 1) * WAVE + lane) * 3 + 2] = F[2];
-    }
-    __syncthreads();
-    if (w == 0 && i < a.n) {
-        for (int v = 0; v < RF_WAVES - 1; ++v) {
-            F[0] += red[(v * WAVE + lane) * 3];
-            F[1] += red[(v * WAVE + lane) * 3 + 1];
-            F[2] += red[(v * WAVE + lane) * 3 + 2];
-        }
-        if (a.store) {
-            a.force[3 * i] = F[0];
-            a.force[3 * i + 1] = F[1];
-            a.force[3 * i + 2] = F[2];
-        } else {
-            a.force[3 * i] += F[0];
-            a.force[3 * i + 1] += F[1];
-            a.force[3 * i + 2] += F[2];
+        for (int k = 0; k < (LUSTIG ? 16 : 12); ++k) {
+            const double t = wave_sum(o[k]);
+            if (threadIdx.x == 0) part[(size_t)k * a.red.cap] = t;
         }
     }
 }
 
-// Scratch of the reciprocal-space passes: per-k coefficients, (chunk, k)
-// partials, per-atom phases and moments.
-struct RecipScratch { double* kf; double* part; double* e1; };
+// Force on atom i, sum_k (b C q sin - b S q cos) k (:609-658).  FF: also the
+// block's sum of F . d (T_RC_FF).
+template <typename R, int KS, bool FF>
+__global__ __launch_bounds__(KS_THREADS) void k_recip_force(RecipArgs a) {
+    extern __shared__ double lds[];
+    const int i0 = blockIdx.x * KS_TILE;
+    const RecipPhases at{a.e1};
+    const double g = ks_force<R, KS>(a.kr, at, static_cast<const R*>(a.kf), i0, a.n, lds);
+    const int i = i0 + (int)threadIdx.x / 3, d = threadIdx.x % 3;
+    double ff[1] = {0.0};
+    if (threadIdx.x < 3 * KS_TILE && i < a.n) {
+        const double f = a.q[i] * g * a.vk[d];
+        if (a.store) a.force[3 * i + d] = f;
+        else a.force[3 * i + d] += f;
+        if constexpr (FF) ff[0] = f * (a.pos[3 * i + d] - a.com[3 * a.mol[i] + d]);
+    }
+    if constexpr (FF) {
+        __syncthreads();
+        block_part<1>(ff, a.red, RS_RECIP_FF);
+    }
+}
+
+template <typename R, bool FF>
+static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
+    const dim3 g((a.n + KS_TILE - 1) / KS_TILE), b(KS_THREADS);
+    const size_t lds = ks_force_lds<R>(a.kr);
+    switch (a.kr.steps()) {
+        case 1: hipLaunchKernelGGL((k_recip_force<R, 1, FF>), g, b, lds, s, a); break;
+        case 2: hipLaunchKernelGGL((k_recip_force<R, 2, FF>), g, b, lds, s, a); break;
+        case 3: hipLaunchKernelGGL((k_recip_force<R, 3, FF>), g, b, lds, s, a); break;
+        case 4: hipLaunchKernelGGL((k_recip_force<R, 4, FF>), g, b, lds, s, a); break;
+        case 5: hipLaunchKernelGGL((k_recip_force<R, 5, FF>), g, b, lds, s, a); break;
+        case 6: hipLaunchKernelGGL((k_recip_force<R, 6, FF>), g, b, lds, s, a); break;
+        case 7: hipLaunchKernelGGL((k_recip_force<R, 7, FF>), g, b, lds, s, a); break;
+        case 8: hipLaunchKernelGGL((k_recip_force<R, 8, FF>), g, b, lds, s, a); break;
+        default: hipLaunchKernelGGL((k_recip_force<R, 0, FF>), g, b, lds, s, a); break;
+    }
+}
+
+template <typename R, int NW>
+static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes) {
+    if (passes & RECIP_SFAC) {
+        // A chunk's (tile, weight) pairs go side by side over blocks only where
+        // the chunks alone leave CUs idle, since each block fills its own table.
+        const int nvt = a.kr.tiles() * NW, per = KS_WAVES * a.vpw, groups = (nvt + per - 1) / per;
+        int gy = std::min(groups, std::max(1, 256 / a.chunks));
+        gy = (groups + (groups + gy - 1) / gy - 1) / ((groups + gy - 1) / gy);   // no block with one group more
+        const size_t lds = ks_table_bytes<R>(a.kr, NW) * ks_tables<R>(a.kr, NW, a.per / KS_TILE);
+        hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(KS_THREADS), lds, s, a);
+    }
+    if (passes & RECIP_REDUCE) {
+        // a wave per dozen chunks, fewer where the row's sums are many: the
+        // loads of one wave follow each other, the epilogue waits for all
+        const size_t per_wave = sizeof(double) * NW * 4 * a.kr.n1;
+        const int waves = std::max(4, std::min({16, (a.chunks + 11) / 12, (int)(LDS_MAX / 2 / per_wave)}));
+        hipLaunchKernelGGL((k_recip_reduce<R, NW>), dim3(a.kr.tiles() * KS_ROWS), dim3(waves * WAVE), waves * per_wave,
+                           s, a);
+    }
+}
+
+// Scratch of the reciprocal-space passes: the force pass's coefficients, the
+// chunks' partials, per-atom phases.
+struct RecipScratch { double* kf; double* part; double* e1; int chunks; };
 
 static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const RecipScratch& sc);
 
 int ewald_recip(Ctx* c, int prec, int lustig, unsigned passes) {
-    return ewald_recip_with(c, prec, lustig, passes, RecipScratch{c->d_kf, c->d_sfac_part, c->d_e1});
+    return ewald_recip_with(c, prec, lustig, passes, RecipScratch{c->d_kf, c->d_sfac_part, c->d_e1, c->sfac_chunks});
 }
 
 // ---- the allocation-free form's scratch -------------------------------------
@@ -690,75 +521,63 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
     RecipArgs a;
     a.n = c->n;
     a.K = c->K;
-    a.ng = c->n_kgrp;
-    a.chunks = c->sfac_chunks;
-    a.per = (c->n + a.chunks - 1) / a.chunks;
-    for (int d = 0; d < 3; ++d) {
-        a.nmax[d] = c->nmax[d];
-        a.vk[d] = 2.0 * PI / c->box.L[d];
-    }
+    a.kr.nrows = c->n_krows;
+    a.kr.nx1 = c->nmax[0] + 1;
+    a.kr.ny1 = c->nmax[1] + 1;
+    a.kr.n1 = c->nmax[2] + 1;
+    a.kr.ts = ks_stride(a.kr.powers());
+    a.kr.xy = c->d_kxy;
+    // whole tiles per chunk
+    const int nt = (c->n + KS_TILE - 1) / KS_TILE;
+    const int most = lustig ? std::min(sc.chunks, SF_CHUNKS_LUSTIG) : sc.chunks;
+    a.per = (nt + most - 1) / most * KS_TILE;
+    a.chunks = (c->n + a.per - 1) / a.per;
+    a.vpw = a.chunks < 128 ? 1 : KS_VT;   // one tile per wave while blocks are few
+    for (int d = 0; d < 3; ++d) a.vk[d] = 2.0 * PI / c->box.L[d];
     a.pos = c->d_pos;
     a.q = c->d_q;
     a.mol = c->d_mol;
     a.com = c->d_com;
-    a.kvec = c->d_kvec;
-    a.kmod2 = c->d_kmod2;
     a.expk = c->d_expk;
-    a.grp = c->d_kgrp;
-    a.split = c->d_ksplit;
     a.part = sc.part;
     a.kf = sc.kf;
     a.e1 = reinterpret_cast<double2*>(sc.e1);
-    a.am = reinterpret_cast<double4*>(sc.e1 + e1_am_offset(c->n));
     a.store = c->recip_store ? 1 : 0;
     a.force = c->recip_store ? c->d_frecip : c->d_force;
-    a.terms = c->d_terms;
     a.red = c->red;
     a.alphaR4 = 1.0 / (4.0 * (c->ew.alpha * c->ew.alpha));
     const double volume = c->box.L[0] * c->box.L[1] * c->box.L[2];
     a.pi4V = 4.0 * PI * (1.0 / volume);
     a.pi8V = 2.0 * a.pi4V;
     const bool mixed = prec == SMD_PREC_MIXED;
-    const int f = mixed ? 1 : 0;
-    if (passes & RECIP_SFAC) {
-        ProfScope ps(c, "recip_sfac");
-        hipLaunchKernelGGL(k_recip_phase, dim3((3 * c->n + 255) / 256), dim3(256), 0, c->stream, c->n, c->d_pos,
-                           a.vk[0], a.vk[1], a.vk[2], a.e1, c->d_q, c->d_mol, c->d_com, a.am);
-        const dim3 g1((a.ng + WAVE - 1) / WAVE, a.chunks);
-        const dim3 b1(SF_WAVES * WAVE);
-        // mixed: FP32 phases, products and per-wave sums over the chunk's
-        // atoms; FP64 from the cross-wave sum on
-        const size_t lds = c->sfac_lds[f];
+    for (unsigned pass : {(unsigned)RECIP_SFAC, (unsigned)RECIP_REDUCE}) {
+        if (!(passes & pass)) continue;
+        ProfScope ps(c, pass == RECIP_SFAC ? "recip_sfac" : "recip_reduce");
         if (mixed) {
-            if (lustig) hipLaunchKernelGGL((k_recip_sfac<float, true>), g1, b1, lds, c->stream, a);
-            else hipLaunchKernelGGL((k_recip_sfac<float, false>), g1, b1, lds, c->stream, a);
+            if (lustig) launch_recip_sums<float, NSUM>(c->stream, a, pass);
+            else launch_recip_sums<float, 1>(c->stream, a, pass);
         } else {
-            if (lustig) hipLaunchKernelGGL((k_recip_sfac<double, true>), g1, b1, lds, c->stream, a);
-            else hipLaunchKernelGGL((k_recip_sfac<double, false>), g1, b1, lds, c->stream, a);
-        }
-    }
-    if (passes & RECIP_REDUCE) {
-        ProfScope ps(c, "recip_reduce");
-        const dim3 gk((a.K + RK_PER_BLOCK - 1) / RK_PER_BLOCK);
-        if (mixed) {
-            if (lustig) hipLaunchKernelGGL((k_recip_reduce<float, true>), gk, dim3(256), 0, c->stream, a);
-            else hipLaunchKernelGGL((k_recip_reduce<float, false>), gk, dim3(256), 0, c->stream, a);
-        } else {
-            if (lustig) hipLaunchKernelGGL((k_recip_reduce<double, true>), gk, dim3(256), 0, c->stream, a);
-            else hipLaunchKernelGGL((k_recip_reduce<double, false>), gk, dim3(256), 0, c->stream, a);
+            if (lustig) launch_recip_sums<double, NSUM>(c->stream, a, pass);
+            else launch_recip_sums<double, 1>(c->stream, a, pass);
         }
         SMD_HIP(c, hipGetLastError());
-        const int rc = red_finish(c, RS_RECIP, gk.x, 16, a.terms + T_RC_E);
-        if (rc) return rc;
+        if (pass == RECIP_REDUCE) {
+            const int rc = red_finish(c, RS_RECIP, a.kr.tiles() * KS_ROWS, lustig ? 16 : 12, c->d_terms + T_RC_E);
+            if (rc) return rc;
+        }
     }
     if (passes & RECIP_FORCE) {
         ProfScope ps(c, "recip_force");
-        const dim3 g2((c->n + WAVE - 1) / WAVE);
-        const size_t lds = c->force_lds[f];
-        if (mixed) hipLaunchKernelGGL((k_recip_force<float>), g2, dim3(RF_WAVES * WAVE), lds, c->stream, a);
-        else hipLaunchKernelGGL((k_recip_force<double>), g2, dim3(RF_WAVES * WAVE), lds, c->stream, a);
+        if (mixed) {
+            if (lustig) launch_recip_force<float, false>(c->stream, a);
+            else launch_recip_force<float, true>(c->stream, a);
+        } else {
+            if (lustig) launch_recip_force<double, false>(c->stream, a);
+            else launch_recip_force<double, true>(c->stream, a);
+        }
+        SMD_HIP(c, hipGetLastError());
+        if (!lustig) return red_finish(c, RS_RECIP_FF, (a.n + KS_TILE - 1) / KS_TILE, 1, c->d_terms + T_RC_FF);
     }
-    SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
 
@@ -861,15 +680,26 @@ extern "C" int smd_ewald_compute_long_static(smd_ctx* c, int prec, smd_ewald_lon
     if (prec != SMD_PREC_FP64 && prec != SMD_PREC_MIXED) return fail(c, SMD_EINVAL, "bad precision %d", prec);
     if (!c->static_scratch) return fail(c, SMD_ESTATE, "static scratch not resolved for device %d", c->device);
     auto up = [](size_t v) { return (v + 31) / 32 * 32; };   // 256-byte segments
-    const size_t n_e1 = up(e1_am_offset(c->n) + 4 * (size_t)c->n);
-    const size_t n_kf = up(2 * (size_t)c->K);
-    const size_t n_part = up((size_t)NSUM * c->K * c->sfac_chunks);
-    const size_t need = n_e1 + n_kf + n_part;
-    if (need > STATIC_SCRATCH_DOUBLES)
+    // Room: 80 bytes per atom, 16 per k and 80 per (k, chunk), with a chunk
+    // per 64 k-runs and CU but at least 32 atoms in each.
+    const int gt = (c->n_kruns + WAVE - 1) / WAVE;
+    const int quota = std::max(1, 256 / gt);
+    const int per = std::max(32, (c->n + quota - 1) / quota);
+    const size_t need = up(((6 * (size_t)c->n + 3) & ~(size_t)3) + 4 * (size_t)c->n) + up(2 * (size_t)c->K) +
+                        up((size_t)10 * c->K * ((c->n + per - 1) / per));
+    const size_t n_e1 = up(6 * (size_t)c->n);
+    KsRows kr{};
+    kr.nrows = c->n_krows;
+    kr.n1 = c->nmax[2] + 1;
+    const size_t n_kf = up(kr.coef_entries());
+    // as many chunks as the rest of the array holds
+    const size_t rest = n_e1 + n_kf < STATIC_SCRATCH_DOUBLES ? STATIC_SCRATCH_DOUBLES - n_e1 - n_kf : 0;
+    const int chunks = (int)std::min<size_t>(c->sfac_chunks, rest / c->k_part);
+    if (need > STATIC_SCRATCH_DOUBLES || chunks < 1)
         return fail(c, SMD_ECAPACITY,
                     "static scratch holds %zu bytes; %d atoms and %d k-vectors need %zu (use smd_ewald_compute_long)",
                     (size_t)SMD_STATIC_SCRATCH_BYTES, c->n, c->K, need * sizeof(double));
-    const RecipScratch sc{c->static_scratch + n_e1, c->static_scratch + n_e1 + n_kf, c->static_scratch};
+    const RecipScratch sc{c->static_scratch + n_e1, c->static_scratch + n_e1 + n_kf, c->static_scratch, chunks};
     hipLaunchKernelGGL(k_clear_terms, dim3(1), dim3(256), 0, c->stream, c->d_terms, (int)T_COUNT);
     SMD_HIP(c, hipGetLastError());
     int rc = ewald_recip_with(c, prec, 1, RECIP_ALL, sc);

@@ -805,7 +805,7 @@ int md_step_enqueue(Ctx* c, bool do_long) {
         {
             StreamSwap sw(c, c->stream2);
             c->recip_store = true;
-            rc = ewald_recip(c, p.prec, 1);
+            rc = ewald_recip(c, p.prec, 0);
             c->recip_store = false;
         }
         if (rc) return rc;
@@ -818,7 +818,7 @@ int md_step_enqueue(Ctx* c, bool do_long) {
     if ((rc = ewald_intra(c, 1))) return rc;
     if (p.ewald.surface && (rc = ewald_surface(c))) return rc;
     if (fork) SMD_HIP(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
-    else if (do_long && (rc = ewald_recip(c, p.prec, 1))) return rc;
+    else if (do_long && (rc = ewald_recip(c, p.prec, 0))) return rc;
     if ((rc = red_flush(c))) return rc;
     // drift removal, SHAKE (adds d_frecip), clears the rebuild flag; then the
     // kinetic and pressure sums, the NH update and the per-step rewrap
@@ -994,7 +994,7 @@ extern "C" int smd_md_init(smd_ctx* c, const smd_md_params* p) {
             return rc;
         if ((rc = ewald_intra(c, 1))) return rc;
         if (p->ewald.surface && (rc = ewald_surface(c))) return rc;
-        if ((rc = ewald_recip(c, p->prec, 1))) return rc;
+        if ((rc = ewald_recip(c, p->prec, 0))) return rc;
     } else if ((rc = pairs_lj(c, p->cutoff, p->switch_on, p->constraint_mode ? 1 : 0, 1, p->prec, false))) {
         return rc;
     }
@@ -1048,7 +1048,7 @@ extern "C" int smd_md_time_family(smd_ctx* c, const char* family, int reps, doub
     c->pack_reuse = pairs_fam;
     if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
     for (int r = 0; e == hipSuccess && rc == SMD_OK && r < reps; ++r)
-        rc = pass ? ewald_recip(c, p.prec, 1, pass)
+        rc = pass ? ewald_recip(c, p.prec, 0, pass)
                   : pairs_lj_ewald(c, nullptr, nullptr, p.cutoff, p.ewald.alpha, p.ewald.real_cut,
                                    p.ewald.use_constraint, 1, p.prec, true);
     if (e == hipSuccess && rc == SMD_OK) e = hipEventRecord(e1, c->stream);

@@ -1,0 +1,375 @@
+// kspace.h -- reciprocal space of point charges as matrix products.
+//
+// exp(i k.r) = X^nx Y^ny Z^nz with X = exp(i 2 pi x / Lx), ... (for a sheared
+// cell x is the coordinate along the tilted lattice).  The k set is kept as
+// rows (nx, ny), each holding nz = -m..m, and +nz and -nz share everything but
+// a sign: with c_n + i s_n = Z^n and a + i b = q X^nx Y^ny,
+//
+//   structure factors   sum_i {a, b}(row, i) {c_n, s_n}(i)
+//   forces              T(row, i) = sum_n U(row, n) c_n(i) + V(row, n) s_n(i),
+//                       force on i = sum_rows Im(a + i b)(T, T') (nx, ny, nz)
+//
+// are products of a 16-row tile with 16 columns over the inner index (atoms,
+// or the 2 n1 functions c_n, s_n), which the matrix cores take: FP64
+// (v_mfma_f64_16x16x4) in the FP64 form, FP32 (v_mfma_f32_16x16x4) with FP64
+// totals every 64 atoms in the mixed form.  Powers come from an FP64
+// recurrence in both.  Work per (row, atom): 2 multiply-adds per k for the
+// factors, 4 for the forces, the padding of the sphere's rows to n1 included
+// about twice that; a walk along nz with a rotation per k takes 8 and more
+// vector instructions per k, and k times the latency.
+#pragma once
+
+#include <type_traits>
+
+#include "smd_internal.h"
+
+namespace smd {
+
+constexpr int KS_TILE = 64;       // atoms per LDS table
+// Table stride: a wave reads 16 powers of 4 neighbouring atoms, which at
+// stride 4 mod 16 fall on distinct banks (65 put four of them on one);
+// 65 where 68 would take the tables past 64 KiB.
+constexpr int KS_TS = KS_TILE + 4, KS_TS_NARROW = KS_TILE + 1;
+constexpr int KS_WAVES = 8;
+constexpr int KS_THREADS = KS_WAVES * WAVE;
+constexpr int KS_ROWS = 16;       // rows of a matrix tile
+constexpr int KS_VT = 2;          // tiles per wave of the structure-factor pass
+constexpr int KS_MAXSTEP = 8;     // inner steps held in registers by the force pass
+
+template <typename R> struct KsMat;
+template <> struct KsMat<double> {
+    typedef double acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    // row of register r of the product in this lane; the column is lane % 16
+    static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + lane / 16; }
+};
+template <> struct KsMat<float> {
+    typedef float acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane / 16) + r; }
+};
+
+template <typename R> struct KsC { R re, im; };
+template <typename R>
+__device__ __forceinline__ KsC<R> ks_mul(KsC<R> a, KsC<R> b) {
+    return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+
+struct KsRows {
+    int nrows, n1;       // rows; nz = 0..n1-1 and their negatives
+    int nx1, ny1;        // powers of X (0..nx1-1) and of Y (0..ny1-1, conjugated for ny < 0)
+    int ts;              // table stride (ks_stride)
+    const int* xy;       // [nrows] nx << 16 | (ny & 0xffff)
+    __host__ __device__ int tiles() const { return (nrows + KS_ROWS - 1) / KS_ROWS; }
+    __host__ __device__ int powers() const { return nx1 + ny1 + n1; }
+    __host__ __device__ int steps() const { return (2 * n1 + 3) / 4; }   // of four functions
+    __host__ __device__ size_t table_entries() const { return (size_t)powers() * ts; }
+    // per-row coefficients of the force pass: [tile][4][4 steps][16]
+    __host__ __device__ size_t coef_entries() const { return (size_t)tiles() * 4 * steps() * 4 * KS_ROWS; }
+};
+inline int ks_stride(int powers) {
+    return (size_t)powers * KS_TS * 16 + 5 * KS_TILE * 8 <= 65536 ? KS_TS : KS_TS_NARROW;
+}
+__host__ __device__ inline int ks_nx(int v) { return v >> 16; }
+__host__ __device__ inline int ks_ny(int v) { return (int)(short)(v & 0xffff); }
+
+// Powers 0..cnt-1 of (c1, s1) into column u of a table, times f.
+template <typename R>
+__device__ __forceinline__ void ks_powers(KsC<R>* tab, int ts, int u, int cnt, double c1, double s1, double f) {
+    double er = f, ei = 0.0;
+    tab[u] = {(R)er, (R)ei};
+    for (int k = 1; k < cnt; ++k) {
+        const double nr = er * c1 - ei * s1, ni = er * s1 + ei * c1;
+        er = nr; ei = ni;
+        tab[(size_t)k * ts + u] = {(R)er, (R)ei};
+    }
+}
+
+// Tables (with several weights also their values) of the structure-factor
+// pass that fit in the 64 KiB a launch takes without asking, at most
+// KS_TABLES: a block fills them together, so their loads and phases overlap.
+constexpr int KS_TABLES = 4;
+template <typename R>
+__host__ __device__ inline size_t ks_table_bytes(const KsRows& kr, int nw) {
+    return kr.table_entries() * 2 * sizeof(R) + (nw > 1 ? (size_t)nw * KS_TILE * sizeof(R) : 0);
+}
+template <typename R>
+__host__ __device__ inline int ks_tables(const KsRows& kr, int nw, int chunk_tiles) {
+    const int fit = (int)(65536 / ks_table_bytes<R>(kr, nw));
+    const int m = fit < KS_TABLES ? fit : KS_TABLES;
+    return m < 1 ? 1 : (m < chunk_tiles ? m : chunk_tiles);
+}
+
+// Structure factors of atoms [i0, i1) for the (tile, weight) pairs of groups
+// g0, g0 + gs, ... of vpw KS_WAVES (vpw at most KS_VT), by one block with
+// `nt` tables: out[((row NW + w) 4 + p) n1 + n] is the sum over the atoms of
+// w_i times a c_n, a s_n, b c_n, b s_n (p = 0..3), w_i = 1 or, with NW = 5,
+// also d_i and |d_i|^2 (d = r - R_mol).  At gives an atom's phase per axis,
+// its charge and d.  Columns past i1 have charge 0.  Tables that hold the
+// whole chunk stay for all the block's groups.
+template <typename R, int NW, typename At>
+__device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, int i1, int g0, int gs, int vpw,
+                                        int nt, void* lds, double* __restrict__ out) {
+    typedef KsMat<R> M;
+    const size_t te = ks_table_bytes<R>(kr, NW) / sizeof(KsC<R>);   // a table, then its weights
+    KsC<R>* const tabs = static_cast<KsC<R>*>(lds);
+    const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int nvt = kr.tiles() * NW;
+    // a wave per (table, axis or weights); lane u fills column u
+    auto fill = [&](int t0) {
+        constexpr int TASKS = NW > 1 ? 4 : 3;
+        for (int task = w; task < nt * TASKS; task += KS_WAVES) {
+            const int tb = task / TASKS, fp = task % TASKS;
+            const int ia = t0 + tb * KS_TILE + lane;
+            const bool live = ia < i1;
+            KsC<R>* tab = tabs + tb * te;
+            if (fp < 3) {
+                double2 p = make_double2(1.0, 0.0);
+                double f = 1.0;
+                if (live) p = at.phase(ia, fp);
+                if (fp == 0) f = live ? at.charge(ia) : 0.0;
+                const int base = fp == 0 ? 0 : (fp == 1 ? kr.nx1 : kr.nx1 + kr.ny1);
+                ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, lane, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x,
+                             p.y, f);
+            } else {
+                double d[3] = {0.0, 0.0, 0.0};
+                if (live) at.offset(ia, d);
+                R* q = reinterpret_cast<R*>(tab + kr.table_entries()) + lane;
+                q[0] = R(1);
+                q[KS_TILE] = (R)d[0];
+                q[2 * KS_TILE] = (R)d[1];
+                q[3 * KS_TILE] = (R)d[2];
+                q[4 * KS_TILE] = (R)(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+            }
+        }
+    };
+    bool filled = false;
+    const bool stay = i1 - i0 <= nt * KS_TILE;
+    for (int vt0 = g0 * KS_WAVES * vpw; vt0 < nvt; vt0 += gs * KS_WAVES * vpw) {
+        // this wave's pairs and, per pair, this lane's row of the tile
+        int ox[KS_VT], oy[KS_VT], wt[KS_VT];
+        R sy[KS_VT];
+        bool on[KS_VT];
+        double tot[KS_VT][4][4];
+#pragma unroll
+        for (int t = 0; t < KS_VT; ++t) {
+            const int vt = vt0 + w + t * KS_WAVES;
+            on[t] = t < vpw && vt < nvt;
+            const int row = min((on[t] ? vt / NW : 0) * KS_ROWS + lane % 16, kr.nrows - 1);
+            const int v = kr.xy[row];
+            wt[t] = vt % NW;
+            ox[t] = ks_nx(v) * kr.ts;
+            oy[t] = (kr.nx1 + abs(ks_ny(v))) * kr.ts;
+            sy[t] = ks_ny(v) < 0 ? R(-1) : R(1);
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tot[t][p][r] = 0.0;
+        }
+        // columns are n = lane % 16 + 16 c; more than 16 functions take further passes
+        for (int nc = 0; nc * 16 < kr.n1; ++nc) {
+            const int oz = (kr.nx1 + kr.ny1 + min(lane % 16 + 16 * nc, kr.n1 - 1)) * kr.ts;
+            for (int t0 = i0; t0 < i1; t0 += KS_TILE) {
+                const int tb = (t0 - i0) / KS_TILE % nt;
+                if (tb == 0 && !filled) {
+                    __syncthreads();
+                    fill(t0);
+                    __syncthreads();
+                    filled = stay;
+                }
+                const KsC<R>* tab = tabs + tb * te;
+                const R* wts = reinterpret_cast<const R*>(tab + kr.table_entries());
+                // One or both pairs per pass over the table, without a branch
+                // inside, so the reads of later steps are issued ahead of the
+                // products; columns past i1 add zeros.
+                typename M::acc acc[KS_VT][4] = {};
+                auto products = [&](auto pairs) {
+#pragma unroll 4
+                    for (int k = 0; k < KS_TILE / 4; ++k) {
+                        const int u = 4 * k + lane / 16;
+                        const KsC<R> z = tab[oz + u];
+#pragma unroll
+                        for (int t = 0; t < decltype(pairs)::value; ++t) {
+                            KsC<R> y = tab[oy[t] + u];
+                            y.im *= sy[t];
+                            KsC<R> e = ks_mul(tab[ox[t] + u], y);
+                            if constexpr (NW > 1) {
+                                const R f = wts[wt[t] * KS_TILE + u];
+                                e.re *= f;
+                                e.im *= f;
+                            }
+                            acc[t][0] = M::mul(e.re, z.re, acc[t][0]);
+                            acc[t][1] = M::mul(e.re, z.im, acc[t][1]);
+                            acc[t][2] = M::mul(e.im, z.re, acc[t][2]);
+                            acc[t][3] = M::mul(e.im, z.im, acc[t][3]);
+                        }
+                    }
+                };
+                if (on[1]) products(std::integral_constant<int, 2>{});   // wave-uniform
+                else if (on[0]) products(std::integral_constant<int, 1>{});
+#pragma unroll
+                for (int t = 0; t < KS_VT; ++t)
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) tot[t][p][r] += (double)acc[t][p][r];
+            }
+            const int n = lane % 16 + 16 * nc;
+#pragma unroll
+            for (int t = 0; t < KS_VT; ++t) {
+                const int vt = vt0 + w + t * KS_WAVES;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = (vt / NW) * KS_ROWS + M::row(lane, r);
+                    const bool st = on[t] && n < kr.n1 && row < kr.nrows;
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        if (st) out[((size_t)(row * NW + wt[t]) * 4 + p) * kr.n1 + n] = tot[t][p][r];
+                        tot[t][p][r] = 0.0;
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The force pass's coefficients of one (row, n) from G+ = (bC, bS) of +nz and
+// G- of -nz (0 where the set has no such k): functions 2n (c_n) and 2n + 1
+// (s_n) of the four outputs Re T, Im T, Re T', Im T'.
+template <typename R>
+__device__ __forceinline__ void ks_coef(const KsRows& kr, R* __restrict__ coef, int row, int n, double cp, double sp,
+                                        double cm, double sm) {
+    // conj(G+) + conj(G-) and i (conj(G+) - conj(G-))
+    const double ur = cp + cm, ui = -(sp + sm), vr = sp - sm, vi = cp - cm;
+    const int kp = 4 * kr.steps();
+    R* w = coef + ((size_t)(row / KS_ROWS) * 4 * kp + 2 * n) * KS_ROWS + row % KS_ROWS;
+    const size_t o = (size_t)kp * KS_ROWS;
+    const double f = (double)n;
+    w[0] = (R)ur;                 w[KS_ROWS] = (R)vr;
+    w[o] = (R)ui;                 w[o + KS_ROWS] = (R)vi;
+    w[2 * o] = (R)(f * vi);       w[2 * o + KS_ROWS] = (R)(-f * ui);
+    w[3 * o] = (R)(-f * vr);      w[3 * o + KS_ROWS] = (R)(f * ur);
+}
+// Zeros for the functions past 2 n1 and, in rows past the last, all of them.
+template <typename R>
+__device__ __forceinline__ void ks_coef_pad(const KsRows& kr, R* __restrict__ coef, int row, int tid, int nt) {
+    const int kp = 4 * kr.steps(), from = row < kr.nrows ? 2 * kr.n1 : 0;
+    for (int t = tid; t < 4 * (kp - from); t += nt) {
+        const int o = t / (kp - from), k = from + t % (kp - from);
+        coef[(((size_t)(row / KS_ROWS) * 4 + o) * kp + k) * KS_ROWS + row % KS_ROWS] = R(0);
+    }
+}
+
+// The waves' partial forces take the table's place once it has been read.
+template <typename R>
+__host__ __device__ inline size_t ks_force_lds(const KsRows& kr) {
+    const size_t t = kr.table_entries() * 2 * sizeof(R), p = (size_t)KS_WAVES * KS_TILE * 3 * sizeof(double);
+    return t > p ? t : p;
+}
+
+// sum_k (bC sin(k.r) - bS cos(k.r)) (nx, ny, nz) of atoms [i0, i0 + 64), by
+// one block: thread t < 192 returns atom i0 + t / 3, component t % 3.  A wave
+// takes every eighth 16-row tile, its coefficients in registers (KS inner
+// steps; 0: more than KS_MAXSTEP, read per product).
+template <typename R, int KS, typename At>
+__device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const R* __restrict__ coef, int i0, int i1,
+                                           void* lds) {
+    typedef KsMat<R> M;
+    KsC<R>* tab = static_cast<KsC<R>*>(lds);
+    double* part = static_cast<double*>(lds);
+    const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int fu = threadIdx.x % KS_TILE, fp = threadIdx.x / KS_TILE;
+    if (fp < 3) {
+        const int ia = min(i0 + fu, i1 - 1);   // idle columns repeat the last atom; nothing reads them
+        const double2 p = at.phase(ia, fp);
+        const int base = fp == 0 ? 0 : (fp == 1 ? kr.nx1 : kr.nx1 + kr.ny1);
+        ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, fu, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x, p.y, 1.0);
+    }
+    __syncthreads();
+    const KsC<R>* tz = tab + (size_t)(kr.nx1 + kr.ny1) * kr.ts;
+    const int steps = KS ? KS : kr.steps(), kp = 4 * steps;
+    // functions 4 s + lane / 16: part (lane / 16) & 1 of power 2 s + lane / 32
+    const R* tzp = reinterpret_cast<const R*>(tz) + ((lane / 16) & 1);
+    double g[4][3];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) g[a][d] = 0.0;
+    for (int tile = w; tile < kr.tiles(); tile += KS_WAVES) {
+        const R* cw = coef + (size_t)tile * 4 * kp * KS_ROWS + lane;   // function lane / 16 of a step, row lane % 16
+        R A[4][KS ? KS : 1];
+        if constexpr (KS > 0) {
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+#pragma unroll
+                for (int s = 0; s < KS; ++s) A[o][s] = cw[((size_t)o * kp + 4 * s) * KS_ROWS];
+        }
+        int ox[4], oy[4];
+        R sy[4];
+        double nx[4], ny[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int v = kr.xy[min(tile * KS_ROWS + M::row(lane, r), kr.nrows - 1)];
+            ox[r] = ks_nx(v) * kr.ts;
+            oy[r] = (kr.nx1 + abs(ks_ny(v))) * kr.ts;
+            sy[r] = ks_ny(v) < 0 ? R(-1) : R(1);
+            nx[r] = (double)ks_nx(v);
+            ny[r] = (double)ks_ny(v);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int u = 16 * a + lane % 16;
+            typename M::acc T[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+            if constexpr (KS > 0) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const R bz = tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + u)];
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) T[o] = M::mul(A[o][s], bz, T[o]);
+                }
+            } else {
+                for (int s = 0; s < steps; ++s) {
+                    const R bz = tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + u)];
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) T[o] = M::mul(cw[((size_t)o * kp + 4 * s) * KS_ROWS], bz, T[o]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                KsC<R> y = tab[oy[r] + u];
+                y.im *= sy[r];
+                const KsC<R> e = ks_mul(tab[ox[r] + u], y);
+                const double val = (double)(e.im * T[0][r] + e.re * T[1][r]);
+                g[a][0] = fma(val, nx[r], g[a][0]);
+                g[a][1] = fma(val, ny[r], g[a][1]);
+                g[a][2] += (double)(e.im * T[2][r] + e.re * T[3][r]);
+            }
+        }
+    }
+    // the four lanes of an atom hold different rows of the tiles
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            g[a][d] += __shfl_xor(g[a][d], 16, WAVE);
+            g[a][d] += __shfl_xor(g[a][d], 32, WAVE);
+        }
+    __syncthreads();
+    if (lane < 16) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) part[((size_t)w * KS_TILE + 16 * a + lane) * 3 + d] = g[a][d];
+    }
+    __syncthreads();
+    double f = 0.0;
+    if (threadIdx.x < 3 * KS_TILE)
+        for (int v = 0; v < KS_WAVES; ++v) f += part[(size_t)v * KS_TILE * 3 + threadIdx.x];
+    return f;
+}
+
+}  // namespace smd

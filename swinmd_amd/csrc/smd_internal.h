@@ -26,7 +26,7 @@ constexpr double BOLTZ = 0.0083145112;              // src/NEMD_defs.h:108
 // Reduction sites of block_part (see there).
 enum RedSite : int {
     RS_BOND = 0, RS_ANGLE, RS_UB, RS_EW_INTRA, RS_EW_SURF, RS_RECIP, RS_MP_REAL, RS_MP_INTRA, RS_MP_SURF,
-    RS_MP_LONG, RS_IND_REAL, RS_IND_INTRA, RS_IND_SURF, RS_IND_LONG, RS_PAIR_LJ, RS_PAIR_EW, RS_PACKED,
+    RS_MP_LONG, RS_IND_REAL, RS_IND_INTRA, RS_IND_SURF, RS_IND_LONG, RS_PAIR_LJ, RS_PAIR_EW, RS_PACKED, RS_RECIP_FF,
     // the torque kernel's dU/dV and torque sums, one pair per launch of a step
     RS_MP_DUDV, RS_MP_TRQ, RS_MP_DUDV_L, RS_MP_TRQ_L, RS_IND_DUDV, RS_IND_TRQ, RS_IND_DUDV_L, RS_IND_TRQ_L,
     RS_COUNT
@@ -168,19 +168,14 @@ struct Ctx {
     int K = 0;
     int nmax[3] = {0, 0, 0};
     double self_energy = 0, charged_energy = 0;
-    double* d_kvec = nullptr;     // [3K]
-    double* d_kmod2 = nullptr;    // [K]
-    double* d_expk = nullptr;     // [K]
-    int32_t* d_kn = nullptr;      // [3K] integer (nx, ny, nz)
-    int4* d_kgrp = nullptr;       // [n_kgrp] runs of consecutive nz in one (nx, ny) row
-    int32_t* d_ksplit = nullptr;  // [RF_WAVES+1] group ranges of the reciprocal force pass
-    int n_kgrp = 0;
-    double* d_sfac_part = nullptr;  // [chunks][K][10] per-chunk structure-factor sums
-    double* d_kf = nullptr;         // [K] (b C, b S) in the force pass's precision
-    double* d_e1 = nullptr;         // [n][3] complex exp(i 2 pi r_p / L_p), then [n] (q, r - R_mol)
+    double* d_expk = nullptr;     // [n_krows][nmax_z + 1] exp(-k^2 / 4 alpha^2) / k^2
+    int32_t* d_kxy = nullptr;     // [n_krows] nx << 16 | (ny & 0xffff)
+    int n_krows = 0, n_kruns = 0; // (nx, ny) rows; runs of at most eight consecutive nz
+    size_t k_part = 0;            // doubles of one chunk's structure-factor partials
+    double* d_sfac_part = nullptr;  // [chunks][k_part]
+    double* d_kf = nullptr;         // force-pass coefficients, in its precision
+    double* d_e1 = nullptr;         // [n][3] complex exp(i 2 pi r_p / L_p)
     int sfac_chunks = 0;
-    size_t sfac_lds[2] = {0, 0};    // dynamic LDS of the structure-factor pass (FP64, FP32)
-    size_t force_lds[2] = {0, 0};   // dynamic LDS of the force pass (FP64, FP32)
 
     // vdW tables (device)
     double* d_vdw_a = nullptr;    // [ntypes^2] per kind meaning

@@ -45,3 +45,43 @@ def test_rigid_water_step_sizes_match_the_oracle(n):
     for k in ("e_real", "e_long", "e_intra", "atom_ke2"):
         if ref[k]:
             assert rel(rep[k], ref[k]) <= 1e-8, k
+
+
+class _BoxedWater(S.System):
+    """A water system in a box of given edges (System's own is a cube)."""
+    edges = None
+
+    @property
+    def box(self):
+        return np.array(self.edges, dtype=np.float64)
+
+
+# molecules, edges, k cut as a count of the longest edge's waves: one k-row and
+# function, rows past a 16-row tile, atoms past a 64-atom table, more than 16
+# and more than 32 functions of nz, tables at their narrow stride
+@pytest.mark.parametrize("n,edges,waves", [(1, (1.2, 1.2, 1.2), 1.2), (21, (1.4, 1.4, 1.4), 5.2),
+                                           (22, (1.4, 1.4, 1.4), 5.2), (64, (1.3, 1.5, 1.7), 11.2),
+                                           (85, (1.5, 1.5, 7.5), 20.3), (43, (1.0, 1.0, 12.0), 49.5)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_reciprocal_space_shapes_match_the_oracle(n, edges, waves, mixed):
+    """Forces, energy, virial and volume derivatives of EwaldForce.compute_long:
+    1e-10 in FP64, 1e-5 mixed (forces) as in the larger parity tests."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context, EwaldForce
+    s = S.water(n, box=min(edges), seed=n, subset=True, jitter=0.01)
+    s.__class__ = _BoxedWater
+    s.edges = edges
+    s.pos = s.pos * (np.array(edges) / min(edges)) if n > 40 else s.pos
+    kcut = 2 * np.pi * waves / max(edges)
+    print(f"case recip n={n} edges={edges} waves={waves} mixed={mixed}", flush=True)
+    ctx = Context(s)
+    ctx.compute_mol_centers()
+    ew = EwaldForce(ctx, alpha=3.5, real_cut=0.5, kcut=kcut, prec=L.PREC_MIXED if mixed else L.PREC_FP64)
+    f = np.zeros((s.n_atoms, 3))
+    out = ew.compute_long(f)
+    fo, eo = O.Oracle(s).ewald_recip(kcut, 3.5)
+    tol = 1e-5 if mixed else 1e-10
+    assert rel_rms(f, fo) <= tol
+    for k in ("energy", "deriv", "deriv2"):
+        assert abs(out[k] - eo[k]) <= tol * max(abs(eo[k]), abs(eo["energy"])), k
+    assert rel_rms(out["virial"], eo["virial"]) <= tol

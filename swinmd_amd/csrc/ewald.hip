@@ -78,7 +78,6 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     kr.n1 = nmax[2] + 1;
     kr.nx1 = nmax[0] + 1;
     kr.ny1 = nmax[1] + 1;
-    kr.ts = ks_stride(kr.powers());
     std::vector<int32_t> xy;
     std::vector<double> rexp;
     int ng = 0, run = 0;   // runs of at most eight consecutive nz in a row
@@ -97,7 +96,7 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     // The sets this path takes: the powers of 64 atoms, and 16 bytes per k
     // and per run of eight, within 64 KiB.
     const size_t ne = (size_t)nmax[0] + nmax[1] + nmax[2] + 3;
-    if (ne * KS_TS_NARROW * 16 + 5 * KS_TILE * 8 > LDS_MAX || (size_t)(K + ng) * 16 > LDS_MAX)
+    if (ne * ks_stride<double>() * 16 + 5 * KS_TILE * 8 > LDS_MAX || (size_t)(K + ng) * 16 > LDS_MAX)
         return fail(c, SMD_ENOTSUP, "reciprocal space too large for the LDS-resident passes (%d k-vectors, nmax %d %d %d)",
                     K, nmax[0], nmax[1], nmax[2]);
     int rc;
@@ -423,7 +422,7 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
 // Force on atom i, sum_k (b C q sin - b S q cos) k (:609-658).  FF: also the
 // block's sum of F . d (T_RC_FF).
 template <typename R, int KS, bool FF>
-__global__ __launch_bounds__(KS_THREADS) void k_recip_force(RecipArgs a) {
+__global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<R>) void k_recip_force(RecipArgs a) {
     extern __shared__ double lds[];
     const int i0 = blockIdx.x * KS_TILE;
     const RecipPhases at{a.e1};
@@ -444,8 +443,10 @@ __global__ __launch_bounds__(KS_THREADS) void k_recip_force(RecipArgs a) {
 
 template <typename R, bool FF>
 static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
-    const dim3 g((a.n + KS_TILE - 1) / KS_TILE), b(KS_THREADS);
-    const size_t lds = ks_force_lds<R>(a.kr);
+    const dim3 g((a.n + KS_TILE - 1) / KS_TILE);
+    const int waves = ks_waves(a.kr.tiles(), 1, KS_MAXW, 3);
+    const dim3 b(waves * WAVE);
+    const size_t lds = ks_force_lds<R>(a.kr, waves);
     switch (a.kr.steps()) {
         case 1: hipLaunchKernelGGL((k_recip_force<R, 1, FF>), g, b, lds, s, a); break;
         case 2: hipLaunchKernelGGL((k_recip_force<R, 2, FF>), g, b, lds, s, a); break;
@@ -464,11 +465,12 @@ static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes
     if (passes & RECIP_SFAC) {
         // A chunk's (tile, weight) pairs go side by side over blocks only where
         // the chunks alone leave CUs idle, since each block fills its own table.
-        const int nvt = a.kr.tiles() * NW, per = KS_WAVES * a.vpw, groups = (nvt + per - 1) / per;
+        const int nvt = a.kr.tiles() * NW, waves = ks_waves(nvt, a.vpw, KS_MAXW, 3);
+        const int groups = (nvt + waves * a.vpw - 1) / (waves * a.vpw);
         int gy = std::min(groups, std::max(1, 256 / a.chunks));
         gy = (groups + (groups + gy - 1) / gy - 1) / ((groups + gy - 1) / gy);   // no block with one group more
         const size_t lds = ks_table_bytes<R>(a.kr, NW) * ks_tables<R>(a.kr, NW, a.per / KS_TILE);
-        hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(KS_THREADS), lds, s, a);
+        hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(waves * WAVE), lds, s, a);
     }
     if (passes & RECIP_REDUCE) {
         // a wave per dozen chunks, fewer where the row's sums are many: the
@@ -525,7 +527,7 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
     a.kr.nx1 = c->nmax[0] + 1;
     a.kr.ny1 = c->nmax[1] + 1;
     a.kr.n1 = c->nmax[2] + 1;
-    a.kr.ts = ks_stride(a.kr.powers());
+    a.kr.ts = prec == SMD_PREC_MIXED ? ks_stride<float>() : ks_stride<double>();
     a.kr.xy = c->d_kxy;
     // whole tiles per chunk
     const int nt = (c->n + KS_TILE - 1) / KS_TILE;

@@ -26,12 +26,11 @@
 namespace smd {
 
 constexpr int KS_TILE = 64;       // atoms per LDS table
-// Table stride: a wave reads 16 powers of 4 neighbouring atoms, which at
-// stride 4 mod 16 fall on distinct banks (65 put four of them on one);
-// 65 where 68 would take the tables past 64 KiB.
-constexpr int KS_TS = KS_TILE + 4, KS_TS_NARROW = KS_TILE + 1;
-constexpr int KS_WAVES = 8;
-constexpr int KS_THREADS = KS_WAVES * WAVE;
+constexpr int KS_MAXW = 8;        // waves of a block, at most
+constexpr int KS_THREADS = KS_MAXW * WAVE;
+// Waves per SIMD the force pass is compiled for: FP32 fits four without
+// spilling (two blocks of eight per CU), FP64 three.
+template <typename R> constexpr int KS_FORCE_OCC = sizeof(R) == 8 ? 3 : 4;
 constexpr int KS_ROWS = 16;       // rows of a matrix tile
 constexpr int KS_VT = 2;          // tiles per wave of the structure-factor pass
 constexpr int KS_MAXSTEP = 8;     // inner steps held in registers by the force pass
@@ -53,7 +52,22 @@ template <> struct KsMat<float> {
     static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane / 16) + r; }
 };
 
-template <typename R> struct KsC { R re, im; };
+template <typename R> struct alignas(2 * sizeof(R)) KsC { R re, im; };
+
+// Table stride: a wave reads 16 powers of 4 neighbouring atoms.  Sixteen-byte
+// entries are read 16 lanes at a time, which an odd stride puts on distinct
+// banks; eight-byte ones 32 at a time, 16 powers of 2 atoms, which 2 mod 32
+// does.
+template <typename R>
+__host__ __device__ constexpr int ks_stride() { return KS_TILE + (sizeof(R) == 8 ? 1 : 2); }
+
+// Waves of a block for `units` tiles, `per` of them per wave at a time, so
+// that no wave has one more than the others where that can be avoided.
+inline int ks_waves(int units, int per, int most, int least) {
+    const int passes = (units + most * per - 1) / (most * per);
+    const int w = (units + passes * per - 1) / (passes * per);
+    return w < least ? least : w;
+}
 template <typename R>
 __device__ __forceinline__ KsC<R> ks_mul(KsC<R> a, KsC<R> b) {
     return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
@@ -62,7 +76,7 @@ __device__ __forceinline__ KsC<R> ks_mul(KsC<R> a, KsC<R> b) {
 struct KsRows {
     int nrows, n1;       // rows; nz = 0..n1-1 and their negatives
     int nx1, ny1;        // powers of X (0..nx1-1) and of Y (0..ny1-1, conjugated for ny < 0)
-    int ts;              // table stride (ks_stride)
+    int ts;              // table stride (ks_stride of the pass's precision)
     const int* xy;       // [nrows] nx << 16 | (ny & 0xffff)
     __host__ __device__ int tiles() const { return (nrows + KS_ROWS - 1) / KS_ROWS; }
     __host__ __device__ int powers() const { return nx1 + ny1 + n1; }
@@ -71,9 +85,6 @@ struct KsRows {
     // per-row coefficients of the force pass: [tile][4][4 steps][16]
     __host__ __device__ size_t coef_entries() const { return (size_t)tiles() * 4 * steps() * 4 * KS_ROWS; }
 };
-inline int ks_stride(int powers) {
-    return (size_t)powers * KS_TS * 16 + 5 * KS_TILE * 8 <= 65536 ? KS_TS : KS_TS_NARROW;
-}
 __host__ __device__ inline int ks_nx(int v) { return v >> 16; }
 __host__ __device__ inline int ks_ny(int v) { return (int)(short)(v & 0xffff); }
 
@@ -105,7 +116,7 @@ __host__ __device__ inline int ks_tables(const KsRows& kr, int nw, int chunk_til
 }
 
 // Structure factors of atoms [i0, i1) for the (tile, weight) pairs of groups
-// g0, g0 + gs, ... of vpw KS_WAVES (vpw at most KS_VT), by one block with
+// g0, g0 + gs, ... of vpw per wave (vpw at most KS_VT), by one block with
 // `nt` tables: out[((row NW + w) 4 + p) n1 + n] is the sum over the atoms of
 // w_i times a c_n, a s_n, b c_n, b s_n (p = 0..3), w_i = 1 or, with NW = 5,
 // also d_i and |d_i|^2 (d = r - R_mol).  At gives an atom's phase per axis,
@@ -118,11 +129,11 @@ __device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, 
     const size_t te = ks_table_bytes<R>(kr, NW) / sizeof(KsC<R>);   // a table, then its weights
     KsC<R>* const tabs = static_cast<KsC<R>*>(lds);
     const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int nvt = kr.tiles() * NW;
+    const int nvt = kr.tiles() * NW, nw = blockDim.x / WAVE;
     // a wave per (table, axis or weights); lane u fills column u
     auto fill = [&](int t0) {
         constexpr int TASKS = NW > 1 ? 4 : 3;
-        for (int task = w; task < nt * TASKS; task += KS_WAVES) {
+        for (int task = w; task < nt * TASKS; task += nw) {
             const int tb = task / TASKS, fp = task % TASKS;
             const int ia = t0 + tb * KS_TILE + lane;
             const bool live = ia < i1;
@@ -149,15 +160,19 @@ __device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, 
     };
     bool filled = false;
     const bool stay = i1 - i0 <= nt * KS_TILE;
-    for (int vt0 = g0 * KS_WAVES * vpw; vt0 < nvt; vt0 += gs * KS_WAVES * vpw) {
+    for (int vt0 = g0 * nw * vpw; vt0 < nvt; vt0 += gs * nw * vpw) {
         // this wave's pairs and, per pair, this lane's row of the tile
         int ox[KS_VT], oy[KS_VT], wt[KS_VT];
         R sy[KS_VT];
         bool on[KS_VT];
-        double tot[KS_VT][4][4];
+        // FP64 products add up in their accumulators; FP32 ones enter FP64
+        // sums after every table
+        constexpr bool SPLIT = sizeof(R) == 4;
+        typename M::acc acc[KS_VT][4];
+        double tot[SPLIT ? KS_VT : 1][4][4];
 #pragma unroll
         for (int t = 0; t < KS_VT; ++t) {
-            const int vt = vt0 + w + t * KS_WAVES;
+            const int vt = vt0 + w + t * nw;
             on[t] = t < vpw && vt < nvt;
             const int row = min((on[t] ? vt / NW : 0) * KS_ROWS + lane % 16, kr.nrows - 1);
             const int v = kr.xy[row];
@@ -168,7 +183,10 @@ __device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, 
 #pragma unroll
             for (int p = 0; p < 4; ++p)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) tot[t][p][r] = 0.0;
+                for (int r = 0; r < 4; ++r) {
+                    acc[t][p][r] = R(0);
+                    if constexpr (SPLIT) tot[t][p][r] = 0.0;
+                }
         }
         // columns are n = lane % 16 + 16 c; more than 16 functions take further passes
         for (int nc = 0; nc * 16 < kr.n1; ++nc) {
@@ -186,7 +204,6 @@ __device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, 
                 // One or both pairs per pass over the table, without a branch
                 // inside, so the reads of later steps are issued ahead of the
                 // products; columns past i1 add zeros.
-                typename M::acc acc[KS_VT][4] = {};
                 auto products = [&](auto pairs) {
 #pragma unroll 4
                     for (int k = 0; k < KS_TILE / 4; ++k) {
@@ -211,25 +228,36 @@ __device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, 
                 };
                 if (on[1]) products(std::integral_constant<int, 2>{});   // wave-uniform
                 else if (on[0]) products(std::integral_constant<int, 1>{});
+                if constexpr (SPLIT) {
 #pragma unroll
-                for (int t = 0; t < KS_VT; ++t)
+                    for (int t = 0; t < KS_VT; ++t)
 #pragma unroll
-                    for (int p = 0; p < 4; ++p)
+                        for (int p = 0; p < 4; ++p)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) tot[t][p][r] += (double)acc[t][p][r];
+                            for (int r = 0; r < 4; ++r) {
+                                tot[t][p][r] += (double)acc[t][p][r];
+                                acc[t][p][r] = R(0);
+                            }
+                }
             }
             const int n = lane % 16 + 16 * nc;
 #pragma unroll
             for (int t = 0; t < KS_VT; ++t) {
-                const int vt = vt0 + w + t * KS_WAVES;
+                const int vt = vt0 + w + t * nw;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = (vt / NW) * KS_ROWS + M::row(lane, r);
                     const bool st = on[t] && n < kr.n1 && row < kr.nrows;
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
-                        if (st) out[((size_t)(row * NW + wt[t]) * 4 + p) * kr.n1 + n] = tot[t][p][r];
-                        tot[t][p][r] = 0.0;
+                        double* o = out + ((size_t)(row * NW + wt[t]) * 4 + p) * kr.n1 + n;
+                        if constexpr (SPLIT) {
+                            if (st) *o = tot[t][p][r];
+                            tot[t][p][r] = 0.0;
+                        } else {
+                            if (st) *o = acc[t][p][r];
+                            acc[t][p][r] = R(0);
+                        }
                     }
                 }
             }
@@ -264,42 +292,39 @@ __device__ __forceinline__ void ks_coef_pad(const KsRows& kr, R* __restrict__ co
     }
 }
 
-// The waves' partial forces take the table's place once it has been read.
+// The table, then the waves' partial forces.
 template <typename R>
-__host__ __device__ inline size_t ks_force_lds(const KsRows& kr) {
-    const size_t t = kr.table_entries() * 2 * sizeof(R), p = (size_t)KS_WAVES * KS_TILE * 3 * sizeof(double);
-    return t > p ? t : p;
+__host__ __device__ inline size_t ks_force_table(const KsRows& kr) { return (kr.table_entries() * 2 * sizeof(R) + 15) / 16 * 16; }
+template <typename R>
+inline size_t ks_force_lds(const KsRows& kr, int waves) {
+    return ks_force_table<R>(kr) + (size_t)waves * KS_TILE * 3 * sizeof(double);
 }
 
 // sum_k (bC sin(k.r) - bS cos(k.r)) (nx, ny, nz) of atoms [i0, i0 + 64), by
-// one block: thread t < 192 returns atom i0 + t / 3, component t % 3.  A wave
-// takes every eighth 16-row tile, its coefficients in registers (KS inner
+// one block of three waves or more: thread t < 192 returns atom i0 + t / 3,
+// component t % 3.  The waves take the 16-row tiles in turn, its coefficients in registers (KS inner
 // steps; 0: more than KS_MAXSTEP, read per product).
 template <typename R, int KS, typename At>
 __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const R* __restrict__ coef, int i0, int i1,
                                            void* lds) {
     typedef KsMat<R> M;
     KsC<R>* tab = static_cast<KsC<R>*>(lds);
-    double* part = static_cast<double*>(lds);
     const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int fu = threadIdx.x % KS_TILE, fp = threadIdx.x / KS_TILE;
+    const int fu = threadIdx.x % KS_TILE, fp = threadIdx.x / KS_TILE, nw = blockDim.x / WAVE;
     if (fp < 3) {
         const int ia = min(i0 + fu, i1 - 1);   // idle columns repeat the last atom; nothing reads them
         const double2 p = at.phase(ia, fp);
         const int base = fp == 0 ? 0 : (fp == 1 ? kr.nx1 : kr.nx1 + kr.ny1);
-        ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, fu, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x, p.y, 1.0);
+        ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, fu, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x,
+                     p.y, 1.0);
     }
     __syncthreads();
     const KsC<R>* tz = tab + (size_t)(kr.nx1 + kr.ny1) * kr.ts;
     const int steps = KS ? KS : kr.steps(), kp = 4 * steps;
     // functions 4 s + lane / 16: part (lane / 16) & 1 of power 2 s + lane / 32
     const R* tzp = reinterpret_cast<const R*>(tz) + ((lane / 16) & 1);
-    double g[4][3];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) g[a][d] = 0.0;
-    for (int tile = w; tile < kr.tiles(); tile += KS_WAVES) {
+    double* part = reinterpret_cast<double*>(static_cast<char*>(lds) + ks_force_table<R>(kr)) + (size_t)w * KS_TILE * 3;
+    for (int tile = w; tile < kr.tiles(); tile += nw) {
         const R* cw = coef + (size_t)tile * 4 * kp * KS_ROWS + lane;   // function lane / 16 of a step, row lane % 16
         R A[4][KS ? KS : 1];
         if constexpr (KS > 0) {
@@ -320,9 +345,9 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
             nx[r] = (double)ks_nx(v);
             ny[r] = (double)ks_ny(v);
         }
-#pragma unroll
         for (int a = 0; a < 4; ++a) {
             const int u = 16 * a + lane % 16;
+            double g[3] = {0.0, 0.0, 0.0};
             typename M::acc T[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
             if constexpr (KS > 0) {
 #pragma unroll
@@ -344,31 +369,29 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
                 y.im *= sy[r];
                 const KsC<R> e = ks_mul(tab[ox[r] + u], y);
                 const double val = (double)(e.im * T[0][r] + e.re * T[1][r]);
-                g[a][0] = fma(val, nx[r], g[a][0]);
-                g[a][1] = fma(val, ny[r], g[a][1]);
-                g[a][2] += (double)(e.im * T[2][r] + e.re * T[3][r]);
+                g[0] = fma(val, nx[r], g[0]);
+                g[1] = fma(val, ny[r], g[1]);
+                g[2] += (double)(e.im * T[2][r] + e.re * T[3][r]);
+            }
+            // the four lanes of an atom hold different rows of the tile
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                g[d] += __shfl_xor(g[d], 16, WAVE);
+                g[d] += __shfl_xor(g[d], 32, WAVE);
+            }
+            if (lane < 16) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    double* o = part + 3 * u + d;
+                    *o = tile == w ? g[d] : *o + g[d];
+                }
             }
         }
-    }
-    // the four lanes of an atom hold different rows of the tiles
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            g[a][d] += __shfl_xor(g[a][d], 16, WAVE);
-            g[a][d] += __shfl_xor(g[a][d], 32, WAVE);
-        }
-    __syncthreads();
-    if (lane < 16) {
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int d = 0; d < 3; ++d) part[((size_t)w * KS_TILE + 16 * a + lane) * 3 + d] = g[a][d];
     }
     __syncthreads();
     double f = 0.0;
     if (threadIdx.x < 3 * KS_TILE)
-        for (int v = 0; v < KS_WAVES; ++v) f += part[(size_t)v * KS_TILE * 3 + threadIdx.x];
+        for (int v = 0; v < min(nw, kr.tiles()); ++v) f += part[(ptrdiff_t)(v - w) * KS_TILE * 3 + threadIdx.x];
     return f;
 }
 

@@ -40,6 +40,7 @@
 #include <string>
 #include <vector>
 
+#include "kspace.h"
 #include "shake.h"
 #include "smd_internal.h"
 
@@ -68,7 +69,9 @@ struct Rep {
     int32_t pb0, pb1;             // pair-kernel blocks
     int32_t fb0, fb1;             // reciprocal-finish blocks
     int32_t sb0, sb1;             // SHAKE blocks
-    int32_t hmax, nyb, nzmax, pad1;
+    int32_t hmax, nyb, nzmax, rcap;   // rcap: (h, k) rows the cell can have at any tilt, a multiple of 16
+    int64_t ebase, cbase;         // first exp factor (rcap * (nzmax + 1) of them) and force-pass coefficient
+    int32_t rowbase, pad1;        // first row
     double L, invL, gamma, kcut, e_self, volume;
 };
 
@@ -77,7 +80,7 @@ struct RepState {
     double tilt, fnh, fnh_minus;
     double drift[3];
     int32_t K, need, since, apply_drift;
-    int32_t pad0, pending, max_row, pad;   // pending: rebuild at the next step
+    int32_t nrows, pending, max_row, pad;   // pending: rebuild at the next step
     unsigned long long maxd2;     // bits of the largest |d|^2 of the last step (non-negative doubles order as integers)
     int64_t steps, list_updates;
 };
@@ -90,6 +93,7 @@ struct Params {
     double pre2;                  // (rlist + 2 r_OH)^2: the list's O-O prefilter
     double two_roh;               // 2 r_OH with a rounding margin
     int32_t max_count, nose_hoover, nb_cap, n;
+    int32_t rows_on;              // reciprocal space by rows (kspace.h), else the direct passes
 };
 
 struct Args {
@@ -110,6 +114,10 @@ struct Args {
     int32_t* nb_cnt;              // [n]
     double4* kvec;                // [sum kcap] (kx, ky, kz, exp(-k^2/4a^2)/k^2)
     double2* kf;                  // [sum kcap] (b C, b S) for the force pass
+    int32_t* rowxy;               // [sum rcap] rows (h, k) of the current k set
+    double* rowexp;               // exp(-k^2 / 4 a^2) / k^2 per (row, l), 0 outside the set
+    double* coef;                 // force-pass coefficients (ks_coef)
+    double2* e1;                  // [n][3] phases of the fractional coordinates
     double* sf_part;              // structure-factor partials
     double* pair_part;            // [NPAIR][n_pair_blocks]
     double* kf_part;              // [NKF][n_fin_blocks]
@@ -166,6 +174,71 @@ __device__ __forceinline__ double new_tilt(const Rep& r, double tilt, double dt)
 
 // ---- step head: list trigger and the sheared k set -----------------------
 
+// The replica's rows: (h, k) with a k-vector inside the cutoff, l = -m..m in
+// each, compacted in (h, k) order from the candidates h in [0, hmax], k in
+// [-nyb, nyb] (a superset at every tilt); then their exp factors.
+__device__ __forceinline__ KsRows rep_rows(const Args& a, const Rep& rp, int nrows) {
+    KsRows kr;
+    kr.nrows = nrows;
+    kr.nx1 = rp.hmax + 1;
+    kr.ny1 = rp.nyb + 1;
+    kr.n1 = rp.nzmax + 1;
+    kr.ts = ks_stride<double>();
+    kr.xy = a.rowxy + rp.rowbase;
+    return kr;
+}
+
+__device__ void begin_rows(const Args& a, const Rep& rp, RepState& s) {
+    __shared__ int wtot[256 / WAVE];
+    __shared__ int kcount;
+    const double tilt = s.tilt, v = 2.0 * PI / rp.L, kCut2 = rp.kcut * rp.kcut;
+    const int ny_n = 2 * rp.nyb + 1, total = (rp.hmax + 1) * ny_n, n1 = rp.nzmax + 1;
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    int32_t* xy = a.rowxy + rp.rowbase;
+    if (threadIdx.x == 0) kcount = 0;
+    int count = 0;
+    for (int base = 0; base < total; base += blockDim.x) {
+        const int c = base + threadIdx.x, nx = c / ny_n, ny = c % ny_n - rp.nyb;
+        bool take = false;
+        if (c < total && (nx > 0 || ny >= 0)) {
+            const double kx = nx * v, ky = (ny - nx * tilt / rp.L) * v;
+            // (0, 0) has no l = 0; it is a row when l = 1 is inside
+            const double kz = nx == 0 && ny == 0 ? v : 0.0;
+            take = kx * kx + ky * ky + kz * kz < kCut2;
+        }
+        const unsigned long long m = __ballot(take);
+        if (lane == 0) wtot[w] = __popcll(m);
+        __syncthreads();
+        int off = count;
+        for (int q = 0; q < w; ++q) off += wtot[q];
+        for (int q = 0; q < (int)(blockDim.x / WAVE); ++q) count += wtot[q];
+        const int slot = off + __popcll(m & ((1ull << lane) - 1ull));
+        if (take && slot < rp.rcap) xy[slot] = (nx << 16) | (ny & 0xffff);
+        __syncthreads();
+    }
+    const int rows = min(count, rp.rcap);
+    const double alphaR4 = 1.0 / (4.0 * (a.p.alpha * a.p.alpha));
+    int mine = 0;
+    for (int t = threadIdx.x; t < rows * n1; t += blockDim.x) {
+        const int row = t / n1, n = t % n1;
+        const int nx = ks_nx(xy[row]), ny = ks_ny(xy[row]);
+        const double kx = nx * v, ky = (ny - nx * tilt / rp.L) * v, kz = n * v;
+        const double k2 = kx * kx + ky * ky + kz * kz;
+        const bool zero = nx == 0 && ny == 0;
+        const bool in = k2 < kCut2 && !(zero && n == 0);
+        a.rowexp[rp.ebase + t] = in ? exp(-k2 * alphaR4) / k2 : 0.0;
+        mine += in ? (n == 0 || zero ? 1 : 2) : 0;
+    }
+    mine = wave_sum(mine);
+    if (lane == 0) atomicAdd(&kcount, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s.K = min(kcount, rp.kcap);
+        s.nrows = rows;
+        if (kcount > rp.kcap || count > rp.rcap) atomicOr(a.err, E_KCAP);
+    }
+}
+
 // One block per replica.  Decides whether the replica's list is rebuilt this
 // step, and enumerates the reciprocal lattice of the current cell with
 // |k| < kcut in (h, k, l) order, one of each +-k pair, by an ordered
@@ -192,6 +265,10 @@ __global__ __launch_bounds__(256) void k_begin(Args a) {
             if (a.count_update) s.list_updates++;
         }
         s.maxd2 = 0ull;
+    }
+    if (a.p.rows_on) {
+        begin_rows(a, rp, s);
+        return;
     }
     const double tilt = s.tilt;
     const double alphaR4 = 1.0 / (4.0 * (a.p.alpha * a.p.alpha));
@@ -573,6 +650,127 @@ __global__ __launch_bounds__(256) void k_kforce(Args a, int tile) {
     }
 }
 
+// ---- the same by rows, on the matrix cores ---------------------------------
+//
+// k.r = 2 pi (h (x - t y / L) + k y + l z) / L: with x along the tilted
+// lattice the phases factor as they do in an orthogonal cell, so kspace.h's
+// products apply, in FP64 in both precisions.  73,689 molecules, 1,535 k each,
+// alone: factors 132, sums 18, forces 169, the k set 6 us, against the direct
+// mixed passes' 194, 6, 250 and 21.
+
+struct BatchAtoms {
+    const Args& a;
+    const Rep& rp;
+    double tilt;
+    // the fractional coordinate's phase, kept for the force pass
+    __device__ __forceinline__ double2 phase(int i, int p) const {
+        double u = a.pos[3 * i + p];
+        if (p == 0) u -= tilt * rp.invL * a.pos[3 * i + 1];
+        double s, c;
+        sincos(2.0 * PI * (u * rp.invL), &s, &c);
+        const double2 e = make_double2(c, s);
+        a.e1[3 * i + p] = e;
+        return e;
+    }
+    __device__ __forceinline__ double charge(int i) const { return a.p.q[i % 3]; }
+    __device__ __forceinline__ void offset(int, double (&)[3]) const {}
+};
+struct BatchPhases {
+    const double2* e1;
+    __device__ __forceinline__ double2 phase(int i, int p) const { return e1[3 * i + p]; }
+};
+
+// One block per (replica, chunk): its structure factors, [row][4][n1].
+__global__ __launch_bounds__(KS_THREADS) void k_rows_sfac(Args a) {
+    extern __shared__ double lds[];
+    const int4 bm = a.sf_blk[blockIdx.x];
+    const Rep rp = a.rep[bm.x];
+    const KsRows kr = rep_rows(a, rp, a.st[bm.x].nrows);
+    if (kr.nrows == 0) return;   // block-uniform: no k inside the cutoff
+    const int c0 = rp.a0 + bm.z * a.sf_chunk, c1 = min(c0 + a.sf_chunk, rp.a1);
+    const BatchAtoms at{a, rp, a.st[bm.x].tilt};
+    ks_sfac<double, 1>(kr, at, c0, c1, 0, 1, KS_VT, ks_tables<double>(kr, 1, a.sf_chunk / KS_TILE), lds,
+                       a.sf_part + rp.pbase + (int64_t)bm.z * rp.rcap * 4 * kr.n1);
+}
+
+// One wave per row of a replica: the chunks' sums in order, the energy and
+// virial terms (EwaldForce.cpp:529-698) and the force pass's coefficients
+// with b = 8 pi / V exp(..)/k^2; rows past the last clear theirs.
+__global__ __launch_bounds__(256) void k_rows_fin(Args a) {
+    __shared__ double sum[256 / WAVE][4 * WAVE];
+    const int2 bm = a.fin_blk[blockIdx.x];
+    const Rep rp = a.rep[bm.x];
+    const KsRows kr = rep_rows(a, rp, a.st[bm.x].nrows);
+    const double tilt = a.st[bm.x].tilt;
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    const int row = bm.y * (256 / WAVE) + w;
+    double* coef = a.coef + rp.cbase;
+    double v[NKF];
+#pragma unroll
+    for (int q = 0; q < NKF; ++q) v[q] = 0.0;
+    if (row < kr.tiles() * KS_ROWS) ks_coef_pad<double>(kr, coef, row, lane, WAVE);
+    const int nv = 4 * kr.n1;
+    if (row < kr.nrows)
+        for (int t = lane; t < nv; t += WAVE) {
+            const double* p = a.sf_part + rp.pbase + (int64_t)row * nv + t;
+            const int64_t stride = (int64_t)rp.rcap * nv;
+            double s = 0.0;
+#pragma unroll 4
+            for (int c = 0; c < rp.nch; ++c) s += p[c * stride];
+            sum[w][t] = s;
+        }
+    __syncthreads();
+    if (row < kr.nrows && lane < kr.n1) {
+        const int n = lane, nx = ks_nx(kr.xy[row]), ny = ks_ny(kr.xy[row]);
+        const double ek = a.rowexp[rp.ebase + (int64_t)row * kr.n1 + n];
+        const double u = 2.0 * PI / rp.L, kx = nx * u, ky = (ny - nx * tilt / rp.L) * u;
+        const double alphaR4 = 1.0 / (4.0 * (a.p.alpha * a.p.alpha));
+        const double pi4V = 4.0 * PI / rp.volume, b = 2.0 * pi4V * ek;
+        double p[4], G[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) p[q] = sum[w][q * kr.n1 + n];
+        const int signs = ek == 0.0 ? 0 : (n == 0 || (nx == 0 && ny == 0) ? 1 : 2);
+        for (int s = 0; s < signs; ++s) {
+            const double sg = s ? -1.0 : 1.0, kz = sg * n * u;
+            const double C = p[0] - sg * p[3], S = p[2] + sg * p[1];
+            const double k2 = kx * kx + ky * ky + kz * kz;
+            const double te = pi4V * ek * (S * S + C * C);
+            const double coeff = 2.0 * (alphaR4 + 1.0 / k2);
+            v[0] += te;
+            v[1] += te - te * coeff * kx * kx;
+            v[2] += -te * coeff * kx * ky;
+            v[3] += -te * coeff * kx * kz;
+            v[4] += te - te * coeff * ky * ky;
+            v[5] += -te * coeff * ky * kz;
+            v[6] += te - te * coeff * kz * kz;
+            G[s][0] = b * C;
+            G[s][1] = b * S;
+        }
+        ks_coef<double>(kr, coef, row, n, G[0][0], G[0][1], G[1][0], G[1][1]);
+    }
+    block_store<NKF>(v, a.kf_part, a.n_fin_blk);
+}
+
+// Forces of 64 atoms of one replica.
+template <int KS>
+__global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<double>) void k_rows_force(Args a) {
+    extern __shared__ double lds[];
+    const int2 bm = a.kf_blk[blockIdx.x];
+    const Rep rp = a.rep[bm.x];
+    const KsRows kr = rep_rows(a, rp, a.st[bm.x].nrows);
+    const BatchPhases at{a.e1};
+    const double g = ks_force<double, KS>(kr, at, a.coef + rp.cbase, bm.y, rp.a1, lds);
+    __syncthreads();
+    if (threadIdx.x < 3 * KS_TILE) lds[threadIdx.x] = g;
+    __syncthreads();
+    const int i = bm.y + (int)threadIdx.x / 3, d = threadIdx.x % 3;
+    if (threadIdx.x < 3 * KS_TILE && i < rp.a1) {
+        // k_y = (k - h t / L) 2 pi / L
+        const double f = d == 1 ? g - a.st[bm.x].tilt * rp.invL * lds[threadIdx.x - 1] : g;
+        a.frec[3 * i + d] = a.p.q[i % 3] * (2.0 * PI * rp.invL) * f;
+    }
+}
+
 // ---- SHAKE with SLLOD, kinetics, rewrap, and the replica's epilogue -------
 
 // One thread per molecule.  vtMinus loses the drift the previous epilogue
@@ -885,6 +1083,9 @@ struct smd_batch {
     int32_t *d_nb = nullptr, *d_nb_cnt = nullptr;
     double4* d_kvec = nullptr;
     double2* d_kf = nullptr;
+    int32_t* d_rowxy = nullptr;
+    double *d_rowexp = nullptr, *d_coef = nullptr;
+    double2* d_e1 = nullptr;
     double *d_sf_part = nullptr, *d_pair_part = nullptr, *d_kf_part = nullptr, *d_sh_part = nullptr;
     size_t sf_part_cap = 0, pair_part_cap = 0;
     int2 *d_pair_blk = nullptr, *d_fin_blk = nullptr, *d_kf_blk = nullptr, *d_sh_blk = nullptr;
@@ -893,6 +1094,9 @@ struct smd_batch {
     size_t pair_blk_cap = 0, sf_blk_cap = 0;
     int n_pair_blk = 0, n_sf_blk = 0, n_fin_blk = 0, n_kf_blk = 0, n_sh_blk = 0, n_list_blk = 0;
     int ktot = 0;
+    size_t rows_lds[2] = {0, 0};   // dynamic LDS of the row passes: factors, forces
+    int rows_waves[2] = {3, 3};    // and their waves per block
+    int rows_steps = 0;
     hipGraphExec_t graph = nullptr;
     bool have_state = false, started = false;
 };
@@ -943,6 +1147,7 @@ static int build_tables(smd_batch* b) {
     std::vector<int2> pair_blk, fin_blk, kf_blk, sh_blk, list_blk;
     std::vector<int4> sf_blk;
     int64_t pbase = 0;
+    b->rows_lds[0] = 0;
     for (int r = 0; r < b->R; ++r) {
         Rep& rp = b->rep[r];
         const int na = rp.a1 - rp.a0;
@@ -951,14 +1156,24 @@ static int build_tables(smd_batch* b) {
         rp.pb1 = (int)pair_blk.size();
         rp.nch = (na + CH - 1) / CH;
         rp.pbase = pbase;
-        pbase += 2 * (int64_t)rp.nch * rp.kcap;
-        const int kt = (rp.kcap + 255) / 256;
+        const bool rows = b->prm.rows_on;
+        if (rows) {
+            KsRows kr{};
+            kr.nx1 = rp.hmax + 1;
+            kr.ny1 = rp.nyb + 1;
+            kr.n1 = rp.nzmax + 1;
+            kr.ts = ks_stride<double>();
+            b->rows_lds[0] = std::max(b->rows_lds[0], ks_table_bytes<double>(kr, 1) * ks_tables<double>(kr, 1, CH / KS_TILE));
+        }
+        pbase += rows ? (int64_t)rp.nch * rp.rcap * 4 * (rp.nzmax + 1) : 2 * (int64_t)rp.nch * rp.kcap;
+        const int kt = rows ? 1 : (rp.kcap + 255) / 256;
+        const int ft = rows ? rp.rcap / (256 / WAVE) : kt;
         for (int t = 0; t < kt; ++t)
             for (int c = 0; c < rp.nch; ++c) sf_blk.push_back(make_int4(r, t, c, 0));
         rp.fb0 = (int)fin_blk.size();
-        for (int t = 0; t < kt; ++t) fin_blk.push_back(make_int2(r, t));
+        for (int t = 0; t < ft; ++t) fin_blk.push_back(make_int2(r, t));
         rp.fb1 = (int)fin_blk.size();
-        for (int i = rp.a0; i < rp.a1; i += 256) kf_blk.push_back(make_int2(r, i));
+        for (int i = rp.a0; i < rp.a1; i += rows ? KS_TILE : 256) kf_blk.push_back(make_int2(r, i));
         rp.sb0 = (int)sh_blk.size();
         for (int m = rp.m0; m < rp.m1; m += KIN_BLOCK) sh_blk.push_back(make_int2(r, m));
         rp.sb1 = (int)sh_blk.size();
@@ -1014,6 +1229,7 @@ static Args make_args(smd_batch* b) {
     a.fpair = b->d_fpair; a.frec = b->d_frec; a.com = b->d_com; a.mom = b->d_mom;
     a.nb = b->d_nb; a.nb_cnt = b->d_nb_cnt;
     a.kvec = b->d_kvec; a.kf = b->d_kf;
+    a.rowxy = b->d_rowxy; a.rowexp = b->d_rowexp; a.coef = b->d_coef; a.e1 = b->d_e1;
     a.sf_part = b->d_sf_part; a.pair_part = b->d_pair_part; a.kf_part = b->d_kf_part; a.sh_part = b->d_sh_part;
     a.pair_blk = b->d_pair_blk; a.sf_blk = b->d_sf_blk; a.fin_blk = b->d_fin_blk; a.kf_blk = b->d_kf_blk;
     a.sh_blk = b->d_sh_blk;
@@ -1038,6 +1254,22 @@ static void launch_pairs(hipStream_t s, const Args& a, int G, int nblk) {
 
 enum Pass : unsigned { P_BEGIN = 1, P_LIST = 2, P_PAIRS = 4, P_SFAC = 8, P_KFIN = 16, P_KFORCE = 32 };
 
+// Inner steps in registers when every replica has the same number of them.
+static void launch_rows_force(smd_batch* b, hipStream_t s, const Args& a) {
+    const dim3 g(b->n_kf_blk), t(b->rows_waves[1] * WAVE);
+    const size_t lds = b->rows_lds[1];
+    switch (b->rows_steps) {
+    case 2: hipLaunchKernelGGL(k_rows_force<2>, g, t, lds, s, a); break;
+    case 3: hipLaunchKernelGGL(k_rows_force<3>, g, t, lds, s, a); break;
+    case 4: hipLaunchKernelGGL(k_rows_force<4>, g, t, lds, s, a); break;
+    case 5: hipLaunchKernelGGL(k_rows_force<5>, g, t, lds, s, a); break;
+    case 6: hipLaunchKernelGGL(k_rows_force<6>, g, t, lds, s, a); break;
+    case 7: hipLaunchKernelGGL(k_rows_force<7>, g, t, lds, s, a); break;
+    case 8: hipLaunchKernelGGL(k_rows_force<8>, g, t, lds, s, a); break;
+    default: hipLaunchKernelGGL(k_rows_force<0>, g, t, lds, s, a); break;
+    }
+}
+
 static void launch_pass(smd_batch* b, hipStream_t s, const Args& a, unsigned pass) {
     const bool mixed = b->prec == SMD_PREC_MIXED;
     switch (pass) {
@@ -1048,13 +1280,24 @@ static void launch_pass(smd_batch* b, hipStream_t s, const Args& a, unsigned pas
         else launch_pairs<double>(s, a, b->tiles.pair_lanes, b->n_pair_blk);
         break;
     case P_SFAC: {
+        if (b->prm.rows_on) {
+            hipLaunchKernelGGL(k_rows_sfac, dim3(b->n_sf_blk), dim3(b->rows_waves[0] * WAVE), b->rows_lds[0], s, a);
+            break;
+        }
         const size_t lds = sizeof(double4) * b->tiles.sfac_chunk;
         if (mixed) hipLaunchKernelGGL(k_sfac<float>, dim3(b->n_sf_blk), dim3(SF_THREADS), lds, s, a);
         else hipLaunchKernelGGL(k_sfac<double>, dim3(b->n_sf_blk), dim3(SF_THREADS), lds, s, a);
         break;
     }
-    case P_KFIN: hipLaunchKernelGGL(k_kfin, dim3(b->n_fin_blk), dim3(256), 0, s, a); break;
+    case P_KFIN:
+        if (b->prm.rows_on) hipLaunchKernelGGL(k_rows_fin, dim3(b->n_fin_blk), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(k_kfin, dim3(b->n_fin_blk), dim3(256), 0, s, a);
+        break;
     case P_KFORCE: {
+        if (b->prm.rows_on) {
+            launch_rows_force(b, s, a);
+            break;
+        }
         const int tile = b->tiles.kforce_tile;
         const size_t lds = sizeof(double) * 5 * tile;
         if (mixed) hipLaunchKernelGGL(k_kforce<float>, dim3(b->n_kf_blk), dim3(256), lds, s, a, tile);
@@ -1145,7 +1388,11 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
     b->R = p->n_replicas;
     b->prec = p->prec;
     const double rl = p->cutoff + p->cut_buff;
-    int a = 0, m = 0, kb = 0;
+    int a = 0, m = 0, kb = 0, rb = 0;
+    int64_t eb = 0, cb = 0;
+    // rows where a table of every replica's powers fits the LDS a launch takes
+    // without asking (about 19 waves along the edge), else the direct passes
+    bool rows_ok = true;
     double dens = 0.0;
     for (int r = 0; r < b->R; ++r) {
         const int nmr = p->n_mols[r];
@@ -1169,6 +1416,27 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
         rp.kcap = ((int)(half * 1.15 + 4.0 * PI * nR * nR * 0.5) + 64 + 63) / 64 * 64;
         rp.kbase = kb;
         kb += rp.kcap;
+        // rows: lattice points of half the disk of radius nR, with room for its rim
+        rp.rcap = ((int)(0.5 * PI * nR * nR * 1.15 + 4.0 * nR) + 16 + 15) / 16 * 16;
+        KsRows kr{};
+        kr.nrows = rp.rcap;
+        kr.nx1 = rp.hmax + 1;
+        kr.ny1 = rp.nyb + 1;
+        kr.n1 = rp.nzmax + 1;
+        kr.ts = ks_stride<double>();
+        rp.rowbase = rb;
+        rp.ebase = eb;
+        rp.cbase = cb;
+        rb += rp.rcap;
+        eb += (int64_t)rp.rcap * kr.n1;
+        cb += (int64_t)kr.coef_entries();
+        rows_ok = rows_ok && ks_table_bytes<double>(kr, 1) <= 65536 && kr.n1 <= WAVE;
+        // block shapes for the row tiles of an unsheared cell (half the disk)
+        const int tiles = ((int)(0.5 * PI * nR * nR + nR) + KS_ROWS) / KS_ROWS;
+        b->rows_waves[0] = std::max(b->rows_waves[0], ks_waves(tiles, KS_VT, KS_MAXW, 3));
+        b->rows_waves[1] = std::max(b->rows_waves[1], ks_waves(tiles, 1, KS_MAXW, 3));
+        b->rows_lds[1] = std::max(b->rows_lds[1], ks_force_lds<double>(kr, KS_MAXW));
+        b->rows_steps = r == 0 || b->rows_steps == kr.steps() ? kr.steps() : 0;
         rp.e_self = -(double)nmr * (2 * p->q_h * p->q_h + p->q_o * p->q_o) * p->alpha / SQRT_PI;
         b->rep.push_back(rp);
         b->nm.push_back(nmr);
@@ -1195,6 +1463,7 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
     q.max_count = p->max_count;
     q.nose_hoover = p->nose_hoover;
     q.n = a;
+    q.rows_on = rows_ok ? 1 : 0;
     int cap = p->nb_cap;
     if (cap <= 0) cap = (int)(dens * (4.0 / 3.0) * PI * rl * rl * rl * 1.35) + 64;
     q.nb_cap = (cap + 63) / 64 * 64;
@@ -1211,8 +1480,12 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
         (rc = dalloc(b, b->d_vtm, n3)) || (rc = dalloc(b, b->d_vel, n3)) || (rc = dalloc(b, b->d_disp, n3)) ||
         (rc = dalloc(b, b->d_fpair, n3)) || (rc = dalloc(b, b->d_frec, n3)) || (rc = dalloc(b, b->d_com, 3 * (size_t)m)) ||
         (rc = dalloc(b, b->d_mom, 3 * (size_t)m)) || (rc = dalloc(b, b->d_nb, (size_t)a * q.nb_cap)) ||
-        (rc = dalloc(b, b->d_nb_cnt, a)) || (rc = dalloc(b, b->d_kvec, kb)) || (rc = dalloc(b, b->d_kf, kb)))
+        (rc = dalloc(b, b->d_nb_cnt, a)))
         return rc;
+    if (rows_ok) rc = dalloc(b, b->d_rowxy, rb) || dalloc(b, b->d_rowexp, eb) || dalloc(b, b->d_coef, cb) ||
+                      dalloc(b, b->d_e1, n3) ? SMD_ENOMEM : SMD_OK;
+    else rc = dalloc(b, b->d_kvec, kb) || dalloc(b, b->d_kf, kb) ? SMD_ENOMEM : SMD_OK;
+    if (rc) return rc;
     BHIP(b, hipMemset(b->d_err, 0, sizeof(unsigned)));
     BHIP(b, hipMemset(b->d_out, 0, sizeof(smd_batch_report) * b->R));
     BHIP(b, hipMemset(b->d_nb_cnt, 0, sizeof(int32_t) * a));
@@ -1226,6 +1499,7 @@ extern "C" void smd_batch_destroy(smd_batch* b) {
     drop_graph(b);
     void* ptrs[] = {b->d_rep, b->d_st, b->d_out, b->d_err, b->d_pos, b->d_vtm, b->d_vel, b->d_disp,
                     b->d_fpair, b->d_frec, b->d_com, b->d_mom, b->d_nb, b->d_nb_cnt, b->d_kvec, b->d_kf,
+                    b->d_rowxy, b->d_rowexp, b->d_coef, b->d_e1,
                     b->d_sf_part, b->d_pair_part, b->d_kf_part, b->d_sh_part, b->d_pair_blk, b->d_fin_blk,
                     b->d_kf_blk, b->d_sh_blk, b->d_sf_blk, b->d_list_blk};
     for (void* p : ptrs)

@@ -85,3 +85,32 @@ def test_reciprocal_space_shapes_match_the_oracle(n, edges, waves, mixed):
     for k in ("energy", "deriv", "deriv2"):
         assert abs(out[k] - eo[k]) <= tol * max(abs(eo[k]), abs(eo["energy"])), k
     assert rel_rms(out["virial"], eo["virial"]) <= tol
+
+
+# cutoffs of one k-row and up, the last that the row passes' LDS takes (16
+# waves along the edge), the direct passes past it, and two replicas whose
+# rows differ in their number of functions
+@pytest.mark.parametrize("n2", [(1,), (20, 81), (256,), (306,)])
+def test_sheared_reciprocal_space_matches_the_oracle(n2):
+    """Two steps at a tilt: forces and energies 1e-8, the same k count."""
+    from oracle import oracle as O
+    from swinmd_amd.nemd import ShearBatch
+    systems = [S.water(n, density_mol=RHO, seed=n, subset=True) for n in (256, 275)[:len(n2)]]
+    kcut = [S.kcut_for(k, s.box[0]) for k, s in zip(n2, systems)]
+    gam, tilt = [3.0, -2.0][:len(n2)], [0.31, -0.2][:len(n2)]
+    vels = [O.Oracle(s).init_velocity(300.0, 5, per_atom=False, ndf=3 * s.n_mols - 3) for s in systems]
+    print(f"case shear n2={n2}", flush=True)
+    b = ShearBatch(systems, gam, cutoff=0.8, cut_buff=0.08, alpha=3.5, kcut=kcut, dt=0.002, temperature=300.0,
+                   coupl=0.1)
+    b.set_state([s.pos for s in systems], vels, tilt)
+    b.start()
+    b.run(2)
+    st, rep = b.state(), b.reports()
+    for r, s in enumerate(systems):
+        want = O.sllod_run(O.Oracle(s), dict(cutoff=0.8, cut_buff=0.08, alpha=3.5, kcut=kcut[r], dt=0.002,
+                                             temperature=300.0, coupl=0.1), gam[r], 2, velocity=vels[r], tilt=tilt[r])
+        assert rep[r]["n_kvec"] == want["K"]
+        assert rel(rep[r]["e_long"], want["e_long"]) <= 1e-8
+        assert rel_rms(b.split(st["force"])[r], want["force"]) <= 1e-8
+        assert rel_rms(b.split(st["pos"])[r], want["pos"]) <= 1e-10
+        assert np.max(np.abs(rep[r]["virial"] - want["virial"])) <= 1e-7 * np.max(np.abs(want["virial"]))

@@ -599,14 +599,16 @@ int smd_md_time_family(smd_ctx* ctx, const char* family, int reps, double* avg_u
  * the joint pass).
  * "md_fused_shake" (0/1, default 1): the MD step runs SHAKE and the kinetic
  * and pressure sums as one kernel (0: two kernels).
- * "cg_lanes" (8, 16 or 32, default 16): lanes sharing one row of the CG's A v.
+ * "cg_lanes" (8, 16 or 32; by size if not set): lanes sharing one row of the
+ * CG's A v.
  * "cg_graph" (0/1, default 1): smd_induce replays each batch of CG
  * iterations from a captured hipGraph (0: direct launches, for profilers).
  * "cg_batch" (1..64, default 16): CG iterations per batch, i.e. between the
  * host's checks of the stop flag.
  * "pair_lanes": lanes sharing one atom's row
  * in the pair kernels (both the packed mixed kernel and the general one),
- * 4, 8, 16, 32 or 64, or 0 (default: 16 for FP32 pair math, 32 for FP64).
+ * 4, 8, 16, 32 or 64, or 0 (default: by size, from 16 for FP32 pair math and
+ * 32 for FP64).
  * Drops a captured MD
  * graph.  SMD_EINVAL for an unknown name or value. */
 int smd_set_tuning(smd_ctx* ctx, const char* name, int value);

@@ -9,8 +9,8 @@ forms against each other:
                   kernels (1) or on the step's stream (0);
   md_fused_shake  SHAKE and the kinetic and pressure sums as one kernel (1)
                   or two (0);
-  pair_lanes      lanes per atom row of the pair kernel (0: 16 for the
-                  mixed form, 32 for FP64).
+  pair_lanes      lanes per atom row of the pair kernel (0: by size, from 16
+                  for the mixed form and 32 for FP64).
 The tuner times the step under every combination on the live system, for
 its size, cutoff and k-set on this GPU, and keeps the fastest.  The
 trajectory runs on while it measures, so a few hundred steps of the run are

@@ -30,7 +30,6 @@
 
 namespace smd {
 
-constexpr int IND_LANES = 16;      // lanes per atom row in the field and T.mu kernels
 constexpr int CG_THREADS = 256;    // threads per block of the vector kernels
 constexpr int BLK_MOLS = 64;       // molecules per block of the block preconditioner's vector kernels
 constexpr int BLK_THREADS = 9 * BLK_MOLS;   // a thread per dipole component (nine waves)
@@ -738,18 +737,17 @@ __global__ __launch_bounds__(256) void k_apply_pos32(IndArgs a, const float4* __
 // k_apply_table with `lanes` lanes per row (8, 16 or 32).
 static void launch_apply(Ctx* c, int lanes, const IndArgs& a, const double* v, double* out, const double* dotv,
                          double* part, CgTop top) {
-    const dim3 grid((unsigned)(((int64_t)c->n * lanes + 255) / 256)), b256(256);
-    if (lanes == 8) hipLaunchKernelGGL((k_apply_table<8>), grid, b256, 0, c->stream, a, v, out, dotv, part, top);
-    else if (lanes == 32) hipLaunchKernelGGL((k_apply_table<32>), grid, b256, 0, c->stream, a, v, out, dotv, part, top);
-    else hipLaunchKernelGGL((k_apply_table<16>), grid, b256, 0, c->stream, a, v, out, dotv, part, top);
+    const dim3 grid((unsigned)(((int64_t)c->n * lanes + 255) / 256));
+    with_lanes(lanes, [&](auto g) {
+        hipLaunchKernelGGL((k_apply_table<decltype(g)::value>), grid, dim3(256), 0, c->stream, a, v, out, dotv, part, top);
+    });
 }
-
 static void launch_apply32(Ctx* c, int lanes, const IndArgs& a, const float4* v32, const double* v, double* out,
                            double* part, CgTop top) {
-    const dim3 grid((unsigned)(((int64_t)c->n * lanes + 255) / 256)), b256(256);
-    if (lanes == 8) hipLaunchKernelGGL((k_apply_pos32<8>), grid, b256, 0, c->stream, a, v32, v, out, part, top);
-    else if (lanes == 32) hipLaunchKernelGGL((k_apply_pos32<32>), grid, b256, 0, c->stream, a, v32, v, out, part, top);
-    else hipLaunchKernelGGL((k_apply_pos32<16>), grid, b256, 0, c->stream, a, v32, v, out, part, top);
+    const dim3 grid((unsigned)(((int64_t)c->n * lanes + 255) / 256));
+    with_lanes(lanes, [&](auto g) {
+        hipLaunchKernelGGL((k_apply_pos32<decltype(g)::value>), grid, dim3(256), 0, c->stream, a, v32, v, out, part, top);
+    });
 }
 
 // ---- CG -------------------------------------------------------------------------
@@ -1299,10 +1297,13 @@ int frames_run(Ctx* c) {
 int induce_direct_apply(Ctx* c, const smd_induce_params* p, double* x, double* z) {
     IndArgs a = ind_args(c, p);
     const int dim = 3 * c->n;
-    const dim3 grid_rows((unsigned)(((int64_t)c->n * IND_LANES + 255) / 256));
+    const int lanes = row_lanes(c->n);
+    const dim3 grid_rows((unsigned)(((int64_t)c->n * lanes + 255) / 256));
     hipLaunchKernelGGL(k_direct, dim3((dim + 255) / 256), dim3(256), 0, c->stream, dim, c->d_polar, c->d_e0, x,
                        (float*)nullptr);
-    hipLaunchKernelGGL((k_apply_a<IND_LANES>), grid_rows, dim3(256), 0, c->stream, a, x, z);
+    with_lanes(lanes, [&](auto g) {
+        hipLaunchKernelGGL((k_apply_a<decltype(g)::value>), grid_rows, dim3(256), 0, c->stream, a, x, z);
+    });
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
@@ -1340,7 +1341,7 @@ static CgArgs cg_args(Ctx* c, const smd_induce_params* p) {
     g.hdone = c->d_cg_done;
     g.e0 = c->d_e0;
     g.polar = c->d_polar;
-    g.nparts_mv = (int)(((int64_t)n * c->cg_lanes + 255) / 256);   // blocks of the A v kernel
+    g.nparts_mv = (int)(((int64_t)n * cg_lanes(c) + 255) / 256);   // blocks of the A v kernel
     g.nmol = c->nmol;
     g.blk = p->precond == 2 ? c->d_pc_blk : nullptr;
     g.nparts_vec = p->precond == 2 ? (c->nmol + BLK_MOLS - 1) / BLK_MOLS : (dim + CG_THREADS - 1) / CG_THREADS;
@@ -1368,8 +1369,8 @@ static CgTop blk_top(const CgArgs& g) {
 // A v of the solve in its precision; v32 is v's FP32 copy (mixed).
 static void solve_apply(Ctx* c, const smd_induce_params* p, const IndArgs& a, const double* v, const float4* v32,
                         double* out, double* part, CgTop top) {
-    if (p->prec == SMD_PREC_MIXED) launch_apply32(c, c->cg_lanes, a, v32, v, out, part, top);
-    else launch_apply(c, c->cg_lanes, a, v, out, part ? v : nullptr, part, top);
+    if (p->prec == SMD_PREC_MIXED) launch_apply32(c, cg_lanes(c), a, v32, v, out, part, top);
+    else launch_apply(c, cg_lanes(c), a, v, out, part ? v : nullptr, part, top);
 }
 
 // Enqueues everything of a solve up to the first CG iteration: frames (when
@@ -1389,7 +1390,8 @@ int induce_field(Ctx* c, const smd_induce_params* p, bool frames) {
     IndArgs a = ind_args(c, p);
     const int n = c->n, dim = 3 * n;
     const dim3 b256(256);
-    const dim3 grid_rows((unsigned)(((int64_t)n * IND_LANES + 255) / 256));
+    const int lanes = row_lanes(n);
+    const dim3 grid_rows((unsigned)(((int64_t)n * lanes + 255) / 256));
     const dim3 grid_vec((dim + CG_THREADS - 1) / CG_THREADS);
     {
         ProfScope ps(c, "ind_field");
@@ -1398,11 +1400,16 @@ int induce_field(Ctx* c, const smd_induce_params* p, bool frames) {
             hipLaunchKernelGGL(k_pack_ind32, dim3((n + 255) / 256), b256, 0, c->stream, a);
             // the learned guess's charge shells come out of the same pass
             float* shells = p->guess == 3 ? c->d_shell32 : nullptr;
-            hipLaunchKernelGGL((k_field_table32<IND_LANES>), grid_rows, b256, 0, c->stream, a, shells);
+            with_lanes(lanes, [&](auto g) {
+                hipLaunchKernelGGL((k_field_table32<decltype(g)::value>), grid_rows, b256, 0, c->stream, a, shells);
+            });
             c->ind_shells_valid = shells != nullptr;
         } else {
-            hipLaunchKernelGGL((k_field<IND_LANES>), grid_rows, b256, 0, c->stream, a);
-            if (p->do_min) hipLaunchKernelGGL((k_ind_table<IND_LANES>), grid_rows, b256, 0, c->stream, a);
+            with_lanes(lanes, [&](auto g) {
+                hipLaunchKernelGGL((k_field<decltype(g)::value>), grid_rows, b256, 0, c->stream, a);
+                if (p->do_min)
+                    hipLaunchKernelGGL((k_ind_table<decltype(g)::value>), grid_rows, b256, 0, c->stream, a);
+            });
         }
     }
     SMD_HIP(c, hipGetLastError());
@@ -1485,7 +1492,7 @@ static void cg_iterations(Ctx* c, const smd_induce_params* p, const IndArgs& a, 
                 hipLaunchKernelGGL(k_pcg_dir<0>, grid_vec, bt, 0, c->stream, g);
             }
         } else {
-            launch_apply(c, c->cg_lanes, a, g.v, g.z, g.v, g.p_vz, CgTop{g.state, g.p_dv, g.nparts_vec, g.tol});
+            launch_apply(c, cg_lanes(c), a, g.v, g.z, g.v, g.p_vz, CgTop{g.state, g.p_dv, g.nparts_vec, g.tol});
             if (k & 1) {
                 hipLaunchKernelGGL(k_cg_step<1>, grid_vec, bt, 0, c->stream, g);
                 hipLaunchKernelGGL(k_cg_dir<1>, grid_vec, bt, 0, c->stream, g);
@@ -1510,7 +1517,8 @@ int induce_batches(Ctx* c, const smd_induce_params* p, int batches) {
     }
     std::string key;
     auto put = [&key](const void* q, size_t bytes) { key.append(static_cast<const char*>(q), bytes); };
-    put(&c->cg_lanes, sizeof c->cg_lanes);
+    const int lanes = cg_lanes(c);
+    put(&lanes, sizeof lanes);
     put(&c->cg_batch, sizeof c->cg_batch);
     put(&p->precond, sizeof p->precond);
     put(&p->prec, sizeof p->prec);
@@ -1617,8 +1625,8 @@ extern "C" int smd_induce_time_apply(smd_ctx* c, int reps, double* avg_us) {
     SMD_HIP(c, hipEventCreate(&e1));
     SMD_HIP(c, hipEventRecord(e0, c->stream));
     for (int k = 0; k < reps; ++k) {
-        if (mixed) launch_apply32(c, c->cg_lanes, a, c->d_cg32, c->d_mu, z, nullptr, CgTop{nullptr, nullptr, 0, 0.0});
-        else launch_apply(c, c->cg_lanes, a, c->d_mu, z, nullptr, nullptr, CgTop{nullptr, nullptr, 0, 0.0});
+        if (mixed) launch_apply32(c, cg_lanes(c), a, c->d_cg32, c->d_mu, z, nullptr, CgTop{nullptr, nullptr, 0, 0.0});
+        else launch_apply(c, cg_lanes(c), a, c->d_mu, z, nullptr, nullptr, CgTop{nullptr, nullptr, 0, 0.0});
     }
     SMD_HIP(c, hipEventRecord(e1, c->stream));
     SMD_HIP(c, hipEventSynchronize(e1));
@@ -1637,7 +1645,7 @@ extern "C" int smd_set_multipoles(smd_ctx* c, const double* dip_local, const dou
     if (n_atoms != c->n) return fail(c, SMD_EINVAL, "count %lld != %d", (long long)n_atoms, c->n);
     const int n = c->n;
     if (!c->d_dipl) {
-        const int parts = std::max((int)(((int64_t)n * 32 + 255) / 256), (3 * n + CG_THREADS - 1) / CG_THREADS);   // up to 32 lanes per row
+        const int parts = std::max((int)(((int64_t)n * 64 + 255) / 256), (3 * n + CG_THREADS - 1) / CG_THREADS);   // up to 64 lanes per row
         auto A = [&](auto*& p, size_t bytes) -> int {
             if (hipMalloc(&p, bytes) != hipSuccess) return fail(c, SMD_ENOMEM, "induction allocation of %zu bytes", bytes);
             return SMD_OK;

@@ -38,7 +38,6 @@ namespace smd {
 
 constexpr double COULOMBS = 138.93548501;      // COUlOMBS, src/NEMD_defs.h:104
 constexpr double SQRT_COULOMB_MP = 11.78708976;
-constexpr int MP_LANES = 16;                   // lanes per atom row in real space
 constexpr int MP_NSUM = 20;                    // structure-factor sums per k
 constexpr int MP_SF_THREADS = 256;             // k per block of the structure-factor pass
 constexpr int MP_RF_THREADS = 256;             // atoms per block of the force pass
@@ -391,22 +390,33 @@ __global__ __launch_bounds__(256) void k_pack_sites32(MpArgs a, float4* __restri
                                                       float4* __restrict__ pind32, int with_pind);
 
 // Real-space kernels in the context's precision for these classes (FP64, or
-// FP32 pair math from packed records with FP64 accumulation); the mixed form
-// first packs the records (and, for induction, the induced dipoles).
+// FP32 pair math from packed records with FP64 accumulation; packed by
+// pack_sites), over the coupling table where the arguments carry it.  Gives
+// the grid's blocks.
+static unsigned real_kernel(Ctx* c, const MpArgs& a, bool induction) {
+    const int lanes = row_lanes(c->n);
+    const dim3 gr((unsigned)(((int64_t)c->n * lanes + 255) / 256)), b256(256);
+    with_lanes(lanes, [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        if (c->mp_prec == SMD_PREC_MIXED) {
+            if (induction && a.tj) hipLaunchKernelGGL((k_ind_real_tab<G>), gr, b256, 0, c->stream, a);
+            else if (induction) hipLaunchKernelGGL((k_ind_real<G, float>), gr, b256, 0, c->stream, a);
+            else if (a.tj) hipLaunchKernelGGL((k_mp_real_tab<G>), gr, b256, 0, c->stream, a);
+            else hipLaunchKernelGGL((k_mp_real<G, float>), gr, b256, 0, c->stream, a);
+        } else {
+            if (induction) hipLaunchKernelGGL((k_ind_real<G, double>), gr, b256, 0, c->stream, a);
+            else hipLaunchKernelGGL((k_mp_real<G, double>), gr, b256, 0, c->stream, a);
+        }
+    });
+    return gr.x;
+}
+
 static int launch_real(Ctx* c, const MpArgs& a, bool induction) {
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256)), b256(256);
-    if (c->mp_prec == SMD_PREC_MIXED) {
-        hipLaunchKernelGGL(k_pack_sites32, dim3((c->n + 255) / 256), b256, 0, c->stream, a, c->d_site32, c->d_pind32,
-                           induction ? 1 : 0);
-        if (induction && a.tj) hipLaunchKernelGGL((k_ind_real_tab<MP_LANES>), gr, b256, 0, c->stream, a);
-        else if (induction) hipLaunchKernelGGL((k_ind_real<MP_LANES, float>), gr, b256, 0, c->stream, a);
-        else if (a.tj) hipLaunchKernelGGL((k_mp_real_tab<MP_LANES>), gr, b256, 0, c->stream, a);
-        else hipLaunchKernelGGL((k_mp_real<MP_LANES, float>), gr, b256, 0, c->stream, a);
-    } else {
-        if (induction) hipLaunchKernelGGL((k_ind_real<MP_LANES, double>), gr, b256, 0, c->stream, a);
-        else hipLaunchKernelGGL((k_mp_real<MP_LANES, double>), gr, b256, 0, c->stream, a);
-    }
-    return red_finish(c, induction ? RS_IND_REAL : RS_MP_REAL, gr.x, 11, a.terms + M_REAL_E);
+    if (c->mp_prec == SMD_PREC_MIXED)
+        hipLaunchKernelGGL(k_pack_sites32, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, a, c->d_site32,
+                           c->d_pind32, induction ? 1 : 0);
+    const unsigned nb = real_kernel(c, a, induction);
+    return red_finish(c, induction ? RS_IND_REAL : RS_MP_REAL, nb, 11, a.terms + M_REAL_E);
 }
 
 __global__ __launch_bounds__(256) void k_mp_torques(MpArgs a, unsigned parts, int site);
@@ -950,7 +960,6 @@ int multipole_short(Ctx* c, smd_mp_out* out) {
     MpArgs a = mp_args(c);
     const dim3 b256(256);
     const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256));
     ProfScope ps(c, "mp_short");
     SMD_HIP(c, hipMemsetAsync(c->d_mp_terms, 0, sizeof(double) * M_COUNT, c->stream));
     if ((rc = frames_run(c))) return rc;
@@ -1910,7 +1919,6 @@ int induction_short(Ctx* c, smd_indf_out* out) {
     MpArgs a = ind_args(c);
     const dim3 b256(256);
     const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256));
     ProfScope ps(c, "ind_short");
     SMD_HIP(c, hipMemsetAsync(c->d_mp_terms, 0, sizeof(double) * M_COUNT, c->stream));
     if ((rc = frames_run(c))) return rc;
@@ -2094,7 +2102,6 @@ int multipole_enqueue(Ctx* c, double* terms) {
     a.terms = terms;
     const dim3 b256(256);
     const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256));
     hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, terms);
     // the k-space sums and per-site partial forces on the second stream,
     // beside the real-space kernels (they touch none of the same buffers)
@@ -2120,7 +2127,6 @@ int induction_enqueue(Ctx* c, double* terms) {
     a.terms = terms;
     const dim3 b256(256);
     const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256));
     hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, terms);
     const bool fork = polar_fork_begin(c);
     int rc_long = fork ? mp_long_sums(c, a, false) : SMD_OK;
@@ -2353,25 +2359,14 @@ extern "C" int smd_polar_time_kernel(smd_ctx* c, const char* name, int reps, dou
         a.tj = c->d_it_j;
         a.tstride = c->it_stride;
     }
-    const dim3 gr((unsigned)(((int64_t)c->n * MP_LANES + 255) / 256)), b256(256);
-    const bool mixed = c->mp_prec == SMD_PREC_MIXED;
-    if (mixed)
-        hipLaunchKernelGGL(k_pack_sites32, dim3((c->n + 255) / 256), b256, 0, c->stream, a, c->d_site32, c->d_pind32, 1);
+    if (c->mp_prec == SMD_PREC_MIXED)
+        hipLaunchKernelGGL(k_pack_sites32, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, a, c->d_site32,
+                           c->d_pind32, 1);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SMD_HIP(c, hipEventCreate(&e0));
     SMD_HIP(c, hipEventCreate(&e1));
     SMD_HIP(c, hipEventRecord(e0, c->stream));
-    for (int r = 0; r < reps; ++r) {
-        if (ind) {
-            if (tab) hipLaunchKernelGGL((k_ind_real_tab<MP_LANES>), gr, b256, 0, c->stream, a);
-            else if (mixed) hipLaunchKernelGGL((k_ind_real<MP_LANES, float>), gr, b256, 0, c->stream, a);
-            else hipLaunchKernelGGL((k_ind_real<MP_LANES, double>), gr, b256, 0, c->stream, a);
-        } else {
-            if (tab) hipLaunchKernelGGL((k_mp_real_tab<MP_LANES>), gr, b256, 0, c->stream, a);
-            else if (mixed) hipLaunchKernelGGL((k_mp_real<MP_LANES, float>), gr, b256, 0, c->stream, a);
-            else hipLaunchKernelGGL((k_mp_real<MP_LANES, double>), gr, b256, 0, c->stream, a);
-        }
-    }
+    for (int r = 0; r < reps; ++r) (void)real_kernel(c, a, ind);
     SMD_HIP(c, hipEventRecord(e1, c->stream));
     SMD_HIP(c, hipEventSynchronize(e1));
     float ms = 0.f;

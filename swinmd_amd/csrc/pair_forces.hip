@@ -502,6 +502,12 @@ __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
 
 // ---------------------------------------------------------------------------
 
+// Lanes per atom row: the set ones, or by size (row_lanes), from 32 for FP64
+// pair math (measured best on the 12,288-atom water list).
+static int pair_row_lanes(const Ctx* c, int prec) {
+    return c->pair_lanes ? c->pair_lanes : std::max(prec == SMD_PREC_MIXED ? 16 : 32, row_lanes(c->n));
+}
+
 template <int VDW, bool EWALD, int G>
 static void launch_pairs_g(Ctx* c, const PairArgs& a, int prec, int lustig) {
     const int threads = 256;
@@ -519,9 +525,7 @@ static void launch_pairs_g(Ctx* c, const PairArgs& a, int prec, int lustig) {
 template <int VDW, bool EWALD>
 static hipError_t launch_pairs(Ctx* c, const PairArgs& a, int prec, int lustig) {
     ProfScope ps(c, "pairs");
-    // measured best on the 12,288-atom water list: 16 lanes for FP32 pair
-    // math, 32 for FP64
-    const int lanes = c->pair_lanes ? c->pair_lanes : (prec == SMD_PREC_MIXED ? 16 : 32);
+    const int lanes = pair_row_lanes(c, prec);
     switch (lanes) {
         case 4: launch_pairs_g<VDW, EWALD, 4>(c, a, prec, lustig); break;
         case 8: launch_pairs_g<VDW, EWALD, 8>(c, a, prec, lustig); break;
@@ -1093,8 +1097,7 @@ static int pairs_packed(Ctx* c, const PairArgs& pa, int lustig) {
     if (!c->pack_reuse)
         hipLaunchKernelGGL(k_pack_sites, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->d_pos, c->d_q,
                            c->d_type, c->d_mol, c->d_com, c->box, rec, tm, off);
-    const int pl = c->pair_lanes;
-    const int lanes = pl == 4 || pl == 8 || pl == 32 || pl == 64 ? pl : 16;
+    const int lanes = pair_row_lanes(c, SMD_PREC_MIXED);
     const dim3 grid((unsigned)(((int64_t)n * lanes + 255) / 256));
 #define SMD_PACKED(G)                                                                              \
     do {                                                                                           \

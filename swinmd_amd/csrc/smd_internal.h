@@ -214,7 +214,7 @@ struct Ctx {
     int* d_cg_state = nullptr;    // [4] done, iterations, stop reason
     double* d_cg_scal = nullptr;  // [4] last residual norm
     int cg_graph = 1;                   // replay CG batches from a captured graph
-    int cg_lanes = 16;                  // lanes per row of the CG's A v
+    int cg_lanes = 0;                   // lanes per row of the CG's A v (0: by size)
     int cg_batch = 16;                  // CG iterations per captured batch
     hipGraphExec_t cg_exec = nullptr;   // a captured batch of CG iterations
     std::string cg_key;                 // the kernel arguments it was captured with
@@ -270,7 +270,7 @@ struct Ctx {
     int md_fused_shake = 1;           // the MD step's SHAKE and kinetics in one kernel
 
     Prof prof;
-    int pair_lanes = 0;           // lanes per atom row in the pair kernels (0: by precision)
+    int pair_lanes = 0;           // lanes per atom row in the pair kernels (0: by size and precision)
     int pair_packed = 1;
     bool pack_reuse = false;
     // Ensemble::accumulate stress sums of the MD step: [0] counter,
@@ -312,6 +312,33 @@ struct Ctx {
     bool ind_real_table = false;    // Induction's mixed real space may walk the current solve's coupling table
     bool mp_real_table = false;     // Multipole's mixed real space may walk the current solve's coupling table
 };
+
+// Lanes per atom row of the kernels that walk a neighbour list's or coupling
+// table's rows: 16, or 32 and 64 where n rows of 16 are fewer than three
+// wavefronts for each of the 1,024 SIMDs, since then the kernel lasts as long
+// as one lane's chain of pairs and shorter chains on more lanes are free.
+// More lanes than that only add to the sums over a row's lanes.  Measured with
+// 16 / 32 / 64 lanes in us, FP64 water of
+//                        3,072 sites      6,144 sites      12,288 sites
+//   induced real space   122 / 100 / 75   174 / 153 / 149  265 / 286 / 290
+//   permanent            101 /  88 / 61   147 / 129 / 124  227 / 240 / 235
+//   field                 40 /  29 / 20    53 /  38 /  36   63 /  61 /  62
+//   A v of the solve    10.7 / 10.4 / 10 15.5 / 14.0 / 15.7 25.4 / 26.0 / 31.8
+//   pairs (LJ + Ewald)    45 /  31 / 21                      56 /  53 /  51
+// and of the mixed form's induced real space 84 / 44 / 28, 78 / 52 / 52 and
+// 97 / 91 / 97.
+inline int row_lanes(int n) { return n >= 12288 ? 16 : n >= 6144 ? 32 : 64; }
+inline int cg_lanes(const Ctx* c) { return c->cg_lanes ? c->cg_lanes : row_lanes(c->n); }
+
+// f(std::integral_constant<int, lanes>) for a row kernel's lanes.
+template <typename F> void with_lanes(int lanes, F f) {
+    switch (lanes) {
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 32: f(std::integral_constant<int, 32>{}); break;
+        case 64: f(std::integral_constant<int, 64>{}); break;
+        default: f(std::integral_constant<int, 16>{}); break;
+    }
+}
 
 }  // namespace smd
 

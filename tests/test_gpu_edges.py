@@ -114,3 +114,43 @@ def test_sheared_reciprocal_space_matches_the_oracle(n2):
         assert rel_rms(b.split(st["force"])[r], want["force"]) <= 1e-8
         assert rel_rms(b.split(st["pos"])[r], want["pos"]) <= 1e-10
         assert np.max(np.abs(rep[r]["virial"] - want["virial"])) <= 1e-7 * np.max(np.abs(want["virial"]))
+
+
+@pytest.mark.parametrize("n", [256, 512])
+@pytest.mark.parametrize("prec", [L.PREC_FP64, L.PREC_MIXED])
+def test_row_lanes_by_size_give_the_small_boxes_forces(n, prec):
+    """Eight copies of a box are the same infinite lattice, so every copy's
+    short-range forces, fields and induced dipoles are the small box's: 768
+    and 1,536 sites run 64 lanes per atom row, their copies 32 (6,144 sites,
+    the line itself) and 16 (12,288, the other line).  FP64 1e-10 (rounding of
+    another order), mixed 1e-5 (the form's own bar)."""
+    from swinmd_amd.forces import Context, EwaldForce, Induction, LJForce, Multipole
+    print(f"case {n} waters and eight copies, prec {prec}", flush=True)
+    base = S.water(n, density_mol=RHO, seed=5, subset=True, r_oh=0.09572, hoh_deg=108.5, types=S.AMOEBA_TYPES)
+    big = S.water(8 * n, density_mol=RHO, seed=5, subset=True, r_oh=0.09572, hoh_deg=108.5, types=S.AMOEBA_TYPES)
+    Lb = base.box[0]
+    shifts = [(i - 0.5, j - 0.5, k - 0.5) for i in range(2) for j in range(2) for k in range(2)]
+    big.pos = np.concatenate([base.pos + Lb * np.array(s) for s in shifts])
+    solve_tol = 1e-12 if prec == L.PREC_FP64 else 1e-6
+    out = []
+    for s in (base, big):
+        ctx = Context(s)
+        ctx.compute_mol_centers()
+        ctx.set_pairlist(0.7, 0.05, s is big)
+        kcut = S.kcut_for(3, s.box[0])
+        pc, mpf, indf = (np.zeros((s.n_atoms, 3)) for _ in range(3))
+        LJForce(ctx, cutoff=0.7, prec=prec).compute(pc)
+        EwaldForce(ctx, alpha=3.5, real_cut=0.7, kcut=kcut, prec=prec).compute(pc)
+        mp = Multipole(ctx, alpha=3.5, real_cut=0.7, kcut=kcut, prec=prec)
+        a = mp.compute(mpf)
+        ind = Induction(ctx, cutoff_ind=0.7, a_damp=0.39, damp_tij=True, do_min=True, tol=solve_tol * L.DEBYE_E_NM,
+                        precond=2, guess=2, prec=prec)
+        ind.setup_terms(alpha=3.5, real_cut=0.7, kcut=kcut, prec=prec)
+        ind.induce()
+        b = ind.compute(indf)
+        _, _, e0, mu = ind.results()
+        out.append((pc, mpf, indf, e0, mu, np.array([a["real_energy"], b["real_energy"]])))
+    tol = 1e-10 if prec == L.PREC_FP64 else 1e-5
+    for name, x, y in zip(("pairs", "multipole", "induction", "e0", "mu"), out[0], out[1]):
+        assert rel_rms(np.asarray(y).reshape(8, -1), np.tile(np.asarray(x).reshape(1, -1), (8, 1))) <= tol, name
+    assert np.abs(out[1][5] / (8 * out[0][5]) - 1).max() <= tol

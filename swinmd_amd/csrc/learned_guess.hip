@@ -19,16 +19,16 @@
 // standardised inputs and outputs.
 //
 // Matrix products run on the matrix cores as
-// v_mfma_f32_16x16x16_bf16: BF16 operands, FP32 accumulation.  Fragment
+// v_mfma_f32_16x16x32_bf16: BF16 operands, FP32 accumulation.  Fragment
 // layout of lane l (r = l % 16, g = l / 16):
-//   A[r][4g .. 4g+3],  B[4g .. 4g+3][r],  D[4g + t][r] for t = 0..3.
+//   A[r][8g .. 8g+7],  B[8g .. 8g+7][r],  D[4g + t][r] for t = 0..3.
 // One wave carries 16 rows through every layer; activations pass between
 // layers through LDS, because D's layout is A's transposed.
 //  * The training step is one kernel per batch: forward, loss, backward to
-//    the first layer.  It keeps the pre-activations in registers and writes
-//    the BF16 layer inputs and back-propagated gradients feature-major.
-//  * The weight gradient then runs one wave per 16 x 16 tile of dW and batch
-//    slice, each tile an MFMA product over the batch.
+//    the first layer.  It keeps the SiLU's derivatives in registers and
+//    writes the BF16 layer inputs and back-propagated gradients as the
+//    weight gradient's operand fragments.
+//  * The weight gradient is then a matrix product over the batch, in slices.
 //  * Adam sums the slices in a fixed order, so a training run is
 //    deterministic.
 #include <algorithm>
@@ -50,13 +50,11 @@ constexpr int MF = 32, MH = 128, MO = 3, MOP = 16;   // features, hidden width, 
 // padded to 16 rows that stay zero), then the four bias vectors.
 constexpr int OFF_W1 = 0, OFF_W2 = 4096, OFF_W3 = 20480, OFF_W4 = 36864, W_INT = 38912;
 constexpr int OFF_B1 = 38912, OFF_B2 = 39040, OFF_B3 = 39168, OFF_B4 = 39296, P_INT = 39312;
-// the transposed BF16 copies [in][out] sit at the same offsets
+// the BF16 copies, in fragments, have the matrices at the same offsets
 constexpr int NPUB = 37635;        // W1 b1 W2 b2 W3 b3 W4[3] b4[3]
 constexpr int NNORM = 2 * MF + 2 * MO;
-constexpr int MLP_WAVES = 4;       // waves (of 16 rows) per block
 constexpr int LDS_STRIDE = 136;    // BF16 per LDS row: 128 + 8, rows stay 16-byte aligned
-constexpr int WG_TILES = 16 + 64 + 64 + 8;
-constexpr int WG_SPLITS = 16;      // batch slices of the weight gradient
+constexpr int WG_SPLITS = 64;      // most batch slices of the weight gradient
 constexpr int DESC_LANES = 16;
 constexpr double SQRT_COULOMB_LG = 11.78708976;   // SQRTCOULOMBCONSTANT, src/NEMD_defs.h:103
 constexpr double POLMIN_LG = 0.00000001;          // Induction.cpp:195
@@ -68,31 +66,62 @@ __device__ __forceinline__ uint16_t f2bf(float f) {   // nearest, ties to even
 }
 __device__ __forceinline__ float bf2f(short h) { return __uint_as_float((uint32_t)(uint16_t)h << 16); }
 
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
 __device__ __forceinline__ v4f mfma16(v4s a, v4s b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ v4f mfma32(v8bf a, v8bf b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ v8bf ld8(const uint16_t* p) { return *reinterpret_cast<const v8bf*>(p); }
+
+// A wave's LDS writes before its later LDS reads (of other lanes' values),
+// and its reads before its next writes.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 struct MlpArgs {
-    int rows, rows16;          // valid rows, rows padded to 16
+    int rows, rows32;          // valid rows, rows padded to 32
     const int32_t* idx;        // row -> sample of x and tgt (null: identity)
     const uint16_t* x;         // [*][32] standardised inputs, BF16
-    const uint16_t* wb;        // BF16 weights [out][in]
-    const uint16_t* wt;        // BF16 weights [in][out]
+    const uint16_t* wb;        // BF16 weights [out][in], in fragments (w_index)
+    const uint16_t* wt;        // BF16 weights [in][out], in fragments (wt_index)
     const float* w;            // FP32 masters (biases)
     float* y;                  // [rows][3]
-    // training
+    // training: in fragments of the weight gradient's products (frag_out)
     const float* tgt;          // [*][3] standardised targets
-    uint16_t* xt;              // [32][rows16] layer-1 inputs, feature-major
-    uint16_t* ht;              // [3][128][rows16] inputs of layers 2-4
-    uint16_t* dzt;             // [3][128][rows16] dL/dz of layers 1-3, then [16][rows16] of layer 4
+    uint16_t* xt;              // inputs of layer 1, 32 features
+    uint16_t* ht;              // [3] inputs of layers 2-4, 128 features
+    uint16_t* dzt;             // [3] dL/dz of layers 1-3, 128 features, then 16 of layer 4
     double* loss_part;         // [blocks] sums of squared errors
     float scale;               // 2 / (3 rows)
 };
 
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float dsilu_f(float z) {
-    const float s = 1.0f / (1.0f + expf(-z));
-    return s * (1.0f + z * (1.0f - s));
+// Sigmoid s and SiLU h = z s in about half the instructions of 1.0f / (1.0f +
+// expf(-z)) and z / (1.0f + expf(-z)): exp(-z) = 2^n 2^f with -z log2(e) = n + f
+// formed in two floats, and the quotients from the hardware's reciprocal with
+// one correction each, which also gives back what 1 + e lost in rounding.
+// The corrections are left out where |z| is so large that s is 1 or not a
+// normal number.  Relative error against 64 bits over z in [-30, 30]: of s
+// rms 2.8e-8, at most 1.2e-7 (the quotients above 3.3e-8, 1.6e-7); of h
+// 3.0e-8, 1.4e-7 (3.5e-8, 1.8e-7).
+__device__ __forceinline__ void silu_parts(float z, float& s, float& h) {
+    constexpr float L_HI = 1.44269502e+00f, L_LO = 1.92596303e-08f;
+    const float x = __builtin_fmaxf(-z, -104.0f);
+    const float n = __builtin_rintf(x * L_HI);
+    const float f = __builtin_fmaf(x, L_LO, __builtin_fmaf(x, L_HI, -n));
+    const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+    const float d = 1.0f + e, b = d - 1.0f, lost = (1.0f - (d - b)) + (e - b);   // 1 + e = d + lost
+    const bool mid = __builtin_fabsf(z) < 87.0f;
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float s1 = __builtin_fmaf(__builtin_fmaf(-lost, r, __builtin_fmaf(-d, r, 1.0f)), r, r);
+    s = mid ? s1 : r;
+    const float q = z * s;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-lost, q, __builtin_fmaf(-d, q, z)), s, q);
+    h = mid ? q1 : q;
 }
 
 // acc[c] = bias of the 16 columns of tile c, for every row
@@ -104,319 +133,332 @@ __device__ __forceinline__ void bias_init(v4f (&acc)[8], const float* b, int r) 
     }
 }
 
-// acc += A (16 x K, from LDS rows) . W^T tiles, W [128][K] BF16 row-major
-template <int K>
-__device__ __forceinline__ void dense_lds(v4f (&acc)[8], const uint16_t* lds, const uint16_t* W, int r, int g) {
-#pragma unroll
-    for (int ks = 0; ks < K / 16; ++ks) {
-        const v4s av = *reinterpret_cast<const v4s*>(lds + r * LDS_STRIDE + ks * 16 + 4 * g);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const v4s bv = *reinterpret_cast<const v4s*>(W + (size_t)(c * 16 + r) * K + ks * 16 + 4 * g);
-            acc[c] = mfma16(av, bv, acc[c]);
-        }
-    }
+// n BF16 (a multiple of 8) from global to LDS, 16 bytes per thread and step
+__device__ __forceinline__ void stage(uint16_t* dst, const uint16_t* src, int n) {
+    for (int t = 8 * threadIdx.x; t < n; t += 8 * blockDim.x)
+        *reinterpret_cast<uint4*>(dst + t) = *reinterpret_cast<const uint4*>(src + t);
 }
 
-// SiLU of a hidden layer's pre-activations into LDS (row 4g+t, column
-// 16c+r); when training, the BF16 activations also go feature-major to ht.
+// A fragments of 16 rows x 128 columns from the wave's LDS rows
+__device__ __forceinline__ void rows_in(v8bf (&av)[4], const uint16_t* lds, int r, int g) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) av[ks] = ld8(lds + r * LDS_STRIDE + ks * 32 + 8 * g);
+}
+
+// acc += A . W^T of column tile c, K = 128, W's fragments in LDS
+__device__ __forceinline__ v4f dense_tile(v4f acc, const v8bf (&av)[4], const uint16_t* W, int c, int lane) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) acc = mfma32(av[ks], ld8(W + ((c * 4 + ks) * WAVE + lane) * 8), acc);
+    return acc;
+}
+
+// Place of column tile c of `tiles`, rows 4g..4g+3 of a 16-row tile, in the
+// training step's buffers: a weight-gradient product's operand fragment of 32
+// rows is lane l's 8 values of two neighbouring row tiles, so a matrix
+// product reads 1 KB in a row and nothing is transposed (the order of the 32
+// rows inside the product is free as long as both operands use it).
+__device__ __forceinline__ uint16_t* frag_out(uint16_t* base, int tiles, int row_tile, int c, int lane) {
+    return base + ((size_t)(row_tile >> 1) * tiles + c) * 512 + lane * 8 + (row_tile & 1) * 4;
+}
+
+// SiLU of a hidden layer's pre-activations into the wave's LDS rows (row
+// 4g+t, column 16c+r), in BF16.  When training they also go to `frag`, and
+// acc becomes silu'(z), all that the backward pass needs of z.
 template <bool TRAIN>
-__device__ __forceinline__ void hidden_out(const MlpArgs& a, int l, const v4f (&acc)[8], uint16_t* lds, int row0,
-                                           bool live, int r, int g) {
+__device__ __forceinline__ void hidden_out(v4f (&acc)[8], uint16_t* lds, uint16_t* frag, int row_tile, bool live,
+                                           int lane) {
+    const int r = lane & 15, g = lane >> 4;
+    wave_lds_order();   // the layer's input, in the same rows, has been read
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const int col = c * 16 + r;
         v4s hb;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint16_t h = f2bf(silu_f(acc[c][t]));
+            const float z = acc[c][t];
+            float s, hf;
+            silu_parts(z, s, hf);
+            const uint16_t h = f2bf(hf);
             hb[t] = (short)h;
-            lds[(4 * g + t) * LDS_STRIDE + col] = h;
+            lds[(4 * g + t) * LDS_STRIDE + c * 16 + r] = h;
+            if (TRAIN) acc[c][t] = s * (1.0f + z * (1.0f - s));
         }
-        if (TRAIN && live)
-            *reinterpret_cast<v4s*>(a.ht + (size_t)l * MH * a.rows16 + (size_t)col * a.rows16 + row0 + 4 * g) = hb;
+        if (TRAIN && live) *reinterpret_cast<v4s*>(frag_out(frag, 8, row_tile, c, lane)) = hb;
     }
+    wave_lds_order();
 }
 
-// Backward through a hidden layer: dz = (dh) * silu'(z), dh[16 x 128] from
-// the A fragments in LDS (K columns) times W^T tiles Wt [128][K] of the layer
-// above; dz to LDS (when out_lds) and feature-major to dzt.
-template <int K>
-__device__ __forceinline__ void back_layer(const MlpArgs& a, int l, const uint16_t* lds_in, uint16_t* lds_out,
-                                           const uint16_t* Wt, const v4f (&z)[8], int row0, bool live, int r,
-                                           int g) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        v4f acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < K / 16; ++ks) {
-            const v4s av = *reinterpret_cast<const v4s*>(lds_in + r * LDS_STRIDE + ks * 16 + 4 * g);
-            const v4s bv = *reinterpret_cast<const v4s*>(Wt + (size_t)(c * 16 + r) * K + ks * 16 + 4 * g);
-            acc = mfma16(av, bv, acc);
-        }
-        const int col = c * 16 + r;
-        v4s db;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const uint16_t d = f2bf(acc[t] * dsilu_f(z[c][t]));
-            db[t] = (short)d;
-            if (lds_out) lds_out[(4 * g + t) * LDS_STRIDE + col] = d;
-        }
-        if (live)
-            *reinterpret_cast<v4s*>(a.dzt + (size_t)l * MH * a.rows16 + (size_t)col * a.rows16 + row0 + 4 * g) = db;
-    }
-}
-
-// Forward of 16 rows per wave; with TRAIN also the loss and the backward pass.
-// Every wave runs every step (rows past rows16 compute on zeros and store
-// nothing) so that the block barriers stay uniform.
+// The forward pass's layers up to the outputs o of one wave's 16 rows, which
+// enter as the A fragment ax; z1..z3 of a training step hold silu' after it.
 template <bool TRAIN>
-__global__ __launch_bounds__(256) void k_mlp_rows(MlpArgs a) {
-    __shared__ __align__(16) uint16_t act[MLP_WAVES][2][16 * LDS_STRIDE];
-    __shared__ double lsum[MLP_WAVES];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+__device__ __forceinline__ v4f mlp_forward(const MlpArgs& a, const uint16_t* wl, uint16_t* lds, v8bf ax, v4f (&z1)[8],
+                                           v4f (&z2)[8], v4f (&z3)[8], int row_tile, bool live, int lane) {
     const int r = lane & 15, g = lane >> 4;
-    const int row0 = (blockIdx.x * MLP_WAVES + wv) * 16;
-    const bool live = row0 < a.rows16;
-    uint16_t* L0 = act[wv][0];
-    uint16_t* L1 = act[wv][1];
-
-    v4s ax[2];
-    {
-        const int row = row0 + r;
-        if (live && row < a.rows) {
-            const int s = a.idx ? a.idx[row] : row;
-            const uint16_t* xr = a.x + (size_t)s * MF;
-            ax[0] = *reinterpret_cast<const v4s*>(xr + 4 * g);
-            ax[1] = *reinterpret_cast<const v4s*>(xr + 16 + 4 * g);
-        } else {
-            ax[0] = v4s{0, 0, 0, 0};
-            ax[1] = v4s{0, 0, 0, 0};
-        }
-        if (TRAIN && live)
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) a.xt[(size_t)(ks * 16 + 4 * g + t) * a.rows16 + row] = (uint16_t)ax[ks][t];
-    }
-    v4f z1[8], z2[8], z3[8];
+    const size_t layer = (size_t)MH * a.rows32;
+    v8bf av[4];
     bias_init(z1, a.w + OFF_B1, r);
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const v4s bv = *reinterpret_cast<const v4s*>(a.wb + OFF_W1 + (size_t)(c * 16 + r) * MF + ks * 16 + 4 * g);
-            z1[c] = mfma16(ax[ks], bv, z1[c]);
-        }
-    hidden_out<TRAIN>(a, 0, z1, L0, row0, live, r, g);
-    __syncthreads();
+    for (int c = 0; c < 8; ++c) z1[c] = mfma32(ax, ld8(wl + OFF_W1 + (c * WAVE + lane) * 8), z1[c]);
+    hidden_out<TRAIN>(z1, lds, a.ht, row_tile, live, lane);
+    rows_in(av, lds, r, g);
     bias_init(z2, a.w + OFF_B2, r);
-    dense_lds<MH>(z2, L0, a.wb + OFF_W2, r, g);
-    hidden_out<TRAIN>(a, 1, z2, L1, row0, live, r, g);
-    __syncthreads();
-    bias_init(z3, a.w + OFF_B3, r);
-    dense_lds<MH>(z3, L1, a.wb + OFF_W3, r, g);
-    __syncthreads();                       // every lane has read L0 (layer 2's input)
-    hidden_out<TRAIN>(a, 2, z3, L0, row0, live, r, g);
-    __syncthreads();
-    v4f o;
-    {
-        const float b = a.w[OFF_B4 + r];
-        o = v4f{b, b, b, b};
 #pragma unroll
-        for (int ks = 0; ks < MH / 16; ++ks) {
-            const v4s av = *reinterpret_cast<const v4s*>(L0 + r * LDS_STRIDE + ks * 16 + 4 * g);
-            const v4s bv = *reinterpret_cast<const v4s*>(a.wb + OFF_W4 + (size_t)r * MH + ks * 16 + 4 * g);
-            o = mfma16(av, bv, o);
-        }
-    }
-    // o[t] = output r of row row0 + 4g + t
-    if (live && r < MO)
+    for (int c = 0; c < 8; ++c) z2[c] = dense_tile(z2[c], av, wl + OFF_W2, c, lane);
+    hidden_out<TRAIN>(z2, lds, a.ht + layer, row_tile, live, lane);
+    rows_in(av, lds, r, g);
+    bias_init(z3, a.w + OFF_B3, r);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) z3[c] = dense_tile(z3[c], av, wl + OFF_W3, c, lane);
+    hidden_out<TRAIN>(z3, lds, a.ht + 2 * layer, row_tile, live, lane);
+    rows_in(av, lds, r, g);
+    const float b = a.w[OFF_B4 + r];
+    const v4f o = dense_tile(v4f{b, b, b, b}, av, wl + OFF_W4, 0, lane);
+    // o[t] = output r of row 16 row_tile + 4g + t
+    if (r < MO)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int row = row0 + 4 * g + t;
+            const int row = 16 * row_tile + 4 * g + t;
             if (row < a.rows) a.y[(size_t)row * MO + r] = o[t];
         }
-    if (!TRAIN) return;
+    return o;
+}
+
+// The wave's 16 rows of x as an A fragment; rows past the end are zeros.
+__device__ __forceinline__ uint4 rows_x(const MlpArgs& a, int row, int g) {
+    if (row >= a.rows) return make_uint4(0u, 0u, 0u, 0u);
+    const int s = a.idx ? a.idx[row] : row;
+    return *reinterpret_cast<const uint4*>(a.x + (size_t)s * MF + 8 * g);
+}
+
+// dz of a hidden layer, column tile c: dh times silu', to the wave's LDS rows
+// (when LDS) and to the weight gradient's fragments.
+template <bool LDS>
+__device__ __forceinline__ void back_out(const v4f& dh, const v4f& ds, uint16_t* lds, uint16_t* frag, int row_tile, int c,
+                                         bool live, int lane) {
+    const int r = lane & 15, g = lane >> 4;
+    v4s db;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const uint16_t d = f2bf(dh[t] * ds[t]);
+        db[t] = (short)d;
+        if (LDS) lds[(4 * g + t) * LDS_STRIDE + c * 16 + r] = d;
+    }
+    if (live) *reinterpret_cast<v4s*>(frag_out(frag, 8, row_tile, c, lane)) = db;
+}
+
+// Forward, loss and backward of W x 16 rows.  Every wave runs every step
+// (rows past rows32 compute on zeros and store nothing) so that the block
+// barriers stay uniform.  What it costs is the weights' way to the matrix
+// cores, the 96 sigmoids per lane and the latency of the layers' chain: the
+// weights are read once per block, in fragment order (a linear copy, and
+// conflict-free 16-byte reads), the forward copies making room for the
+// transposed ones; activations pass between layers through the wave's own
+// LDS rows, without block barriers; and the sigmoid is computed once, the
+// forward pass keeping silu'(z) instead of z.  24,576 rows: 32 us; with
+// weights read by every wave from L2, the sigmoid formed twice by the
+// library's functions and 32-byte pieces of feature-major stores it was 99.
+template <int W>
+__global__ __launch_bounds__(W * WAVE) void k_mlp_train(MlpArgs a) {
+    __shared__ __align__(16) uint16_t wl[W_INT];
+    __shared__ __align__(16) uint16_t act[W][16 * LDS_STRIDE];
+    __shared__ double lsum[W];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int tile = blockIdx.x * W + wv;
+    const bool live = 16 * tile < a.rows32;
+    const size_t layer = (size_t)MH * a.rows32;
+    uint16_t* L = act[wv];
+    stage(wl, a.wb, W_INT);
+    const uint4 xin = rows_x(a, 16 * tile + r, g);
+    *reinterpret_cast<uint4*>(L + r * LDS_STRIDE + 8 * g) = xin;
+    wave_lds_order();
+    if (live)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            v4s xb;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) xb[t] = (short)L[(4 * g + t) * LDS_STRIDE + c * 16 + r];
+            *reinterpret_cast<v4s*>(frag_out(a.xt, 2, tile, c, lane)) = xb;
+        }
+    __syncthreads();   // the weights are in LDS
+    v4f z1[8], z2[8], z3[8];
+    const v4f o = mlp_forward<true>(a, wl, L, __builtin_bit_cast(v8bf, xin), z1, z2, z3, tile, live, lane);
 
     // loss and dL/dy; dL/dy of padded rows and outputs is zero
     double se = 0.0;
     v4s dyb;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        const int row = row0 + 4 * g + t;
+        const int row = 16 * tile + 4 * g + t;
         float d = 0.f;
-        if (live && r < MO && row < a.rows) {
+        if (r < MO && row < a.rows) {
             const int s = a.idx ? a.idx[row] : row;
             d = o[t] - a.tgt[(size_t)s * MO + r];
             se += (double)d * (double)d;
         }
-        const uint16_t h = f2bf(a.scale * d);
-        dyb[t] = (short)h;
+        dyb[t] = (short)f2bf(a.scale * d);
     }
-    __syncthreads();                       // every lane has read L0 (layer 4's input)
+    wave_lds_order();
 #pragma unroll
-    for (int t = 0; t < 4; ++t) L1[(4 * g + t) * LDS_STRIDE + r] = (uint16_t)dyb[t];
-    if (live)
-        *reinterpret_cast<v4s*>(a.dzt + (size_t)3 * MH * a.rows16 + (size_t)r * a.rows16 + row0 + 4 * g) = dyb;
+    for (int t = 0; t < 4; ++t) L[(4 * g + t) * LDS_STRIDE + r] = (uint16_t)dyb[t];
+    if (live) *reinterpret_cast<v4s*>(frag_out(a.dzt + 3 * layer, 1, tile, 0, lane)) = dyb;
     se = wave_sum(se);
     if (lane == 0) lsum[wv] = se;
-    __syncthreads();
-    if (threadIdx.x == 0) a.loss_part[blockIdx.x] = (lsum[0] + lsum[1]) + (lsum[2] + lsum[3]);
-    // layer 3: dh3 = dy . W4 (K = 16), W4^T [128][16]
-    back_layer<MOP>(a, 2, L1, L0, a.wt + OFF_W4, z3, row0, live, r, g);
-    __syncthreads();
-    back_layer<MH>(a, 1, L0, L1, a.wt + OFF_W3, z2, row0, live, r, g);
-    __syncthreads();
-    back_layer<MH>(a, 0, L1, nullptr, a.wt + OFF_W2, z1, row0, live, r, g);
-}
-
-// ---- inference: weights staged in LDS, 16x16x32 matrix products ----------
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ v4f mfma32(v8bf a, v8bf b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// v_mfma_f32_16x16x32_bf16 fragments of lane l (r = l % 16, g = l / 16):
-//   A[r][8g .. 8g+7],  B[8g .. 8g+7][r],  D[4g + t][r] for t = 0..3.
-// Each block stages the four BF16 weight matrices in LDS once (rows padded
-// by 8 so that the 16 rows a fragment read touches fall in different banks)
-// and carries INF_WAVES x 16 rows through the network, 16 per wave.
-constexpr int INF_WAVES = 8;
-constexpr int W1_STRIDE = MF + 8;                       // BF16 per LDS row of W1
-constexpr int INF_W1 = 0, INF_W2 = MH * W1_STRIDE, INF_W3 = INF_W2 + MH * LDS_STRIDE,
-              INF_W4 = INF_W3 + MH * LDS_STRIDE, INF_WSIZE = INF_W4 + MOP * LDS_STRIDE;
-
-__device__ __forceinline__ v8bf ld8(const uint16_t* p) { return *reinterpret_cast<const v8bf*>(p); }
-
-// rows x cols BF16 (row-major, cols a multiple of 8) from global to LDS with
-// the given LDS row stride, 16 bytes per thread and step
-__device__ __forceinline__ void stage(uint16_t* dst, int stride, const uint16_t* src, int rows, int cols) {
-    const int per_row = cols / 8;
-    for (int t = threadIdx.x; t < rows * per_row; t += blockDim.x) {
-        const int row = t / per_row, c8 = t % per_row;
-        *reinterpret_cast<uint4*>(dst + row * stride + 8 * c8) =
-            *reinterpret_cast<const uint4*>(src + (size_t)row * cols + 8 * c8);
+    __syncthreads();   // every wave is through with the forward weights
+    if (threadIdx.x == 0) {
+        double s = lsum[0];
+        for (int w = 1; w < W; ++w) s += lsum[w];
+        a.loss_part[blockIdx.x] = s;
     }
-}
-
-// acc += A (16 x 128, LDS rows) . W^T over 8 column tiles, W [128][128] in LDS
-__device__ __forceinline__ void dense128(v4f (&acc)[8], const uint16_t* lds, const uint16_t* W, int r, int g) {
+    stage(wl + OFF_W2, a.wt + OFF_W2, W_INT - OFF_W2);
+    __syncthreads();
+    // layer 3: dh3 = dy . W4 (K = 16)
+    {
+        const v4s av = *reinterpret_cast<const v4s*>(L + r * LDS_STRIDE + 4 * g);
+        wave_lds_order();
 #pragma unroll
-    for (int ks = 0; ks < MH / 32; ++ks) {
-        const v8bf av = ld8(lds + r * LDS_STRIDE + ks * 32 + 8 * g);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] = mfma32(av, ld8(W + (c * 16 + r) * LDS_STRIDE + ks * 32 + 8 * g), acc[c]);
+        for (int c = 0; c < 8; ++c) {
+            const v4s bv = *reinterpret_cast<const v4s*>(wl + OFF_W4 + (c * WAVE + lane) * 4);
+            back_out<true>(mfma16(av, bv, v4f{0.f, 0.f, 0.f, 0.f}), z3[c], L, a.dzt + 2 * layer, tile, c, live, lane);
+        }
+        wave_lds_order();
     }
-}
-
-__device__ __forceinline__ void silu_lds(const v4f (&acc)[8], uint16_t* lds, int r, int g) {
+    v8bf av[4];
+    rows_in(av, L, r, g);
+    wave_lds_order();
 #pragma unroll
     for (int c = 0; c < 8; ++c)
+        back_out<true>(dense_tile(v4f{0.f, 0.f, 0.f, 0.f}, av, wl + OFF_W3, c, lane), z2[c], L, a.dzt + layer, tile, c,
+                       live, lane);
+    wave_lds_order();
+    rows_in(av, L, r, g);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) lds[(4 * g + t) * LDS_STRIDE + c * 16 + r] = f2bf(silu_f(acc[c][t]));
+    for (int c = 0; c < 8; ++c)
+        back_out<false>(dense_tile(v4f{0.f, 0.f, 0.f, 0.f}, av, wl + OFF_W2, c, lane), z1[c], nullptr, a.dzt, tile, c,
+                        live, lane);
 }
 
+// Inference: each block stages the weights once and carries INF_WAVES x 16
+// rows through the network, 16 per wave.
+constexpr int INF_WAVES = 8;
 __global__ __launch_bounds__(INF_WAVES * WAVE) void k_mlp_infer(MlpArgs a) {
-    __shared__ __align__(16) uint16_t wl[INF_WSIZE];
-    __shared__ __align__(16) uint16_t act[INF_WAVES][2][16 * LDS_STRIDE];
-    stage(wl + INF_W1, W1_STRIDE, a.wb + OFF_W1, MH, MF);
-    stage(wl + INF_W2, LDS_STRIDE, a.wb + OFF_W2, MH, MH);
-    stage(wl + INF_W3, LDS_STRIDE, a.wb + OFF_W3, MH, MH);
-    stage(wl + INF_W4, LDS_STRIDE, a.wb + OFF_W4, MOP, MH);
+    __shared__ __align__(16) uint16_t wl[W_INT];
+    __shared__ __align__(16) uint16_t act[INF_WAVES][16 * LDS_STRIDE];
+    stage(wl, a.wb, W_INT);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int r = lane & 15, g = lane >> 4;
-    const int row0 = (blockIdx.x * INF_WAVES + wv) * 16;
-    uint16_t* L0 = act[wv][0];
-    uint16_t* L1 = act[wv][1];
-    uint4 xin = make_uint4(0u, 0u, 0u, 0u);   // rows past the end compute on zeros
-    {
-        const int row = row0 + r;
-        if (row < a.rows) {
-            const int sidx = a.idx ? a.idx[row] : row;
-            xin = *reinterpret_cast<const uint4*>(a.x + (size_t)sidx * MF + 8 * g);
-        }
-    }
-    const v8bf ax = __builtin_bit_cast(v8bf, xin);
+    const int tile = blockIdx.x * INF_WAVES + wv;
+    const uint4 xin = rows_x(a, 16 * tile + (lane & 15), lane >> 4);
     __syncthreads();   // the weights are in LDS
-    // every wave runs every layer, so the barriers between them stay uniform
-    v4f z[8];
-    bias_init(z, a.w + OFF_B1, r);
+    v4f z1[8], z2[8], z3[8];
+    mlp_forward<false>(a, wl, act[wv], __builtin_bit_cast(v8bf, xin), z1, z2, z3, tile, false, lane);
+}
+
+// One wave's MT x KT tiles of dW[m][k] = sum_n dz[n][m] in[n][k] over the row
+// pairs p0..p1 (32 rows each), and with `bias` the sums of dz.  The next
+// pair's fragments are on their way while the products of this one run.
+template <int MT, int KT>
+__device__ __forceinline__ void wgrad_tiles(const uint16_t* dz, int dtiles, int mt0, const uint16_t* in, int itiles, int kt0,
+                                            int p0, int p1, float* W, int K, float* bias, int lane) {
+    const int r = lane & 15, g = lane >> 4;
+    v4f acc[MT][KT];
+    float bs[MT];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) z[c] = mfma32(ax, ld8(wl + INF_W1 + (c * 16 + r) * W1_STRIDE + 8 * g), z[c]);
-    silu_lds(z, L0, r, g);
-    __syncthreads();
-    bias_init(z, a.w + OFF_B2, r);
-    dense128(z, L0, wl + INF_W2, r, g);
-    silu_lds(z, L1, r, g);
-    __syncthreads();
-    bias_init(z, a.w + OFF_B3, r);
-    dense128(z, L1, wl + INF_W3, r, g);
-    __syncthreads();   // every lane has read L0 (layer 2's input)
-    silu_lds(z, L0, r, g);
-    __syncthreads();
-    v4f o;
-    {
-        const float b = a.w[OFF_B4 + r];
-        o = v4f{b, b, b, b};
+    for (int i = 0; i < MT; ++i) {
+        bs[i] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < MH / 32; ++ks)
-            o = mfma32(ld8(L0 + r * LDS_STRIDE + ks * 32 + 8 * g), ld8(wl + INF_W4 + r * LDS_STRIDE + ks * 32 + 8 * g), o);
+        for (int k = 0; k < KT; ++k) acc[i][k] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    if (r < MO)
+    const uint16_t* ap = dz + ((size_t)p0 * dtiles + mt0) * 512 + lane * 8;
+    const uint16_t* bp = in + ((size_t)p0 * itiles + kt0) * 512 + lane * 8;
+    v8bf av[MT], bv[KT];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int row = row0 + 4 * g + t;
-            if (row < a.rows) a.y[(size_t)row * MO + r] = o[t];
+    for (int i = 0; i < MT; ++i) av[i] = ld8(ap + i * 512);
+#pragma unroll
+    for (int k = 0; k < KT; ++k) bv[k] = ld8(bp + k * 512);
+    for (int p = p0; p < p1; ++p) {
+        const int step = p + 1 < p1 ? 512 : 0;   // the last pair is read again, unused
+        ap += (size_t)step * dtiles;
+        bp += (size_t)step * itiles;
+        v8bf an[MT], bn[KT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) an[i] = ld8(ap + i * 512);
+#pragma unroll
+        for (int k = 0; k < KT; ++k) bn[k] = ld8(bp + k * 512);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int k = 0; k < KT; ++k) acc[i][k] = mfma32(av[i], bv[k], acc[i][k]);
+        if (bias)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                float s[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) s[j] = (float)av[i][j];
+                bs[i] += ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+            }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) av[i] = an[i];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) bv[k] = bn[k];
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                W[(size_t)((mt0 + i) * 16 + 4 * g + q) * K + (kt0 + k) * 16 + r] = acc[i][k][q];
+        if (bias) {
+            float s = bs[i];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (g == 0) bias[(mt0 + i) * 16 + r] = s;
         }
-}
-
-// dW[m][k] = sum_n dz[m][n] in[k][n] over one batch slice, one wave per tile;
-// tiles with k0 = 0 also sum dz for the bias.  Writes every entry of its
-// slice's partial vector.
-__global__ __launch_bounds__(64) void k_mlp_wgrad(MlpArgs a, float* part, int chunk) {
-    int t = blockIdx.x, l;
-    if (t < 16) l = 0;
-    else if (t < 80) { l = 1; t -= 16; }
-    else if (t < 144) { l = 2; t -= 80; }
-    else { l = 3; t -= 144; }
-    const int K = l == 0 ? MF : MH;
-    const int kt_n = K / 16, mt = t / kt_n, kt = t % kt_n;
-    const int woff = l == 0 ? OFF_W1 : l == 1 ? OFF_W2 : l == 2 ? OFF_W3 : OFF_W4;
-    const int boff = l == 0 ? OFF_B1 : l == 1 ? OFF_B2 : l == 2 ? OFF_B3 : OFF_B4;
-    const uint16_t* dz = a.dzt + (size_t)l * MH * a.rows16;
-    const uint16_t* in = l == 0 ? a.xt : a.ht + (size_t)(l - 1) * MH * a.rows16;
-    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-    const uint16_t* arow = dz + (size_t)(mt * 16 + r) * a.rows16 + 4 * g;
-    const uint16_t* brow = in + (size_t)(kt * 16 + r) * a.rows16 + 4 * g;
-    const int n0 = blockIdx.y * chunk, n1 = min(a.rows16, n0 + chunk);
-    v4f acc{0.f, 0.f, 0.f, 0.f};
-    float bs = 0.f;
-    for (int n = n0; n < n1; n += 16) {
-        const v4s av = *reinterpret_cast<const v4s*>(arow + n);
-        const v4s bv = *reinterpret_cast<const v4s*>(brow + n);
-        acc = mfma16(av, bv, acc);
-        bs += (bf2f(av[0]) + bf2f(av[1])) + (bf2f(av[2]) + bf2f(av[3]));
-    }
-    float* p = part + (size_t)blockIdx.y * P_INT;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) p[woff + (size_t)(mt * 16 + 4 * g + q) * K + kt * 16 + r] = acc[q];
-    if (kt == 0) {
-        bs += __shfl_xor(bs, 16);
-        bs += __shfl_xor(bs, 32);
-        if (g == 0) p[boff + mt * 16 + r] = bs;
     }
 }
 
-// Index of master parameter p < W_INT in the transposed copy.
-__device__ __forceinline__ int transposed_index(int p) {
-    if (p < OFF_W2) return OFF_W1 + (p % MF) * MH + p / MF;
-    if (p < OFF_W3) { const int q = p - OFF_W2; return OFF_W2 + (q % MH) * MH + q / MH; }
-    if (p < OFF_W4) { const int q = p - OFF_W3; return OFF_W3 + (q % MH) * MH + q / MH; }
-    const int q = p - OFF_W4;
-    return OFF_W4 + (q % MH) * MOP + q / MH;
+// The weight gradient over one slice of the batch, blockIdx.y, written whole
+// to the slice's partial vector: a block per square layer (a wave a 64 x 64
+// quarter, so each fragment feeds four matrix products) and one for the first
+// and last layers, two waves each.  Bound by reading the operands (38 MB at
+// 24,576 rows, twice per square layer): 11 us; a wave per 16 x 16 tile read
+// them 239 MB in all and took 57.
+__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpArgs a, float* part, int chunk) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p0 = blockIdx.y * chunk, p1 = min(a.rows32 / 32, p0 + chunk);
+    const size_t layer = (size_t)MH * a.rows32;
+    float* P = part + (size_t)blockIdx.y * P_INT;
+    if (blockIdx.x < 2) {
+        const int l = blockIdx.x + 1, mt = (w >> 1) * 4, kt = (w & 1) * 4;
+        wgrad_tiles<4, 4>(a.dzt + l * layer, 8, mt, a.ht + (l - 1) * layer, 8, kt, p0, p1, P + (l == 1 ? OFF_W2 : OFF_W3),
+                          MH, kt == 0 ? P + (l == 1 ? OFF_B2 : OFF_B3) : nullptr, lane);
+    } else if (w < 2) {
+        wgrad_tiles<4, 2>(a.dzt, 8, 4 * w, a.xt, 2, 0, p0, p1, P + OFF_W1, MF, P + OFF_B1, lane);
+    } else {
+        wgrad_tiles<1, 4>(a.dzt + 3 * layer, 1, 0, a.ht + 2 * layer, 8, 4 * (w - 2), p0, p1, P + OFF_W4, MH,
+                          w == 2 ? P + OFF_B4 : nullptr, lane);
+    }
+}
+
+// Place of W[m][k] in a copy of fragments of the products' B operand: tile
+// of 16 rows m, K slab of 32, lane (m % 16, (k % 32) / 8), 8 values.
+__device__ __forceinline__ int frag_index(int m, int k, int K) {
+    return (((m >> 4) * (K >> 5) + (k >> 5)) * WAVE + ((k >> 3) & 3) * 16 + (m & 15)) * 8 + (k & 7);
+}
+// Master parameter p < W_INT in the [out][in] copy
+__device__ __forceinline__ int w_index(int p) {
+    if (p < OFF_W2) return OFF_W1 + frag_index(p / MF, p % MF, MF);
+    const int off = p < OFF_W3 ? OFF_W2 : p < OFF_W4 ? OFF_W3 : OFF_W4, q = p - off;
+    return off + frag_index(q / MH, q % MH, MH);
+}
+// and, from OFF_W2 on, in the [in][out] copy (the first layer passes nothing
+// back); the last layer's 16 outputs make fragments of K = 16, 4 values a lane
+__device__ __forceinline__ int wt_index(int p) {
+    if (p >= OFF_W4) {
+        const int m = (p - OFF_W4) / MH, k = (p - OFF_W4) % MH;
+        return OFF_W4 + ((k >> 4) * WAVE + (m >> 2) * 16 + (k & 15)) * 4 + (m & 3);
+    }
+    const int off = p < OFF_W3 ? OFF_W2 : OFF_W3, q = p - off;
+    return off + frag_index(q % MH, q / MH, MH);
 }
 
 struct AdamArgs {
@@ -428,27 +470,37 @@ struct AdamArgs {
     int update;                // 0: only refresh the BF16 copies from w
 };
 
+// A wave per 64 parameters adds a quarter of the slices each, and the first
+// adds the quarters: the slices' loads are what this kernel waits for (64
+// slices 5.9 us; a thread per parameter took 6.4 for 16).
 __global__ __launch_bounds__(256) void k_mlp_adam(AdamArgs a) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P_INT) return;
-    float w = a.w[p];
+    __shared__ float quarter[4][WAVE];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p = blockIdx.x * WAVE + lane;
+    float sum = 0.f;
+    if (a.part && p < P_INT)
+#pragma unroll 4
+        for (int s = w; s < a.splits; s += 4) sum += a.part[(size_t)s * P_INT + p];
+    quarter[w][lane] = sum;
+    __syncthreads();
+    if (w != 0 || p >= P_INT) return;
+    float wp = a.w[p];
     if (a.part) {
-        float gsum = 0.f;
-        for (int s = 0; s < a.splits; ++s) gsum += a.part[(size_t)s * P_INT + p];
+        const float gsum = (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
         if (a.grad_out) { a.grad_out[p] = gsum; return; }
         if (a.update) {
             const float m = a.b1 * a.m[p] + (1.f - a.b1) * gsum;
             const float v = a.b2 * a.v[p] + (1.f - a.b2) * gsum * gsum;
             a.m[p] = m;
             a.v[p] = v;
-            w -= a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
-            a.w[p] = w;
+            wp -= a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
+            a.w[p] = wp;
         }
     }
     if (p < W_INT) {
-        const uint16_t h = f2bf(w);
-        a.wb[p] = h;
-        a.wt[transposed_index(p)] = h;
+        const uint16_t h = f2bf(wp);
+        a.wb[w_index(p)] = h;
+        if (p >= OFF_W2) a.wt[wt_index(p)] = h;
     }
 }
 
@@ -766,20 +818,20 @@ struct Mlp {
     float* w = nullptr;        // FP32 masters [P_INT]
     float* am = nullptr;       // Adam moments [P_INT]
     float* av = nullptr;
-    uint16_t* wb = nullptr;    // BF16 [W_INT]
-    uint16_t* wt = nullptr;    // BF16 transposed [W_INT]
+    uint16_t* wb = nullptr;    // BF16 [W_INT], in fragments
+    uint16_t* wt = nullptr;    // BF16 transposed [W_INT], in fragments
     float* norm = nullptr;     // [NNORM]
     bool norm_set = false;
     float* part = nullptr;     // [WG_SPLITS][P_INT]
     float* grad = nullptr;     // [P_INT]
-    // row buffers for up to cap rows (a multiple of 16)
+    // row buffers for up to cap rows (a multiple of 32)
     int64_t cap = 0;
     uint16_t* x = nullptr;     // [cap][32]
     float* y = nullptr;        // [cap][3]
     float* tgt = nullptr;      // [cap][3]
-    uint16_t* xt = nullptr;    // [32][cap]
-    uint16_t* ht = nullptr;    // [3][128][cap]
-    uint16_t* dzt = nullptr;   // [3 * 128 + 16][cap]
+    uint16_t* xt = nullptr;    // 32 cap
+    uint16_t* ht = nullptr;    // 3 * 128 cap
+    uint16_t* dzt = nullptr;   // (3 * 128 + 16) cap
     double* loss_part = nullptr;   // [cap / 64]
     // per-site buffers of the context's n sites
     double* frame = nullptr;   // [n][9]
@@ -824,14 +876,14 @@ void mlp_release(Ctx* c) {
     c->mlp = nullptr;
 }
 
-static int64_t round16(int64_t v) { return (v + 15) / 16 * 16; }
+static int64_t round32(int64_t v) { return (v + 31) / 32 * 32; }
 
-static int ensure_rows(Ctx* c, int64_t rows16) {
+static int ensure_rows(Ctx* c, int64_t rows32) {
     Mlp* m = c->mlp;
-    if (rows16 <= m->cap) return SMD_OK;
+    if (rows32 <= m->cap) return SMD_OK;
     SMD_HIP(c, hipStreamSynchronize(c->stream));
     free_rows(m);
-    const int64_t cap = std::max<int64_t>(rows16, 1024);
+    const int64_t cap = std::max<int64_t>(rows32, 1024);
     SMD_HIP(c, hipMalloc(&m->x, sizeof(uint16_t) * MF * cap));
     SMD_HIP(c, hipMalloc(&m->y, sizeof(float) * MO * cap));
     SMD_HIP(c, hipMalloc(&m->tgt, sizeof(float) * MO * cap));
@@ -839,8 +891,6 @@ static int ensure_rows(Ctx* c, int64_t rows16) {
     SMD_HIP(c, hipMalloc(&m->ht, sizeof(uint16_t) * 3 * MH * cap));
     SMD_HIP(c, hipMalloc(&m->dzt, sizeof(uint16_t) * (3 * MH + MOP) * cap));
     SMD_HIP(c, hipMalloc(&m->loss_part, sizeof(double) * (cap / 64 + 1)));
-    // rows 3..15 of layer 4's dL/dz are never written and must read as zero
-    SMD_HIP(c, hipMemsetAsync(m->dzt, 0, sizeof(uint16_t) * (3 * MH + MOP) * cap, c->stream));
     m->cap = cap;
     return SMD_OK;
 }
@@ -848,7 +898,7 @@ static int ensure_rows(Ctx* c, int64_t rows16) {
 static MlpArgs rows_args(Mlp* m, int64_t rows, const int32_t* idx, const uint16_t* x, const float* tgt) {
     MlpArgs a{};
     a.rows = (int)rows;
-    a.rows16 = (int)round16(rows);
+    a.rows32 = (int)round32(rows);
     a.idx = idx;
     a.x = x;
     a.wb = m->wb;
@@ -864,23 +914,41 @@ static MlpArgs rows_args(Mlp* m, int64_t rows, const int32_t* idx, const uint16_
     return a;
 }
 
-static unsigned row_blocks(int64_t rows16) { return (unsigned)((rows16 + 16 * MLP_WAVES - 1) / (16 * MLP_WAVES)); }
+// Waves per block of the training pass: 8, so that one copy of the weights
+// serves 128 rows, or 4 where twice the blocks still leave CUs without one.
+static int train_waves(int64_t rows32) { return rows32 <= 64 * 256 ? 4 : 8; }
+static unsigned row_blocks(int64_t rows32) {
+    const int w = 16 * train_waves(rows32);
+    return (unsigned)((rows32 + w - 1) / w);
+}
+
+// Batch slices of the weight gradient, each of `chunk` pairs of row tiles (two
+// at least): as many as there are buffers for, since a slice lasts as long as
+// its chain of loads.
+static int wgrad_slices(int64_t rows32, int* chunk) {
+    const int pairs = (int)(rows32 / 32);
+    *chunk = std::max(2, (pairs + WG_SPLITS - 1) / WG_SPLITS);
+    return (pairs + *chunk - 1) / *chunk;
+}
 
 // One forward + backward over rows, then the weight gradient's slices into part.
 static int train_pass(Ctx* c, const MlpArgs& a) {
     Mlp* m = c->mlp;
-    hipLaunchKernelGGL(k_mlp_rows<true>, dim3(row_blocks(a.rows16)), dim3(256), 0, c->stream, a);
-    const int slices = std::max(1, std::min(WG_SPLITS, a.rows16 / 16));
-    const int chunk = (int)round16((a.rows16 + slices - 1) / slices);
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(WG_TILES, WG_SPLITS), dim3(64), 0, c->stream, a, m->part, chunk);
+    const dim3 grid(row_blocks(a.rows32));
+    if (train_waves(a.rows32) == 8) hipLaunchKernelGGL(k_mlp_train<8>, grid, dim3(512), 0, c->stream, a);
+    else hipLaunchKernelGGL(k_mlp_train<4>, grid, dim3(256), 0, c->stream, a);
+    int chunk;
+    const int slices = wgrad_slices(a.rows32, &chunk);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(3, slices), dim3(256), 0, c->stream, a, m->part, chunk);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
 
-static AdamArgs adam_args(Mlp* m) {
+static AdamArgs adam_args(Mlp* m, int64_t rows32 = 0) {
     AdamArgs a{};
     a.w = m->w; a.m = m->am; a.v = m->av; a.wb = m->wb; a.wt = m->wt;
-    a.part = m->part; a.splits = WG_SPLITS;
+    int chunk;
+    a.part = m->part; a.splits = wgrad_slices(rows32, &chunk);
     a.b1 = 0.9f; a.b2 = 0.999f; a.eps = 1e-8f;
     return a;
 }
@@ -888,7 +956,7 @@ static AdamArgs adam_args(Mlp* m) {
 static int refresh_copies(Ctx* c) {
     AdamArgs a = adam_args(c->mlp);
     a.part = nullptr;
-    hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + 255) / 256), dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + WAVE - 1) / WAVE), dim3(256), 0, c->stream, a);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
@@ -968,10 +1036,10 @@ int mlp_guess(Ctx* c, double* x, const double* z, float* x32) {
     if (!m || !m->norm_set) return fail(c, SMD_ESTATE, "learned guess: no trained network (smd_mlp_train or smd_mlp_set_norm)");
     int rc;
     if ((rc = check_sites(c))) return rc;
-    if ((rc = ensure_rows(c, round16(c->n)))) return rc;
+    if ((rc = ensure_rows(c, round32(c->n)))) return rc;
     if ((rc = descriptors_run(c, x, z, nullptr, m->x))) return rc;
     MlpArgs a = rows_args(m, c->n, nullptr, m->x, nullptr);
-    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((a.rows16 + 16 * INF_WAVES - 1) / (16 * INF_WAVES))),
+    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((a.rows32 + 16 * INF_WAVES - 1) / (16 * INF_WAVES))),
                        dim3(INF_WAVES * WAVE), 0, c->stream, a);
     hipLaunchKernelGGL(k_guess, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->n, m->frame, c->d_polar,
                        c->d_e0, m->y, m->norm, x, x32);
@@ -1116,11 +1184,11 @@ int smd_mlp_forward(smd_ctx* c, const float* x, int64_t rows, float* y) {
     int rc;
     if ((rc = require(c))) return rc;
     if (rows <= 0 || rows > (1 << 26)) return fail(c, SMD_EINVAL, "smd_mlp_forward: rows %lld", (long long)rows);
-    if ((rc = ensure_rows(c, round16(rows)))) return rc;
+    if ((rc = ensure_rows(c, round32(rows)))) return rc;
     if ((rc = upload_rows(c, x, rows))) return rc;
     Mlp* m = c->mlp;
     MlpArgs a = rows_args(m, rows, nullptr, m->x, nullptr);
-    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((a.rows16 + 16 * INF_WAVES - 1) / (16 * INF_WAVES))),
+    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((a.rows32 + 16 * INF_WAVES - 1) / (16 * INF_WAVES))),
                        dim3(INF_WAVES * WAVE), 0, c->stream, a);
     SMD_HIP(c, hipGetLastError());
     SMD_HIP(c, hipMemcpyAsync(y, m->y, sizeof(float) * MO * rows, hipMemcpyDeviceToHost, c->stream));
@@ -1134,16 +1202,16 @@ int smd_mlp_loss_grad(smd_ctx* c, const float* x, const float* target, int64_t r
     if ((rc = require(c))) return rc;
     if (rows <= 0 || rows > (1 << 26)) return fail(c, SMD_EINVAL, "smd_mlp_loss_grad: rows %lld", (long long)rows);
     Mlp* m = c->mlp;
-    if ((rc = ensure_rows(c, round16(rows)))) return rc;
+    if ((rc = ensure_rows(c, round32(rows)))) return rc;
     if ((rc = upload_rows(c, x, rows))) return rc;
     SMD_HIP(c, hipMemcpyAsync(m->tgt, target, sizeof(float) * MO * rows, hipMemcpyHostToDevice, c->stream));
     MlpArgs a = rows_args(m, rows, nullptr, m->x, m->tgt);
     if ((rc = train_pass(c, a))) return rc;
-    AdamArgs ad = adam_args(m);
+    AdamArgs ad = adam_args(m, a.rows32);
     ad.grad_out = m->grad;
-    hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + 255) / 256), dim3(256), 0, c->stream, ad);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + WAVE - 1) / WAVE), dim3(256), 0, c->stream, ad);
     SMD_HIP(c, hipGetLastError());
-    const unsigned nb = row_blocks(a.rows16);
+    const unsigned nb = row_blocks(a.rows32);
     std::vector<double> lp(nb);
     std::vector<float> g(P_INT);
     SMD_HIP(c, hipMemcpyAsync(lp.data(), m->loss_part, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
@@ -1163,7 +1231,7 @@ int smd_mlp_descriptors(smd_ctx* c, float* desc, int64_t n_atoms) {
     int rc;
     if ((rc = require(c))) return rc;
     if (n_atoms != c->n) return fail(c, SMD_EINVAL, "smd_mlp_descriptors: %lld atoms, context has %d", (long long)n_atoms, c->n);
-    if ((rc = ensure_rows(c, round16(c->n)))) return rc;
+    if ((rc = ensure_rows(c, round32(c->n)))) return rc;
     float* raw = nullptr;
     SMD_HIP(c, hipMalloc(&raw, sizeof(float) * MF * (size_t)c->n));
     rc = state_descriptors(c, raw);
@@ -1229,7 +1297,7 @@ int smd_mlp_train(smd_ctx* c, const smd_mlp_train_params* p, smd_mlp_train_repor
                     (double)p->lr, (double)p->lr_final);
     const int64_t N = m->ds_rows;
     const int64_t B = std::min<int64_t>(p->batch, N);
-    if ((rc = ensure_rows(c, round16(B)))) return rc;
+    if ((rc = ensure_rows(c, round32(B)))) return rc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SMD_HIP(c, hipEventCreate(&e0));
     SMD_HIP(c, hipEventCreate(&e1));
@@ -1272,15 +1340,17 @@ int smd_mlp_train(smd_ctx* c, const smd_mlp_train_params* p, smd_mlp_train_repor
             const int64_t r0 = b * B, rows = std::min(B, N - r0);
             MlpArgs a = rows_args(m, rows, m->perm + r0, m->ds_xn, m->ds_tn);
             if ((rc = train_pass(c, a))) break;
+            int chunk;
+            ad.splits = wgrad_slices(a.rows32, &chunk);
             ++m->adam_t;
             const double t = (double)m->adam_t;
             const double frac = (double)(m->adam_t - 1) / (double)std::max<int64_t>(1, total - 1);
             ad.lr = (float)(p->lr_final + 0.5 * (p->lr - p->lr_final) * (1.0 + std::cos(3.14159265358979323846 * frac)));
             ad.c1 = (float)(1.0 / (1.0 - std::pow(0.9, t)));
             ad.c2 = (float)(1.0 / (1.0 - std::pow(0.999, t)));
-            hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + 255) / 256), dim3(256), 0, c->stream, ad);
+            hipLaunchKernelGGL(k_mlp_adam, dim3((P_INT + WAVE - 1) / WAVE), dim3(256), 0, c->stream, ad);
             if (record) {
-                const unsigned nb = row_blocks(a.rows16);
+                const unsigned nb = row_blocks(a.rows32);
                 std::vector<double> lp(nb);
                 SMD_HIP(c, hipMemcpyAsync(lp.data(), m->loss_part, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
                 SMD_HIP(c, hipStreamSynchronize(c->stream));

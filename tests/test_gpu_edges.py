@@ -154,3 +154,32 @@ def test_row_lanes_by_size_give_the_small_boxes_forces(n, prec):
     for name, x, y in zip(("pairs", "multipole", "induction", "e0", "mu"), out[0], out[1]):
         assert rel_rms(np.asarray(y).reshape(8, -1), np.tile(np.asarray(x).reshape(1, -1), (8, 1))) <= tol, name
     assert np.abs(out[1][5] / (8 * out[0][5]) - 1).max() <= tol
+
+
+# one row, a row more than a 16-row tile and than a pair of tiles, a slice of
+# one pair left over, and both sides of the line between 4 and 8 waves a block
+@pytest.mark.parametrize("rows", [1, 17, 33, 2081, 16384, 16385])
+def test_network_gradient_rows_match_the_oracle(rows):
+    """Loss, gradients of every layer and outputs, oracle with BF16 products;
+    the bars are those of the other batches."""
+    from oracle import learned_guess as G
+    from swinmd_amd.forces import Context, LearnedGuess
+    print(f"case network gradient rows {rows}", flush=True)
+    ctx = Context(S.water(27, density_mol=RHO, seed=2, types=S.AMOEBA_TYPES))
+    net = LearnedGuess(ctx, seed=3)
+    rng = np.random.default_rng(rows)
+    p32 = G.init_params(7).astype(np.float32)
+    p32[G.NPARAMS - 3:] = [0.3, -0.1, 0.2]
+    net.set_params(p32)
+    x = rng.normal(size=(rows, G.NF)).astype(np.float32)
+    t = rng.normal(scale=0.5, size=(rows, G.NO)).astype(np.float32)
+    loss, g = net.loss_grad(x, t)
+    wl, wg = G.loss_grad(p32.astype(np.float64), x.astype(np.float64), t.astype(np.float64), emulate=True)
+    assert abs(loss - wl) <= 1e-4 * wl
+    assert rel_rms(g, wg) <= 2e-3
+    offs = np.cumsum([0] + [int(np.prod(s)) for _, s in G.PUB_SHAPES])
+    for b, (name, _) in enumerate(G.PUB_SHAPES):
+        gb, wb = g[offs[b]:offs[b + 1]], wg[offs[b]:offs[b + 1]]
+        assert rel_rms(gb, wb) <= 1e-2, name
+    assert rel_rms(net.forward(x), G.forward(p32.astype(np.float64), x.astype(np.float64))[0]) <= 1e-3
+    ctx.close()

@@ -76,13 +76,6 @@ __device__ __forceinline__ v4f mfma32(v8bf a, v8bf b, v4f c) {
 }
 __device__ __forceinline__ v8bf ld8(const uint16_t* p) { return *reinterpret_cast<const v8bf*>(p); }
 
-// A wave's LDS writes before its later LDS reads (of other lanes' values),
-// and its reads before its next writes.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 struct MlpArgs {
     int rows, rows32;          // valid rows, rows padded to 32
     const int32_t* idx;        // row -> sample of x and tgt (null: identity)

@@ -13,8 +13,8 @@
 // the back, so every atom's row holds all its partners and the pair kernels
 // need no atomics.  Cell grid: one pass per step assigns atoms to cells, scans
 // the counts and compacts each cell's atoms in index order; the pairs are then
-// found per (cell, neighbour cell) block from LDS-staged positions (see
-// k_list_cells).  Without cells, one wavefront per atom tests all atoms.
+// tested once per pair of cells and each atom's row made from the hits (see
+// k_list_hits, k_list_rows).  Without cells, one wavefront per atom tests all atoms.
 #include <algorithm>
 #include <climits>
 
@@ -105,14 +105,14 @@ __global__ __launch_bounds__(128) void k_cell_assign(int nmol, const int32_t* __
 // One block per cell: its start (the sum of the counts of lower cells) and
 // its atoms compacted in index order (set_atom appends in atom order,
 // CellManager.cpp:145-170); it stops once the cell is full.  The counts are
-// cleared later, by the counting pass of the list build.
+// cleared later, by k_list_hits.
 constexpr int FILL_THREADS = 1024;
 constexpr int FILL_WAVES = FILL_THREADS / WAVE;
 
 __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, const int32_t* __restrict__ cell_of,
                                                             const int32_t* __restrict__ cnt,
                                                             int32_t* __restrict__ start, int32_t* __restrict__ atoms,
-                                                            const int* gate) {
+                                                            int32_t* __restrict__ slot, const int* gate) {
     if (gate && !*gate) return;
     __shared__ int32_t wsum[FILL_WAVES];
     const int c = blockIdx.x;
@@ -145,7 +145,11 @@ __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, co
             off += k < w ? wsum[k] : 0;
             tot += wsum[k];
         }
-        if (hit && base + off + __popcll(m & below) < end) atoms[base + off + __popcll(m & below)] = a;
+        const int at = base + off + __popcll(m & below);
+        if (hit && at < end) {
+            atoms[at] = a;
+            slot[a] = at;
+        }
         base += tot;
         __syncthreads();
     }
@@ -163,7 +167,7 @@ struct ListArgs {
     int32_t* nb_own;
     int32_t stride;
     unsigned* status;
-    uint32_t* mask;    // [27][mask_words][n] hit bits of the cell-pair pass, by cell-order slot
+    uint64_t* mask;    // [27][mask_words][n] hit bits of the cell-pair pass, by cell-order slot
     int mask_words;
 };
 
@@ -234,206 +238,256 @@ __device__ __forceinline__ Excl load_excl(const ListArgs& a, int i) {
 
 // ---- cell-pair list build ----------------------------------------------------
 //
-// Block (c, s) pairs the atoms of cell c with the atoms of its s-th
-// neighbour: s = 0 the cell itself (no PBC, CellManager.cpp:257-279), s =
-// 1..13 the forward stencil (the reference's row of the atom in c), s =
-// 14..26 the backward stencil (the same pairs seen from the other atom).  The
-// neighbour's positions are staged in LDS and each thread owns one atom of c.
-// A counting pass stores, per atom, the hits of each segment (self j>i, self
-// j<i, forward 1..13, backward 1..13); the writing pass repeats the test and
-// writes each hit at its final slot, so row i's front segment is the
-// reference's row in its order.
+// Cell c is paired with its neighbour s: s = 0 the cell itself (no PBC,
+// CellManager.cpp:257-279), s = 1..13 the forward stencil (the reference's row
+// of the atom in c), s = 14..26 the backward stencil (the same pairs seen from
+// the other atom).  k_list_hits tests every pair of atoms once and records
+// both atoms' hits as bits; k_list_rows, a wave per atom, turns an atom's bits
+// into its row.
 
-constexpr int LB_THREADS = 256;   // atoms of cell c per pass of a block
-constexpr int LB_STAGE = 256;     // neighbour atoms staged in LDS at a time
-constexpr int LB_MASK_MAX = 1024; // neighbour-cell atom indices staged for the mask expansion
-constexpr int NSEG = 28;          // per-atom hit counters
+constexpr int LB_THREADS = 256;
+constexpr int LB_WAVES = LB_THREADS / WAVE;
 
-// Neighbour s of cell c and, per axis, the multiple of L (-1, 0, +1) that
-// brings a partner in that cell next to the atom when the stencil wrapped
-// around the box.
-__device__ __forceinline__ int neighbour_cell(const CellGrid& g, int c, int s, int wrap[3]) {
-    wrap[0] = wrap[1] = wrap[2] = 0;
+// Neighbour s of cell c, around the box.
+__device__ __forceinline__ int neighbour_cell(const CellGrid& g, int c, int s) {
     if (s == 0) return c;
     const int sgn = s <= 13 ? 1 : -1;
     const int k = s <= 13 ? s - 1 : s - 14;
     const int cz = c / g.nxy, cy = (c % g.nxy) / g.n[0], cx = c % g.n[0];
     int xx = cx + sgn * c_stencil[k][0], yy = cy + sgn * c_stencil[k][1], zz = cz + sgn * c_stencil[k][2];
-    if (xx >= g.n[0]) { xx = 0; wrap[0] = 1; } else if (xx < 0) { xx = g.n[0] - 1; wrap[0] = -1; }
-    if (yy >= g.n[1]) { yy = 0; wrap[1] = 1; } else if (yy < 0) { yy = g.n[1] - 1; wrap[1] = -1; }
-    if (zz >= g.n[2]) { zz = 0; wrap[2] = 1; } else if (zz < 0) { zz = g.n[2] - 1; wrap[2] = -1; }
+    if (xx >= g.n[0]) xx = 0; else if (xx < 0) xx = g.n[0] - 1;
+    if (yy >= g.n[1]) yy = 0; else if (yy < 0) yy = g.n[1] - 1;
+    if (zz >= g.n[2]) zz = 0; else if (zz < 0) zz = g.n[2] - 1;
     return zz * g.nxy + yy * g.n[0] + xx;
 }
 
-// Tests up to 32 staged candidates against atom i and returns their hit
-// bits.  SELF: the cell itself (no PBC; j > i owned).  Otherwise the pair
-// vector is shifted by the stencil's wrap: |d + shift| < L/2 on every axis
-// is the reference's single PBC step (a value exactly at -L/2 takes the
-// exact path), and every hit has the block's ownership.  The first pass only
-// counts; the second writes each hit at its slot.
-template <bool WRITE, bool SELF>
-__device__ __forceinline__ uint32_t test_word(const ListArgs& a, const double4* __restrict__ sj, int nb, int i,
-                                              double px, double py, double pz, double shx, double shy, double shz,
-                                              const Excl& ex, bool fits, int32_t* row, int& own_at, int& non_at,
-                                              bool block_owned = true) {
-    uint32_t word = 0;
-#pragma unroll 4
-    for (int b = 0; b < nb; ++b) {
-        const double4 q = sj[b];
-        const int j = (int)q.w;
-        double dx = q.x - px, dy = q.y - py, dz = q.z - pz;
-        if constexpr (!SELF) {
-            const double ex_ = dx + shx, ey_ = dy + shy, ez_ = dz + shz;
-            const bool inside = (fabs(ex_) < a.box.h[0]) & (fabs(ey_) < a.box.h[1]) & (fabs(ez_) < a.box.h[2]);
-            dx = inside ? ex_ : dx;
-            dy = inside ? ey_ : dy;
-            dz = inside ? ez_ : dz;
-            if (!inside) pbc(dx, dy, dz, a.box);
-        }
-        if (len2_exact(dx, dy, dz) < a.rlist2 && (!SELF || j != i) && !excluded(ex, j)) {
-            const bool owned = SELF ? (j > i) : block_owned;
-            if constexpr (WRITE) {
-                if (fits) {
-                    if (owned) row[own_at] = j;
-                    else row[a.stride - 1 - non_at] = j;
-                }
-            } else {
-                word |= 1u << b;
-            }
-            own_at += owned ? 1 : 0;
-            non_at += owned ? 0 : 1;
-        }
+// The reference's distance test of a pair vector.  In the cell itself
+// (SELF) it takes no PBC; for a neighbour, apply_pbc's loop makes at most one
+// step of L when |d| < 1.5 L (NEAR), which d - L rint(d / L) makes too, in
+// the same single operation.  The two may differ for |d| next to L/2 only,
+// where neither result is inside a list radius of at most L/3 (a grid has at
+// least three cells per axis).  Every operation is odd in d, so the test
+// gives the same answer from either atom.
+template <bool SELF, bool NEAR>
+__device__ __forceinline__ bool list_hit(const ListArgs& a, double dx, double dy, double dz) {
+    if constexpr (!SELF) {
+        if constexpr (NEAR) pbc_near(dx, dy, dz, a.box);
+        else pbc(dx, dy, dz, a.box);
     }
-    return word;
+    return len2_exact(dx, dy, dz) < a.rlist2;
 }
 
-template <bool WRITE>
-__global__ __launch_bounds__(LB_THREADS) void k_list_cells(ListArgs a, CellGrid g, const int32_t* __restrict__ start,
-                                                           const int32_t* __restrict__ catoms, int32_t* __restrict__ seg,
-                                                           int32_t* cell_cnt, const int* gate) {
+// One wave's tile: 64 atoms of cell c, one per lane, against nb (up to 64)
+// atoms of the neighbour in LDS (whose rows past nb repeat an atom).  Returns
+// the lane's hits as bits; back gets, in lane b, the hits of candidate b over
+// the 64 atoms (the ballot of the same test), so the backward stencil costs
+// no tests of its own.
+template <bool SELF, bool NEAR>
+__device__ __forceinline__ uint64_t hit_tile(const ListArgs& a, const double (*sj)[3], int nb, double px, double py,
+                                             double pz, bool act, uint64_t& back) {
+    uint32_t word[2] = {0u, 0u}, blo = 0, bhi = 0;
+    const int lane = threadIdx.x % WAVE;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+        // four candidates at a time, so that their chains overlap
+        for (int b = 32 * half; b < 32 * half + 32 && b < nb; b += 4) {
+            bool hit[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                hit[u] = list_hit<SELF, NEAR>(a, sj[b + u][0] - px, sj[b + u][1] - py, sj[b + u][2] - pz) && act;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                word[half] |= hit[u] ? 1u << ((b + u) & 31) : 0u;
+                const uint64_t m = __ballot(hit[u]);
+                const bool mine = lane == b + u;
+                blo = mine ? (uint32_t)m : blo;
+                bhi = mine ? (uint32_t)(m >> 32) : bhi;
+            }
+        }
+    back = ((uint64_t)bhi << 32) | blo;
+    const uint64_t all = ((uint64_t)word[1] << 32) | word[0];
+    return nb < WAVE ? all & ((1ull << nb) - 1ull) : all;
+}
+
+// Hits of all pairs of cell blockIdx.x and its neighbour blockIdx.y (0..13),
+// in tiles of 64 x 64 atoms, a wave each; word (s, t) of an atom holds its
+// hits among atoms 64 t.. of neighbour s.  Exclusions and the atom itself are
+// left in; k_list_rows takes them out.  Bound by the FP64 test, about 25
+// instructions a pair: 42 us for 4,096 waters in 64 cells (17.4 million
+// pairs), 18 for 1,021 in 27; testing each pair from both atoms, a block per
+// neighbour, took 63 and 46.
+__global__ __launch_bounds__(LB_THREADS) void k_list_hits(ListArgs a, CellGrid g, const int32_t* __restrict__ start,
+                                                          const int32_t* __restrict__ catoms, int32_t* cell_cnt,
+                                                          const int* gate) {
     if (gate && !*gate) return;
-    __shared__ double4 sj[LB_STAGE];   // x, y, z, atom index
+    __shared__ double sj[LB_WAVES][WAVE][3];
     const int c = blockIdx.x, s = blockIdx.y;
     // the cell counts were last read by k_cell_fill: clear them for the next build
-    if constexpr (!WRITE)
-        if (c == 0 && s == 0)
-            for (int k = threadIdx.x; k < g.ncell; k += blockDim.x) cell_cnt[k] = 0;
-    int wrap[3];
-    const int nc = neighbour_cell(g, c, s, wrap);
-    // A partner across a wrapped face sits about L away: apply_pbc's loop
-    // then makes exactly one step, d + shift (shift = +L when the stencil
-    // wrapped past the upper face, since d = x_j - x_i is then near -L).
-    // Whenever d + shift lands in [-L/2, L/2) it is apply_pbc's result, the
-    // same single operation; otherwise the loops run.
-    const double shx = wrap[0] * a.box.L[0], shy = wrap[1] * a.box.L[1], shz = wrap[2] * a.box.L[2];
+    if (c == 0 && s == 0 && blockIdx.z == 0)
+        for (int k = threadIdx.x; k < g.ncell; k += blockDim.x) cell_cnt[k] = 0;
+    const int nc = neighbour_cell(g, c, s);
     const int ib = start[c], ie = start[c + 1];
     const int jb = start[nc], je = start[nc + 1];
-    const int n = a.n;
-    // the counting pass records its hits as bits when the neighbour cell fits
-    // the mask; the writing pass then expands the bits instead of testing again
-    const bool use_mask = je - jb <= 32 * a.mask_words;
-    // the writing pass reads the neighbour cell's atom indices from LDS
-    __shared__ int32_t sidx[LB_MASK_MAX];
-    const bool lds_idx = WRITE && use_mask && je - jb <= LB_MASK_MAX;
-    if (lds_idx) {
-        for (int t = threadIdx.x; t < je - jb; t += blockDim.x) sidx[t] = catoms[jb + t];
-        __syncthreads();
-    }
-    for (int i0 = ib; i0 < ie; i0 += LB_THREADS) {
-        const int k = i0 + threadIdx.x;
-        const bool act = k < ie;
-        const int i = act ? catoms[k] : 0;
-        double px = 0, py = 0, pz = 0;
-        Excl ex{};
-        int own_at = 0, non_at = 0;   // counts (first pass) or next slots (second pass)
-        bool fits = true;
-        // word w of this atom's hits: mrow[w * n] (slot-major, so a wave's
-        // stores of one word are contiguous)
-        uint32_t* mrow = a.mask + (size_t)s * a.mask_words * n + k;
-        if (act) {
-            px = a.pos[3 * i]; py = a.pos[3 * i + 1]; pz = a.pos[3 * i + 2];
-            ex = load_excl(a, i);
-            if constexpr (WRITE) {
-                // k_seg_offsets left each segment's first slot in seg
-                fits = a.nb_cnt[i] <= a.stride;
-                const int at = s == 0 ? 0 : seg[s * n + i];
-                own_at = at;
-                non_at = at;
-            }
+    const int ti_n = (ie - ib + WAVE - 1) / WAVE, tj_n = (je - jb + WAVE - 1) / WAVE;
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    const size_t n = a.n;
+    for (int t = blockIdx.z * LB_WAVES + w; t < ti_n * tj_n; t += gridDim.z * LB_WAVES) {
+        const int ti = t / tj_n, tj = t % tj_n;
+        if ((s == 0 && tj < ti) || (ti >= a.mask_words && tj >= a.mask_words)) continue;
+        // the wave's time is one candidate's times the candidates': the
+        // larger side takes the lanes
+        const int ki = ib + ti * WAVE, kj = jb + tj * WAVE;
+        const bool swap = min(WAVE, ie - ki) < min(WAVE, je - kj);
+        const int kl = swap ? kj : ki, kl_end = swap ? je : ie, tl = swap ? tj : ti, sl = s == 0 ? 0 : swap ? s + 13 : s;
+        const int kc = swap ? ki : kj, kc_end = swap ? ie : je, tc = swap ? ti : tj, sc = s == 0 ? 0 : swap ? s : s + 13;
+        const bool act = kl + lane < kl_end;
+        const int i = catoms[act ? kl + lane : kl], j = catoms[min(kc + lane, kc_end - 1)];
+        const double px = a.pos[3 * i], py = a.pos[3 * i + 1], pz = a.pos[3 * i + 2];
+        // |x| < 3/4 L on every axis keeps each pair's |d| under 1.5 L
+        bool near = fabs(px) < 0.75 * a.box.L[0] && fabs(py) < 0.75 * a.box.L[1] && fabs(pz) < 0.75 * a.box.L[2];
+        wave_lds_order();   // the tile before this one has been read
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double x = a.pos[3 * j + d];
+            sj[w][lane][d] = x;
+            near = near && fabs(x) < 0.75 * a.box.L[d];
         }
-        int32_t* row = a.nb + (int64_t)i * a.stride;
-        if (WRITE && use_mask) {
-            // expand the recorded hits in candidate order
-            if (act && fits) {
-                const int nw = (je - jb + 31) / 32;
-                for (int w = 0; w < nw; ++w) {
-                    uint32_t bits = mrow[(size_t)w * n];
-                    while (bits) {
-                        const int b = __ffs(bits) - 1;
-                        bits &= bits - 1u;
-                        const int j = lds_idx ? sidx[32 * w + b] : catoms[jb + 32 * w + b];
-                        const bool owned = s == 0 ? (j > i) : (s <= 13);
-                        if (owned) row[own_at++] = j;
-                        else row[a.stride - 1 - non_at++] = j;
-                    }
-                }
-            }
-            continue;
-        }
-        for (int j0 = jb; j0 < je; j0 += LB_STAGE) {
-            const int nj = min(LB_STAGE, je - j0);
-            __syncthreads();
-            for (int t = threadIdx.x; t < nj; t += blockDim.x) {
-                const int j = catoms[j0 + t];
-                sj[t] = make_double4(a.pos[3 * j], a.pos[3 * j + 1], a.pos[3 * j + 2], (double)j);
-            }
-            __syncthreads();
-            if (act) {
-                // candidates in words of 32: word w0/32 of the hit mask is
-                // stored once its 32 candidates are tested
-                for (int w0 = 0; w0 < nj; w0 += 32) {
-                    const int nb = min(32, nj - w0);
-                    const uint32_t word = s == 0
-                        ? test_word<WRITE, true>(a, sj + w0, nb, i, px, py, pz, 0.0, 0.0, 0.0, ex, fits, row,
-                                                 own_at, non_at)
-                        : test_word<WRITE, false>(a, sj + w0, nb, i, px, py, pz, shx, shy, shz, ex, fits, row,
-                                                  own_at, non_at, s <= 13);
-                    if (!WRITE && use_mask) mrow[(size_t)((j0 - jb + w0) >> 5) * n] = word;
-                }
-            }
-        }
-        if constexpr (!WRITE) {
-            if (act) {
-                if (s == 0) { seg[i] = own_at; seg[n + i] = non_at; }
-                else seg[(s + 1) * n + i] = s <= 13 ? own_at : non_at;
-            }
-        }
+        wave_lds_order();
+        const int nb = min(WAVE, kc_end - kc);
+        uint64_t back = 0, word;
+        if (s == 0) word = hit_tile<true, true>(a, sj[w], nb, px, py, pz, act, back);
+        else if (__all(near)) word = hit_tile<false, true>(a, sj[w], nb, px, py, pz, act, back);
+        else word = hit_tile<false, false>(a, sj[w], nb, px, py, pz, act, back);
+        if (act && tc < a.mask_words) a.mask[((size_t)sl * a.mask_words + tc) * n + kl + lane] = word;
+        if ((s > 0 || ti != tj) && lane < nb && tl < a.mask_words)
+            a.mask[((size_t)sc * a.mask_words + tl) * n + kc + lane] = back;
     }
 }
 
-// Between the two passes: per atom, the first slot of each stencil cell's
-// segment -- owned hits (same cell j > i, forward cells 1..13) from the front
-// of the row in stencil order, the others (same cell j < i, backward cells
-// 14..26) from the back -- written over the counts; the row totals.
-__global__ __launch_bounds__(256) void k_seg_offsets(ListArgs a, int32_t* __restrict__ seg, const int* gate) {
+// Row of each atom, in cell order, from its hit bits, a wave per atom: lanes
+// take the neighbours' candidates in stencil order (ten for the own cell, of
+// which most atoms are hits, two for each of the others), so a scan over the
+// lanes' counts gives every lane the slots of its hits.  Owned hits (same
+// cell j > i, forward cells) fill the row from the front, the others from the
+// back; both segments are in the reference's order.  Words of atoms past the
+// mask (a neighbour of more than 64 mask_words atoms) are tested here.
+// The places are put in order in LDS, so that the row leaves in whole cache
+// lines: 45 us at 4,096 waters (430 partners a row), 20 at 1,021; a lane per
+// atom and neighbour, each storing to its own row, took 52 and 36 and a pass
+// for the slots before it.
+constexpr int LR_THREADS = 1024;
+constexpr int ROW_LDS = 1024;   // longest row put in order in LDS
+__global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g, const int32_t* __restrict__ start,
+                                                          const int32_t* __restrict__ catoms,
+                                                          const int32_t* __restrict__ cell_of,
+                                                          const int32_t* __restrict__ slot, const int* gate) {
     if (gate && !*gate) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = a.n;
-    if (i >= n) return;
-    int cnt[NSEG];
+    constexpr int SELF_LANES = 10, WORDS = 4, EXCL = 4;
+    static_assert(SELF_LANES % 2 == 0 && SELF_LANES + 52 <= WAVE, "lanes of 27 neighbours");
+    __shared__ int32_t ranked[LR_THREADS / WAVE][ROW_LDS];
+    const int lane = threadIdx.x % WAVE;
+    const int k = blockIdx.x * (LR_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    if (k >= a.n) return;
+    const int s = lane < SELF_LANES ? 0 : 1 + (lane - SELF_LANES) / 2;
+    const int q = s == 0 ? lane : lane & 1, Q = s == 0 ? SELF_LANES : 2;
+    const size_t n = a.n;
+    const int i = catoms[k], c = cell_of[i];
+    int jb = 0, je = 0, h0 = 0, h1 = 0;
+    if (s <= 26) {
+        const int nc = neighbour_cell(g, c, s);
+        jb = start[nc];
+        je = start[nc + 1];
+        const int nh = (je - jb + 31) / 32;
+        h0 = q * nh / Q;
+        h1 = (q + 1) * nh / Q;
+    }
+    const int e0 = a.excl_off[i], ne = a.excl_off[i + 1] - e0;
+    int out[EXCL];   // the first excluded atoms' places
 #pragma unroll
-    for (int t = 0; t < NSEG; ++t) cnt[t] = seg[t * n + i];
-    // cnt[0], cnt[1]: same cell, owned and not; cnt[s + 1]: stencil cell s
-    int own_at = cnt[0], non_at = cnt[1];
-    seg[i] = 0;
+    for (int e = 0; e < EXCL; ++e) out[e] = e < ne ? slot[a.excl[e0 + e]] : -1;
+    const uint32_t* mask = reinterpret_cast<const uint32_t*>(a.mask + (size_t)s * a.mask_words * n + k);
+    // the lane's hits among candidates 32 h.. of its neighbour
+    auto hits = [&](int h) {
+        uint32_t word = 0;
+        const int base = jb + 32 * h;
+        if (h < 2 * a.mask_words) {
+            word = mask[2 * n * (h >> 1) + (h & 1)];
+        } else {
+            for (int b = 0; b < 32 && base + b < je; ++b) {
+                const int j = catoms[base + b];
+                const double dx = a.pos[3 * j] - a.pos[3 * i], dy = a.pos[3 * j + 1] - a.pos[3 * i + 1],
+                             dz = a.pos[3 * j + 2] - a.pos[3 * i + 2];
+                const bool hit = s == 0 ? list_hit<true, false>(a, dx, dy, dz) : list_hit<false, false>(a, dx, dy, dz);
+                word |= hit ? 1u << b : 0u;
+            }
+        }
+        if (s == 0 && (unsigned)(k - base) < 32u) word &= ~(1u << (k - base));
 #pragma unroll
-    for (int s = 1; s <= 13; ++s) { seg[s * n + i] = own_at; own_at += cnt[s + 1]; }
+        for (int e = 0; e < EXCL; ++e)
+            if ((unsigned)(out[e] - base) < 32u) word &= ~(1u << (out[e] - base));
+        for (int e = EXCL; e < ne; ++e) {
+            const int at = slot[a.excl[e0 + e]] - base;
+            if ((unsigned)at < 32u) word &= ~(1u << at);
+        }
+        return word;
+    };
+    // which of them row i owns: forward cells, and in its own cell the atoms
+    // after it (a cell's atoms are in index order)
+    auto owned = [&](int h) {
+        if (s > 0) return s <= 13 ? ~0u : 0u;
+        const int at = k - (jb + 32 * h);
+        return at < 0 ? ~0u : at >= 31 ? 0u : ~0u << (at + 1);
+    };
+    uint32_t words[WORDS];   // the lane's first words, their loads issued together
+    int own = 0, non = 0;
 #pragma unroll
-    for (int s = 14; s <= 26; ++s) { seg[s * n + i] = non_at; non_at += cnt[s + 1]; }
-    const int total = own_at + non_at;
-    a.nb_cnt[i] = total;
-    a.nb_own[i] = own_at;
-    if (total > a.stride) atomicOr(a.status, ST_LIST_OVERFLOW);
+    for (int u = 0; u < WORDS; ++u) words[u] = h0 + u < h1 ? hits(h0 + u) : 0u;
+#pragma unroll
+    for (int u = 0; u < WORDS; ++u) {
+        own += __popc(words[u] & owned(h0 + u));
+        non += __popc(words[u] & ~owned(h0 + u));
+    }
+    for (int h = h0 + WORDS; h < h1; ++h) {
+        const uint32_t word = hits(h), mine = owned(h);
+        own += __popc(word & mine);
+        non += __popc(word & ~mine);
+    }
+    int own_at = own, non_at = non;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int x = __shfl_up(own_at, o), y = __shfl_up(non_at, o);
+        own_at += lane >= o ? x : 0;
+        non_at += lane >= o ? y : 0;
+    }
+    const int own_all = __shfl(own_at, WAVE - 1), all = own_all + __shfl(non_at, WAVE - 1);
+    own_at -= own;
+    non_at -= non;
+    if (lane == 0) {
+        a.nb_cnt[i] = all;
+        a.nb_own[i] = own_all;
+        if (all > a.stride) atomicOr(a.status, ST_LIST_OVERFLOW);
+    }
+    if (all > a.stride) return;
+    int32_t* row = a.nb + (int64_t)i * a.stride;
+    int32_t* order = ranked[threadIdx.x / WAVE];
+    const bool in_lds = all <= ROW_LDS;
+    auto place = [&](int h, uint32_t bits) {
+        const uint32_t mine = owned(h);
+        while (bits) {
+            const int b = __ffs(bits) - 1, at = jb + 32 * h + b;
+            bits &= bits - 1u;
+            const bool own_hit = mine >> b & 1u;
+            const int to = own_hit ? own_at++ : own_all + non_at++;
+            if (in_lds) order[to] = at;
+            else row[own_hit ? to : a.stride - 1 - (to - own_all)] = catoms[at];
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < WORDS; ++u) place(h0 + u, words[u]);
+    for (int h = h0 + WORDS; h < h1; ++h) place(h, hits(h));
+    if (!in_lds) return;
+    wave_lds_order();
+    for (int t = lane; t < all; t += WAVE) row[t < own_all ? t : a.stride - 1 - (t - own_all)] = catoms[order[t]];
 }
 
 // Ensemble::build_pairlist (src/Ensemble.cpp:492-525): all j != i with the
@@ -544,13 +598,15 @@ static int launch_list(Ctx* c, const int* gate, bool md_prep) {
                                g, c->box, pr, c->d_cell_of, c->d_cell_cnt, gate);
         if (c->list_fork) SMD_HIP(c, hipEventRecord(c->list_fork, c->stream));   // positions are final here
         hipLaunchKernelGGL(k_cell_fill, dim3(nc), dim3(FILL_THREADS), 0, c->stream, c->n, nc, c->d_cell_of,
-                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, gate);
-        const dim3 gl(nc, 27);
-        hipLaunchKernelGGL((k_list_cells<false>), gl, dim3(LB_THREADS), 0, c->stream, a, g, c->d_cell_start,
-                           c->d_cell_atoms, c->d_list_seg, c->d_cell_cnt, gate);
-        hipLaunchKernelGGL(k_seg_offsets, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, a, c->d_list_seg, gate);
-        hipLaunchKernelGGL((k_list_cells<true>), gl, dim3(LB_THREADS), 0, c->stream, a, g, c->d_cell_start,
-                           c->d_cell_atoms, c->d_list_seg, c->d_cell_cnt, gate);
+                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, c->d_cell_slot, gate);
+        // tiles of a cell pair beyond four go to further blocks
+        const int tiles = (c->n / nc + WAVE - 1) / WAVE;
+        const dim3 gl(nc, 14, std::min(8, (tiles * tiles + LB_WAVES - 1) / LB_WAVES));
+        hipLaunchKernelGGL(k_list_hits, gl, dim3(LB_THREADS), 0, c->stream, a, g, c->d_cell_start, c->d_cell_atoms,
+                           c->d_cell_cnt, gate);
+        constexpr int per = LR_THREADS / WAVE;
+        hipLaunchKernelGGL(k_list_rows, dim3((c->n + per - 1) / per), dim3(LR_THREADS), 0, c->stream, a, g,
+                           c->d_cell_start, c->d_cell_atoms, c->d_cell_of, c->d_cell_slot, gate);
     } else {
         if (md_prep)
             hipLaunchKernelGGL(k_rebuild_prep, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, c->nmol,
@@ -583,17 +639,17 @@ int pairlist_build(Ctx* c, double cutoff, double cut_buff, int use_cells, bool o
             if (c->d_cell_start) (void)hipFree(c->d_cell_start);
             SMD_HIP(c, hipMalloc(&c->d_cell_cnt, sizeof(int32_t) * (nc + 1)));
             SMD_HIP(c, hipMalloc(&c->d_cell_start, sizeof(int32_t) * (nc + 1)));
-            // the counting pass clears the counts after each use; they start at zero
+            // k_list_hits clears the counts after each use; they start at zero
             SMD_HIP(c, hipMemset(c->d_cell_cnt, 0, sizeof(int32_t) * (nc + 1)));
             c->cell_alloc = nc + 1;
         }
         // hit bits for neighbour cells of up to twice the mean occupancy
-        const int words = (2 * c->n / nc + 31) / 32 + 1;
+        const int words = (2 * c->n / nc + 63) / 64 + 1;
         if (words > c->list_mask_words) {
             if (c->d_list_mask) (void)hipFree(c->d_list_mask);
             c->d_list_mask = nullptr;
             c->list_mask_words = 0;
-            const size_t bytes = sizeof(uint32_t) * 27 * (size_t)c->n * words;
+            const size_t bytes = sizeof(uint64_t) * 27 * (size_t)c->n * words;
             if (hipMalloc(&c->d_list_mask, bytes) != hipSuccess)
                 return fail(c, SMD_ENOMEM, "pair-list mask allocation of %zu bytes failed", bytes);
             c->list_mask_words = words;

@@ -147,8 +147,8 @@ struct Ctx {
     int32_t* d_cell_cnt = nullptr;    // [ncell+1]
     int32_t* d_cell_start = nullptr;  // [ncell+1]
     int32_t* d_cell_atoms = nullptr;  // [n]
-    int32_t* d_list_seg = nullptr;    // [28][n] per-atom hit counts of the cell-pair segments
-    uint32_t* d_list_mask = nullptr;  // [27][n][list_mask_words] hit bits of the cell-pair pass
+    int32_t* d_cell_slot = nullptr;   // [n] place of each atom in d_cell_atoms
+    uint64_t* d_list_mask = nullptr;  // [27][list_mask_words][n] hit bits of the cell-pair pass
     int list_mask_words = 0;
     int32_t* d_nb = nullptr;          // [n * stride]
     int32_t* d_nb_cnt = nullptr;      // [n] full row length
@@ -437,6 +437,13 @@ __device__ __forceinline__ void pbc_near(double& x, double& y, double& z, const 
     x -= b.L[0] * rint(x * b.inv[0]);
     y -= b.L[1] * rint(y * b.inv[1]);
     z -= b.L[2] * rint(z * b.inv[2]);
+}
+
+// A wave's LDS writes before its later LDS reads (of other lanes' values),
+// and its reads before its next writes.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // Vector3::length2 (src/utils/Vector3.h:190-192) with each product and sum

@@ -183,3 +183,34 @@ def test_network_gradient_rows_match_the_oracle(rows):
         assert rel_rms(gb, wb) <= 1e-2, name
     assert rel_rms(net.forward(x), G.forward(p32.astype(np.float64), x.astype(np.float64))[0]) <= 1e-3
     ctx.close()
+
+
+@pytest.mark.parametrize("case", ["few", "uniform", "crowded", "outside"])
+def test_cell_list_rows_match_the_oracle(case):
+    """Rows of the cell-built list, in order, for few atoms a cell, for tiles
+    with every remainder, for one cell beyond its share of the hit bits with
+    rows too long for LDS, and for atoms more than 3/4 of a box away; with up
+    to nine exclusions on an atom."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context
+    n = {"few": 40, "uniform": 3100, "crowded": 1700, "outside": 900}[case]
+    print(f"case cell list {case} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    s = S.lj_fcc(1)
+    s.density = n / 27.0                       # a box of 3
+    if case == "outside":
+        pos = rng.uniform(-4.0, 4.0, (n, 3))
+    else:
+        pos = rng.uniform(-1.5, 1.5, (n, 3))
+    if case == "crowded":
+        pos[:1400] = rng.uniform(0.6, 1.4, (1400, 3))
+    s.pos, s.type, s.mol = pos, np.zeros(n, dtype=np.int32), np.arange(n, dtype=np.int32)
+    s.bonds = [(0, k, 0) for k in range(1, 10)] + [(k, k + 1, 0) for k in range(20, n - 1, 3)]
+    off, nb, used = O.Oracle(s).pairlist(0.85, 0.1, True)
+    assert used
+    ctx = Context(s)
+    ctx.set_pairlist(0.85, 0.1, True)
+    goff, gnb = ctx.pairlist()
+    np.testing.assert_array_equal(goff, off)
+    np.testing.assert_array_equal(gnb, nb)
+    ctx.close()

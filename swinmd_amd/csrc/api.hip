@@ -72,44 +72,35 @@ int red_finish(Ctx* c, int site, unsigned nblocks, int nv, double* dst) {
     return SMD_OK;
 }
 
-constexpr int FLUSH_MAX = 24;
-struct FlushList {
-    const double* part[FLUSH_MAX];
-    double* dst[FLUSH_MAX];
-    int nb[FLUSH_MAX];
-    int nv[FLUSH_MAX];
-    int cap;
-};
-
 // Block b adds queued finish b: one wave per value, as k_red_finish.
 __global__ __launch_bounds__(1024) void k_red_flush(FlushList f) {
     const int b = blockIdx.x;
-    const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    for (int k = w; k < f.nv[b]; k += blockDim.x / WAVE) {
-        const double* p = f.part[b] + (size_t)k * f.cap;
-        double s = 0.0;
-#pragma unroll 8
-        for (int i = lane; i < f.nb[b]; i += WAVE) s += p[i];
-        s = wave_sum(s);
-        if (lane == 0) f.dst[b][k] += s;
-    }
+    for (int k = threadIdx.x / WAVE; k < f.nv[b]; k += blockDim.x / WAVE) flush_value(f, b, k);
 }
 
-int red_flush(Ctx* c) {
-    const size_t n = c->red_pending.size();
-    if (n == 0) return SMD_OK;
-    if (n > (size_t)FLUSH_MAX) return fail(c, SMD_ESTATE, "%zu queued reductions exceed %d", n, FLUSH_MAX);
-    FlushList f{};
+// The queued finishes, emptied into f.
+int red_take(Ctx* c, FlushList& f) {
+    f = FlushList{};
     f.cap = c->red.cap;
-    for (size_t q = 0; q < n; ++q) {
-        const RedPending& r = c->red_pending[q];
+    if (c->red_pending.size() > (size_t)FLUSH_MAX)
+        return fail(c, SMD_ESTATE, "%zu queued reductions exceed %d", c->red_pending.size(), FLUSH_MAX);
+    for (const RedPending& r : c->red_pending) {
+        const int q = f.count++;
         f.part[q] = c->red.base + (size_t)r.site * RED_NV * c->red.cap;
         f.dst[q] = r.dst;
         f.nb[q] = (int)r.nb;
         f.nv[q] = r.nv;
+        f.values += r.nv;
     }
     c->red_pending.clear();
-    hipLaunchKernelGGL(k_red_flush, dim3((unsigned)n), dim3(1024), 0, c->stream, f);
+    return SMD_OK;
+}
+
+int red_flush(Ctx* c) {
+    FlushList f;
+    int rc = red_take(c, f);
+    if (rc || f.count == 0) return rc;
+    hipLaunchKernelGGL(k_red_flush, dim3((unsigned)f.count), dim3(1024), 0, c->stream, f);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
@@ -233,6 +224,8 @@ extern "C" int smd_ctx_create(smd_ctx** out, const smd_topology* t, int device) 
     c->nmol = nm;
     c->ntypes = t->n_types;
     c->h_mol_start = ms;
+    c->one_site = true;
+    for (size_t m = 0; m + 1 < ms.size(); ++m) c->one_site = c->one_site && ms[m + 1] - ms[m] == 1;
     c->h_type.assign(t->atom_type, t->atom_type + n);
     c->h_mass.assign(t->mass, t->mass + n);
     c->h_q.assign(t->scaled_charge, t->scaled_charge + n);

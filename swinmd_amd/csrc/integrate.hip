@@ -52,6 +52,7 @@ struct IntegArgs {
     double* part_kin;        // [KIN_PARTS][gridDim] kinetics kernels
     double* part_sh;         // [9][gridDim] k_shake
     int nb_vom;
+    int nb_kin;              // blocks of molecules of the kinetics kernel
     int zero_force;          // k_step_head also clears the forces (the polarizable step)
 };
 
@@ -249,32 +250,18 @@ __global__ __launch_bounds__(256) void k_shake(IntegArgs a) {
     block_store<9>(v, a.part_sh, gridDim.x);
 }
 
-__global__ __launch_bounds__(256) void k_lf_atoms(IntegArgs a) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double vc[3] = {0.0, 0.0, 0.0};
-    if (a.md_step) {
-        drift_velocity(a, vc);
-        if (i == 0) a.flag[0] = 0;   // every consumer of the rebuild flag has run
-    }
-    if (i >= a.n) return;
-    const double fnh = a.fnh_on_device ? a.scalars[0] : a.fnh_host;
-    const double mr = 1.0 / a.mass[i];
-    // the drift removal of LFIntegrator::run (:354-379) on vtMinus and the
-    // velocity (zero outside the MD step)
-    for (int d = 0; d < 3; ++d) {
-        a.vtm[3 * i + d] -= vc[d];
-        a.vel[3 * i + d] -= vc[d];
-    }
-    double vp[3];
+// Half-step velocity vp and velocity vel after the step of one atom, from
+// vt (t - dt/2) and vel with the drift taken off.
+__device__ __forceinline__ void lf_velocity(const IntegArgs& a, double fnh, double mr, const double (&vt)[3],
+                                            const double (&F)[3], double (&vel)[3], double (&vp)[3]) {
     if (a.nose_hoover) {
-        double vel[3] = {a.vel[3 * i], a.vel[3 * i + 1], a.vel[3 * i + 2]};
         double velcheck = 1.0;
         int cnt = 0;
         while (velcheck > 1E-10 && cnt < 11) {
             double vv = 0.0, half[3];
             for (int d = 0; d < 3; ++d) {
-                vp[d] = a.vtm[3 * i + d] + a.dt * (mr * a.force[3 * i + d] - fnh * vel[d]);
-                half[d] = (vp[d] + a.vtm[3 * i + d]) * 0.5;
+                vp[d] = vt[d] + a.dt * (mr * F[d] - fnh * vel[d]);
+                half[d] = (vp[d] + vt[d]) * 0.5;
                 const double dv = half[d] - vel[d];
                 vv += dv * dv;
             }
@@ -284,16 +271,61 @@ __global__ __launch_bounds__(256) void k_lf_atoms(IntegArgs a) {
         }
         if (cnt == 10) atomicOr(a.status, ST_NH_ITER);
     } else {
-        for (int d = 0; d < 3; ++d) vp[d] = a.vtm[3 * i + d] + a.dt * mr * a.force[3 * i + d];
+        for (int d = 0; d < 3; ++d) vp[d] = vt[d] + a.dt * mr * F[d];
     }
+    for (int d = 0; d < 3; ++d) vel[d] = (vp[d] + vt[d]) * 0.5;
+}
+
+// Atom i's update: vt and vel are stored; pn is its new position.
+struct LfIn {
+    double vt[3], vel[3], F[3], pos[3], disp[3], real[3], m, fnh;
+};
+__device__ __forceinline__ void lf_load(const IntegArgs& a, int i, LfIn& in) {
+    in.fnh = a.fnh_on_device ? a.scalars[0] : a.fnh_host;
+    in.m = a.mass[i];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        in.vt[d] = a.vtm[3 * i + d];
+        in.vel[d] = a.vel[3 * i + d];
+        in.F[d] = a.force[3 * i + d];
+        in.pos[d] = a.pos[3 * i + d];
+        in.disp[d] = a.disp[3 * i + d];
+        in.real[d] = a.real[3 * i + d];
+    }
+}
+__device__ __forceinline__ void lf_atom(const IntegArgs& a, int i, LfIn& in, const double (&vc)[3], double (&pn)[3],
+                                        double (&vel)[3]) {
+    double vp[3];
+    // the drift removal of LFIntegrator::run (:354-379) on vtMinus and the
+    // velocity (zero outside the MD step)
+    for (int d = 0; d < 3; ++d) {
+        in.vt[d] -= vc[d];
+        vel[d] = in.vel[d] - vc[d];
+    }
+    lf_velocity(a, in.fnh, 1.0 / in.m, in.vt, in.F, vel, vp);
     for (int d = 0; d < 3; ++d) {
         const double dr = a.dt * vp[d];
-        a.pos[3 * i + d] += dr;
-        a.disp[3 * i + d] += dr;
-        a.real[3 * i + d] += dr;
-        a.vel[3 * i + d] = (vp[d] + a.vtm[3 * i + d]) * 0.5;
+        pn[d] = in.pos[d] + dr;
+        a.disp[3 * i + d] = in.disp[d] + dr;
+        a.real[3 * i + d] = in.real[d] + dr;
+        a.vel[3 * i + d] = vel[d];
         a.vtm[3 * i + d] = vp[d];
     }
+}
+
+__global__ __launch_bounds__(256) void k_lf_atoms(IntegArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double vc[3] = {0.0, 0.0, 0.0};
+    LfIn in;
+    if (i < a.n) lf_load(a, i, in);
+    if (a.md_step) {
+        drift_velocity(a, vc);
+        if (i == 0) a.flag[0] = 0;   // every consumer of the rebuild flag has run
+    }
+    if (i >= a.n) return;
+    double pn[3], vel[3];
+    lf_atom(a, i, in, vc, pn, vel);
+    for (int d = 0; d < 3; ++d) a.pos[3 * i + d] = pn[d];
 }
 
 // LF Nose-Hoover friction update (LFIntegrator::run :688-709): fnh, fnhmi.
@@ -309,35 +341,46 @@ __device__ __forceinline__ void nh_friction(const IntegArgs& a, double ke_atom, 
     a.scalars[1] = fp;
 }
 
+// One wave per block: the kinetic and pressure sums are wave reductions
+// spread over as many CUs as there are waves of molecules.
+constexpr int KIN_THREADS = 64;
+
+// Rows of Ctx::part_kin: the kinetic sums (2), the pressure sums (21), the
+// SHAKE virial (9).
+constexpr int KP_KE = 0, KP_PR = 2, KP_SH = 23;
+
 // Integrator::computePressure (src/Integrator.cpp:205-270), the shake-virial
-// correction of LFIntegrator::run (:805-814), myAvLus.P (:730-743) and the
-// stress sums of Ensemble::accumulate (src/Ensemble.cpp:814-894) for the MD
-// step, from the step's sums; one thread.  Ensemble::virial is the force
-// terms' virials subtracted, the long-range virial added without its ZZ
-// component (EwaldForce::compute_long copies i < ZZ, EwaldForce.cpp:194).
-__device__ void md_pressure(const IntegArgs& a, const double* t) {
+// correction of LFIntegrator::run (:805-814) and myAvLus.P (:730-743) for the
+// MD step, from the step's sums t.  Ensemble::virial is the force terms'
+// virials subtracted, the long-range virial added without its ZZ component
+// (EwaldForce::compute_long copies i < ZZ, EwaldForce.cpp:194).
+// Component k of the tensors:
+__device__ __forceinline__ void md_pressure_tensor(const IntegArgs& a, const double* t, int k, double* atom_p,
+                                                   double* mol_p) {
     const double V = a.box.L[0] * a.box.L[1] * a.box.L[2];
-    const int sym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};   // (xx xy xz yy yz zz) -> 3x3
-    double vir[9], atomP[9], molP[9];
-    const double dt2 = a.dt * a.dt;
-    for (int k = 0; k < 9; ++k) {
-        vir[k] = -t[T_LJ_VIR + k] - t[T_EW_VIR + k] - (a.surface ? t[T_SU_VIR + k] : 0.0) +
+    const int x = k / 3, y = k % 3, lo = min(x, y), hi = max(x, y);
+    const int sym = lo == 0 ? hi : lo + hi + 1;   // (xx xy xz yy yz zz) of 3x3
+    double vir = -t[T_LJ_VIR + k] - t[T_EW_VIR + k] - (a.surface ? t[T_SU_VIR + k] : 0.0) +
                  (k < 8 ? t[T_RC_VIR + k] : 0.0);
-        const double molv = vir[k] - t[T_PR_MC + k];
-        atomP[k] = (t[T_PR_KA + sym[k]] + vir[k]) / V;
-        molP[k] = (t[T_PR_KM + sym[k]] + molv) / V;
-        a.terms[T_PR_MOLVIR + k] = molv;
-    }
-    for (int k = 0; k < 9; ++k) {
-        const double sh = t[T_SH_VIR + k] / dt2;
-        vir[k] += sh;
-        atomP[k] += sh / V;
-        a.terms[T_PR_VIR + k] = vir[k];
-        a.terms[T_PR_ATOM + k] = atomP[k];
-        a.terms[T_PR_MOL + k] = molP[k];
-    }
-    // molVirt with the terms this step has: LJ, Ewald real, intramolecular,
-    // surface and reciprocal volume derivatives (LFIntegrator.cpp:730-733)
+    const double molv = vir - t[T_PR_MC + k];
+    double atomP = (t[T_PR_KA + sym] + vir) / V;
+    const double molP = (t[T_PR_KM + sym] + molv) / V;
+    const double dt2 = a.dt * a.dt;
+    const double sh = t[T_SH_VIR + k] / dt2;
+    vir += sh;
+    atomP += sh / V;
+    a.terms[T_PR_MOLVIR + k] = molv;
+    a.terms[T_PR_VIR + k] = vir;
+    a.terms[T_PR_ATOM + k] = atomP;
+    a.terms[T_PR_MOL + k] = molP;
+    atom_p[k] = atomP;
+    mol_p[k] = molP;
+}
+
+// and molVirt with the terms this step has: LJ, Ewald real, intramolecular,
+// surface and reciprocal volume derivatives (LFIntegrator.cpp:730-733)
+__device__ __forceinline__ double md_pressure_mol(const IntegArgs& a, const double* t) {
+    const double V = a.box.L[0] * a.box.L[1] * a.box.L[2];
     // LJForce sets ljdUlus only with computeLustig (src/forces/LJForce.cpp:
     // 238-247); EwaldForce's derivatives are always formed, its molDeriv only
     // for unconstrained molecules (EwaldForce.cpp:780-784)
@@ -361,49 +404,75 @@ __device__ void md_pressure(const IntegArgs& a, const double* t) {
     a.terms[T_PR_LUS + 2] = longDeriv;
     a.terms[T_PR_LUS + 3] = molDeriv;
     a.terms[T_PR_LUS + 4] = surf;
-    double* st = a.stress;
-    st[0] += 1.0;
-    if (st[0] > a.stress_after) {
-        st[1] += 1.0;
-        st[2] += molPt;
-        st[3] += (atomP[1] + atomP[3]) * 0.5;
-        st[4] += (atomP[3] - atomP[1]) * 0.5;
-        st[5] += (atomP[0] - atomP[4]);
-        st[6] += (atomP[4] - atomP[8]);
-        st[7] += (molP[0] + molP[4] + molP[8]) / 3.0;
-        st[8] += (molP[1] + molP[3]) * 0.5;
-        st[9] += (molP[3] - molP[1]) * 0.5;
-        st[10] += (molP[0] - molP[4]);
-        st[11] += (molP[4] - molP[8]);
-    }
+    return molPt;
 }
 
-// One wave per block: the kinetic and pressure sums are wave reductions
-// spread over as many CUs as there are waves of molecules.
-constexpr int KIN_THREADS = 64;
-
-// Rows of Ctx::part_kin: the kinetic sums (2), the pressure sums (21), the
-// SHAKE virial (9).
-constexpr int KP_KE = 0, KP_PR = 2, KP_SH = 23;
+// Stress sum k > 0 of Ensemble::accumulate (src/Ensemble.cpp:814-894): what
+// one sample adds.
+__device__ __forceinline__ double stress_sample(int k, double molPt, const double* atomP, const double* molP) {
+    switch (k) {
+        case 1: return 1.0;
+        case 2: return molPt;
+        case 3: return (atomP[1] + atomP[3]) * 0.5;
+        case 4: return (atomP[3] - atomP[1]) * 0.5;
+        case 5: return atomP[0] - atomP[4];
+        case 6: return atomP[4] - atomP[8];
+        case 7: return (molP[0] + molP[4] + molP[8]) / 3.0;
+        case 8: return (molP[1] + molP[3]) * 0.5;
+        case 9: return (molP[3] - molP[1]) * 0.5;
+        case 10: return molP[0] - molP[4];
+        default: return molP[4] - molP[8];
+    }
+}
 
 // The kinetics kernels' totals (kinetic sums, in the MD step the pressure
 // sums and, after SHAKE, its virial) and, in the MD step, the Nose-Hoover
 // update, the pressure tensors and the stress sums.
-// One block of FINISH_THREADS after the kinetics kernel, on its stream.
+// One block of FINISH_THREADS after the kinetics kernel, on its stream, so
+// its time is a chain of latencies: everything it reads is loaded at the top,
+// two rows of partials per wave, and the epilogue's divisions run in separate
+// waves (the friction, each tensor component, the molecular pressure): 4.8 us,
+// 6.6 to 8 with one thread for all of it.
 __global__ __launch_bounds__(FINISH_THREADS) void k_kin_finish(IntegArgs a, int nb, int shake_rows) {
-    rows_total(a.part_kin + (size_t)KP_KE * nb, nb, nb, 2, a.terms + T_KE_ATOM);
-    if (a.md_step) rows_total(a.part_kin + (size_t)KP_PR * nb, nb, nb, 21, a.terms + T_PR_MC);
-    if (shake_rows) rows_total(a.part_kin + (size_t)KP_SH * nb, nb, nb, 9, a.terms + T_SH_VIR);
+    constexpr int WAVES = FINISH_THREADS / WAVE;
+    static_assert(2 * WAVES >= KIN_PARTS && FINISH_THREADS >= T_COUNT && WAVES >= 3, "k_kin_finish's shares");
+    __shared__ double tl[T_COUNT], tot[2 * WAVES], atomP[9], molP[9], molPt;
+    const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const double term = threadIdx.x < T_COUNT ? a.terms[threadIdx.x] : 0.0;
+    const double st = a.md_step && threadIdx.x < 12 ? a.stress[threadIdx.x] : 0.0;
+    const int rows = !a.md_step ? 2 : shake_rows ? KIN_PARTS : KP_SH;
+    const double* p0 = a.part_kin + (size_t)min(w, rows - 1) * nb;
+    const double* p1 = a.part_kin + (size_t)min(w + WAVES, rows - 1) * nb;
+    double s0 = 0.0, s1 = 0.0;
+#pragma unroll 4
+    for (int i = lane; i < nb; i += WAVE) {
+        s0 += p0[i];
+        s1 += p1[i];
+    }
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    if (lane == 0) {
+        tot[w] = s0;
+        tot[w + WAVES] = s1;
+    }
+    if (threadIdx.x < T_COUNT) tl[threadIdx.x] = term;
+    __syncthreads();
+    if (threadIdx.x < rows) {
+        const int k = threadIdx.x;
+        const int to = k < KP_PR ? T_KE_ATOM + k : k < KP_SH ? T_PR_MC + (k - KP_PR) : T_SH_VIR + (k - KP_SH);
+        tl[to] += tot[k];
+        a.terms[to] = tl[to];
+    }
     if (!a.md_step) return;
-    // the step's sums, read once by the whole block (the epilogue's thread
-    // then works from LDS, not from a chain of dependent global loads)
-    __shared__ double tl[T_COUNT];
     __syncthreads();
-    for (int k = threadIdx.x; k < T_COUNT; k += blockDim.x) tl[k] = a.terms[k];
+    if (w == 0 && lane < 9) md_pressure_tensor(a, tl, lane, atomP, molP);
+    if (w == 1 && lane == 0) nh_friction(a, tl[T_KE_ATOM], tl[T_KE_MOL]);
+    if (w == 2 && lane == 0) molPt = md_pressure_mol(a, tl);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        nh_friction(a, tl[T_KE_ATOM], tl[T_KE_MOL]);
-        md_pressure(a, tl);
+    if (threadIdx.x < 12) {
+        const double calls = __shfl(st, 0) + 1.0;
+        if (threadIdx.x == 0) a.stress[0] = calls;
+        else if (calls > a.stress_after) a.stress[threadIdx.x] = st + stress_sample(threadIdx.x, molPt, atomP, molP);
     }
 }
 
@@ -470,10 +539,61 @@ __global__ __launch_bounds__(KIN_THREADS) void k_kinetics(IntegArgs a, int rewra
     if (a.md_step) block_store<21>(pr, a.part_kin + (size_t)KP_PR * nb, nb);
 }
 
+// MD step, molecules of one site: the update of k_lf_atoms and, from the
+// values still in registers, the sums of k_kinetics.  As in k_shake_kinetics
+// the blocks past nb_kin add the queued partials.  Three kernels of 7.0, 6.2
+// and 3.8 us (864 atoms), each a launch and a chain of loads, became one of 5.0.
+__global__ __launch_bounds__(KIN_THREADS) void k_lf_kinetics(IntegArgs a, FlushList f) {
+    if ((int)blockIdx.x >= a.nb_kin) { flush_any(f, blockIdx.x - a.nb_kin); return; }
+    double sum[KP_SH];   // the first rows of part_kin
+#pragma unroll
+    for (int k = 0; k < KP_SH; ++k) sum[k] = 0.0;
+    double* v = sum + KP_KE;
+    double* pr = sum + KP_PR;
+    double vc[3];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    LfIn in;
+    if (i < a.n) lf_load(a, i, in);
+    drift_velocity(a, vc);
+    if (i == 0) a.flag[0] = 0;   // every consumer of the rebuild flag has run
+    if (i < a.n) {
+        double pn[3], vel[3], P[3], C[3], p[3], dr[3], vv = 0.0;
+        lf_atom(a, i, in, vc, pn, vel);
+        const double m = in.m, rm = 1.0 / m;
+        for (int d = 0; d < 3; ++d) {
+            P[d] = m * vel[d];
+            C[d] = m * pn[d] / m;
+            vv += vel[d] * vel[d];
+            p[d] = vel[d] * m;
+            dr[d] = pn[d] - C[d];
+        }
+        v[0] = vv * m;
+        v[1] = (P[0] * P[0] + P[1] * P[1] + P[2] * P[2]) / m;
+        for (int x = 0; x < 3; ++x)
+            for (int y = 0; y < 3; ++y) pr[3 * x + y] = in.F[y] * dr[x];
+        pr[9] = p[0] * rm * p[0]; pr[10] = p[0] * rm * p[1]; pr[11] = p[0] * rm * p[2];
+        pr[12] = p[1] * rm * p[1]; pr[13] = p[1] * rm * p[2]; pr[14] = p[2] * rm * p[2];
+        pr[15] = P[0] * rm * P[0]; pr[16] = P[0] * rm * P[1]; pr[17] = P[0] * rm * P[2];
+        pr[18] = P[1] * rm * P[1]; pr[19] = P[1] * rm * P[2]; pr[20] = P[2] * rm * P[2];
+        double cx = C[0], cy = C[1], cz = C[2];
+        pbc(cx, cy, cz, a.box);
+        const double sh[3] = {cx - C[0], cy - C[1], cz - C[2]}, cw[3] = {cx, cy, cz};
+        for (int d = 0; d < 3; ++d) {
+            a.mom[3 * i + d] = P[d];
+            a.pos[3 * i + d] = pn[d] + sh[d];
+            a.com[3 * i + d] = cw[d];
+        }
+    }
+    wave_store<KP_SH>(sum, a.part_kin, a.nb_kin);
+}
+
 // MD step, rigid water: SHAKE of each molecule and, from the positions and
 // velocities still in registers, its kinetic and pressure sums (the
 // arithmetic of k_kinetics), then the step's epilogue in the last block.
-__global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int rewrap) {
+// The blocks past the molecules' nb_kin add the force terms' queued partials,
+// which the sweeps hide (k_kin_finish reads both).
+__global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int rewrap, FlushList f) {
+    if ((int)blockIdx.x >= a.nb_kin) { flush_any(f, blockIdx.x - a.nb_kin); return; }
     double sv[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     double sum[KIN_PARTS];   // rows of part_kin
 #pragma unroll
@@ -538,7 +658,7 @@ __global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int
     }
 #pragma unroll
     for (int k = 0; k < 9; ++k) sum[KP_SH + k] = sv[k];
-    wave_store<KIN_PARTS>(sum, a.part_kin, gridDim.x);
+    wave_store<KIN_PARTS>(sum, a.part_kin, a.nb_kin);
 }
 
 __global__ __launch_bounds__(256) void k_mol_centers(int nmol, const int32_t* __restrict__ ms,
@@ -710,22 +830,45 @@ int kinetics_run(Ctx* c, bool rewrap, const smd_integrator_params* md) {
     return SMD_OK;
 }
 
-// The MD step's SHAKE and kinetics in one kernel (rigid 3-site water).
-static int shake_kinetics_run(Ctx* c, const smd_integrator_params* md) {
+// Arguments of a kernel that integrates the MD step and forms its sums.
+static IntegArgs step_args(Ctx* c, const smd_integrator_params* md) {
     IntegArgs a = integ_args(c, md);
     a.fnh_on_device = 1;
     a.md_step = 1;
-    a.frecip = c->shake_frecip ? c->d_frecip : nullptr;
     a.ndf = md_ndf(c);
     a.surface = c->md.ewald_on ? c->md.ewald.surface : 0;
-    a.use_constraint = c->md.ewald_on ? c->md.ewald.use_constraint : 1;
+    a.use_constraint = c->md.ewald_on ? c->md.ewald.use_constraint : (c->md.constraint_mode ? 1 : 0);
     a.lustig = c->md.lustig;
     a.stress = c->d_stress;
     a.stress_after = 0.15 * (double)c->md.total_steps;
+    a.nb_kin = (c->nmol + KIN_THREADS - 1) / KIN_THREADS;
+    return a;
+}
+
+// The MD step's update and kinetics of one-site molecules in one kernel.
+static int lf_kinetics_run(Ctx* c, const smd_integrator_params* md) {
+    IntegArgs a = step_args(c, md);
+    FlushList f;
+    int rc = red_take(c, f);
+    if (rc) return rc;
     ProfScope ps(c, "shake_kinetics");
-    const int nb = (c->nmol + KIN_THREADS - 1) / KIN_THREADS;
-    hipLaunchKernelGGL(k_shake_kinetics, dim3(nb), dim3(KIN_THREADS), 0, c->stream, a, 1);
-    hipLaunchKernelGGL(k_kin_finish, dim3(1), dim3(FINISH_THREADS), 0, c->stream, a, nb, 1);
+    hipLaunchKernelGGL(k_lf_kinetics, dim3(a.nb_kin + f.values), dim3(KIN_THREADS), 0, c->stream, a, f);
+    hipLaunchKernelGGL(k_kin_finish, dim3(1), dim3(FINISH_THREADS), 0, c->stream, a, a.nb_kin, 0);
+    SMD_HIP(c, hipGetLastError());
+    return SMD_OK;
+}
+
+// The MD step's SHAKE and kinetics in one kernel (rigid 3-site water).
+static int shake_kinetics_run(Ctx* c, const smd_integrator_params* md) {
+    IntegArgs a = step_args(c, md);
+    a.frecip = c->shake_frecip ? c->d_frecip : nullptr;
+    a.use_constraint = c->md.ewald_on ? c->md.ewald.use_constraint : 1;
+    FlushList f;
+    int rc = red_take(c, f);
+    if (rc) return rc;
+    ProfScope ps(c, "shake_kinetics");
+    hipLaunchKernelGGL(k_shake_kinetics, dim3(a.nb_kin + f.values), dim3(KIN_THREADS), 0, c->stream, a, 1, f);
+    hipLaunchKernelGGL(k_kin_finish, dim3(1), dim3(FINISH_THREADS), 0, c->stream, a, a.nb_kin, 1);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
@@ -790,12 +933,14 @@ int md_step_enqueue(Ctx* c, bool do_long) {
         // pressure sums, the NH update and the per-step rewrap
         int rc = pairlist_build(c, p.cutoff, p.cut_buff, p.use_cells, true);
         if (!rc) rc = pairs_lj(c, p.cutoff, p.switch_on, p.constraint_mode ? 1 : 0, p.lustig, p.prec, true);
+        if (!rc && !p.constraint_mode && c->one_site) return lf_kinetics_run(c, &p.integ);
         if (!rc) rc = red_flush(c);
         if (!rc) rc = p.constraint_mode ? shake_run(c, &p.integ, true, 0.0, true) : lf_atoms_run(c, &p.integ, 0.0, true);
         if (!rc) rc = kinetics_run(c, true, &p.integ);
         return rc;
     }
     const bool fork = do_long && c->recip_overlap;
+    const bool intra_beside = fork && c->ew.use_constraint;
     c->list_fork = fork ? c->ev_fork : nullptr;
     int rc = pairlist_build(c, p.cutoff, p.cut_buff, p.use_cells, true);
     c->list_fork = nullptr;
@@ -807,6 +952,8 @@ int md_step_enqueue(Ctx* c, bool do_long) {
             c->recip_store = true;
             rc = ewald_recip(c, p.prec, 0);
             c->recip_store = false;
+            // constrained molecules' intramolecular terms are sums only
+            if (!rc && intra_beside) rc = ewald_intra(c, 1);
         }
         if (rc) return rc;
         SMD_HIP(c, hipEventRecord(c->ev_join, c->stream2));
@@ -815,17 +962,16 @@ int md_step_enqueue(Ctx* c, bool do_long) {
     rc = pairs_lj_ewald(c, nullptr, nullptr, p.cutoff, p.ewald.alpha, p.ewald.real_cut, p.ewald.use_constraint,
                         1, p.prec, true);
     if (rc) return rc;
-    if ((rc = ewald_intra(c, 1))) return rc;
+    if (!intra_beside && (rc = ewald_intra(c, 1))) return rc;
     if (p.ewald.surface && (rc = ewald_surface(c))) return rc;
     if (fork) SMD_HIP(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
     else if (do_long && (rc = ewald_recip(c, p.prec, 0))) return rc;
-    if ((rc = red_flush(c))) return rc;
     // drift removal, SHAKE (adds d_frecip), clears the rebuild flag; then the
     // kinetic and pressure sums, the NH update and the per-step rewrap
     c->shake_frecip = fork;
     if (c->md_fused_shake) {
         rc = shake_kinetics_run(c, &p.integ);
-    } else {
+    } else if (!(rc = red_flush(c))) {
         rc = shake_run(c, &p.integ, true, 0.0, true);
         if (!rc) rc = kinetics_run(c, true, &p.integ);
     }

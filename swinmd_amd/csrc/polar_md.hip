@@ -139,9 +139,8 @@ static int part_c(Ctx* c) {
         }
         c->ind_real_table = false;
         c->mp_real_table = false;
-        if (!rc) rc = red_flush(c);
+        if (!rc) rc = md_tail_enqueue(c);   // which adds the queued partials
     }
-    if (!rc) rc = md_tail_enqueue(c);
     return rc;
 }
 

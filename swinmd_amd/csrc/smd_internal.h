@@ -129,6 +129,7 @@ struct Ctx {
     bool red_defer = false;       // red_finish queues instead of launching (red_flush launches)
     std::vector<RedPending> red_pending;
     double* static_scratch = nullptr;   // this device's address of ewald.hip's static scratch array
+    bool one_site = false;        // every molecule has one atom
     double* part_vom = nullptr;   // [4][nb_atoms]: k_step_head
     double* part_kin = nullptr;   // [KIN_PARTS][nb_mols64]: kinetics kernels
     double* part_sh = nullptr;    // [9][nb_mols]: k_shake
@@ -594,6 +595,36 @@ __device__ __forceinline__ void rows_total(const double* __restrict__ part, int 
     }
 }
 
+// Queued finishes for one launch: their partials' rows and destinations.
+constexpr int FLUSH_MAX = 24;
+struct FlushList {
+    const double* part[FLUSH_MAX];
+    double* dst[FLUSH_MAX];
+    int nb[FLUSH_MAX];
+    int nv[FLUSH_MAX];
+    int cap;
+    int count, values;   // finishes, values of all of them
+};
+
+// Value k of queued finish b, by one wave.
+__device__ __forceinline__ void flush_value(const FlushList& f, int b, int k) {
+    const int lane = threadIdx.x % WAVE;
+    const double* p = f.part[b] + (size_t)k * f.cap;
+    double s = 0.0;
+#pragma unroll 8
+    for (int i = lane; i < f.nb[b]; i += WAVE) s += p[i];
+    s = wave_sum(s);
+    if (lane == 0) f.dst[b][k] += s;
+}
+
+// Value v of all of them, by one wave: for kernels that carry a flush in
+// blocks of their own, beside work that does not need its results.
+__device__ __forceinline__ void flush_any(const FlushList& f, int v) {
+    int b = 0;
+    while (b < f.count && v >= f.nv[b]) v -= f.nv[b++];
+    if (b < f.count) flush_value(f, b, v);
+}
+
 template <int NV>
 __device__ __forceinline__ void block_part(double (&v)[NV], const Red& r, int site) {
     static_assert(NV <= RED_NV, "block_part: too many values for a reduction site");
@@ -638,6 +669,7 @@ int rows_finish(Ctx* c, hipStream_t s, const double* part, int stride, int nb, i
 // Launches one kernel that adds every queued finish (in queue order, each in
 // block order) and clears the queue; no-op when the queue is empty.
 int red_flush(Ctx* c);
+int red_take(Ctx* c, FlushList& f);
 // Queues finishes for the scope (a step's kernels), dropping any left over.
 struct RedDefer {
     Ctx* c;

@@ -214,3 +214,34 @@ def test_cell_list_rows_match_the_oracle(case):
     np.testing.assert_array_equal(goff, off)
     np.testing.assert_array_equal(gnb, nb)
     ctx.close()
+
+
+@pytest.mark.parametrize("cells", [1, 2, 3, 4])
+def test_lj_step_sizes_match_the_oracle(cells):
+    """4, 32, 108 and 256 atoms: part of a block of the update and kinetics
+    kernel, and whole blocks with and without a remainder; 10 steps in
+    reduced units with list rebuilds, the trajectory tests' bars."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context, WaterMD
+    s = S.lj_fcc(cells, jitter=0.02)
+    half = 0.5 * s.box[0]
+    c = dict(cutoff=min(2.5, 0.8 * half), cut_buff=0.02, dt=0.004, temperature=0.8 / 0.0083145112, coupl=0.5,
+             constraint=False, ewald=False, switch_on=True, use_cells=half > 1.5 * 2.52, atom_thermo=True)
+    print(f"case lj step {s.n_atoms} atoms", flush=True)
+    o = O.Oracle(s)
+    vel = o.init_velocity(c["temperature"], 2, per_atom=True, ndf=3 * s.n_atoms - 3)
+    ref = O.md_from_cfg(o, c, 10, velocity=vel)
+    ctx = Context(s)
+    ctx.set_velocities(vel)
+    md = WaterMD(ctx, cutoff=c["cutoff"], cut_buff=c["cut_buff"], dt=c["dt"], temperature=c["temperature"],
+                 coupl=c["coupl"], atom_thermo=True, constraint=False, ewald=False, switch_on=True,
+                 use_cells=c["use_cells"])
+    md.init()
+    md.run(4)
+    rep = md.run(6)
+    assert rep["list_updates"] == ref["list_updates"]
+    assert rel_rms(ctx.positions(), ref["pos"]) <= 1e-10
+    assert rel_rms(ctx.velocities(), ref["vel"]) <= 1e-8
+    for k in ("e_lj", "atom_ke2"):
+        assert rel(rep[k], ref[k]) <= 1e-8, k
+    ctx.close()

@@ -1308,9 +1308,13 @@ static void launch_pass(smd_batch* b, hipStream_t s, const Args& a, unsigned pas
     }
 }
 
-// The step: head, then the pair branch (list, pairs) and the reciprocal
-// branch (structure factors, per-k finish, forces), on two streams when
-// overlap is on, then SHAKE and the epilogues.
+// The step: head, then the reciprocal branch (structure factors, per-k
+// finish, forces) and the pair branch (list, pairs), on two streams when
+// overlap is on, then SHAKE and the epilogues.  The pair branch takes the
+// second stream, so that the structure factors' few large blocks are in place
+// before the list's thousands of small ones: the other way round they waited
+// for room until the pairs were done, and a step of 64 replicas (75,900
+// waters) took 983 us instead of 937.
 static int enqueue_step(smd_batch* b) {
     Args a = make_args(b);
     a.count_update = 1;
@@ -1322,11 +1326,11 @@ static int enqueue_step(smd_batch* b) {
         BHIP(b, hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
         s2 = b->stream2;
     }
-    launch_pass(b, b->stream, a, P_LIST);
-    launch_pass(b, b->stream, a, P_PAIRS);
-    launch_pass(b, s2, a, P_SFAC);
-    launch_pass(b, s2, a, P_KFIN);
-    launch_pass(b, s2, a, P_KFORCE);
+    launch_pass(b, b->stream, a, P_SFAC);
+    launch_pass(b, b->stream, a, P_KFIN);
+    launch_pass(b, b->stream, a, P_KFORCE);
+    launch_pass(b, s2, a, P_LIST);
+    launch_pass(b, s2, a, P_PAIRS);
     if (b->tiles.overlap) {
         BHIP(b, hipEventRecord(b->ev_join, b->stream2));
         BHIP(b, hipStreamWaitEvent(b->stream, b->ev_join, 0));

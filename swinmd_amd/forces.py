@@ -94,7 +94,7 @@ class Context:
         self.check(fn(self.h, _ptr(a), n))
 
     def _vec_out(self, fn, n):
-        out = np.zeros((n, 3))
+        out = np.empty((n, 3))
         self.check(fn(self.h, _ptr(out), n))
         return out
 

@@ -102,8 +102,8 @@ class ShearBatch:
         self.check(self.lib.smd_batch_run(self.h, int(nsteps)))
 
     def state(self):
-        out = {k: np.zeros((self.n, 3)) for k in ("pos", "vel", "vtm", "force")}
-        tilt = np.zeros(len(self.systems))
+        out = {k: np.empty((self.n, 3)) for k in ("pos", "vel", "vtm", "force")}
+        tilt = np.empty(len(self.systems))
         self.check(self.lib.smd_batch_get_state(self.h, _ptr(out["pos"]), _ptr(out["vel"]), _ptr(out["vtm"]),
                                                 _ptr(out["force"]), _ptr(tilt)))
         out["tilt"] = tilt

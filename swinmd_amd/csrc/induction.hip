@@ -85,7 +85,7 @@ __device__ __forceinline__ double dot3(d3 a, d3 b) { return a.x * b.x + a.y * b.
 __device__ __forceinline__ double len3(d3 a) { return sqrt(a.x * a.x + a.y * a.y + a.z * a.z); }
 
 // One thread per water (sites H1, O, H2).
-__global__ __launch_bounds__(256) void k_frames(IndArgs a) {
+__global__ __launch_bounds__(MOL_THREADS) void k_frames(IndArgs a) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= a.nmol) return;
     const int a0 = a.mol_start[m];
@@ -944,7 +944,7 @@ __device__ __forceinline__ int tri(int i, int j) { return i * (i + 1) / 2 + j; }
 __device__ __forceinline__ int stri(int i, int j) { return i >= j ? tri(i, j) : tri(j, i); }
 
 // Assembles, factors and inverts each molecule's block: thread per molecule.
-__global__ __launch_bounds__(256) void k_block_pc(IndArgs a, double* __restrict__ blk, int nmol) {
+__global__ __launch_bounds__(MOL_THREADS) void k_block_pc(IndArgs a, double* __restrict__ blk, int nmol) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= nmol) return;
     double B[45];
@@ -1288,7 +1288,7 @@ int frames_run(Ctx* c) {
     smd_induce_params p{};
     p.cutoff_ind = 1.0;
     IndArgs a = ind_args(c, &p);
-    hipLaunchKernelGGL(k_frames, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(k_frames, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, a);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
 }
@@ -1395,7 +1395,7 @@ int induce_field(Ctx* c, const smd_induce_params* p, bool frames) {
     const dim3 grid_vec((dim + CG_THREADS - 1) / CG_THREADS);
     {
         ProfScope ps(c, "ind_field");
-        if (frames) hipLaunchKernelGGL(k_frames, dim3((c->nmol + 255) / 256), b256, 0, c->stream, a);
+        if (frames) hipLaunchKernelGGL(k_frames, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, a);
         if (p->do_min && a.mixed) {
             hipLaunchKernelGGL(k_pack_ind32, dim3((n + 255) / 256), b256, 0, c->stream, a);
             // the learned guess's charge shells come out of the same pass
@@ -1457,7 +1457,7 @@ int induce_start(Ctx* c, const smd_induce_params* p) {
     if (mixed && !copied) hipLaunchKernelGGL(k_to_f32, grid_vec, b256, 0, c->stream, dim, g.x, x32);
     solve_apply(c, p, a, g.x, g.v32, g.z, nullptr, plain);
     if (p->precond == 2) {
-        hipLaunchKernelGGL(k_block_pc, dim3((c->nmol + 255) / 256), b256, 0, c->stream, a, c->d_pc_blk, c->nmol);
+        hipLaunchKernelGGL(k_block_pc, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, a, c->d_pc_blk, c->nmol);
         hipLaunchKernelGGL(k_pcg_start_blk, dim3(g.nparts_vec), dim3(BLK_THREADS), 0, c->stream, g);
         solve_apply(c, p, a, g.u, g.v32, g.z, g.p_vz, blk_top(g));   // w = A u, with the stopping test
     } else if (p->precond) hipLaunchKernelGGL(k_pcg_start, grid_vec, dim3(CG_THREADS), 0, c->stream, g);

@@ -419,12 +419,12 @@ static int launch_real(Ctx* c, const MpArgs& a, bool induction) {
     return red_finish(c, induction ? RS_IND_REAL : RS_MP_REAL, nb, 11, a.terms + M_REAL_E);
 }
 
-__global__ __launch_bounds__(256) void k_mp_torques(MpArgs a, unsigned parts, int site);
+__global__ __launch_bounds__(MOL_THREADS) void k_mp_torques(MpArgs a, unsigned parts, int site);
 
 // Torques to forces, then the sums of its dU/dV and torque terms (sites
 // `site` and `site + 1`: each launch of a step has its own pair).
 static int launch_torques(Ctx* c, const MpArgs& a, dim3 g, unsigned parts, int site) {
-    hipLaunchKernelGGL(k_mp_torques, g, dim3(256), 0, c->stream, a, parts, site);
+    hipLaunchKernelGGL(k_mp_torques, g, dim3(MOL_THREADS), 0, c->stream, a, parts, site);
     int rc = red_finish(c, site, g.x, 5, a.terms + M_DUDV);
     if (!rc) rc = red_finish(c, site + 1, g.x, 5, a.terms + M_TRQ);
     return rc;
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void k_mp_site_sums(MpArgs a) {
 
 // One thread per molecule: excluded pairs inside it with erf-screened D_l
 // (intraMolCorrect :1350-1600).  Forces and torques only without constraints.
-__global__ __launch_bounds__(256) void k_mp_intra(MpArgs a) {
+__global__ __launch_bounds__(MOL_THREADS) void k_mp_intra(MpArgs a) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     double v[2] = {0.0, 0.0};
     if (m < a.nmol) {
@@ -594,7 +594,7 @@ __device__ __forceinline__ V3 h_site(V3 rh, V3 ro, V3 tau, double& dudv) {
 
 // One thread per water; the torque-array parts set in `parts` (bit p for
 // part p), each part's dU/dV summed into its own slot.
-__global__ __launch_bounds__(256) void k_mp_torques(MpArgs a, unsigned parts, int site) {
+__global__ __launch_bounds__(MOL_THREADS) void k_mp_torques(MpArgs a, unsigned parts, int site) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     double dv[5] = {0, 0, 0, 0, 0}, tn[5] = {0, 0, 0, 0, 0};
     if (m < a.nmol) {
@@ -959,14 +959,14 @@ int multipole_short(Ctx* c, smd_mp_out* out) {
                     c->list_cutoff + c->list_buff);
     MpArgs a = mp_args(c);
     const dim3 b256(256);
-    const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 ga((c->n + 255) / 256), gm(mol_blocks(c));
     ProfScope ps(c, "mp_short");
     SMD_HIP(c, hipMemsetAsync(c->d_mp_terms, 0, sizeof(double) * M_COUNT, c->stream));
     if ((rc = frames_run(c))) return rc;
     hipLaunchKernelGGL(k_mp_site_sums, ga, b256, 0, c->stream, a);
     if ((rc = site_sums_finish(c, a, ga.x, false))) return rc;
     if ((rc = launch_real(c, a, false))) return rc;
-    hipLaunchKernelGGL(k_mp_intra, gm, b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_mp_intra, gm, dim3(MOL_THREADS), 0, c->stream, a);
     if ((rc = red_finish(c, RS_MP_INTRA, gm.x, 2, a.terms + M_INTRA_E))) return rc;
     const double volume = a.volume, volumer = 1.0 / volume;
     const double coeff = 2.0 * PI * volumer / 3.0;
@@ -1027,7 +1027,7 @@ int multipole_long(Ctx* c, smd_mp_long_out* out) {
     if (c->mp_prec == SMD_PREC_MIXED) hipLaunchKernelGGL((k_mp_kforce<float>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
         else hipLaunchKernelGGL((k_mp_kforce<double>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
     hipLaunchKernelGGL(k_kforce_sum, dim3((c->n + 255) / 256), b256, 0, c->stream, a);
-    if (c->mp.torques && (rc = launch_torques(c, a, dim3((c->nmol + 255) / 256), 8u, RS_MP_DUDV_L))) return rc;
+    if (c->mp.torques && (rc = launch_torques(c, a, dim3(mol_blocks(c)), 8u, RS_MP_DUDV_L))) return rc;
     SMD_HIP(c, hipGetLastError());
     double t[M_COUNT];
     if ((rc = mp_read_terms(c, t))) return rc;
@@ -1419,7 +1419,7 @@ __global__ __launch_bounds__(256) void k_ind_site_sums(MpArgs a) {
 
 // One thread per molecule: excluded pairs inside it (intraMolCorrect
 // :1850-1985).  Forces and torques only without constraints.
-__global__ __launch_bounds__(256) void k_ind_intra(MpArgs a) {
+__global__ __launch_bounds__(MOL_THREADS) void k_ind_intra(MpArgs a) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     double v[2] = {0.0, 0.0};
     if (m < a.nmol) {
@@ -1918,14 +1918,14 @@ int induction_short(Ctx* c, smd_indf_out* out) {
                     c->list_cutoff + c->list_buff);
     MpArgs a = ind_args(c);
     const dim3 b256(256);
-    const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 ga((c->n + 255) / 256), gm(mol_blocks(c));
     ProfScope ps(c, "ind_short");
     SMD_HIP(c, hipMemsetAsync(c->d_mp_terms, 0, sizeof(double) * M_COUNT, c->stream));
     if ((rc = frames_run(c))) return rc;
     hipLaunchKernelGGL(k_ind_site_sums, ga, b256, 0, c->stream, a);
     if ((rc = site_sums_finish(c, a, ga.x, true))) return rc;
     if ((rc = launch_real(c, a, true))) return rc;
-    hipLaunchKernelGGL(k_ind_intra, gm, b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_ind_intra, gm, dim3(MOL_THREADS), 0, c->stream, a);
     if ((rc = red_finish(c, RS_IND_INTRA, gm.x, 2, a.terms + M_INTRA_E))) return rc;
     const double volume = a.volume, volumer = 1.0 / volume;
     const double coeff = 2.0 * PI * volumer / 3.0;
@@ -1986,7 +1986,7 @@ int induction_long(Ctx* c, smd_mp_long_out* out) {
     if (c->mp_prec == SMD_PREC_MIXED) hipLaunchKernelGGL((k_ind_kforce<float>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
         else hipLaunchKernelGGL((k_ind_kforce<double>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
     hipLaunchKernelGGL(k_kforce_sum, dim3((c->n + 255) / 256), b256, 0, c->stream, a);
-    if (c->indf.torques && (rc = launch_torques(c, a, dim3((c->nmol + 255) / 256), 8u, RS_IND_DUDV_L))) return rc;
+    if (c->indf.torques && (rc = launch_torques(c, a, dim3(mol_blocks(c)), 8u, RS_IND_DUDV_L))) return rc;
     SMD_HIP(c, hipGetLastError());
     double t[M_COUNT];
     if ((rc = mp_read_terms(c, t))) return rc;
@@ -2063,12 +2063,12 @@ void polar_join(Ctx* c) { (void)hipStreamWaitEvent(c->stream, c->ev_join, 0); }
 // space, intramolecular, surface, their torques), into a.terms and d_force.
 static int mp_short_enqueue(Ctx* c, const MpArgs& a) {
     int rc;
-    const dim3 b256(256), ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 b256(256), ga((c->n + 255) / 256), gm(mol_blocks(c));
     ProfScope ps(c, "mp_short");
     hipLaunchKernelGGL(k_mp_site_sums, ga, b256, 0, c->stream, a);
     if ((rc = site_sums_finish(c, a, ga.x, false))) return rc;
     if ((rc = launch_real(c, a, false))) return rc;
-    hipLaunchKernelGGL(k_mp_intra, gm, b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_mp_intra, gm, dim3(MOL_THREADS), 0, c->stream, a);
     if ((rc = red_finish(c, RS_MP_INTRA, gm.x, 2, a.terms + M_INTRA_E))) return rc;
     if (c->mp.surface) {
         hipLaunchKernelGGL(k_mp_surface, ga, b256, 0, c->stream, a, 2.0 * PI * (1.0 / a.volume) / 3.0);
@@ -2080,12 +2080,12 @@ static int mp_short_enqueue(Ctx* c, const MpArgs& a) {
 
 static int ind_short_enqueue(Ctx* c, const MpArgs& a) {
     int rc;
-    const dim3 b256(256), ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 b256(256), ga((c->n + 255) / 256), gm(mol_blocks(c));
     ProfScope ps(c, "ind_short");
     hipLaunchKernelGGL(k_ind_site_sums, ga, b256, 0, c->stream, a);
     if ((rc = site_sums_finish(c, a, ga.x, true))) return rc;
     if ((rc = launch_real(c, a, true))) return rc;
-    hipLaunchKernelGGL(k_ind_intra, gm, b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_ind_intra, gm, dim3(MOL_THREADS), 0, c->stream, a);
     if ((rc = red_finish(c, RS_IND_INTRA, gm.x, 2, a.terms + M_INTRA_E))) return rc;
     if (c->indf.surface) {
         hipLaunchKernelGGL(k_ind_surface, ga, b256, 0, c->stream, a, 2.0 * PI * (1.0 / a.volume) / 3.0);
@@ -2101,7 +2101,7 @@ int multipole_enqueue(Ctx* c, double* terms) {
     MpArgs a = mp_args(c);
     a.terms = terms;
     const dim3 b256(256);
-    const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 ga((c->n + 255) / 256), gm(mol_blocks(c));
     hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, terms);
     // the k-space sums and per-site partial forces on the second stream,
     // beside the real-space kernels (they touch none of the same buffers)
@@ -2126,7 +2126,7 @@ int induction_enqueue(Ctx* c, double* terms) {
     MpArgs a = ind_args(c);
     a.terms = terms;
     const dim3 b256(256);
-    const dim3 ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 ga((c->n + 255) / 256), gm(mol_blocks(c));
     hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, terms);
     const bool fork = polar_fork_begin(c);
     int rc_long = fork ? mp_long_sums(c, a, false) : SMD_OK;
@@ -2196,7 +2196,7 @@ int polar_joint_enqueue(Ctx* c, double* mp_t, double* ind_t, bool with_mp_short,
     ai.terms = ind_t;
     use_table(c, am, c->mp_real_table);
     use_table(c, ai, c->ind_real_table);
-    const dim3 b256(256), ga((c->n + 255) / 256), gm((c->nmol + 255) / 256);
+    const dim3 b256(256), ga((c->n + 255) / 256), gm(mol_blocks(c));
     if (with_mp_short) hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, mp_t);
     hipLaunchKernelGGL(k_zero_terms, dim3(1), b256, 0, c->stream, ind_t);
     auto long_sums = [&]() -> int {

@@ -711,7 +711,7 @@ __global__ void k_virtual_sites(int nmol, const int32_t* __restrict__ mol_start,
 // Moves the force on each virtual site back onto its atom and host atom
 // (BuffvdWForce.cpp:262-274, BuckinghamForce.cpp:217-238); one thread per
 // molecule, so the molecule's atoms have a single writer.
-__global__ __launch_bounds__(256) void k_redistribute(int nmol, const int32_t* __restrict__ mol_start,
+__global__ __launch_bounds__(MOL_THREADS) void k_redistribute(int nmol, const int32_t* __restrict__ mol_start,
                                                       const double* __restrict__ fa, const double* __restrict__ fb,
                                                       const int32_t* __restrict__ host,
                                                       const double* __restrict__ fvirt, double* __restrict__ force) {
@@ -742,12 +742,12 @@ int vdw_run(Ctx* c, const smd_vdw_params* p, int prec, smd_vdw_out* out, bool re
     case SMD_VDW_MIE: e = launch_pairs<V_MIE, false>(c, a, prec, lustig); break;
     case SMD_VDW_BUCK:
     case SMD_VDW_BUFF147:
-        hipLaunchKernelGGL(k_virtual_sites, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, c->nmol,
+        hipLaunchKernelGGL(k_virtual_sites, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, c->nmol,
                            c->d_mol_start, c->d_type, c->d_pos, c->d_epos, p->kind, p->hfactor, p->co2_bond);
         e = (p->kind == SMD_VDW_BUCK) ? launch_pairs<V_BUCK, false>(c, a, prec, lustig)
                                       : launch_pairs<V_BUFF, false>(c, a, prec, lustig);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_redistribute, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, c->nmol,
+            hipLaunchKernelGGL(k_redistribute, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, c->nmol,
                                c->d_mol_start, c->d_fa, c->d_fb, c->d_host, c->d_fvirt, c->d_force);
             e = hipGetLastError();
         }
@@ -1174,7 +1174,7 @@ int vdw_enqueue(Ctx* c, const smd_vdw_params* p, int prec) {
     switch (p->kind) {
     case SMD_VDW_LJ: e = launch_pairs<V_LJ, false>(c, a, prec, lustig); break;
     case SMD_VDW_BUFF147:
-        hipLaunchKernelGGL(k_virtual_sites, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, c->nmol,
+        hipLaunchKernelGGL(k_virtual_sites, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, c->nmol,
                            c->d_mol_start, c->d_type, c->d_pos, c->d_epos, p->kind, p->hfactor, p->co2_bond);
         if (prec == SMD_PREC_MIXED && c->d_vrec) {
             hipLaunchKernelGGL(k_pack_vsites, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->n, c->d_epos,
@@ -1184,7 +1184,7 @@ int vdw_enqueue(Ctx* c, const smd_vdw_params* p, int prec) {
         }
         e = launch_pairs<V_BUFF, false>(c, a, prec, lustig);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_redistribute, dim3((c->nmol + 255) / 256), dim3(256), 0, c->stream, c->nmol,
+            hipLaunchKernelGGL(k_redistribute, dim3(mol_blocks(c)), dim3(MOL_THREADS), 0, c->stream, c->nmol,
                                c->d_mol_start, c->d_fa, c->d_fb, c->d_host, c->d_fvirt, c->d_force);
             e = hipGetLastError();
         }

@@ -331,6 +331,15 @@ struct Ctx {
 inline int row_lanes(int n) { return n >= 12288 ? 16 : n >= 6144 ? 32 : 64; }
 inline int cg_lanes(const Ctx* c) { return c->cg_lanes ? c->cg_lanes : row_lanes(c->n); }
 
+// Threads per block of the kernels with a thread per molecule: one wave, so
+// that 8,192 molecules reach 128 CUs and not 32; each lasts as long as its
+// thread's chain of loads and FP64 arithmetic.  Against 256 threads, at 1,024
+// and 8,192 waters in us: torques 8.7 -> 7.2 and 9.3 -> 7.6, block
+// preconditioner 10.1 -> 7.2 and 28 -> 19, redistribution 5.2 -> 3.9 and
+// 14.4 -> 10.5, intramolecular terms about the same.
+constexpr int MOL_THREADS = 64;
+inline unsigned mol_blocks(const Ctx* c) { return (unsigned)((c->nmol + MOL_THREADS - 1) / MOL_THREADS); }
+
 // f(std::integral_constant<int, lanes>) for a row kernel's lanes.
 template <typename F> void with_lanes(int lanes, F f) {
     switch (lanes) {

@@ -854,22 +854,18 @@ __global__ __launch_bounds__(WAVE) void k_mp_kforce(MpArgs a) {
 
 // The k-range partials of each site in order: force added, k-space torque
 // stored (torque-array part 3).
+// A thread per value, so that the loads of the ranges are whole lines and
+// many are in flight: 1,024 waters with 43 ranges 5.6 us, a thread per site
+// 16.
 __global__ __launch_bounds__(256) void k_kforce_sum(MpArgs a) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n) return;
-    double F[6] = {0, 0, 0, 0, 0, 0};
-    for (int s = 0; s < a.ksplit; ++s) {
-        const double* p = a.fpart + ((size_t)s * a.n + i) * 6;
-#pragma unroll
-        for (int x = 0; x < 6; ++x) F[x] += p[x];
-    }
-    a.force[3 * i] += COULOMBS * F[0];
-    a.force[3 * i + 1] += COULOMBS * F[1];
-    a.force[3 * i + 2] += COULOMBS * F[2];
-    double* tr = a.trq + 9 * (size_t)a.n;
-    tr[3 * i] = COULOMBS * F[3];
-    tr[3 * i + 1] = COULOMBS * F[4];
-    tr[3 * i + 2] = COULOMBS * F[5];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 6 * a.n) return;
+    const int i = t / 6, x = t % 6;
+    double f = 0.0;
+#pragma unroll 8
+    for (int s = 0; s < a.ksplit; ++s) f += a.fpart[(size_t)s * a.n * 6 + t];
+    if (x < 3) a.force[3 * i + x] += COULOMBS * f;
+    else a.trq[9 * (size_t)a.n + 3 * i + x - 3] = COULOMBS * f;
 }
 
 // ---- host side ---------------------------------------------------------------------
@@ -1026,7 +1022,7 @@ int multipole_long(Ctx* c, smd_mp_long_out* out) {
     if ((rc = red_finish(c, RS_MP_LONG, (a.K + 3) / 4, 9, a.terms + M_LONG_E))) return rc;
     if (c->mp_prec == SMD_PREC_MIXED) hipLaunchKernelGGL((k_mp_kforce<float>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
         else hipLaunchKernelGGL((k_mp_kforce<double>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
-    hipLaunchKernelGGL(k_kforce_sum, dim3((c->n + 255) / 256), b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_kforce_sum, dim3((6 * c->n + 255) / 256), b256, 0, c->stream, a);
     if (c->mp.torques && (rc = launch_torques(c, a, dim3(mol_blocks(c)), 8u, RS_MP_DUDV_L))) return rc;
     SMD_HIP(c, hipGetLastError());
     double t[M_COUNT];
@@ -1985,7 +1981,7 @@ int induction_long(Ctx* c, smd_mp_long_out* out) {
     if ((rc = red_finish(c, RS_IND_LONG, (a.K + 3) / 4, 9, a.terms + M_LONG_E))) return rc;
     if (c->mp_prec == SMD_PREC_MIXED) hipLaunchKernelGGL((k_ind_kforce<float>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
         else hipLaunchKernelGGL((k_ind_kforce<double>), dim3((c->n + WAVE - 1) / WAVE, a.ksplit), dim3(WAVE), 0, c->stream, a);
-    hipLaunchKernelGGL(k_kforce_sum, dim3((c->n + 255) / 256), b256, 0, c->stream, a);
+    hipLaunchKernelGGL(k_kforce_sum, dim3((6 * c->n + 255) / 256), b256, 0, c->stream, a);
     if (c->indf.torques && (rc = launch_torques(c, a, dim3(mol_blocks(c)), 8u, RS_IND_DUDV_L))) return rc;
     SMD_HIP(c, hipGetLastError());
     double t[M_COUNT];
@@ -2114,7 +2110,7 @@ int multipole_enqueue(Ctx* c, double* terms) {
     else if ((rc = mp_long_sums(c, a, true))) return rc;
     {
         ProfScope ps(c, "mp_long");
-        hipLaunchKernelGGL(k_kforce_sum, ga, b256, 0, c->stream, a);
+        hipLaunchKernelGGL(k_kforce_sum, dim3((6 * c->n + 255) / 256), b256, 0, c->stream, a);
         if (c->mp.torques && (rc = launch_torques(c, a, gm, 8u, RS_MP_DUDV_L))) return rc;
     }
     SMD_HIP(c, hipGetLastError());
@@ -2137,7 +2133,7 @@ int induction_enqueue(Ctx* c, double* terms) {
     else if ((rc = mp_long_sums(c, a, false))) return rc;
     {
         ProfScope ps(c, "ind_long");
-        hipLaunchKernelGGL(k_kforce_sum, ga, b256, 0, c->stream, a);
+        hipLaunchKernelGGL(k_kforce_sum, dim3((6 * c->n + 255) / 256), b256, 0, c->stream, a);
         if (c->indf.torques && (rc = launch_torques(c, a, gm, 8u, RS_IND_DUDV_L))) return rc;
     }
     SMD_HIP(c, hipGetLastError());
@@ -2231,7 +2227,7 @@ int polar_joint_enqueue(Ctx* c, double* mp_t, double* ind_t, bool with_mp_short,
     else if ((rc = long_sums())) return rc;
     {
         ProfScope ps(c, "ind_long");
-        hipLaunchKernelGGL(k_kforce_sum, ga, b256, 0, c->stream, ai);
+        hipLaunchKernelGGL(k_kforce_sum, dim3((6 * c->n + 255) / 256), b256, 0, c->stream, ai);
         if (c->indf.torques && (rc = launch_torques(c, ai, gm, 8u, RS_IND_DUDV_L))) return rc;
     }
     SMD_HIP(c, hipGetLastError());

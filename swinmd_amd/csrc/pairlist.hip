@@ -375,6 +375,9 @@ __global__ __launch_bounds__(LB_THREADS) void k_list_hits(ListArgs a, CellGrid g
 // lines: 45 us at 4,096 waters (430 partners a row), 20 at 1,021; a lane per
 // atom and neighbour, each storing to its own row, took 52 and 36 and a pass
 // for the slots before it.
+// A row longer than the stride is cut to it and filled: owned atoms to its
+// end, the others in the slots the owned leave.  In the MD step the pair
+// kernels walk the row, up to the stride, before the host reads the status.
 constexpr int LR_THREADS = 1024;
 constexpr int ROW_LDS = 1024;   // longest row put in order in LDS
 __global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g, const int32_t* __restrict__ start,
@@ -467,8 +470,11 @@ __global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g
         a.nb_own[i] = own_all;
         if (all > a.stride) atomicOr(a.status, ST_LIST_OVERFLOW);
     }
-    if (all > a.stride) return;
     int32_t* row = a.nb + (int64_t)i * a.stride;
+    auto store = [&](int t, int at) {   // the t-th hit, owned ones first
+        const int to = t < own_all ? t : a.stride - 1 - (t - own_all);
+        if (t < own_all ? to < a.stride : to >= own_all) row[to] = catoms[at];
+    };
     int32_t* order = ranked[threadIdx.x / WAVE];
     const bool in_lds = all <= ROW_LDS;
     auto place = [&](int h, uint32_t bits) {
@@ -479,7 +485,7 @@ __global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g
             const bool own_hit = mine >> b & 1u;
             const int to = own_hit ? own_at++ : own_all + non_at++;
             if (in_lds) order[to] = at;
-            else row[own_hit ? to : a.stride - 1 - (to - own_all)] = catoms[at];
+            else store(to, at);
         }
     };
 #pragma unroll
@@ -487,7 +493,7 @@ __global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g
     for (int h = h0 + WORDS; h < h1; ++h) place(h, hits(h));
     if (!in_lds) return;
     wave_lds_order();
-    for (int t = lane; t < all; t += WAVE) row[t < own_all ? t : a.stride - 1 - (t - own_all)] = catoms[order[t]];
+    for (int t = lane; t < all; t += WAVE) store(t, order[t]);
 }
 
 // Ensemble::build_pairlist (src/Ensemble.cpp:492-525): all j != i with the

@@ -245,3 +245,37 @@ def test_lj_step_sizes_match_the_oracle(cells):
     for k in ("e_lj", "atom_ke2"):
         assert rel(rep[k], ref[k]) <= 1e-8, k
     ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["lj", "water"])
+@pytest.mark.parametrize("cells", [True, False])
+@pytest.mark.parametrize("prec", [L.PREC_FP64, L.PREC_MIXED])
+def test_rows_outgrowing_the_list_in_a_step_are_an_error(kind, cells, prec):
+    """Atoms in a box of 4 fall towards its middle, every distance shrinking by
+    the same factor, so that rows pass the capacity fixed when the step was
+    set up (1.5 times the first rows, and more) in a rebuild inside the run.
+    The pair kernels of that step and the next walk the cut rows; the run
+    ends with the capacity's error."""
+    from swinmd_amd._lib import SMD_ECAPACITY, SmdError
+    from swinmd_amd.forces import Context, WaterMD
+    print(f"case outgrown rows {kind} cells={cells} prec={prec}", flush=True)
+    dt, steps, shrink = 0.002, 10, 0.5 if kind == "lj" else 0.6
+    if kind == "lj":
+        s = S.lj_fcc(5, rho=500 / 64.0, sigma=0.15, eps=1e-6)
+        com = s.pos
+    else:
+        s = S.water(343, box=4.0, seed=4, subset=True, jitter=0.0)
+        com = np.repeat(s.pos.reshape(-1, 3, 3).mean(1), 3, axis=0)
+    ctx = Context(s)
+    vel = -com * (1 - shrink) / (steps * dt)
+    # the thermostat holds the fall's own kinetic energy
+    temperature = float((s.mass[:, None] * vel ** 2).sum() / ((3 if kind == "lj" else 2) * s.n_atoms * 0.0083145112))
+    ctx.set_velocities(vel)
+    md = WaterMD(ctx, cutoff=0.9, cut_buff=0.1, dt=dt, temperature=temperature, coupl=10.0, use_cells=cells, prec=prec,
+                 constraint=kind == "water", ewald=kind == "water", kcut=S.kcut_for(3, 4.0))
+    md.init()
+    assert md.run(2)["list_updates"] >= 1
+    with pytest.raises(SmdError) as e:
+        md.run(steps)
+    assert e.value.code == SMD_ECAPACITY
+    ctx.close()

@@ -178,7 +178,7 @@ __device__ __forceinline__ void shake_mol(const IntegArgs& a, int m, const Shake
     } else {
         // Coordinate form of the same sweeps with the minimum image of each
         // bond.  The update is predicated instead of branched: an inactive
-        // constraint moves its atoms by exactly 0.0.
+        // constraint and a failed molecule move by exactly 0.0.
         const double tol_2 = 2 * a.tol;
         int count = 0;
         while (!done && count < a.max_count && !failed) {
@@ -194,7 +194,7 @@ __device__ __forceinline__ void shake_mol(const IntegArgs& a, int m, const Shake
                 const bool act = fabs(diff) > in.bl[b] * tol_2;
                 failed = failed || (act && rno < in.bl[b] * a.tol);
                 const double q = diff / (2 * rno * (mr[b] + mr[nx]));
-                const double factor = act ? q : 0.0;
+                const double factor = act && !failed ? q : 0.0;
                 wv[b][0] += factor * nX; wv[b][1] += factor * nY; wv[b][2] += factor * nZ;
                 const double fX = factor * oX, fY = factor * oY, fZ = factor * oZ;
                 rn[b][0] += mr[b] * fX; rn[b][1] += mr[b] * fY; rn[b][2] += mr[b] * fZ;

@@ -22,8 +22,9 @@
 
 namespace smd {
 
-// q = n / d to about an ulp: hardware reciprocal, one Newton step, then the
-// quotient corrected by its residual.  d > 0 and normal.
+// q = n / d to about an ulp: hardware reciprocal, two Newton steps, then the
+// quotient corrected by its residual.  d > 0 and normal; the sweeps drop the
+// quotients of any other.
 __device__ __forceinline__ double quotient(double n, double d) {
     double r = __builtin_amdgcn_rcp(d);
     r = fma(fma(-d, r, 1.0), r, r);
@@ -70,7 +71,8 @@ __device__ __forceinline__ void shake_sweeps(const double (&od)[3][3], const dou
             const bool act = fabs(diff) > bl[b] * tol_2;
             failed = failed || (act && rno < bl[b] * tol);
             const double q = quotient(diff, rno * hm[b]);
-            const double f = act ? q : 0.0;
+            // a failed molecule moves no further: its positions stay finite
+            const double f = act && !failed ? q : 0.0;
             done = done && !act;
 #pragma unroll
             for (int j = 0; j < 3; ++j) W[b][j] = fma(f, lam[j], W[b][j]);

@@ -279,3 +279,67 @@ def test_rows_outgrowing_the_list_in_a_step_are_an_error(kind, cells, prec):
         md.run(steps)
     assert e.value.code == SMD_ECAPACITY
     ctx.close()
+
+
+def _turned_over(s, m, dt):
+    """Velocities that take molecule m's first hydrogen past its oxygen in one
+    step: the new bond is twice as long and points 0.01 of it back, which
+    SHAKE refuses (LFIntegrator.cpp:1519-1523) at its first constraint."""
+    v = np.zeros((s.n_atoms, 3))
+    bond = s.pos[3 * m] - s.pos[3 * m + 1]
+    side = np.cross(bond, [0.3, 0.5, 0.8])
+    new = -0.01 * bond + 2 * np.linalg.norm(bond) * side / np.linalg.norm(side)
+    v[3 * m] = (new - bond) / dt
+    return v
+
+
+@pytest.mark.parametrize("wrap", [False, True])
+def test_a_step_shake_refuses_leaves_its_molecule_unmoved(wrap):
+    """The run ends with the constraint error, and the refused molecule is
+    where its velocities took it, within the forces' dt^2 F / m < 0.01 nm, not
+    where the refused quotient would put it, 15 nm away.  wrap: a molecule
+    across the box face, where the sweeps take minimum images."""
+    from swinmd_amd._lib import SMD_ESHAKE, SmdError
+    from swinmd_amd.forces import Context, WaterMD
+    s, cfg = _water_cfg(64)
+    print(f"case refused step wrap={wrap}", flush=True)
+    box, dt = s.box[0], 1e-4
+    if wrap:   # hydrogens and oxygens of one molecule on either side of a face
+        s.pos = s.pos - s.pos[0] * [1, 0, 0] + [0.5 * box - 1e-3, 0, 0]
+        s.pos = s.pos - box * np.rint(s.pos / box)
+    ctx = Context(s)
+    vel = _turned_over(s, 0, dt)
+    if wrap:
+        whole = s.pos[:3] - box * np.rint((s.pos[:3] - s.pos[1]) / box)
+        assert np.abs(whole - s.pos[:3]).max() > 1
+    ctx.set_velocities(vel)
+    md = WaterMD(ctx, **{**{k: cfg[k] for k in ("cutoff", "cut_buff", "alpha", "kcut", "use_cells")}, "dt": dt,
+                         "temperature": 300.0, "coupl": 1e3})
+    md.init()
+    with pytest.raises(SmdError) as e:
+        md.run(1)
+    assert e.value.code == SMD_ESHAKE
+    d = ctx.positions()[:3] - (s.pos[:3] + dt * vel[:3])
+    d -= box * np.rint(d / box)
+    assert np.abs(d).max() < 0.01
+    ctx.close()
+
+
+def test_a_replica_step_shake_refuses_leaves_its_molecule_unmoved():
+    """As the step above, for the sheared replicas' step."""
+    from swinmd_amd._lib import SMD_ESHAKE, SmdError
+    from swinmd_amd.nemd import ShearBatch
+    s = S.water(256, density_mol=RHO, seed=8, subset=True)
+    print("case refused replica step", flush=True)
+    box, dt = s.box[0], 1e-4
+    vel = _turned_over(s, 7, dt)
+    b = ShearBatch([s], [0.5], cutoff=0.8, cut_buff=0.08, alpha=3.5, n2max=20, dt=dt, temperature=300.0, coupl=1e3)
+    b.set_state([s.pos], [vel], [0.0])
+    b.start()
+    with pytest.raises(SmdError) as e:
+        b.run(1)
+    assert e.value.code == SMD_ESHAKE
+    d = b.state()["pos"][21:24] - (s.pos[21:24] + dt * vel[21:24])
+    d -= box * np.rint(d / box)
+    assert np.abs(d).max() < 0.01
+    b.close()

@@ -55,18 +55,22 @@ int rows_finish(Ctx* c, hipStream_t s, const double* part, int stride, int nb, i
     return SMD_OK;
 }
 
-int red_finish(Ctx* c, int site, unsigned nblocks, int nv, double* dst) {
+int red_finish(Ctx* c, int site, unsigned nblocks, int nv, double* dst, int first) {
     if ((int)nblocks > c->red.cap)
         return fail(c, SMD_ECAPACITY, "reduction over %u blocks exceeds the arena's %d", nblocks, c->red.cap);
     if (nblocks == 0) return SMD_OK;
     if (c->red_defer) {
-        for (const RedPending& q : c->red_pending)
-            if (q.site == site) return fail(c, SMD_ESTATE, "reduction site %d queued twice in one step", site);
-        c->red_pending.push_back(RedPending{site, nblocks, nv, dst});
+        for (const RedPending& q : c->red_pending) {
+            if (q.site == site && first < q.first + q.nv && q.first < first + nv)
+                return fail(c, SMD_ESTATE, "reduction site %d queued twice in one step", site);
+            if (dst < q.dst + q.nv && q.dst < dst + nv)
+                return fail(c, SMD_ESTATE, "reduction sites %d and %d queued for one sum", q.site, site);
+        }
+        c->red_pending.push_back(RedPending{site, first, nblocks, nv, dst});
         return SMD_OK;
     }
     hipLaunchKernelGGL(k_red_finish, dim3(1), dim3(FINISH_THREADS), 0, c->stream,
-                       c->red.base + (size_t)site * RED_NV * c->red.cap, c->red.cap, (int)nblocks, nv, dst, 1 << 30,
+                       c->red.base + ((size_t)site * RED_NV + first) * c->red.cap, c->red.cap, (int)nblocks, nv, dst, 1 << 30,
                        (double*)nullptr);
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
@@ -86,7 +90,7 @@ int red_take(Ctx* c, FlushList& f) {
         return fail(c, SMD_ESTATE, "%zu queued reductions exceed %d", c->red_pending.size(), FLUSH_MAX);
     for (const RedPending& r : c->red_pending) {
         const int q = f.count++;
-        f.part[q] = c->red.base + (size_t)r.site * RED_NV * c->red.cap;
+        f.part[q] = c->red.base + ((size_t)r.site * RED_NV + r.first) * c->red.cap;
         f.dst[q] = r.dst;
         f.nb[q] = (int)r.nb;
         f.nv[q] = r.nv;

@@ -422,11 +422,19 @@ static int launch_real(Ctx* c, const MpArgs& a, bool induction) {
 __global__ __launch_bounds__(MOL_THREADS) void k_mp_torques(MpArgs a, unsigned parts, int site);
 
 // Torques to forces, then the sums of its dU/dV and torque terms (sites
-// `site` and `site + 1`: each launch of a step has its own pair).
+// `site` and `site + 1`: each launch of a step has its own pair).  Queued, a
+// finish per run of parts that this launch formed: the step's other launch
+// adds the others, in the same flush.
 static int launch_torques(Ctx* c, const MpArgs& a, dim3 g, unsigned parts, int site) {
     hipLaunchKernelGGL(k_mp_torques, g, dim3(MOL_THREADS), 0, c->stream, a, parts, site);
-    int rc = red_finish(c, site, g.x, 5, a.terms + M_DUDV);
-    if (!rc) rc = red_finish(c, site + 1, g.x, 5, a.terms + M_TRQ);
+    int rc = SMD_OK;
+    for (int p = 0, e; p < 5 && !rc; p = e) {
+        e = p + 1;
+        if (c->red_defer && !(parts >> p & 1u)) continue;
+        while (e < 5 && (!c->red_defer || parts >> e & 1u)) ++e;
+        rc = red_finish(c, site, g.x, e - p, a.terms + M_DUDV + p, p);
+        if (!rc) rc = red_finish(c, site + 1, g.x, e - p, a.terms + M_TRQ + p, p);
+    }
     return rc;
 }
 

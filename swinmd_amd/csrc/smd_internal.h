@@ -40,7 +40,7 @@ inline size_t red_doubles(int cap) { return (size_t)RS_COUNT * RED_NV * cap; }
 // A finish that waits for red_flush (inside a step, where one kernel then
 // adds every site's partials).
 struct RedPending {
-    int site;
+    int site, first;   // values first.. first + nv - 1 of the site
     unsigned nb;
     int nv;
     double* dst;
@@ -664,9 +664,11 @@ int ewald_surface(Ctx* c);
 enum : unsigned { RECIP_SFAC = 1u, RECIP_REDUCE = 2u, RECIP_FORCE = 4u, RECIP_ALL = 7u };
 int ewald_recip(Ctx* c, int prec, int lustig, unsigned passes = RECIP_ALL);
 int static_scratch_init(Ctx* c);
-// Adds the nv block partials of a site's last launch (nblocks blocks) to dst,
-// in block order, on the context's stream.
-int red_finish(Ctx* c, int site, unsigned nblocks, int nv, double* dst);
+// Adds the block partials of nv values of a site's last launch (nblocks
+// blocks), from value `first` on, to dst, in block order, on the context's
+// stream.  Queued finishes (RedDefer) are added side by side: no two may share
+// a destination.
+int red_finish(Ctx* c, int site, unsigned nblocks, int nv, double* dst, int first = 0);
 // Adds rows [0, nrows) of block partials part[k * stride + b], b < nb, to
 // dst in block order: one block of FINISH_THREADS on stream s, after the
 // kernel that stored them (in place of a last-block ticket, whose

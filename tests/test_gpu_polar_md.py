@@ -67,6 +67,28 @@ def test_polar_md_matches_reference(use_graph, joint, overlap, m_sums):
     assert rel_rms(md_real(ctx), fx.vec("end_real_pos")) <= 1e-10
 
 
+def test_polar_step_forms_with_surface_terms_agree():
+    """Two steps with torques and both classes' surface terms, which fill every
+    part of the torque sums: a launch of a step that queued a sum of the
+    other's would be refused.  The forms add the same forces in other orders:
+    1e-9."""
+    fx = Fixture("amoeba216_md10_polar")
+    fx.cfg["surface"] = True
+    out = []
+    for joint, overlap in ((1, 1), (0, 1), (1, 0)):
+        print(f"case surface terms joint {joint} overlap {overlap}", flush=True)
+        ctx = _ctx(fx.system)
+        ctx.set_tuning("polar_joint_long", joint)
+        ctx.set_tuning("recip_overlap", overlap)
+        ctx.set_velocities(fx.vec("init_vel"))
+        _, md = _polar_md(fx, ctx, True)
+        md.init()
+        md.run(2)
+        out.append(ctx.forces())
+    for f in out[1:]:
+        assert rel_rms(f, out[0]) <= 1e-9
+
+
 def test_polar_md_1024_from_the_lattice_start_matches_reference():
     """start() + 3 steps of the 1,024-molecule polarizable water from its
     lattice start (cutoff 0.9 nm, |n|^2 <= 81, cell list), the reference's

@@ -840,7 +840,8 @@ typedef struct {
 typedef struct {
     int32_t pair_lanes;           /* lanes per atom row of the pair kernel */
     int32_t sfac_chunk;           /* atoms per block of the structure-factor pass */
-    int32_t kforce_tile;          /* k-vectors per LDS tile of the reciprocal force pass */
+    int32_t kforce_tile;          /* k-vectors per LDS tile of the direct reciprocal force pass (k sets too
+                                     large for the row passes' tables; unused by those) */
     int32_t overlap;              /* 1: pair and reciprocal passes on two graph branches */
     int32_t use_graph;            /* 1: one captured graph launch per step; 0: direct launches */
 } smd_batch_tiles;
@@ -860,7 +861,8 @@ int smd_batch_get_reports(smd_batch* b, smd_batch_report* rep);   /* [R] */
 int smd_batch_set_tiles(smd_batch* b, const smd_batch_tiles* t);
 int smd_batch_get_tiles(const smd_batch* b, smd_batch_tiles* t);
 /* Times every candidate tile shape on the current state (each kernel alone,
- * HIP events, reps launches) and keeps the fastest.  times_us receives
+ * HIP events, reps launches) and keeps the fastest; kforce_tile only where the
+ * direct passes run.  times_us receives
  * n_cand rows of (pair_lanes, sfac_chunk, kforce_tile, pair us, sfac us,
  * kforce us) when not NULL; *n_cand is its capacity in rows on entry. */
 int smd_batch_autotune(smd_batch* b, int reps, double* times_us, int32_t* n_cand);

@@ -1749,8 +1749,10 @@ extern "C" int smd_batch_autotune(smd_batch* b, int reps, double* times_us, int3
         rows.insert(rows.end(), {0.0, (double)c, 0.0, 0.0, us, 0.0});
         if (us < bt) { bt = us; best.sfac_chunk = c; }
     }
+    // the row force pass has no k tiles: nothing to choose
     bt = 1e30;
     for (int k : ktiles) {
+        if (b->prm.rows_on) break;
         smd_batch_tiles t = best;
         t.kforce_tile = k;
         if ((rc = smd_batch_set_tiles(b, &t))) return rc;

@@ -343,3 +343,54 @@ def test_a_replica_step_shake_refuses_leaves_its_molecule_unmoved():
     d -= box * np.rint(d / box)
     assert np.abs(d).max() < 0.01
     b.close()
+
+
+@pytest.mark.parametrize("n2", [20, 306])
+def test_autotuner_times_the_tiles_that_the_passes_read(n2):
+    """The row force pass has no k tiles, so they are neither timed nor
+    changed; past its tables' size the direct pass has."""
+    from swinmd_amd.nemd import ShearBatch
+    s = S.water(256, density_mol=RHO, seed=9, subset=True)
+    print(f"case autotuned tiles n2={n2}", flush=True)
+    b = ShearBatch([s], [1.0], cutoff=0.8, cut_buff=0.08, alpha=3.5, n2max=n2, dt=0.002)
+    b.set_tiles(kforce_tile=192)
+    b.set_state([s.pos], [np.zeros_like(s.pos)], [0.0])
+    b.start()
+    best, table = b.autotune(reps=2)
+    timed = [row["kforce_tile"] for row in table if "kforce_tile" in row]
+    assert sum("pair_lanes" in row for row in table) == 4 and sum("sfac_chunk" in row for row in table) == 3
+    if n2 == 20:
+        assert not timed and best["kforce_tile"] == 192
+    else:
+        assert len(timed) == 3 and best["kforce_tile"] in timed
+    b.close()
+
+
+@pytest.mark.parametrize("prec,tiles", [(L.PREC_FP64, dict(kforce_tile=64, sfac_chunk=64)),
+                                        (L.PREC_FP64, dict(kforce_tile=1536, sfac_chunk=512)), (L.PREC_MIXED, {}),
+                                        (L.PREC_MIXED, dict(kforce_tile=128, sfac_chunk=256))])
+def test_direct_sheared_reciprocal_passes_match_the_oracle(prec, tiles):
+    """The passes for k sets past the row tables, in both precisions and with
+    tiles that end inside the k set and the atoms: forces and energies after
+    two steps at a tilt, FP64 1e-8, mixed 1e-5 (the form's own bar)."""
+    from oracle import oracle as O
+    from swinmd_amd.nemd import ShearBatch
+    s = S.water(275, density_mol=RHO, seed=275, subset=True)
+    kcut = S.kcut_for(306, s.box[0])
+    vel = O.Oracle(s).init_velocity(300.0, 5, per_atom=False, ndf=3 * s.n_mols - 3)
+    print(f"case direct sheared passes prec={prec} {tiles}", flush=True)
+    b = ShearBatch([s], [3.0], cutoff=0.8, cut_buff=0.08, alpha=3.5, kcut=[kcut], dt=0.002, temperature=300.0,
+                   coupl=0.1, prec=prec)
+    if tiles:
+        b.set_tiles(**tiles)
+    b.set_state([s.pos], [vel], [0.31])
+    b.start()
+    b.run(2)
+    st, rep = b.state(), b.reports()[0]
+    want = O.sllod_run(O.Oracle(s), dict(cutoff=0.8, cut_buff=0.08, alpha=3.5, kcut=kcut, dt=0.002,
+                                         temperature=300.0, coupl=0.1), 3.0, 2, velocity=vel, tilt=0.31)
+    tol = 1e-8 if prec == L.PREC_FP64 else 1e-5
+    assert rep["n_kvec"] == want["K"]
+    assert rel(rep["e_long"], want["e_long"]) <= tol
+    assert rel_rms(st["force"], want["force"]) <= tol
+    b.close()

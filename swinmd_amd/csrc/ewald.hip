@@ -28,7 +28,6 @@
 
 namespace smd {
 
-constexpr size_t LDS_MAX = 65536;
 constexpr int NSUM = 5;        // weights of the structure factors with Lustig terms: 1, d, |d|^2
 constexpr int SF_CHUNKS = 256; // atom chunks of the structure-factor pass, at most: one block per CU
 // With Lustig terms a chunk's partials are 211 KB (1,535 k): at 192 chunks
@@ -93,10 +92,10 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
         rexp[rexp.size() - kr.n1 + std::abs(kn[3 * k + 2])] = ek[k];
     }
     kr.nrows = (int)xy.size();
-    // The sets this path takes: the powers of 64 atoms, and 16 bytes per k
-    // and per run of eight, within 64 KiB.
+    // The sets this path takes: the powers and weights of 64 atoms, and 16
+    // bytes per k and per run of eight, within 64 KiB.
     const size_t ne = (size_t)nmax[0] + nmax[1] + nmax[2] + 3;
-    if (ne * ks_stride<double>() * 16 + 5 * KS_TILE * 8 > LDS_MAX || (size_t)(K + ng) * 16 > LDS_MAX)
+    if (ne * ks_stride<double>() * 16 + 5 * KS_TILE * 8 > KS_TABLE_LDS || (size_t)(K + ng) * 16 > KS_TABLE_LDS)
         return fail(c, SMD_ENOTSUP, "reciprocal space too large for the LDS-resident passes (%d k-vectors, nmax %d %d %d)",
                     K, nmax[0], nmax[1], nmax[2]);
     int rc;
@@ -476,7 +475,7 @@ static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes
         // a wave per dozen chunks, fewer where the row's sums are many: the
         // loads of one wave follow each other, the epilogue waits for all
         const size_t per_wave = sizeof(double) * NW * 4 * a.kr.n1;
-        const int waves = std::max(4, std::min({16, (a.chunks + 11) / 12, (int)(LDS_MAX / 2 / per_wave)}));
+        const int waves = std::max(4, std::min({16, (a.chunks + 11) / 12, (int)(KS_TABLE_LDS / 2 / per_wave)}));
         hipLaunchKernelGGL((k_recip_reduce<R, NW>), dim3(a.kr.tiles() * KS_ROWS), dim3(waves * WAVE), waves * per_wave,
                            s, a);
     }
@@ -682,8 +681,10 @@ extern "C" int smd_ewald_compute_long_static(smd_ctx* c, int prec, smd_ewald_lon
     if (prec != SMD_PREC_FP64 && prec != SMD_PREC_MIXED) return fail(c, SMD_EINVAL, "bad precision %d", prec);
     if (!c->static_scratch) return fail(c, SMD_ESTATE, "static scratch not resolved for device %d", c->device);
     auto up = [](size_t v) { return (v + 31) / 32 * 32; };   // 256-byte segments
-    // Room: 80 bytes per atom, 16 per k and 80 per (k, chunk), with a chunk
-    // per 64 k-runs and CU but at least 32 atoms in each.
+    // The documented room: 80 bytes per atom, 16 per k and 80 per (k, chunk),
+    // with a chunk per 64 k-runs and CU but at least 32 atoms in each.  The
+    // passes take 48 per atom, the coefficients and the partials; what the
+    // documented room admits leaves them 18 chunks and more.
     const int gt = (c->n_kruns + WAVE - 1) / WAVE;
     const int quota = std::max(1, 256 / gt);
     const int per = std::max(32, (c->n + quota - 1) / quota);

@@ -34,6 +34,10 @@ template <typename R> constexpr int KS_FORCE_OCC = sizeof(R) == 8 ? 3 : 4;
 constexpr int KS_ROWS = 16;       // rows of a matrix tile
 constexpr int KS_VT = 2;          // tiles per wave of the structure-factor pass
 constexpr int KS_MAXSTEP = 8;     // inner steps held in registers by the force pass
+// LDS of a table: two blocks to a CU with the force pass's partials beside it
+// (12 KiB more), which together are what one launch may ask for at most.
+constexpr size_t KS_TABLE_LDS = 65536, KS_CU_LDS = 163840;
+static_assert(2 * (KS_TABLE_LDS + (size_t)KS_MAXW * KS_TILE * 3 * sizeof(double)) <= KS_CU_LDS, "k-space LDS");
 
 template <typename R> struct KsMat;
 template <> struct KsMat<double> {
@@ -101,8 +105,7 @@ __device__ __forceinline__ void ks_powers(KsC<R>* tab, int ts, int u, int cnt, d
 }
 
 // Tables (with several weights also their values) of the structure-factor
-// pass that fit in the 64 KiB a launch takes without asking, at most
-// KS_TABLES: a block fills them together, so their loads and phases overlap.
+// pass that fit in KS_TABLE_LDS, at most KS_TABLES: a block fills them together, so their loads and phases overlap.
 constexpr int KS_TABLES = 4;
 template <typename R>
 __host__ __device__ inline size_t ks_table_bytes(const KsRows& kr, int nw) {
@@ -110,7 +113,7 @@ __host__ __device__ inline size_t ks_table_bytes(const KsRows& kr, int nw) {
 }
 template <typename R>
 __host__ __device__ inline int ks_tables(const KsRows& kr, int nw, int chunk_tiles) {
-    const int fit = (int)(65536 / ks_table_bytes<R>(kr, nw));
+    const int fit = (int)(KS_TABLE_LDS / ks_table_bytes<R>(kr, nw));
     const int m = fit < KS_TABLES ? fit : KS_TABLES;
     return m < 1 ? 1 : (m < chunk_tiles ? m : chunk_tiles);
 }

@@ -1403,8 +1403,8 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
     const double rl = p->cutoff + p->cut_buff;
     int a = 0, m = 0, kb = 0, rb = 0;
     int64_t eb = 0, cb = 0;
-    // rows where a table of every replica's powers fits the LDS a launch takes
-    // without asking (about 19 waves along the edge), else the direct passes
+    // rows where a table of every replica's powers fits KS_TABLE_LDS (16 waves
+    // along the edge), else the direct passes
     bool rows_ok = true;
     double dens = 0.0;
     for (int r = 0; r < b->R; ++r) {
@@ -1443,7 +1443,7 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
         rb += rp.rcap;
         eb += (int64_t)rp.rcap * kr.n1;
         cb += (int64_t)kr.coef_entries();
-        rows_ok = rows_ok && ks_table_bytes<double>(kr, 1) <= 65536 && kr.n1 <= WAVE;
+        rows_ok = rows_ok && ks_table_bytes<double>(kr, 1) <= KS_TABLE_LDS && kr.n1 <= WAVE;
         // block shapes for the row tiles of an unsheared cell (half the disk)
         const int tiles = ((int)(0.5 * PI * nR * nR + nR) + KS_ROWS) / KS_ROWS;
         b->rows_waves[0] = std::max(b->rows_waves[0], ks_waves(tiles, KS_VT, KS_MAXW, 3));

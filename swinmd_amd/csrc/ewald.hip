@@ -105,7 +105,9 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     const int nt = (c->n + KS_TILE - 1) / KS_TILE;
     c->sfac_chunks = std::max(1, std::min(nt, SF_CHUNKS));
     c->k_part = (size_t)kr.nrows * NSUM * 4 * kr.n1;
-    if ((rc = realloc(c->d_sfac_part, sizeof(double) * c->k_part * c->sfac_chunks))) return rc;
+    // the larger of the two forms' partials: NSUM weights, or one of more chunks
+    const int w = std::max(NSUM * std::min(nt, SF_CHUNKS_LUSTIG), c->sfac_chunks);
+    if ((rc = realloc(c->d_sfac_part, sizeof(double) * c->k_part / NSUM * w))) return rc;
     if ((rc = realloc(c->d_e1, sizeof(double) * 6 * (size_t)c->n))) return rc;
     SMD_HIP(c, hipMemcpy(c->d_kxy, xy.data(), sizeof(int32_t) * xy.size(), hipMemcpyHostToDevice));
     SMD_HIP(c, hipMemcpy(c->d_expk, rexp.data(), sizeof(double) * rexp.size(), hipMemcpyHostToDevice));

@@ -394,3 +394,30 @@ def test_direct_sheared_reciprocal_passes_match_the_oracle(prec, tiles):
     assert rel(rep["e_long"], want["e_long"]) <= tol
     assert rel_rms(st["force"], want["force"]) <= tol
     b.close()
+
+
+def test_ewald_setup_takes_the_memory_its_passes_use():
+    """5,462 waters, |n|^2 <= 81: the structure factors' partials are 64 chunks
+    of five weights (14 MB), the phases 0.8 MB; 12 MB for the tables and the
+    allocator's pages."""
+    import ctypes as C
+    from swinmd_amd.forces import Context, EwaldForce
+    s = S.water(5462, density_mol=RHO, seed=1, subset=True)
+    print("case ewald memory", flush=True)
+    ctx = Context(s)
+    ctx.compute_mol_centers()
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def left():
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    before = left()
+    ew = EwaldForce(ctx, alpha=3.5, real_cut=0.9, kcut=S.kcut_for(81, s.box[0]))
+    took = before - left()
+    rows = sum(1 for x in range(10) for y in range(0 if x == 0 else -9, 10) if x * x + y * y <= 81)
+    assert took <= 64 * 5 * 4 * 10 * rows * 8 + 48 * s.n_atoms + 12e6, took
+    # the passes with and without Lustig sums stay inside it
+    assert np.isfinite(ew.compute_long(np.zeros((s.n_atoms, 3)))["energy"])
+    ctx.close()

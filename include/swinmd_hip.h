@@ -599,8 +599,8 @@ int smd_md_time_family(smd_ctx* ctx, const char* family, int reps, double* avg_u
  * the joint pass).
  * "md_fused_shake" (0/1, default 1): the MD step runs SHAKE and the kinetic
  * and pressure sums as one kernel (0: two kernels).
- * "cg_lanes" (8, 16 or 32; by size if not set): lanes sharing one row of the
- * CG's A v.
+ * "cg_lanes" (8, 16 or 32, or 0 (default): by size): lanes sharing one row of
+ * the CG's A v.
  * "cg_graph" (0/1, default 1): smd_induce replays each batch of CG
  * iterations from a captured hipGraph (0: direct launches, for profilers).
  * "cg_batch" (1..64, default 16): CG iterations per batch, i.e. between the

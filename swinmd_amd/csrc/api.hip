@@ -403,7 +403,7 @@ extern "C" int smd_set_tuning(smd_ctx* c, const char* name, int value) {
     if (!c || !name) return SMD_EINVAL;
     if (std::string(name) == "pair_lanes") {
         if (value != 0 && value != 4 && value != 8 && value != 16 && value != 32 && value != 64)
-            return fail(c, SMD_EINVAL, "pair_lanes must be 0 (by precision), 4, 8, 16, 32 or 64 (got %d)", value);
+            return fail(c, SMD_EINVAL, "pair_lanes must be 0 (by size and precision), 4, 8, 16, 32 or 64 (got %d)", value);
         c->pair_lanes = value;
     } else if (std::string(name) == "pair_packed") {
         if (value != 0 && value != 1) return fail(c, SMD_EINVAL, "pair_packed must be 0 or 1 (got %d)", value);
@@ -412,7 +412,8 @@ extern "C" int smd_set_tuning(smd_ctx* c, const char* name, int value) {
         if (value != 0 && value != 1) return fail(c, SMD_EINVAL, "md_fused_shake must be 0 or 1 (got %d)", value);
         c->md_fused_shake = value;
     } else if (std::string(name) == "cg_lanes") {
-        if (value != 8 && value != 16 && value != 32) return fail(c, SMD_EINVAL, "cg_lanes must be 8, 16 or 32 (got %d)", value);
+        if (value != 0 && value != 8 && value != 16 && value != 32)
+            return fail(c, SMD_EINVAL, "cg_lanes must be 0 (by size), 8, 16 or 32 (got %d)", value);
         c->cg_lanes = value;
         if (c->cg_exec) { (void)hipGraphExecDestroy(c->cg_exec); c->cg_exec = nullptr; }
     } else if (std::string(name) == "cg_batch") {

@@ -734,7 +734,7 @@ __global__ __launch_bounds__(256) void k_apply_pos32(IndArgs a, const float4* __
     if (part) block_partial(d, part);   // p.Ap of the CG step
 }
 
-// k_apply_table with `lanes` lanes per row (8, 16 or 32).
+// k_apply_table with `lanes` lanes per row (8, 16, 32 or 64).
 static void launch_apply(Ctx* c, int lanes, const IndArgs& a, const double* v, double* out, const double* dotv,
                          double* part, CgTop top) {
     const dim3 grid((unsigned)(((int64_t)c->n * lanes + 255) / 256));

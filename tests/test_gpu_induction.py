@@ -137,3 +137,24 @@ def test_time_apply_leaves_the_solution_unchanged():
     assert ind.time_apply(5) > 0.0
     assert np.array_equal(ind.results()[3], mu)
     ctx.close()
+
+
+def test_cg_lanes_by_size_can_be_set_again():
+    """0 gives back the default, the lanes by size: the same bits as a solve
+    that never set any; other values are still refused."""
+    from swinmd_amd import _lib as L
+    fx = Fixture("amoeba216_induction_cg")
+    print("case cg_lanes set again", flush=True)
+    ctx, ind = _induction(fx)
+    ind.induce()
+    mu = ind.results()[3].copy()
+    ctx.set_tuning("cg_lanes", 8)
+    ind.induce()
+    assert rel_rms(ind.results()[3], mu) <= 1e-10
+    ctx.set_tuning("cg_lanes", 0)
+    ind.induce()
+    assert np.array_equal(ind.results()[3], mu)
+    for bad in (4, 64, -1):
+        with pytest.raises(L.SmdError):
+            ctx.set_tuning("cg_lanes", bad)
+    ctx.close()

@@ -471,29 +471,31 @@ __global__ __launch_bounds__(LR_THREADS) void k_list_rows(ListArgs a, CellGrid g
         if (all > a.stride) atomicOr(a.status, ST_LIST_OVERFLOW);
     }
     int32_t* row = a.nb + (int64_t)i * a.stride;
-    auto store = [&](int t, int at) {   // the t-th hit, owned ones first
-        const int to = t < own_all ? t : a.stride - 1 - (t - own_all);
-        if (t < own_all ? to < a.stride : to >= own_all) row[to] = catoms[at];
-    };
     int32_t* order = ranked[threadIdx.x / WAVE];
-    const bool in_lds = all <= ROW_LDS;
-    auto place = [&](int h, uint32_t bits) {
-        const uint32_t mine = owned(h);
-        while (bits) {
-            const int b = __ffs(bits) - 1, at = jb + 32 * h + b;
-            bits &= bits - 1u;
-            const bool own_hit = mine >> b & 1u;
-            const int to = own_hit ? own_at++ : own_all + non_at++;
-            if (in_lds) order[to] = at;
-            else store(to, at);
-        }
-    };
+    // the lane's hits, `put` getting each one's rank (owned ones first) and place
+    auto place = [&](auto put) {
+        auto bits_of = [&](int h, uint32_t bits) {
+            const uint32_t mine = owned(h);
+            while (bits) {
+                const int b = __ffs(bits) - 1;
+                bits &= bits - 1u;
+                put(mine >> b & 1u ? own_at++ : own_all + non_at++, jb + 32 * h + b);
+            }
+        };
 #pragma unroll
-    for (int u = 0; u < WORDS; ++u) place(h0 + u, words[u]);
-    for (int h = h0 + WORDS; h < h1; ++h) place(h, hits(h));
-    if (!in_lds) return;
+        for (int u = 0; u < WORDS; ++u) bits_of(h0 + u, words[u]);
+        for (int h = h0 + WORDS; h < h1; ++h) bits_of(h, hits(h));
+    };
+    if (all > ROW_LDS || all > a.stride) {
+        place([&](int t, int at) {
+            const int to = t < own_all ? t : a.stride - 1 - (t - own_all);
+            if (t < own_all ? to < a.stride : to >= own_all) row[to] = catoms[at];
+        });
+        return;
+    }
+    place([&](int t, int at) { order[t] = at; });
     wave_lds_order();
-    for (int t = lane; t < all; t += WAVE) store(t, order[t]);
+    for (int t = lane; t < all; t += WAVE) row[t < own_all ? t : a.stride - 1 - (t - own_all)] = catoms[order[t]];
 }
 
 // Ensemble::build_pairlist (src/Ensemble.cpp:492-525): all j != i with the

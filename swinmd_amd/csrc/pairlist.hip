@@ -535,6 +535,7 @@ static bool cell_setup(double len, const double L[3], int n[3], double rlen[3]) 
 int pairlist_alloc(Ctx* c, int32_t stride) {
     if (stride <= c->stride && c->d_nb) return SMD_OK;
     if (c->d_nb) (void)hipFree(c->d_nb);
+    drop_step_graphs(c);
     c->d_nb = nullptr;
     const size_t bytes = (size_t)c->n * (size_t)stride * sizeof(int32_t);
     if (hipMalloc(&c->d_nb, bytes ? bytes : 4) != hipSuccess) {
@@ -657,6 +658,7 @@ int pairlist_build(Ctx* c, double cutoff, double cut_buff, int use_cells, bool o
             if (c->d_list_mask) (void)hipFree(c->d_list_mask);
             c->d_list_mask = nullptr;
             c->list_mask_words = 0;
+            drop_step_graphs(c);
             const size_t bytes = sizeof(uint64_t) * 27 * (size_t)c->n * words;
             if (hipMalloc(&c->d_list_mask, bytes) != hipSuccess)
                 return fail(c, SMD_ENOMEM, "pair-list mask allocation of %zu bytes failed", bytes);

@@ -680,6 +680,7 @@ int rows_finish(Ctx* c, hipStream_t s, const double* part, int stride, int nb, i
 // Launches one kernel that adds every queued finish (in queue order, each in
 // block order) and clears the queue; no-op when the queue is empty.
 int red_flush(Ctx* c);
+void drop_step_graphs(Ctx* c);
 int red_take(Ctx* c, FlushList& f);
 // Queues finishes for the scope (a step's kernels), dropping any left over.
 struct RedDefer {

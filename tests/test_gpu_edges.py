@@ -421,3 +421,33 @@ def test_ewald_setup_takes_the_memory_its_passes_use():
     # the passes with and without Lustig sums stay inside it
     assert np.isfinite(ew.compute_long(np.zeros((s.n_atoms, 3)))["energy"])
     ctx.close()
+
+
+def test_captured_steps_outlive_a_list_that_grew():
+    """A captured step after host builds that replaced the list's buffers (a
+    crowd of atoms in one cell) runs on the new ones: the same trajectory as
+    without them."""
+    from swinmd_amd.forces import Context, WaterMD
+    s = S.lj_fcc(8)                            # 2,048 atoms, box 13.4
+    print("case captured step and grown list", flush=True)
+    vel = np.random.default_rng(3).normal(0.0, 0.8, (s.n_atoms, 3))
+    crowd = s.pos.copy()
+    crowd[:900] = np.random.default_rng(4).uniform(0.2, 1.8, (900, 3))
+    out = []
+    for grow in (False, True):
+        ctx = Context(s)
+        ctx.set_velocities(vel - vel.mean(0))
+        md = WaterMD(ctx, cutoff=2.5, cut_buff=0.3, dt=0.004, temperature=0.8 / 0.0083145112, coupl=0.5,
+                     constraint=False, ewald=False, switch_on=True)
+        md.init()
+        md.run(3)
+        pos = ctx.positions()
+        if grow:
+            ctx.set_positions(crowd)
+            ctx.set_pairlist(2.5, 0.3, True)
+        ctx.set_positions(pos)
+        ctx.set_pairlist(2.5, 0.3, True)
+        md.run(3)
+        out.append(ctx.positions())
+        ctx.close()
+    assert rel_rms(out[1], out[0]) <= 1e-12

@@ -275,7 +275,7 @@ extern "C" int smd_ctx_create(smd_ctx** out, const smd_topology* t, int device) 
     A(c->d_mom, sizeof(double) * 3 * nm);
     A(c->d_bond2, sizeof(double) * 3 * nm);
     A(c->d_terms, sizeof(double) * T_COUNT);
-    A(c->d_status, sizeof(unsigned));
+    A(c->d_status, 2 * sizeof(unsigned));
     A(c->d_flag, sizeof(int) * 8);
     c->nb_atoms = (n + 255) / 256;
     c->nb_mols = (nm + 255) / 256;

@@ -105,14 +105,16 @@ __global__ __launch_bounds__(128) void k_cell_assign(int nmol, const int32_t* __
 // One block per cell: its start (the sum of the counts of lower cells) and
 // its atoms compacted in index order (set_atom appends in atom order,
 // CellManager.cpp:145-170); it stops once the cell is full.  The counts are
-// cleared later, by k_list_hits.
+// cleared later, by k_list_hits.  A host's build also gets the largest cell
+// past the `held` atoms of the hit bits.
 constexpr int FILL_THREADS = 1024;
 constexpr int FILL_WAVES = FILL_THREADS / WAVE;
 
 __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, const int32_t* __restrict__ cell_of,
                                                             const int32_t* __restrict__ cnt,
                                                             int32_t* __restrict__ start, int32_t* __restrict__ atoms,
-                                                            int32_t* __restrict__ slot, const int* gate) {
+                                                            int32_t* __restrict__ slot, int held, unsigned* largest,
+                                                            const int* gate) {
     if (gate && !*gate) return;
     __shared__ int32_t wsum[FILL_WAVES];
     const int c = blockIdx.x;
@@ -131,6 +133,7 @@ __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, co
     if (threadIdx.x == 0) {
         start[c] = base;
         if (c == ncell - 1) start[ncell] = end;
+        if (largest && end - base > held) atomicMax(largest, (unsigned)(end - base));
     }
     const uint64_t below = (1ull << lane) - 1ull;
     for (int a0 = 0; a0 < n && base < end; a0 += FILL_THREADS) {
@@ -607,7 +610,8 @@ static int launch_list(Ctx* c, const int* gate, bool md_prep) {
                                g, c->box, pr, c->d_cell_of, c->d_cell_cnt, gate);
         if (c->list_fork) SMD_HIP(c, hipEventRecord(c->list_fork, c->stream));   // positions are final here
         hipLaunchKernelGGL(k_cell_fill, dim3(nc), dim3(FILL_THREADS), 0, c->stream, c->n, nc, c->d_cell_of,
-                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, c->d_cell_slot, gate);
+                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, c->d_cell_slot,
+                           WAVE * c->list_mask_words, gate ? nullptr : c->d_status + 1, gate);
         // tiles of a cell pair beyond four go to further blocks
         const int tiles = (c->n / nc + WAVE - 1) / WAVE;
         const dim3 gl(nc, 14, std::min(8, (tiles * tiles + LB_WAVES - 1) / LB_WAVES));
@@ -625,6 +629,26 @@ static int launch_list(Ctx* c, const int* gate, bool md_prep) {
     }
     SMD_HIP(c, hipGetLastError());
     return SMD_OK;
+}
+
+// Hit bits for the largest cell a build found, and a quarter more for the
+// rebuilds inside a step.  Slabs and droplets fill cells far beyond the mean,
+// and k_list_rows tests what the bits do not hold one lane per word.  Calls
+// of 16,000 waters in an eighth of their box, radius 1.3 nm, 1,370 -> 420 us;
+// 4,096 in a 27th, 446 -> 167.  A list row holds about five atoms for each of a cell's,
+// so the bits stay well below the list's own size.  Without the memory the
+// smaller mask stays.
+static void mask_grow(Ctx* c, int largest) {
+    const int words = (largest + largest / 4 + WAVE - 1) / WAVE;
+    uint64_t* mask = nullptr;
+    if (hipMalloc(&mask, sizeof(uint64_t) * 27 * (size_t)c->n * words) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    (void)hipFree(c->d_list_mask);
+    c->d_list_mask = mask;
+    c->list_mask_words = words;
+    drop_step_graphs(c);
 }
 
 // Builds the list.  With on_device_flag the kernels are gated on d_flag[0]
@@ -681,13 +705,14 @@ int pairlist_build(Ctx* c, double cutoff, double cut_buff, int use_cells, bool o
     for (int attempt = 0; attempt < 6; ++attempt) {
         int rc = pairlist_alloc(c, stride);
         if (rc) return rc;
-        SMD_HIP(c, hipMemsetAsync(c->d_status, 0, sizeof(unsigned), c->stream));
+        SMD_HIP(c, hipMemsetAsync(c->d_status, 0, 2 * sizeof(unsigned), c->stream));
         rc = launch_list(c, nullptr, false);
         if (rc) return rc;
-        unsigned st = 0;
-        SMD_HIP(c, hipMemcpyAsync(&st, c->d_status, sizeof st, hipMemcpyDeviceToHost, c->stream));
+        unsigned st[2] = {0, 0};
+        SMD_HIP(c, hipMemcpyAsync(st, c->d_status, sizeof st, hipMemcpyDeviceToHost, c->stream));
         SMD_HIP(c, hipStreamSynchronize(c->stream));
-        if (!(st & ST_LIST_OVERFLOW)) {
+        if (c->list_cells && st[1] > (unsigned)(WAVE * c->list_mask_words)) mask_grow(c, (int)st[1]);
+        if (!(st[0] & ST_LIST_OVERFLOW)) {
             c->list_valid = true;
             return SMD_OK;
         }

@@ -117,7 +117,7 @@ struct Ctx {
     double* d_mom = nullptr;      // [3nmol] Molecule::momenta
     double* d_bond2 = nullptr;    // [3nmol]
     double* d_terms = nullptr;    // [T_COUNT]
-    unsigned* d_status = nullptr;
+    unsigned* d_status = nullptr;  // status bits; the largest cell past the list's hit bits
     int* d_flag = nullptr;        // [8]: 0 rebuild-needed, 1 drift-apply, 2 kinetics ticket,
                                   // 3 SHAKE ticket, 4 surface-sum ticket, 5 multipole/induction site-sum ticket
     // Fixed-order block partials of the sums that feed the trajectory (drift

@@ -423,6 +423,36 @@ def test_ewald_setup_takes_the_memory_its_passes_use():
     ctx.close()
 
 
+@pytest.mark.parametrize("crowd", [0.8, 0.3])
+def test_cell_list_follows_a_crowded_cell(crowd):
+    """Builds before and after the hit bits grow to a crowded cell, and a
+    uniform one after that: rows in order, as the oracle's.  The smaller crowd
+    has rows past the first capacity as well."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context
+    n = 2500
+    print(f"case crowded cell {crowd}", flush=True)
+    rng = np.random.default_rng(11)
+    s = S.lj_fcc(1)
+    s.density = n / 125.0                      # a box of 5
+    even = rng.uniform(-2.5, 2.5, (n, 3))
+    packed = even.copy()
+    packed[:700] = 1.5 + rng.uniform(-0.5, 0.5, (700, 3)) * crowd
+    s.type, s.mol = np.zeros(n, dtype=np.int32), np.arange(n, dtype=np.int32)
+    s.pos = packed
+    ctx = Context(s)
+    for pos in (packed, packed, even, packed):
+        s.pos = pos
+        off, nb, used = O.Oracle(s).pairlist(0.9, 0.1, True)
+        assert used
+        ctx.set_positions(pos)
+        ctx.set_pairlist(0.9, 0.1, True)
+        goff, gnb = ctx.pairlist()
+        np.testing.assert_array_equal(goff, off)
+        np.testing.assert_array_equal(gnb, nb)
+    ctx.close()
+
+
 def test_captured_steps_outlive_a_list_that_grew():
     """A captured step after host builds that replaced the list's buffers (a
     crowd of atoms in one cell) runs on the new ones: the same trajectory as

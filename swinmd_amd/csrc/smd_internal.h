@@ -333,10 +333,9 @@ inline int cg_lanes(const Ctx* c) { return c->cg_lanes ? c->cg_lanes : row_lanes
 
 // Threads per block of the kernels with a thread per molecule: one wave, so
 // that 8,192 molecules reach 128 CUs and not 32; each lasts as long as its
-// thread's chain of loads and FP64 arithmetic.  Against 256 threads, at 1,024
-// and 8,192 waters in us: torques 8.7 -> 7.2 and 9.3 -> 7.6, block
-// preconditioner 10.1 -> 7.2 and 28 -> 19, redistribution 5.2 -> 3.9 and
-// 14.4 -> 10.5, intramolecular terms about the same.
+// thread's chain of loads and FP64 arithmetic.  Alone, against 256 threads, at
+// 1,024 and 8,192 waters in us: torques 7.9 -> 6.8 and 8.0 -> 6.9, lab frames
+// 6.6 -> 5.8 and 7.1 -> 6.0, block preconditioner 9.2 -> 6.9 and 9.5 -> 7.4.
 constexpr int MOL_THREADS = 64;
 inline unsigned mol_blocks(const Ctx* c) { return (unsigned)((c->nmol + MOL_THREADS - 1) / MOL_THREADS); }
 

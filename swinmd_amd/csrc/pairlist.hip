@@ -612,8 +612,9 @@ static int launch_list(Ctx* c, const int* gate, bool md_prep) {
         hipLaunchKernelGGL(k_cell_fill, dim3(nc), dim3(FILL_THREADS), 0, c->stream, c->n, nc, c->d_cell_of,
                            c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, c->d_cell_slot,
                            WAVE * c->list_mask_words, gate ? nullptr : c->d_status + 1, gate);
-        // tiles of a cell pair beyond four go to further blocks
-        const int tiles = (c->n / nc + WAVE - 1) / WAVE;
+        // tiles of a cell pair beyond four go to further blocks; a dilute grid
+        // has less than an atom a cell
+        const int tiles = std::max(1, (c->n / nc + WAVE - 1) / WAVE);
         const dim3 gl(nc, 14, std::min(8, (tiles * tiles + LB_WAVES - 1) / LB_WAVES));
         hipLaunchKernelGGL(k_list_hits, gl, dim3(LB_THREADS), 0, c->stream, a, g, c->d_cell_start, c->d_cell_atoms,
                            c->d_cell_cnt, gate);

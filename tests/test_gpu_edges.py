@@ -481,3 +481,27 @@ def test_captured_steps_outlive_a_list_that_grew():
         out.append(ctx.positions())
         ctx.close()
     assert rel_rms(out[1], out[0]) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [1, 26, 27, 40])
+def test_cell_list_of_fewer_atoms_than_cells(n):
+    """A grid of 27 cells with less than an atom a cell and with one or more:
+    the rows of the oracle; two atoms are neighbours."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context
+    print(f"case dilute cell list n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    s = S.lj_fcc(1)
+    s.density = n / 27.0                       # a box of 3
+    s.pos = rng.uniform(-1.5, 1.5, (n, 3))
+    if n > 1:
+        s.pos[1] = s.pos[0] + [0.1, 0.0, 0.0]
+    s.type, s.mol = np.zeros(n, dtype=np.int32), np.arange(n, dtype=np.int32)
+    off, nb, used = O.Oracle(s).pairlist(0.9, 0.05, True)
+    assert used
+    ctx = Context(s)
+    ctx.set_pairlist(0.9, 0.05, True)
+    goff, gnb = ctx.pairlist()
+    np.testing.assert_array_equal(goff, off)
+    np.testing.assert_array_equal(gnb, nb)
+    ctx.close()

@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <random>
 #include <vector>
@@ -1160,14 +1161,15 @@ int smd_mlp_get_norm(smd_ctx* c, float* norm, int64_t count) {
 }
 
 static int upload_rows(Ctx* c, const float* x, int64_t rows) {
-    std::vector<uint16_t> xb((size_t)rows * MF);
-    for (size_t k = 0; k < xb.size(); ++k) {   // the kernels' rounding, on the host
+    const size_t n = (size_t)rows * MF;
+    const std::unique_ptr<uint16_t[]> xb(new uint16_t[n]);   // not cleared: every entry is written
+    for (size_t k = 0; k < n; ++k) {   // the kernels' rounding, on the host
         uint32_t u;
         std::memcpy(&u, &x[k], 4);
         u += 0x7FFFu + ((u >> 16) & 1u);
         xb[k] = (uint16_t)(u >> 16);
     }
-    SMD_HIP(c, hipMemcpyAsync(c->mlp->x, xb.data(), sizeof(uint16_t) * xb.size(), hipMemcpyHostToDevice, c->stream));
+    SMD_HIP(c, hipMemcpyAsync(c->mlp->x, xb.get(), sizeof(uint16_t) * n, hipMemcpyHostToDevice, c->stream));
     SMD_HIP(c, hipStreamSynchronize(c->stream));
     return SMD_OK;
 }

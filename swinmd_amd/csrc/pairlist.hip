@@ -113,8 +113,7 @@ constexpr int FILL_WAVES = FILL_THREADS / WAVE;
 __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, const int32_t* __restrict__ cell_of,
                                                             const int32_t* __restrict__ cnt,
                                                             int32_t* __restrict__ start, int32_t* __restrict__ atoms,
-                                                            int32_t* __restrict__ slot, int held, unsigned* largest,
-                                                            const int* gate) {
+                                                            int held, unsigned* largest, const int* gate) {
     if (gate && !*gate) return;
     __shared__ int32_t wsum[FILL_WAVES];
     const int c = blockIdx.x;
@@ -148,11 +147,7 @@ __global__ __launch_bounds__(FILL_THREADS) void k_cell_fill(int n, int ncell, co
             off += k < w ? wsum[k] : 0;
             tot += wsum[k];
         }
-        const int at = base + off + __popcll(m & below);
-        if (hit && at < end) {
-            atoms[at] = a;
-            slot[a] = at;
-        }
+        if (hit && base + off + __popcll(m & below) < end) atoms[base + off + __popcll(m & below)] = a;
         base += tot;
         __syncthreads();
     }
@@ -320,7 +315,8 @@ __device__ __forceinline__ uint64_t hit_tile(const ListArgs& a, const double (*s
 // pairs), 18 for 1,021 in 27; testing each pair from both atoms, a block per
 // neighbour, took 63 and 46.
 __global__ __launch_bounds__(LB_THREADS) void k_list_hits(ListArgs a, CellGrid g, const int32_t* __restrict__ start,
-                                                          const int32_t* __restrict__ catoms, int32_t* cell_cnt,
+                                                          const int32_t* __restrict__ catoms,
+                                                          int32_t* __restrict__ slot, int32_t* cell_cnt,
                                                           const int* gate) {
     if (gate && !*gate) return;
     __shared__ double sj[LB_WAVES][WAVE][3];
@@ -336,6 +332,8 @@ __global__ __launch_bounds__(LB_THREADS) void k_list_hits(ListArgs a, CellGrid g
     const size_t n = a.n;
     for (int t = blockIdx.z * LB_WAVES + w; t < ti_n * tj_n; t += gridDim.z * LB_WAVES) {
         const int ti = t / tj_n, tj = t % tj_n;
+        // the places of the cell's atoms, for k_list_rows
+        if (s == 0 && ti == tj && ib + ti * WAVE + lane < ie) slot[catoms[ib + ti * WAVE + lane]] = ib + ti * WAVE + lane;
         if ((s == 0 && tj < ti) || (ti >= a.mask_words && tj >= a.mask_words)) continue;
         // the wave's time is one candidate's times the candidates': the
         // larger side takes the lanes
@@ -375,7 +373,7 @@ __global__ __launch_bounds__(LB_THREADS) void k_list_hits(ListArgs a, CellGrid g
 // back; both segments are in the reference's order.  Words of atoms past the
 // mask (a neighbour of more than 64 mask_words atoms) are tested here.
 // The places are put in order in LDS, so that the row leaves in whole cache
-// lines: 45 us at 4,096 waters (430 partners a row), 20 at 1,021; a lane per
+// lines: 42 us at 4,096 waters (430 partners a row), 20 at 1,021; a lane per
 // atom and neighbour, each storing to its own row, took 52 and 36 and a pass
 // for the slots before it.
 // A row longer than the stride is cut to it and filled: owned atoms to its
@@ -610,14 +608,14 @@ static int launch_list(Ctx* c, const int* gate, bool md_prep) {
                                g, c->box, pr, c->d_cell_of, c->d_cell_cnt, gate);
         if (c->list_fork) SMD_HIP(c, hipEventRecord(c->list_fork, c->stream));   // positions are final here
         hipLaunchKernelGGL(k_cell_fill, dim3(nc), dim3(FILL_THREADS), 0, c->stream, c->n, nc, c->d_cell_of,
-                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, c->d_cell_slot,
-                           WAVE * c->list_mask_words, gate ? nullptr : c->d_status + 1, gate);
+                           c->d_cell_cnt, c->d_cell_start, c->d_cell_atoms, WAVE * c->list_mask_words,
+                           gate ? nullptr : c->d_status + 1, gate);
         // tiles of a cell pair beyond four go to further blocks; a dilute grid
         // has less than an atom a cell
         const int tiles = std::max(1, (c->n / nc + WAVE - 1) / WAVE);
         const dim3 gl(nc, 14, std::min(8, (tiles * tiles + LB_WAVES - 1) / LB_WAVES));
         hipLaunchKernelGGL(k_list_hits, gl, dim3(LB_THREADS), 0, c->stream, a, g, c->d_cell_start, c->d_cell_atoms,
-                           c->d_cell_cnt, gate);
+                           c->d_cell_slot, c->d_cell_cnt, gate);
         constexpr int per = LR_THREADS / WAVE;
         hipLaunchKernelGGL(k_list_rows, dim3((c->n + per - 1) / per), dim3(LR_THREADS), 0, c->stream, a, g,
                            c->d_cell_start, c->d_cell_atoms, c->d_cell_of, c->d_cell_slot, gate);

@@ -8,7 +8,8 @@
 // Reciprocal space: kspace.h.  Three launches:
 //   k_recip_sfac: structure factors of an atom chunk, phases exp(i 2 pi r_p /
 //     L_p) evaluated on the way and kept for the forces.  With Lustig terms
-//     also the sums weighted by d = r - R_mol and |d|^2.
+//     also the sums weighted by d = r - R_mol and |d|^2; in FP64 those take
+//     k_recip_phase and k_recip_walk, on the vector units.
 //   k_recip_reduce: partials summed over chunks in a fixed order, then per k:
 //     energy, volume derivatives and virial (:596-607) and the force pass's
 //     coefficients; the reference's per-atom Lustig sums of the force loop
@@ -28,11 +29,42 @@
 
 namespace smd {
 
-constexpr int NSUM = 5;        // weights of the structure factors with Lustig terms: 1, d, |d|^2
-constexpr int SF_CHUNKS = 256; // atom chunks of the structure-factor pass, at most: one block per CU
-// With Lustig terms a chunk's partials are 211 KB (1,535 k): at 192 chunks
-// writing and summing them took 28.8 + 16.6 us, the products 7.
-constexpr int SF_CHUNKS_LUSTIG = 64;
+constexpr int SF_CHUNKS = 256; // blocks of the structure-factor passes, at most: one per CU
+constexpr int GK = 8;          // k of a run: consecutive nz within one (nx, ny) row
+constexpr int WALK_SUMS = 10;  // per-k sums of k_recip_walk
+constexpr int WALK_WAVES = 8;  // its waves per block: the same runs, different atoms
+
+// The structure factors with Lustig terms: as products (mixed, and FP64 where
+// blocks are few) in chunks of whole tiles, sets.count blocks each; or in FP64
+// by k_recip_walk in chunks of 32 atoms and more, a block per 64 runs each.
+// At most `most` chunks, and a block per CU.
+struct LustigPlan {
+    bool walk;
+    KsSets sets;
+    int per, chunks;
+    size_t part;   // doubles of a chunk's partials
+};
+static LustigPlan lustig_plan(const KsRows& kr, int n, int K, int runs, int most, bool mixed) {
+    const int nt = (n + KS_TILE - 1) / KS_TILE;
+    LustigPlan p;
+    p.sets = ks_weight_sets(kr, nt);
+    p.walk = !mixed && p.sets.split == 2;
+    if (p.walk) {
+        const int c = std::max(1, std::min(most, SF_CHUNKS / ((runs + WAVE - 1) / WAVE)));
+        p.per = std::max(32, (n + c - 1) / c);
+        p.part = (size_t)K * WALK_SUMS;
+    } else {
+        const int c = std::max(1, std::min({nt, most, SF_CHUNKS / p.sets.count}));
+        p.per = (nt + c - 1) / c * KS_TILE;
+        p.part = (size_t)kr.nrows * KS_WEIGHTS * 4 * kr.n1;
+    }
+    p.chunks = (n + p.per - 1) / p.per;
+    return p;
+}
+
+// d_e1 holds the phases [n][3] (complex) and then, 32-byte aligned, the
+// per-atom (q, d) of k_recip_walk.
+static size_t e1_am_offset(int n) { return (6 * (size_t)n + 3) & ~(size_t)3; }
 
 // ---- host setup -----------------------------------------------------------
 
@@ -77,21 +109,26 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     kr.n1 = nmax[2] + 1;
     kr.nx1 = nmax[0] + 1;
     kr.ny1 = nmax[1] + 1;
-    std::vector<int32_t> xy;
+    // runs of at most GK consecutive nz in a row, stored as (first k, count,
+    // nx << 16 | (ny & 0xffff), nz of the first k); the rows' first k
+    std::vector<int32_t> xy, rowk;
     std::vector<double> rexp;
-    int ng = 0, run = 0;   // runs of at most eight consecutive nz in a row
+    std::vector<int4> runs;
     for (int k = 0; k < K; ++k) {
         const int v = (kn[3 * k] << 16) | (kn[3 * k + 1] & 0xffff);
         const bool same = !xy.empty() && xy.back() == v;
-        run = same && kn[3 * k + 2] == kn[3 * k - 1] + 1 && run < 8 ? run + 1 : 1;
-        ng += run == 1 ? 1 : 0;
+        if (same && kn[3 * k + 2] == kn[3 * k - 1] + 1 && runs.back().y < GK) ++runs.back().y;
+        else runs.push_back(make_int4(k, 1, v, kn[3 * k + 2]));
         if (!same) {
             xy.push_back(v);
+            rowk.push_back(k);
             rexp.resize(rexp.size() + kr.n1, 0.0);
         }
         rexp[rexp.size() - kr.n1 + std::abs(kn[3 * k + 2])] = ek[k];
     }
+    rowk.push_back(K);
     kr.nrows = (int)xy.size();
+    const int ng = (int)runs.size();
     // The sets this path takes: the powers and weights of 64 atoms, and 16
     // bytes per k and per run of eight, within 64 KiB.
     const size_t ne = (size_t)nmax[0] + nmax[1] + nmax[2] + 3;
@@ -104,11 +141,18 @@ int ewald_setup(Ctx* c, const smd_ewald_params* p) {
     if ((rc = realloc(c->d_kf, sizeof(double) * kr.coef_entries()))) return rc;
     const int nt = (c->n + KS_TILE - 1) / KS_TILE;
     c->sfac_chunks = std::max(1, std::min(nt, SF_CHUNKS));
-    c->k_part = (size_t)kr.nrows * NSUM * 4 * kr.n1;
-    // the larger of the two forms' partials: NSUM weights, or one of more chunks
-    const int w = std::max(NSUM * std::min(nt, SF_CHUNKS_LUSTIG), c->sfac_chunks);
-    if ((rc = realloc(c->d_sfac_part, sizeof(double) * c->k_part / NSUM * w))) return rc;
-    if ((rc = realloc(c->d_e1, sizeof(double) * 6 * (size_t)c->n))) return rc;
+    // the largest of the forms' partials: one weight, or with Lustig terms
+    size_t part = (size_t)kr.nrows * 4 * kr.n1 * c->sfac_chunks;
+    for (bool mixed : {false, true}) {
+        const LustigPlan p = lustig_plan(kr, c->n, K, ng, SF_CHUNKS, mixed);
+        part = std::max(part, p.part * p.chunks);
+    }
+    if ((rc = realloc(c->d_sfac_part, sizeof(double) * part))) return rc;
+    if ((rc = realloc(c->d_e1, sizeof(double) * (e1_am_offset(c->n) + 4 * (size_t)c->n)))) return rc;
+    if ((rc = realloc(c->d_kruns, sizeof(int4) * runs.size()))) return rc;
+    if ((rc = realloc(c->d_rowk, sizeof(int32_t) * rowk.size()))) return rc;
+    SMD_HIP(c, hipMemcpy(c->d_kruns, runs.data(), sizeof(int4) * runs.size(), hipMemcpyHostToDevice));
+    SMD_HIP(c, hipMemcpy(c->d_rowk, rowk.data(), sizeof(int32_t) * rowk.size(), hipMemcpyHostToDevice));
     SMD_HIP(c, hipMemcpy(c->d_kxy, xy.data(), sizeof(int32_t) * xy.size(), hipMemcpyHostToDevice));
     SMD_HIP(c, hipMemcpy(c->d_expk, rexp.data(), sizeof(double) * rexp.size(), hipMemcpyHostToDevice));
     c->n_krows = kr.nrows;
@@ -259,6 +303,12 @@ int ewald_surface(Ctx* c) {
 struct RecipArgs {
     int n, K, chunks, per;     // atoms per chunk, a multiple of KS_TILE
     int vpw;                   // tiles per wave of the structure factors at a time
+    KsSets sets;               // with Lustig terms
+    int nper;                  // n of a row per block of k_recip_reduce
+    int ng;                    // runs
+    const int4* runs;
+    const int32_t* rowk;       // [nrows + 1] first k of each row
+    double4* am;               // [n] (q, d) per atom, d = r - R_mol
     KsRows kr;
     double vk[3];              // 2 pi / L per axis
     const double* pos;
@@ -266,7 +316,7 @@ struct RecipArgs {
     const int32_t* mol;
     const double* com;
     const double* expk;        // [nrows][n1]
-    double* part;              // [chunk][nrows][weights][4][n1]
+    double* part;              // [chunk][nrows][weights][4][n1], of k_recip_walk [chunk][K][WALK_SUMS]
     void* kf;                  // force-pass coefficients, R
     double2* e1;               // [n][3] exp(i 2 pi r_p / L_p) per atom
     double* force;
@@ -310,54 +360,191 @@ __global__ __launch_bounds__(KS_THREADS) void k_recip_sfac(RecipArgs a) {
     extern __shared__ double lds[];
     const int i0 = blockIdx.x * a.per, i1 = min(a.n, i0 + a.per);
     const RecipAtoms at{a, blockIdx.y == 0};
-    ks_sfac<R, NW>(a.kr, at, i0, i1, blockIdx.y, gridDim.y, a.vpw,
-                   ks_tables<R>(a.kr, NW, a.per / KS_TILE), lds,
-                   a.part + (size_t)blockIdx.x * a.kr.nrows * NW * 4 * a.kr.n1);
+    const int nt = ks_tables<R>(a.kr, NW, a.per / KS_TILE);
+    double* part = a.part + (size_t)blockIdx.x * a.kr.nrows * NW * 4 * a.kr.n1;
+    if constexpr (NW > 1) ks_sfac_weights<R>(a.kr, at, i0, i1, blockIdx.y, a.sets.split, nt, lds, part);
+    else ks_sfac<R>(a.kr, at, i0, i1, blockIdx.y, gridDim.y, a.vpw, nt, lds, part);
 }
 
-// One block per row (and per padding row of the last tile, which only clears
-// its coefficients).  The waves sum an equal share of the chunks each, in
-// order, and their shares are added in order; then thread n takes the row's k
-// with nz = +-n.  Bound by the latency of the chunk loads, so a block is as
-// many waves as the sums' LDS allows.
+// FP64 with Lustig terms, many atoms: the matrix cores multiply FP64 at the
+// vector units' rate on this card, and five weights of 16-row tiles padded to
+// 16 functions are two to three times the arithmetic of a walk over the set
+// itself.  48,000 atoms: 725 k 45 us and the phases 5 (as products 65 to 77),
+// 1,535 k 93 + 6 (83 to 98); few atoms wait for latencies, which the products
+// spread over more blocks: 648 atoms, 1,535 k 13 + 2.5 us (10.5).
+__global__ __launch_bounds__(256) void k_recip_phase(RecipArgs a) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const RecipAtoms at{a, true};
+    if (k < a.n) {
+        double d[3];
+        at.offset(k, d);
+        a.am[k] = make_double4(a.q[k], d[0], d[1], d[2]);
+    }
+    if (k < 3 * a.n) at.phase(k / 3, k % 3);
+}
+
+// A block of WALK_WAVES waves owns 64 runs (one per lane) and a chunk of
+// atoms.  Per 64-atom table a lane starts its run at q X^nx Y^ny Z^nz0 and
+// walks along nz, each term the one before times Z.  Per k: 0 q sin, 1 q cos,
+// 2-4 q cos d, 5-7 q sin d, 8 q cos |d|^2, 9 q sin |d|^2 (reciprocal_term
+// :568-594 and the moments its force loop needs).  The waves split a table's
+// atoms and are added in LDS, in order.
+__global__ __launch_bounds__(WALK_WAVES * WAVE) void k_recip_walk(RecipArgs a) {
+    extern __shared__ double lds[];
+    static_assert(WALK_WAVES * WAVE >= 4 * KS_TILE, "one fill task per thread");
+    KsC<double>* tab = reinterpret_cast<KsC<double>*>(lds);
+    const int ts = a.kr.ts, ey0 = a.kr.nx1, ez0 = ey0 + a.kr.ny1;
+    double* misc = reinterpret_cast<double*>(tab + a.kr.table_entries());   // [5][KS_TILE]: q, d, |d|^2
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    const int g = blockIdx.x * WAVE + lane;
+    const int i0 = blockIdx.y * a.per, i1 = min(a.n, i0 + a.per);
+    const int4 run = g < a.ng ? a.runs[g] : make_int4(0, 0, 0, 0);
+    const int nx = ks_nx(run.z), ny = ks_ny(run.z);
+    const int ox = nx * ts, oy = (ey0 + abs(ny)) * ts, oz = (ez0 + abs(run.w)) * ts;
+    const double sy = ny < 0 ? -1.0 : 1.0, sz = run.w < 0 ? -1.0 : 1.0;
+    double acc[GK][WALK_SUMS];
+#pragma unroll
+    for (int t = 0; t < GK; ++t)
+#pragma unroll
+        for (int u = 0; u < WALK_SUMS; ++u) acc[t][u] = 0.0;
+    // thread fu + KS_TILE fp writes atom fu's powers along axis fp (fp < 3) or
+    // its moments; its inputs for the next table are loaded before the current
+    // one is walked
+    const int fu = threadIdx.x % KS_TILE, fp = threadIdx.x / KS_TILE;
+    double2 pe = make_double2(1.0, 0.0);
+    double4 pm = make_double4(0.0, 0.0, 0.0, 0.0);
+    auto fetch = [&](int t0) {
+        const int ia = t0 + fu;
+        if (fp < 3 && ia < i1) pe = a.e1[3 * ia + fp];
+        else if (fp == 3 && ia < i1) pm = a.am[ia];
+    };
+    fetch(i0);
+    for (int t0 = i0; t0 < i1; t0 += KS_TILE) {
+        const int na = min(KS_TILE, i1 - t0);
+        __syncthreads();
+        if (fp < 3 && fu < na) {
+            const int base = fp == 0 ? 0 : (fp == 1 ? ey0 : ez0);
+            ks_powers<double>(tab + (size_t)base * ts, ts, fu, fp == 0 ? a.kr.nx1 : (fp == 1 ? a.kr.ny1 : a.kr.n1), pe.x,
+                              pe.y, 1.0);
+        } else if (fp == 3 && fu < na) {
+            misc[fu] = pm.x;
+            misc[KS_TILE + fu] = pm.y;
+            misc[2 * KS_TILE + fu] = pm.z;
+            misc[3 * KS_TILE + fu] = pm.w;
+            misc[4 * KS_TILE + fu] = pm.y * pm.y + pm.z * pm.z + pm.w * pm.w;
+        }
+        __syncthreads();
+        fetch(t0 + KS_TILE);
+        if (g < a.ng)
+            for (int u = w; u < na; u += WALK_WAVES) {
+                KsC<double> Y = tab[oy + u], Z = tab[oz + u];
+                Y.im *= sy;
+                Z.im *= sz;
+                KsC<double> e = ks_mul(ks_mul(tab[ox + u], Y), Z);
+                const double q = misc[u];
+                e.re *= q;
+                e.im *= q;
+                // Z itself; without one (n1 = 1) a run has one k
+                const KsC<double> z1 = tab[(ez0 + min(1, a.kr.n1 - 1)) * ts + u];
+                const double dx = misc[KS_TILE + u], dy = misc[2 * KS_TILE + u], dz = misc[3 * KS_TILE + u];
+                const double d2 = misc[4 * KS_TILE + u];
+                // all GK sums are formed (uniform control flow); those past
+                // the run's count are never stored
+#pragma unroll
+                for (int t = 0; t < GK; ++t) {
+                    acc[t][0] += e.im;
+                    acc[t][1] += e.re;
+                    acc[t][2] += e.re * dx; acc[t][3] += e.re * dy; acc[t][4] += e.re * dz;
+                    acc[t][5] += e.im * dx; acc[t][6] += e.im * dy; acc[t][7] += e.im * dz;
+                    acc[t][8] += e.re * d2; acc[t][9] += e.im * d2;
+                    e = ks_mul(e, z1);
+                }
+            }
+    }
+    double* red = lds;   // [(WALK_WAVES - 1) * WAVE][WALK_SUMS]
+#pragma unroll
+    for (int t = 0; t < GK; ++t) {
+        __syncthreads();
+        if (w > 0)
+#pragma unroll
+            for (int u = 0; u < WALK_SUMS; ++u) red[((w - 1) * WAVE + lane) * WALK_SUMS + u] = acc[t][u];
+        __syncthreads();
+        if (w == 0 && t < run.y) {
+            double* p = a.part + ((size_t)blockIdx.y * a.K + run.x + t) * WALK_SUMS;
+#pragma unroll
+            for (int u = 0; u < WALK_SUMS; ++u) {
+                double s = acc[t][u];
+                for (int v = 0; v < WALK_WAVES - 1; ++v) s += red[(v * WAVE + lane) * WALK_SUMS + u];
+                p[u] = s;
+            }
+        }
+    }
+}
+
+// One block per row and nper n (and per padding row of the last tile, which only
+// clears its coefficients).  The waves sum an equal share of the chunks each,
+// in order, and their shares are added in order; then a thread takes the row's
+// k with nz = +-n.  Bound by the latency of the chunk loads, so a block is as
+// many waves as there are shares of a dozen chunks.
+// NW 0: the sums of k_recip_walk.
 template <typename R, int NW>
 __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
     extern __shared__ double lds[];
-    constexpr bool LUSTIG = NW > 1;
-    const int row = blockIdx.x, nv = NW * 4 * a.kr.n1;
+    constexpr bool WALK = NW == 0, LUSTIG = NW != 1;
+    const int parts = (a.kr.n1 + a.nper - 1) / a.nper, row = blockIdx.x / parts, n0 = blockIdx.x % parts * a.nper;
     const int lane = threadIdx.x % WAVE, qt = threadIdx.x / WAVE;
     R* kf = static_cast<R*>(a.kf);
-    ks_coef_pad<R>(a.kr, kf, row, threadIdx.x, blockDim.x);
+    if (n0 == 0) ks_coef_pad<R>(a.kr, kf, row, threadIdx.x, blockDim.x);
     double o[3 + 9 + 4] = {0};   // energy, longDeriv, long2ndDeriv, virial[9], Ff, Ffk2, d2UV1, d2UrR
     if (row < a.kr.nrows) {
-        const int nq = blockDim.x / WAVE;
-        const int c0 = (a.chunks * qt) / nq, c1 = (a.chunks * (qt + 1)) / nq;
-        const size_t stride = (size_t)a.kr.nrows * nv;
-        for (int v = lane; v < nv; v += WAVE) {
-            const double* p = a.part + (size_t)row * nv + v;
+        const int nn = min(a.nper, a.kr.n1 - n0);   // this block's n, at most 58: the set's limit on nmax
+        const int k0 = WALK ? a.rowk[row] : 0, count = WALK ? a.rowk[row + 1] - k0 : 0;
+        // the walk's row runs over nz = -m..m, the first over 1..m
+        const int m = a.kr.xy[row] == 0 ? count : (count - 1) / 2, zero = a.kr.xy[row] == 0 ? -1 : m;   // k of nz = 0
+        // values of +n and of -n (walk) or of all weights and products
+        const int nv = WALK ? 2 * nn * WALK_SUMS : NW * 4 * nn;
+        auto place = [&](int v) -> int64_t {
+            if constexpr (WALK) {
+                const int n = n0 + v / (2 * WALK_SUMS), neg = v / WALK_SUMS & 1, k = zero + (neg ? -n : n);
+                return n <= m && k >= 0 ? (int64_t)(k0 + k) * WALK_SUMS + v % WALK_SUMS : -1;
+            } else {
+                return ((int64_t)row * NW * 4 + v / nn) * a.kr.n1 + n0 + v % nn;
+            }
+        };
+        // wave qt: share qt / vw of the chunks, values qt % vw of vw
+        const int nw = blockDim.x / WAVE, vw = min((nv + WAVE - 1) / WAVE, nw), nq = nw / vw, q = qt / vw;
+        const int c0 = (a.chunks * q) / nq, c1 = (a.chunks * (q + 1)) / nq;
+        const size_t stride = WALK ? (size_t)a.K * WALK_SUMS : (size_t)a.kr.nrows * NW * 4 * a.kr.n1;
+        for (int v = (qt % vw) * WAVE + lane; v < nv && q < nq; v += vw * WAVE) {
+            const int64_t at = place(v);
             double s = 0.0;
+            if (at >= 0) {
+                const double* p = a.part + at;
 #pragma unroll 8
-            for (int ch = c0; ch < c1; ++ch) s += p[(size_t)ch * stride];
-            lds[qt * nv + v] = s;
+                for (int ch = c0; ch < c1; ++ch) s += p[(size_t)ch * stride];
+            }
+            lds[q * nv + v] = s;
         }
         __syncthreads();
         for (int v = threadIdx.x; v < nv; v += blockDim.x) {
             double s = lds[v];
-            for (int q = 1; q < nq; ++q) s += lds[q * nv + v];
+            for (int u = 1; u < nq; ++u) s += lds[u * nv + v];
             lds[v] = s;
         }
         __syncthreads();
-        const int n = threadIdx.x;   // n1 is at most 58: the set's limit on nmax
-        if (n < a.kr.n1) {
+        const int n = n0 + threadIdx.x;
+        if (threadIdx.x < nn) {
             const int v = a.kr.xy[row];
             const int nx = ks_nx(v), ny = ks_ny(v);
             const double ek = a.expk[(size_t)row * a.kr.n1 + n];
             const double kx = nx * a.vk[0], ky = ny * a.vk[1];
-            double sum[NW][4];
+            double sum[WALK ? 1 : NW][4];
+            if constexpr (!WALK) {
 #pragma unroll
-            for (int w = 0; w < NW; ++w)
+                for (int w = 0; w < NW; ++w)
 #pragma unroll
-                for (int p = 0; p < 4; ++p) sum[w][p] = lds[(w * 4 + p) * a.kr.n1 + n];
+                    for (int p = 0; p < 4; ++p) sum[w][p] = lds[(w * 4 + p) * nn + threadIdx.x];
+            }
             const double b = a.pi8V * ek;
             double G[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
             // +nz, and -nz where the half space has it
@@ -366,7 +553,25 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
                 const double sg = s ? -1.0 : 1.0;
                 const double kz = sg * n * a.vk[2];
                 const double k2 = kx * kx + ky * ky + kz * kz;
-                const double cosSum = sum[0][0] - sg * sum[0][3], sinSum = sum[0][2] + sg * sum[0][1];
+                const double* sk = lds + (2 * threadIdx.x + s) * WALK_SUMS;   // of the walk
+                double cosSum, sinSum, cd[4], sd[4];   // and with the weights d, |d|^2
+                if constexpr (WALK) {
+                    sinSum = sk[0];
+                    cosSum = sk[1];
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        cd[w] = sk[w < 3 ? 2 + w : 8];
+                        sd[w] = sk[w < 3 ? 5 + w : 9];
+                    }
+                } else {
+                    cosSum = sum[0][0] - sg * sum[0][3];
+                    sinSum = sum[0][2] + sg * sum[0][1];
+#pragma unroll
+                    for (int w = 0; w < NW - 1; ++w) {
+                        cd[w] = sum[w + 1][0] - sg * sum[w + 1][3];
+                        sd[w] = sum[w + 1][2] + sg * sum[w + 1][1];
+                    }
+                }
                 const double te = a.pi4V * ek * (sinSum * sinSum + cosSum * cosSum);
                 const double coeff = 2.0 * (a.alphaR4 + 1.0 / k2);
                 const double kk = (te * kx) * kx + (te * ky) * ky + (te * kz) * kz;
@@ -383,12 +588,6 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
                 o[3 + 2] += -te * coeff * kx * kz;
                 o[3 + 5] += -te * coeff * ky * kz;
                 if constexpr (LUSTIG) {
-                    double cd[4], sd[4];   // weights d, |d|^2
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        cd[w] = sum[w + 1][0] - sg * sum[w + 1][3];
-                        sd[w] = sum[w + 1][2] + sg * sum[w + 1][1];
-                    }
                     // sum_i val_i (k.d_i) with val_i = b (q_i sin_i C - q_i cos_i S)
                     const double kSD = kx * sd[0] + ky * sd[1] + kz * sd[2];
                     const double kCD = kx * cd[0] + ky * cd[1] + kz * cd[2];
@@ -445,7 +644,7 @@ __global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<R>) void k_recip_force(Rec
 template <typename R, bool FF>
 static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
     const dim3 g((a.n + KS_TILE - 1) / KS_TILE);
-    const int waves = ks_waves(a.kr.tiles(), 1, KS_MAXW, 3);
+    const int waves = ks_force_waves(a.kr, (int)g.x);
     const dim3 b(waves * WAVE);
     const size_t lds = ks_force_lds<R>(a.kr, waves);
     switch (a.kr.steps()) {
@@ -461,25 +660,46 @@ static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
     }
 }
 
+static unsigned recip_reduce_blocks(const RecipArgs& a) {
+    return (unsigned)(a.kr.tiles() * KS_ROWS * ((a.kr.n1 + a.nper - 1) / a.nper));
+}
+
+// NW 0: by k_recip_walk.
 template <typename R, int NW>
 static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes) {
     if (passes & RECIP_SFAC) {
-        // A chunk's (tile, weight) pairs go side by side over blocks only where
-        // the chunks alone leave CUs idle, since each block fills its own table.
-        const int nvt = a.kr.tiles() * NW, waves = ks_waves(nvt, a.vpw, KS_MAXW, 3);
-        const int groups = (nvt + waves * a.vpw - 1) / (waves * a.vpw);
-        int gy = std::min(groups, std::max(1, 256 / a.chunks));
-        gy = (groups + (groups + gy - 1) / gy - 1) / ((groups + gy - 1) / gy);   // no block with one group more
-        const size_t lds = ks_table_bytes<R>(a.kr, NW) * ks_tables<R>(a.kr, NW, a.per / KS_TILE);
-        hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(waves * WAVE), lds, s, a);
+        if constexpr (NW == 0) {
+            hipLaunchKernelGGL(k_recip_phase, dim3((3 * a.n + 255) / 256), dim3(256), 0, s, a);
+            const size_t lds = std::max(ks_table_bytes<double>(a.kr, KS_WEIGHTS),
+                                        (size_t)(WALK_WAVES - 1) * WAVE * WALK_SUMS * sizeof(double));
+            hipLaunchKernelGGL(k_recip_walk, dim3((a.ng + WAVE - 1) / WAVE, a.chunks), dim3(WALK_WAVES * WAVE), lds, s, a);
+        } else {
+            int waves, gy;
+            if constexpr (NW > 1) {
+                waves = a.sets.split * a.sets.units;
+                gy = a.sets.count;
+            } else {
+                // A chunk's tiles go side by side over blocks only where the
+                // chunks alone leave CUs idle, since each block fills its own
+                // table.
+                waves = ks_waves(a.kr.tiles(), a.vpw, KS_MAXW, 3);
+                const int sets = (a.kr.tiles() + waves * a.vpw - 1) / (waves * a.vpw) * a.kr.col_groups();
+                gy = std::min(sets, std::max(1, 256 / a.chunks));
+                gy = (sets + (sets + gy - 1) / gy - 1) / ((sets + gy - 1) / gy);   // no block with one set more
+            }
+            const size_t lds = ks_table_bytes<R>(a.kr, NW) * ks_tables<R>(a.kr, NW, a.per / KS_TILE);
+            hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(waves * WAVE), lds, s, a);
+        }
     }
     if (passes & RECIP_REDUCE) {
-        // a wave per dozen chunks, fewer where the row's sums are many: the
-        // loads of one wave follow each other, the epilogue waits for all
-        const size_t per_wave = sizeof(double) * NW * 4 * a.kr.n1;
-        const int waves = std::max(4, std::min({16, (a.chunks + 11) / 12, (int)(KS_TABLE_LDS / 2 / per_wave)}));
-        hipLaunchKernelGGL((k_recip_reduce<R, NW>), dim3(a.kr.tiles() * KS_ROWS), dim3(waves * WAVE), waves * per_wave,
-                           s, a);
+        // a share of the chunks for every dozen, as far as 16 waves hold all of a
+        // row's sums per share: the loads of one wave follow each other, the
+        // epilogue waits for all
+        const int nn = std::min(a.nper, a.kr.n1), nv = NW == 0 ? 2 * nn * WALK_SUMS : NW * 4 * nn;
+        const int vw = std::min(16, (nv + WAVE - 1) / WAVE);
+        const int nq = std::max(1, std::min(16 / vw, (a.chunks + 11) / 12)), waves = std::max(4, vw * nq);
+        const size_t lds = sizeof(double) * std::max(waves * WAVE, nv);
+        hipLaunchKernelGGL((k_recip_reduce<R, NW>), dim3(recip_reduce_blocks(a)), dim3(waves * WAVE), lds, s, a);
     }
 }
 
@@ -490,7 +710,7 @@ struct RecipScratch { double* kf; double* part; double* e1; int chunks; };
 static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const RecipScratch& sc);
 
 int ewald_recip(Ctx* c, int prec, int lustig, unsigned passes) {
-    return ewald_recip_with(c, prec, lustig, passes, RecipScratch{c->d_kf, c->d_sfac_part, c->d_e1, c->sfac_chunks});
+    return ewald_recip_with(c, prec, lustig, passes, RecipScratch{c->d_kf, c->d_sfac_part, c->d_e1, lustig ? SF_CHUNKS : c->sfac_chunks});
 }
 
 // ---- the allocation-free form's scratch -------------------------------------
@@ -530,12 +750,23 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
     a.kr.n1 = c->nmax[2] + 1;
     a.kr.ts = prec == SMD_PREC_MIXED ? ks_stride<float>() : ks_stride<double>();
     a.kr.xy = c->d_kxy;
-    // whole tiles per chunk
-    const int nt = (c->n + KS_TILE - 1) / KS_TILE;
-    const int most = lustig ? std::min(sc.chunks, SF_CHUNKS_LUSTIG) : sc.chunks;
-    a.per = (nt + most - 1) / most * KS_TILE;
+    a.ng = c->n_kruns;
+    a.runs = c->d_kruns;
+    a.rowk = c->d_rowk;
+    const bool mixed = prec == SMD_PREC_MIXED;
+    bool walk = false;
+    if (lustig) {
+        const LustigPlan p = lustig_plan(a.kr, c->n, c->K, c->n_kruns, sc.chunks, mixed);
+        walk = p.walk;
+        a.sets = p.sets;
+        a.per = p.per;
+    } else {   // whole tiles per chunk
+        const int nt = (c->n + KS_TILE - 1) / KS_TILE;
+        a.per = (nt + sc.chunks - 1) / sc.chunks * KS_TILE;
+    }
     a.chunks = (c->n + a.per - 1) / a.per;
     a.vpw = a.chunks < 128 ? 1 : KS_VT;   // one tile per wave while blocks are few
+    a.nper = a.kr.tiles() * KS_ROWS * a.kr.col_groups() <= c->red.cap ? 16 : a.kr.n1;
     for (int d = 0; d < 3; ++d) a.vk[d] = 2.0 * PI / c->box.L[d];
     a.pos = c->d_pos;
     a.q = c->d_q;
@@ -545,6 +776,7 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
     a.part = sc.part;
     a.kf = sc.kf;
     a.e1 = reinterpret_cast<double2*>(sc.e1);
+    a.am = reinterpret_cast<double4*>(sc.e1 + e1_am_offset(c->n));
     a.store = c->recip_store ? 1 : 0;
     a.force = c->recip_store ? c->d_frecip : c->d_force;
     a.red = c->red;
@@ -552,20 +784,20 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
     const double volume = c->box.L[0] * c->box.L[1] * c->box.L[2];
     a.pi4V = 4.0 * PI * (1.0 / volume);
     a.pi8V = 2.0 * a.pi4V;
-    const bool mixed = prec == SMD_PREC_MIXED;
     for (unsigned pass : {(unsigned)RECIP_SFAC, (unsigned)RECIP_REDUCE}) {
         if (!(passes & pass)) continue;
         ProfScope ps(c, pass == RECIP_SFAC ? "recip_sfac" : "recip_reduce");
         if (mixed) {
-            if (lustig) launch_recip_sums<float, NSUM>(c->stream, a, pass);
+            if (lustig) launch_recip_sums<float, KS_WEIGHTS>(c->stream, a, pass);
             else launch_recip_sums<float, 1>(c->stream, a, pass);
         } else {
-            if (lustig) launch_recip_sums<double, NSUM>(c->stream, a, pass);
+            if (walk) launch_recip_sums<double, 0>(c->stream, a, pass);
+            else if (lustig) launch_recip_sums<double, KS_WEIGHTS>(c->stream, a, pass);
             else launch_recip_sums<double, 1>(c->stream, a, pass);
         }
         SMD_HIP(c, hipGetLastError());
         if (pass == RECIP_REDUCE) {
-            const int rc = red_finish(c, RS_RECIP, a.kr.tiles() * KS_ROWS, lustig ? 16 : 12, c->d_terms + T_RC_E);
+            const int rc = red_finish(c, RS_RECIP, recip_reduce_blocks(a), lustig ? 16 : 12, c->d_terms + T_RC_E);
             if (rc) return rc;
         }
     }
@@ -684,22 +916,23 @@ extern "C" int smd_ewald_compute_long_static(smd_ctx* c, int prec, smd_ewald_lon
     if (!c->static_scratch) return fail(c, SMD_ESTATE, "static scratch not resolved for device %d", c->device);
     auto up = [](size_t v) { return (v + 31) / 32 * 32; };   // 256-byte segments
     // The documented room: 80 bytes per atom, 16 per k and 80 per (k, chunk),
-    // with a chunk per 64 k-runs and CU but at least 32 atoms in each.  The
-    // passes take 48 per atom, the coefficients and the partials; what the
-    // documented room admits leaves them 18 chunks and more.
+    // with a chunk per 64 k-runs and CU but at least 32 atoms in each.  What
+    // it admits leaves the passes, whose coefficients and mixed partials take
+    // more, chunks enough.
     const int gt = (c->n_kruns + WAVE - 1) / WAVE;
     const int quota = std::max(1, 256 / gt);
     const int per = std::max(32, (c->n + quota - 1) / quota);
     const size_t need = up(((6 * (size_t)c->n + 3) & ~(size_t)3) + 4 * (size_t)c->n) + up(2 * (size_t)c->K) +
                         up((size_t)10 * c->K * ((c->n + per - 1) / per));
-    const size_t n_e1 = up(6 * (size_t)c->n);
+    const size_t n_e1 = up(e1_am_offset(c->n) + 4 * (size_t)c->n);
     KsRows kr{};
     kr.nrows = c->n_krows;
     kr.n1 = c->nmax[2] + 1;
     const size_t n_kf = up(kr.coef_entries());
     // as many chunks as the rest of the array holds
     const size_t rest = n_e1 + n_kf < STATIC_SCRATCH_DOUBLES ? STATIC_SCRATCH_DOUBLES - n_e1 - n_kf : 0;
-    const int chunks = (int)std::min<size_t>(c->sfac_chunks, rest / c->k_part);
+    const size_t part = lustig_plan(kr, c->n, c->K, c->n_kruns, SF_CHUNKS, prec == SMD_PREC_MIXED).part;
+    const int chunks = (int)std::min<size_t>(SF_CHUNKS, rest / part);
     if (need > STATIC_SCRATCH_DOUBLES || chunks < 1)
         return fail(c, SMD_ECAPACITY,
                     "static scratch holds %zu bytes; %d atoms and %d k-vectors need %zu (use smd_ewald_compute_long)",

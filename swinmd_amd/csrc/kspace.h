@@ -34,7 +34,7 @@ template <typename R> constexpr int KS_FORCE_OCC = sizeof(R) == 8 ? 3 : 4;
 constexpr int KS_ROWS = 16;       // rows of a matrix tile
 constexpr int KS_VT = 2;          // tiles per wave of the structure-factor pass
 constexpr int KS_MAXSTEP = 8;     // inner steps held in registers by the force pass
-// LDS of a table: two blocks to a CU with the force pass's partials beside it
+// LDS of the tables: two blocks to a CU with the force pass's partials beside them
 // (12 KiB more), which together are what one launch may ask for at most.
 constexpr size_t KS_TABLE_LDS = 65536, KS_CU_LDS = 163840;
 static_assert(2 * (KS_TABLE_LDS + (size_t)KS_MAXW * KS_TILE * 3 * sizeof(double)) <= KS_CU_LDS, "k-space LDS");
@@ -85,6 +85,7 @@ struct KsRows {
     __host__ __device__ int tiles() const { return (nrows + KS_ROWS - 1) / KS_ROWS; }
     __host__ __device__ int powers() const { return nx1 + ny1 + n1; }
     __host__ __device__ int steps() const { return (2 * n1 + 3) / 4; }   // of four functions
+    __host__ __device__ int col_groups() const { return (n1 + 15) / 16; }
     __host__ __device__ size_t table_entries() const { return (size_t)powers() * ts; }
     // per-row coefficients of the force pass: [tile][4][4 steps][16]
     __host__ __device__ size_t coef_entries() const { return (size_t)tiles() * 4 * steps() * 4 * KS_ROWS; }
@@ -104,8 +105,10 @@ __device__ __forceinline__ void ks_powers(KsC<R>* tab, int ts, int u, int cnt, d
     }
 }
 
-// Tables (with several weights also their values) of the structure-factor
-// pass that fit in KS_TABLE_LDS, at most KS_TABLES: a block fills them together, so their loads and phases overlap.
+// Tables (with several weights also their values) of a structure-factor pass
+// that a block fills together, so that their loads and phases overlap: as many
+// as fit in KS_TABLE_LDS, or with several weights in twice that, one block to
+// a CU being what its accumulators leave room for; at most KS_TABLES.
 constexpr int KS_TABLES = 4;
 template <typename R>
 __host__ __device__ inline size_t ks_table_bytes(const KsRows& kr, int nw) {
@@ -113,159 +116,234 @@ __host__ __device__ inline size_t ks_table_bytes(const KsRows& kr, int nw) {
 }
 template <typename R>
 __host__ __device__ inline int ks_tables(const KsRows& kr, int nw, int chunk_tiles) {
-    const int fit = (int)(KS_TABLE_LDS / ks_table_bytes<R>(kr, nw));
+    const int fit = (int)((nw > 1 ? 2 : 1) * KS_TABLE_LDS / ks_table_bytes<R>(kr, nw));
     const int m = fit < KS_TABLES ? fit : KS_TABLES;
     return m < 1 ? 1 : (m < chunk_tiles ? m : chunk_tiles);
 }
 
-// Structure factors of atoms [i0, i1) for the (tile, weight) pairs of groups
-// g0, g0 + gs, ... of vpw per wave (vpw at most KS_VT), by one block with
-// `nt` tables: out[((row NW + w) 4 + p) n1 + n] is the sum over the atoms of
-// w_i times a c_n, a s_n, b c_n, b s_n (p = 0..3), w_i = 1 or, with NW = 5,
-// also d_i and |d_i|^2 (d = r - R_mol).  At gives an atom's phase per axis,
-// its charge and d.  Columns past i1 have charge 0.  Tables that hold the
-// whole chunk stay for all the block's groups.
+// Tables of atoms t0.. up to i1: a wave per (table, axis or weights), lane u
+// filling column u.  Columns past i1 have charge 0.
 template <typename R, int NW, typename At>
-__device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, int i1, int g0, int gs, int vpw,
-                                        int nt, void* lds, double* __restrict__ out) {
-    typedef KsMat<R> M;
+__device__ __forceinline__ void ks_fill(const KsRows& kr, const At& at, int t0, int i1, int nt, KsC<R>* tabs) {
+    constexpr int TASKS = NW > 1 ? 4 : 3;
     const size_t te = ks_table_bytes<R>(kr, NW) / sizeof(KsC<R>);   // a table, then its weights
-    KsC<R>* const tabs = static_cast<KsC<R>*>(lds);
     const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int nvt = kr.tiles() * NW, nw = blockDim.x / WAVE;
-    // a wave per (table, axis or weights); lane u fills column u
-    auto fill = [&](int t0) {
-        constexpr int TASKS = NW > 1 ? 4 : 3;
-        for (int task = w; task < nt * TASKS; task += nw) {
-            const int tb = task / TASKS, fp = task % TASKS;
-            const int ia = t0 + tb * KS_TILE + lane;
-            const bool live = ia < i1;
-            KsC<R>* tab = tabs + tb * te;
-            if (fp < 3) {
-                double2 p = make_double2(1.0, 0.0);
-                double f = 1.0;
-                if (live) p = at.phase(ia, fp);
-                if (fp == 0) f = live ? at.charge(ia) : 0.0;
-                const int base = fp == 0 ? 0 : (fp == 1 ? kr.nx1 : kr.nx1 + kr.ny1);
-                ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, lane, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x,
-                             p.y, f);
-            } else {
-                double d[3] = {0.0, 0.0, 0.0};
-                if (live) at.offset(ia, d);
-                R* q = reinterpret_cast<R*>(tab + kr.table_entries()) + lane;
-                q[0] = R(1);
-                q[KS_TILE] = (R)d[0];
-                q[2 * KS_TILE] = (R)d[1];
-                q[3 * KS_TILE] = (R)d[2];
-                q[4 * KS_TILE] = (R)(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-            }
+    for (int task = w; task < nt * TASKS; task += blockDim.x / WAVE) {
+        const int tb = task / TASKS, fp = task % TASKS;
+        const int ia = t0 + tb * KS_TILE + lane;
+        const bool live = ia < i1;
+        KsC<R>* tab = tabs + tb * te;
+        if (fp < 3) {
+            double2 p = make_double2(1.0, 0.0);
+            double f = 1.0;
+            if (live) p = at.phase(ia, fp);
+            if (fp == 0) f = live ? at.charge(ia) : 0.0;
+            const int base = fp == 0 ? 0 : (fp == 1 ? kr.nx1 : kr.nx1 + kr.ny1);
+            ks_powers<R>(tab + (size_t)base * kr.ts, kr.ts, lane, fp == 0 ? kr.nx1 : (fp == 1 ? kr.ny1 : kr.n1), p.x, p.y,
+                         f);
+        } else {
+            double d[3] = {0.0, 0.0, 0.0};
+            if (live) at.offset(ia, d);
+            R* q = reinterpret_cast<R*>(tab + kr.table_entries()) + lane;
+            q[0] = R(1);
+            q[KS_TILE] = (R)d[0];
+            q[2 * KS_TILE] = (R)d[1];
+            q[3 * KS_TILE] = (R)d[2];
+            q[4 * KS_TILE] = (R)(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
         }
-    };
-    bool filled = false;
-    const bool stay = i1 - i0 <= nt * KS_TILE;
-    for (int vt0 = g0 * nw * vpw; vt0 < nvt; vt0 += gs * nw * vpw) {
-        // this wave's pairs and, per pair, this lane's row of the tile
-        int ox[KS_VT], oy[KS_VT], wt[KS_VT];
-        R sy[KS_VT];
-        bool on[KS_VT];
-        // FP64 products add up in their accumulators; FP32 ones enter FP64
-        // sums after every table
-        constexpr bool SPLIT = sizeof(R) == 4;
-        typename M::acc acc[KS_VT][4];
-        double tot[SPLIT ? KS_VT : 1][4][4];
+    }
+}
+
+// This lane's place in a unit of the structure factors, 16 rows by 16 n.
+template <typename R>
+struct KsUnit {
+    int ox, oy, oz;
+    R sy;
+    __device__ __forceinline__ KsUnit(const KsRows& kr, int tile, int cg) {
+        const int lane = threadIdx.x % WAVE;
+        const int v = kr.xy[min(tile * KS_ROWS + lane % 16, kr.nrows - 1)];
+        ox = ks_nx(v) * kr.ts;
+        oy = (kr.nx1 + abs(ks_ny(v))) * kr.ts;
+        oz = (kr.nx1 + kr.ny1 + min(lane % 16 + 16 * cg, kr.n1 - 1)) * kr.ts;
+        sy = ks_ny(v) < 0 ? R(-1) : R(1);
+    }
+    __device__ __forceinline__ KsC<R> row(const KsC<R>* tab, int u) const {
+        KsC<R> y = tab[oy + u];
+        y.im *= sy;
+        return ks_mul(tab[ox + u], y);
+    }
+};
+
+// Sums of the four products {a, b} {c_n, s_n} of one unit and weight: FP64
+// products add up in their accumulators, FP32 ones enter FP64 sums after every
+// table.
+template <typename R>
+struct KsAcc {
+    static constexpr bool SPLIT = sizeof(R) == 4;
+    typename KsMat<R>::acc acc[4];
+    double tot[SPLIT ? 4 : 1][SPLIT ? 4 : 1];
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-        for (int t = 0; t < KS_VT; ++t) {
-            const int vt = vt0 + w + t * nw;
-            on[t] = t < vpw && vt < nvt;
-            const int row = min((on[t] ? vt / NW : 0) * KS_ROWS + lane % 16, kr.nrows - 1);
-            const int v = kr.xy[row];
-            wt[t] = vt % NW;
-            ox[t] = ks_nx(v) * kr.ts;
-            oy[t] = (kr.nx1 + abs(ks_ny(v))) * kr.ts;
-            sy[t] = ks_ny(v) < 0 ? R(-1) : R(1);
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[p][r] = R(0);
+                if constexpr (SPLIT) tot[p][r] = 0.0;
+            }
+    }
+    __device__ __forceinline__ void add(R er, R ei, KsC<R> z) {
+        typedef KsMat<R> M;
+        acc[0] = M::mul(er, z.re, acc[0]);
+        acc[1] = M::mul(er, z.im, acc[1]);
+        acc[2] = M::mul(ei, z.re, acc[2]);
+        acc[3] = M::mul(ei, z.im, acc[3]);
+    }
+    __device__ __forceinline__ void table_end() {
+        if constexpr (SPLIT) {
 #pragma unroll
             for (int p = 0; p < 4; ++p)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    acc[t][p][r] = R(0);
-                    if constexpr (SPLIT) tot[t][p][r] = 0.0;
+                    tot[p][r] += (double)acc[p][r];
+                    acc[p][r] = R(0);
                 }
-        }
-        // columns are n = lane % 16 + 16 c; more than 16 functions take further passes
-        for (int nc = 0; nc * 16 < kr.n1; ++nc) {
-            const int oz = (kr.nx1 + kr.ny1 + min(lane % 16 + 16 * nc, kr.n1 - 1)) * kr.ts;
-            for (int t0 = i0; t0 < i1; t0 += KS_TILE) {
-                const int tb = (t0 - i0) / KS_TILE % nt;
-                if (tb == 0 && !filled) {
-                    __syncthreads();
-                    fill(t0);
-                    __syncthreads();
-                    filled = stay;
-                }
-                const KsC<R>* tab = tabs + tb * te;
-                const R* wts = reinterpret_cast<const R*>(tab + kr.table_entries());
-                // One or both pairs per pass over the table, without a branch
-                // inside, so the reads of later steps are issued ahead of the
-                // products; columns past i1 add zeros.
-                auto products = [&](auto pairs) {
-#pragma unroll 4
-                    for (int k = 0; k < KS_TILE / 4; ++k) {
-                        const int u = 4 * k + lane / 16;
-                        const KsC<R> z = tab[oz + u];
-#pragma unroll
-                        for (int t = 0; t < decltype(pairs)::value; ++t) {
-                            KsC<R> y = tab[oy[t] + u];
-                            y.im *= sy[t];
-                            KsC<R> e = ks_mul(tab[ox[t] + u], y);
-                            if constexpr (NW > 1) {
-                                const R f = wts[wt[t] * KS_TILE + u];
-                                e.re *= f;
-                                e.im *= f;
-                            }
-                            acc[t][0] = M::mul(e.re, z.re, acc[t][0]);
-                            acc[t][1] = M::mul(e.re, z.im, acc[t][1]);
-                            acc[t][2] = M::mul(e.im, z.re, acc[t][2]);
-                            acc[t][3] = M::mul(e.im, z.im, acc[t][3]);
-                        }
-                    }
-                };
-                if (on[1]) products(std::integral_constant<int, 2>{});   // wave-uniform
-                else if (on[0]) products(std::integral_constant<int, 1>{});
-                if constexpr (SPLIT) {
-#pragma unroll
-                    for (int t = 0; t < KS_VT; ++t)
-#pragma unroll
-                        for (int p = 0; p < 4; ++p)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                tot[t][p][r] += (double)acc[t][p][r];
-                                acc[t][p][r] = R(0);
-                            }
-                }
-            }
-            const int n = lane % 16 + 16 * nc;
-#pragma unroll
-            for (int t = 0; t < KS_VT; ++t) {
-                const int vt = vt0 + w + t * nw;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = (vt / NW) * KS_ROWS + M::row(lane, r);
-                    const bool st = on[t] && n < kr.n1 && row < kr.nrows;
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) {
-                        double* o = out + ((size_t)(row * NW + wt[t]) * 4 + p) * kr.n1 + n;
-                        if constexpr (SPLIT) {
-                            if (st) *o = tot[t][p][r];
-                            tot[t][p][r] = 0.0;
-                        } else {
-                            if (st) *o = acc[t][p][r];
-                            acc[t][p][r] = R(0);
-                        }
-                    }
-                }
-            }
         }
     }
+    // out[((row nw + w) 4 + p) n1 + n]
+    __device__ __forceinline__ void store(const KsRows& kr, double* __restrict__ out, int nw, int tile, int cg, int w) const {
+        const int lane = threadIdx.x % WAVE, n = lane % 16 + 16 * cg;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = tile * KS_ROWS + KsMat<R>::row(lane, r);
+            if (n < kr.n1 && row < kr.nrows)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    double* o = out + ((size_t)(row * nw + w) * 4 + p) * kr.n1 + n;
+                    if constexpr (SPLIT) *o = tot[p][r];
+                    else *o = acc[p][r];
+                }
+        }
+    }
+};
+
+// Structure factors of atoms [i0, i1), by one block with `nt` tables:
+// out[(row 4 + p) n1 + n] is the sum over the atoms of a c_n, a s_n, b c_n,
+// b s_n (p = 0..3).  The block takes the (group of 16 n, vpw tiles per wave)
+// sets g0, g0 + gs, ... (vpw at most KS_VT).  At gives an atom's phase per axis
+// and its charge.  Tables that hold the whole chunk stay for all of the
+// block's sets.
+template <typename R, typename At>
+__device__ __forceinline__ void ks_sfac(const KsRows& kr, const At& at, int i0, int i1, int g0, int gs, int vpw, int nt,
+                                        void* lds, double* __restrict__ out) {
+    const size_t te = ks_table_bytes<R>(kr, 1) / sizeof(KsC<R>);
+    KsC<R>* const tabs = static_cast<KsC<R>*>(lds);
+    const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int nw = blockDim.x / WAVE, groups = (kr.tiles() + nw * vpw - 1) / (nw * vpw);
+    bool filled = false;
+    const bool stay = i1 - i0 <= nt * KS_TILE;
+    for (int g = g0; g < groups * kr.col_groups(); g += gs) {
+        const int cg = g / groups, tile0 = g % groups * nw * vpw + w;
+        const bool on0 = tile0 < kr.tiles(), on1 = vpw > 1 && tile0 + nw < kr.tiles();
+        const KsUnit<R> unit[KS_VT] = {{kr, on0 ? tile0 : 0, cg}, {kr, on1 ? tile0 + nw : 0, cg}};
+        KsAcc<R> sum[KS_VT];
+#pragma unroll
+        for (int t = 0; t < KS_VT; ++t) sum[t].clear();
+        for (int t0 = i0; t0 < i1; t0 += KS_TILE) {
+            const int tb = (t0 - i0) / KS_TILE % nt;
+            if (tb == 0 && !filled) {
+                __syncthreads();
+                ks_fill<R, 1>(kr, at, t0, i1, nt, tabs);
+                __syncthreads();
+                filled = stay;
+            }
+            const KsC<R>* tab = tabs + tb * te;
+            // One or both tiles per pass over the table, without a branch
+            // inside, so the reads of later steps are issued ahead of the
+            // products; columns past i1 add zeros.
+            auto products = [&](auto tiles) {
+#pragma unroll 4
+                for (int k = 0; k < KS_TILE / 4; ++k) {
+                    const int u = 4 * k + lane / 16;
+                    const KsC<R> z = tab[unit[0].oz + u];
+#pragma unroll
+                    for (int t = 0; t < decltype(tiles)::value; ++t) {
+                        const KsC<R> e = unit[t].row(tab, u);
+                        sum[t].add(e.re, e.im, z);
+                    }
+                }
+            };
+            if (on1) products(std::integral_constant<int, 2>{});   // wave-uniform
+            else if (on0) products(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int t = 0; t < KS_VT; ++t) sum[t].table_end();
+        }
+        if (on0) sum[0].store(kr, out, 1, tile0, cg, 0);
+        if (on1) sum[1].store(kr, out, 1, tile0 + nw, cg, 0);
+    }
+}
+
+// The same with the weights 1, d_i and |d_i|^2 (d = r - R_mol, from At's
+// offset): out[((row 5 + w) 4 + p) n1 + n].  A block of `split` h waves takes
+// the h units (tile, group of 16 n) of set g, a wave the unit v % h with a
+// share of the weights: split 2, the first three or the other two, so that a
+// row's values are formed once for its weights, a SIMD holds a wave of each
+// kind and the chunk's atoms pass through the tables once; split 5, one each.
+constexpr int KS_WEIGHTS = 5;
+template <typename R, typename At>
+__device__ __forceinline__ void ks_sfac_weights(const KsRows& kr, const At& at, int i0, int i1, int g, int split, int nt,
+                                                void* lds, double* __restrict__ out) {
+    const size_t te = ks_table_bytes<R>(kr, KS_WEIGHTS) / sizeof(KsC<R>);
+    KsC<R>* const tabs = static_cast<KsC<R>*>(lds);
+    const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int h = blockDim.x / WAVE / split, id = g * h + w % h, part = w / h;
+    const int w0 = split == 2 ? 3 * part : part, nw = split == 2 ? 3 - part : 1;
+    const int tile = id % kr.tiles(), cg = id / kr.tiles();
+    const bool on = cg < kr.col_groups();
+    const KsUnit<R> unit(kr, tile, on ? cg : 0);
+    KsAcc<R> sum[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) sum[t].clear();
+    for (int t0 = i0; t0 < i1; t0 += KS_TILE) {
+        const int tb = (t0 - i0) / KS_TILE % nt;
+        if (tb == 0) {
+            __syncthreads();
+            ks_fill<R, KS_WEIGHTS>(kr, at, t0, i1, nt, tabs);
+            __syncthreads();
+        }
+        const KsC<R>* tab = tabs + tb * te;
+        const R* wts = reinterpret_cast<const R*>(tab + kr.table_entries()) + w0 * KS_TILE;
+        auto products = [&](auto weights) {
+#pragma unroll 2
+            for (int k = 0; k < KS_TILE / 4; ++k) {
+                const int u = 4 * k + lane / 16;
+                const KsC<R> z = tab[unit.oz + u], e = unit.row(tab, u);
+#pragma unroll
+                for (int t = 0; t < decltype(weights)::value; ++t) {
+                    const R f = wts[t * KS_TILE + u];
+                    sum[t].add(e.re * f, e.im * f, z);
+                }
+            }
+        };
+        if (on && nw == 3) products(std::integral_constant<int, 3>{});   // wave-uniform
+        else if (on && nw == 2) products(std::integral_constant<int, 2>{});
+        else if (on) products(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int t = 0; t < 3; ++t) sum[t].table_end();
+    }
+    if (on)
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            if (t < nw) sum[t].store(kr, out, KS_WEIGHTS, tile, cg, w0 + t);
+}
+// Its sets for nt tables of atoms: of at most four units, the same number in
+// all of them but the last; or where there is one unit, or units and tables
+// together make at most two blocks to a CU, a unit each with a wave per weight
+// (3,000 atoms, 1,535 k in FP64: compute_long 56 us, 59 with four units).
+struct KsSets { int count, units, split; };
+inline KsSets ks_weight_sets(const KsRows& kr, int nt) {
+    const int u = kr.tiles() * kr.col_groups(), sets = (u + KS_MAXW / 2 - 1) / (KS_MAXW / 2);
+    if (u == 1 || u * nt <= 512) return {u, 1, KS_WEIGHTS};
+    return {sets, (u + sets - 1) / sets, 2};
 }
 
 // The force pass's coefficients of one (row, n) from G+ = (bC, bS) of +nz and
@@ -303,10 +381,22 @@ inline size_t ks_force_lds(const KsRows& kr, int waves) {
     return ks_force_table<R>(kr) + (size_t)waves * KS_TILE * 3 * sizeof(double);
 }
 
+// Waves of the force pass for so many blocks: the tiles in turn, or where
+// tiles and blocks are few, each tile's four groups of 16 atoms over two or
+// four waves (ks_force_split).
+__host__ __device__ inline int ks_force_split(int tiles, int waves) {
+    return 4 * tiles <= waves ? 4 : (2 * tiles <= waves ? 2 : 1);
+}
+inline int ks_force_waves(const KsRows& kr, int blocks) {
+    const int t = kr.tiles(), split = blocks > 256 ? 1 : ks_force_split(t, KS_MAXW);
+    return split == 1 ? ks_waves(t, 1, KS_MAXW, 3) : (split * t < 3 ? 3 : split * t);
+}
+
 // sum_k (bC sin(k.r) - bS cos(k.r)) (nx, ny, nz) of atoms [i0, i0 + 64), by
 // one block of three waves or more: thread t < 192 returns atom i0 + t / 3,
-// component t % 3.  The waves take the 16-row tiles in turn, its coefficients in registers (KS inner
-// steps; 0: more than KS_MAXSTEP, read per product).
+// component t % 3.  A wave holds a tile's coefficients in registers, all KS
+// inner steps of them, or with KS = 0 (more than KS_MAXSTEP) KS_MAXSTEP (half
+// in FP64) at a time for two groups of atoms.
 template <typename R, int KS, typename At>
 __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const R* __restrict__ coef, int i0, int i1,
                                            void* lds) {
@@ -324,18 +414,13 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
     __syncthreads();
     const KsC<R>* tz = tab + (size_t)(kr.nx1 + kr.ny1) * kr.ts;
     const int steps = KS ? KS : kr.steps(), kp = 4 * steps;
+    const int split = ks_force_split(kr.tiles(), nw), tw = w / split, ntw = nw / split;
+    const int a0 = w % split * (4 / split), a1 = a0 + 4 / split;
     // functions 4 s + lane / 16: part (lane / 16) & 1 of power 2 s + lane / 32
     const R* tzp = reinterpret_cast<const R*>(tz) + ((lane / 16) & 1);
     double* part = reinterpret_cast<double*>(static_cast<char*>(lds) + ks_force_table<R>(kr)) + (size_t)w * KS_TILE * 3;
-    for (int tile = w; tile < kr.tiles(); tile += nw) {
+    for (int tile = tw; tile < kr.tiles(); tile += ntw) {
         const R* cw = coef + (size_t)tile * 4 * kp * KS_ROWS + lane;   // function lane / 16 of a step, row lane % 16
-        R A[4][KS ? KS : 1];
-        if constexpr (KS > 0) {
-#pragma unroll
-            for (int o = 0; o < 4; ++o)
-#pragma unroll
-                for (int s = 0; s < KS; ++s) A[o][s] = cw[((size_t)o * kp + 4 * s) * KS_ROWS];
-        }
         int ox[4], oy[4];
         R sy[4];
         double nx[4], ny[4];
@@ -348,24 +433,10 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
             nx[r] = (double)ks_nx(v);
             ny[r] = (double)ks_ny(v);
         }
-        for (int a = 0; a < 4; ++a) {
+        // the tile's share of the forces on atoms 16 a.. from its T
+        auto add = [&](int a, const typename M::acc (&T)[4]) {
             const int u = 16 * a + lane % 16;
             double g[3] = {0.0, 0.0, 0.0};
-            typename M::acc T[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-            if constexpr (KS > 0) {
-#pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    const R bz = tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + u)];
-#pragma unroll
-                    for (int o = 0; o < 4; ++o) T[o] = M::mul(A[o][s], bz, T[o]);
-                }
-            } else {
-                for (int s = 0; s < steps; ++s) {
-                    const R bz = tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + u)];
-#pragma unroll
-                    for (int o = 0; o < 4; ++o) T[o] = M::mul(cw[((size_t)o * kp + 4 * s) * KS_ROWS], bz, T[o]);
-                }
-            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 KsC<R> y = tab[oy[r] + u];
@@ -386,15 +457,66 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     double* o = part + 3 * u + d;
-                    *o = tile == w ? g[d] : *o + g[d];
+                    *o = tile == tw ? g[d] : *o + g[d];
                 }
+            }
+        };
+        auto function = [&](int s, int a) {
+            return tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + 16 * a + lane % 16)];
+        };
+        if constexpr (KS > 0) {
+            R A[4][KS];
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+#pragma unroll
+                for (int s = 0; s < KS; ++s) A[o][s] = cw[((size_t)o * kp + 4 * s) * KS_ROWS];
+            for (int a = a0; a < a1; ++a) {
+                typename M::acc T[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const R bz = function(s, a);
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) T[o] = M::mul(A[o][s], bz, T[o]);
+                }
+                add(a, T);
+            }
+        } else {
+            constexpr int HELD = sizeof(R) == 8 ? KS_MAXSTEP / 2 : KS_MAXSTEP;
+            // a group past the wave's last repeats it and is not added
+            for (int a = a0; a < a1; a += 2) {
+                const int b = min(a + 1, a1 - 1);
+                typename M::acc T[2][4] = {{{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+                                           {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}}};
+                for (int s0 = 0; s0 < steps; s0 += HELD) {
+                    R A[4][HELD];   // steps past the last: coefficients read again, times no function
+#pragma unroll
+                    for (int o = 0; o < 4; ++o)
+#pragma unroll
+                        for (int s = 0; s < HELD; ++s)
+                            A[o][s] = cw[((size_t)o * kp + 4 * min(s0 + s, steps - 1)) * KS_ROWS];
+#pragma unroll
+                    for (int s = 0; s < HELD; ++s) {
+                        const bool in = s0 + s < steps;
+                        const R ba = in ? function(s0 + s, a) : R(0), bb = in ? function(s0 + s, b) : R(0);
+#pragma unroll
+                        for (int o = 0; o < 4; ++o) {
+                            T[0][o] = M::mul(A[o][s], ba, T[0][o]);
+                            T[1][o] = M::mul(A[o][s], bb, T[1][o]);
+                        }
+                    }
+                }
+                add(a, T[0]);
+                if (b > a) add(b, T[1]);
             }
         }
     }
     __syncthreads();
     double f = 0.0;
-    if (threadIdx.x < 3 * KS_TILE)
-        for (int v = 0; v < min(nw, kr.tiles()); ++v) f += part[(ptrdiff_t)(v - w) * KS_TILE * 3 + threadIdx.x];
+    if (threadIdx.x < 3 * KS_TILE) {
+        const int a = (int)threadIdx.x / 3 / 16, aw = a / (4 / split);   // the waves of this atom's group
+        for (int v = 0; v < min(ntw, kr.tiles()); ++v)
+            f += part[(ptrdiff_t)(v * split + aw - w) * KS_TILE * 3 + threadIdx.x];
+    }
     return f;
 }
 

@@ -689,7 +689,7 @@ __global__ __launch_bounds__(KS_THREADS) void k_rows_sfac(Args a) {
     if (kr.nrows == 0) return;   // block-uniform: no k inside the cutoff
     const int c0 = rp.a0 + bm.z * a.sf_chunk, c1 = min(c0 + a.sf_chunk, rp.a1);
     const BatchAtoms at{a, rp, a.st[bm.x].tilt};
-    ks_sfac<double, 1>(kr, at, c0, c1, 0, 1, KS_VT, ks_tables<double>(kr, 1, a.sf_chunk / KS_TILE), lds,
+    ks_sfac<double>(kr, at, c0, c1, 0, 1, KS_VT, ks_tables<double>(kr, 1, a.sf_chunk / KS_TILE), lds,
                        a.sf_part + rp.pbase + (int64_t)bm.z * rp.rcap * 4 * kr.n1);
 }
 

@@ -172,10 +172,11 @@ struct Ctx {
     double* d_expk = nullptr;     // [n_krows][nmax_z + 1] exp(-k^2 / 4 alpha^2) / k^2
     int32_t* d_kxy = nullptr;     // [n_krows] nx << 16 | (ny & 0xffff)
     int n_krows = 0, n_kruns = 0; // (nx, ny) rows; runs of at most eight consecutive nz
-    size_t k_part = 0;            // doubles of one chunk's structure-factor partials with Lustig terms
+    int4* d_kruns = nullptr;      // [n_kruns] (first k, count, nx << 16 | ny, first nz)
+    int32_t* d_rowk = nullptr;    // [n_krows + 1] first k of each row
     double* d_sfac_part = nullptr;  // [chunks of a pass][its partials]
     double* d_kf = nullptr;         // force-pass coefficients, in its precision
-    double* d_e1 = nullptr;         // [n][3] complex exp(i 2 pi r_p / L_p)
+    double* d_e1 = nullptr;         // [n][3] complex exp(i 2 pi r_p / L_p), then [n] (q, r - R_mol)
     int sfac_chunks = 0;
 
     // vdW tables (device)

@@ -397,9 +397,9 @@ def test_direct_sheared_reciprocal_passes_match_the_oracle(prec, tiles):
 
 
 def test_ewald_setup_takes_the_memory_its_passes_use():
-    """5,462 waters, |n|^2 <= 81: the structure factors' partials are 64 chunks
-    of five weights (14 MB), the phases 0.8 MB; 12 MB for the tables and the
-    allocator's pages."""
+    """5,462 waters, |n|^2 <= 81: the structure factors' partials are 128 chunks
+    of five weights (26 MB: two sets of row tiles a chunk, a block per CU), the
+    phases 0.8 MB; 12 MB for the tables and the allocator's pages."""
     import ctypes as C
     from swinmd_amd.forces import Context, EwaldForce
     s = S.water(5462, density_mol=RHO, seed=1, subset=True)
@@ -417,7 +417,7 @@ def test_ewald_setup_takes_the_memory_its_passes_use():
     ew = EwaldForce(ctx, alpha=3.5, real_cut=0.9, kcut=S.kcut_for(81, s.box[0]))
     took = before - left()
     rows = sum(1 for x in range(10) for y in range(0 if x == 0 else -9, 10) if x * x + y * y <= 81)
-    assert took <= 64 * 5 * 4 * 10 * rows * 8 + 48 * s.n_atoms + 12e6, took
+    assert took <= 128 * 5 * 4 * 10 * rows * 8 + 48 * s.n_atoms + 12e6, took
     # the passes with and without Lustig sums stay inside it
     assert np.isfinite(ew.compute_long(np.zeros((s.n_atoms, 3)))["energy"])
     ctx.close()
@@ -504,4 +504,46 @@ def test_cell_list_of_fewer_atoms_than_cells(n):
     goff, gnb = ctx.pairlist()
     np.testing.assert_array_equal(goff, off)
     np.testing.assert_array_equal(gnb, nb)
+    ctx.close()
+
+
+# molecules, edges, k cut as a count of the longest edge's waves: many units of
+# rows and functions in several sets, functions past 16 with atoms enough for
+# the FP64 walk, five tiles, and one tile over several tables a chunk
+@pytest.mark.parametrize("n,edges,waves", [(1100, (3.2, 3.2, 3.2), 11.85), (1000, (1.5, 1.5, 18.0), 49.5),
+                                           (2200, (4.04, 4.04, 4.04), 7.04), (5600, (5.5, 5.5, 5.5), 2.1)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_lustig_sums_of_many_atoms_match_the_oracle(n, edges, waves, mixed):
+    """Forces, energy, virial and volume derivatives of EwaldForce.compute_long,
+    the bars of the smaller shapes; and the step's k-space, which forms no
+    d-weighted sums, gives the same energy and forces."""
+    from oracle import oracle as O
+    from swinmd_amd.forces import Context, EwaldForce, LJForce, WaterMD
+    s = S.water(n, box=edges[0], seed=n, subset=True, jitter=0.01)
+    s.__class__ = _BoxedWater
+    s.pos = s.pos + (np.repeat(s.pos[1::3], 3, axis=0) * (np.array(edges) / edges[0] - 1))   # whole molecules
+    s.edges = edges
+    kcut = 2 * np.pi * waves / max(edges)
+    prec = L.PREC_MIXED if mixed else L.PREC_FP64
+    print(f"case lustig n={n} edges={edges} waves={waves} mixed={mixed}", flush=True)
+    ctx = Context(s)
+    ctx.compute_mol_centers()
+    ew = EwaldForce(ctx, alpha=3.5, real_cut=0.5, kcut=kcut, prec=prec)
+    f = np.zeros((s.n_atoms, 3))
+    out = ew.compute_long(f)
+    fo, eo = O.Oracle(s).ewald_recip(kcut, 3.5)
+    tol = 1e-5 if mixed else 1e-10
+    assert rel_rms(f, fo) <= tol
+    for k in ("energy", "deriv", "deriv2"):
+        assert abs(out[k] - eo[k]) <= tol * max(abs(eo[k]), abs(eo["energy"])), k
+    assert rel_rms(out["virial"], eo["virial"]) <= tol
+    ctx.set_pairlist(0.5, 0.05, False)
+    LJForce(ctx, cutoff=0.5, prec=prec).compute(f)
+    ew.compute(f)
+    ctx.set_velocities(np.zeros_like(f))
+    md = WaterMD(ctx, cutoff=0.5, cut_buff=0.05, alpha=3.5, kcut=kcut, dt=1e-4, temperature=300.0, use_cells=False,
+                 prec=prec)
+    md.init()
+    assert rel(md.run(1)["e_long"], out["energy"]) <= tol
+    assert rel_rms(ctx.forces(), f) <= tol
     ctx.close()

@@ -626,7 +626,7 @@ __global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<R>) void k_recip_force(Rec
     extern __shared__ double lds[];
     const int i0 = blockIdx.x * KS_TILE;
     const RecipPhases at{a.e1};
-    const double g = ks_force<R, KS>(a.kr, at, static_cast<const R*>(a.kf), i0, a.n, lds);
+    const double g = ks_force<R, KS, true>(a.kr, at, static_cast<const R*>(a.kf), i0, a.n, lds);
     const int i = i0 + (int)threadIdx.x / 3, d = threadIdx.x % 3;
     double ff[1] = {0.0};
     if (threadIdx.x < 3 * KS_TILE && i < a.n) {

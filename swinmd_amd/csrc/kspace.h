@@ -396,8 +396,9 @@ inline int ks_force_waves(const KsRows& kr, int blocks) {
 // one block of three waves or more: thread t < 192 returns atom i0 + t / 3,
 // component t % 3.  A wave holds a tile's coefficients in registers, all KS
 // inner steps of them, or with KS = 0 (more than KS_MAXSTEP) KS_MAXSTEP (half
-// in FP64) at a time for two groups of atoms.
-template <typename R, int KS, typename At>
+// in FP64) at a time for two groups of atoms.  SPLIT: the launch may have split
+// the tiles' atoms over waves.
+template <typename R, int KS, bool SPLIT, typename At>
 __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const R* __restrict__ coef, int i0, int i1,
                                            void* lds) {
     typedef KsMat<R> M;
@@ -414,7 +415,7 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
     __syncthreads();
     const KsC<R>* tz = tab + (size_t)(kr.nx1 + kr.ny1) * kr.ts;
     const int steps = KS ? KS : kr.steps(), kp = 4 * steps;
-    const int split = ks_force_split(kr.tiles(), nw), tw = w / split, ntw = nw / split;
+    const int split = SPLIT ? ks_force_split(kr.tiles(), nw) : 1, tw = w / split, ntw = nw / split;
     const int a0 = w % split * (4 / split), a1 = a0 + 4 / split;
     // functions 4 s + lane / 16: part (lane / 16) & 1 of power 2 s + lane / 32
     const R* tzp = reinterpret_cast<const R*>(tz) + ((lane / 16) & 1);
@@ -470,7 +471,7 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
             for (int o = 0; o < 4; ++o)
 #pragma unroll
                 for (int s = 0; s < KS; ++s) A[o][s] = cw[((size_t)o * kp + 4 * s) * KS_ROWS];
-            for (int a = a0; a < a1; ++a) {
+            auto group = [&](int a) {
                 typename M::acc T[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
                 for (int s = 0; s < KS; ++s) {
@@ -479,7 +480,11 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
                     for (int o = 0; o < 4; ++o) T[o] = M::mul(A[o][s], bz, T[o]);
                 }
                 add(a, T);
-            }
+            };
+            if (split == 1)   // all four, a loop of known length
+                for (int a = 0; a < 4; ++a) group(a);
+            else
+                for (int a = a0; a < a1; ++a) group(a);
         } else {
             constexpr int HELD = sizeof(R) == 8 ? KS_MAXSTEP / 2 : KS_MAXSTEP;
             // a group past the wave's last repeats it and is not added

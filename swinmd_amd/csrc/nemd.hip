@@ -759,7 +759,7 @@ __global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<double>) void k_rows_force
     const Rep rp = a.rep[bm.x];
     const KsRows kr = rep_rows(a, rp, a.st[bm.x].nrows);
     const BatchPhases at{a.e1};
-    const double g = ks_force<double, KS>(kr, at, a.coef + rp.cbase, bm.y, rp.a1, lds);
+    const double g = ks_force<double, KS, false>(kr, at, a.coef + rp.cbase, bm.y, rp.a1, lds);
     __syncthreads();
     if (threadIdx.x < 3 * KS_TILE) lds[threadIdx.x] = g;
     __syncthreads();

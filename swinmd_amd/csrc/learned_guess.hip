@@ -1163,7 +1163,10 @@ int smd_mlp_get_norm(smd_ctx* c, float* norm, int64_t count) {
 static int upload_rows(Ctx* c, const float* x, int64_t rows) {
     const size_t n = (size_t)rows * MF;
     const std::unique_ptr<uint16_t[]> xb(new uint16_t[n]);   // not cleared: every entry is written
-    for (size_t k = 0; k < n; ++k) {   // the kernels' rounding, on the host
+    // the kernels' rounding, on the host; four vectors in flight (forward of
+    // 100,000 rows 600-603 us wherever the loop lands, one at a time 640-680)
+#pragma clang loop interleave_count(4)
+    for (size_t k = 0; k < n; ++k) {
         uint32_t u;
         std::memcpy(&u, &x[k], 4);
         u += 0x7FFFu + ((u >> 16) & 1u);

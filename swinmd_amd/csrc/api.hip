@@ -255,7 +255,7 @@ extern "C" int smd_ctx_create(smd_ctx** out, const smd_topology* t, int device) 
     auto A = [&](auto*& p, size_t bytes) {
         if (!ok) return;
         if (hipMalloc(&p, bytes ? bytes : 8) != hipSuccess) ok = false;
-        else if (hipMemset(p, 0, bytes ? bytes : 8) != hipSuccess) ok = false;
+        else if (hipMemsetAsync(p, 0, bytes ? bytes : 8, c->stream) != hipSuccess) ok = false;
     };
     const int nt2 = t->n_types * t->n_types;
     A(c->d_type, sizeof(int32_t) * n);
@@ -312,7 +312,7 @@ extern "C" int smd_ctx_create(smd_ctx** out, const smd_topology* t, int device) 
         delete c;
         return SMD_ENOMEM;
     }
-    hipError_t e = hipSuccess;
+    hipError_t e = hipStreamSynchronize(c->stream);   // the copies below take the null stream
     auto H = [&](void* dst, const void* src, size_t bytes) {
         if (e == hipSuccess) e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
     };

@@ -1666,8 +1666,8 @@ extern "C" int smd_set_multipoles(smd_ctx* c, const double* dip_local, const dou
             (rc = A(c->d_cg_scal, sizeof(double) * 8)))
             return rc;
         c->cg_parts = parts;
-        SMD_HIP(c, hipMemset(c->d_mu, 0, sizeof(double) * 3 * n));
-        SMD_HIP(c, hipMemset(c->d_e0_prev, 0, sizeof(double) * 3 * n));
+        SMD_HIP(c, hipMemsetAsync(c->d_mu, 0, sizeof(double) * 3 * n, c->stream));
+        SMD_HIP(c, hipMemsetAsync(c->d_e0_prev, 0, sizeof(double) * 3 * n, c->stream));
     }
     SMD_HIP(c, hipStreamSynchronize(c->stream));
     SMD_HIP(c, hipMemcpy(c->d_dipl, dip_local, sizeof(double) * 3 * n, hipMemcpyHostToDevice));

@@ -1105,7 +1105,7 @@ static int kset_build(Ctx* c, Ctx::KSet& ks, double alpha, double kcut, int nsum
         return rc;
     if (!c->d_mp_trq && (rc = R(c->d_mp_trq, sizeof(double) * 15 * (size_t)c->n))) return rc;
     if (!c->d_mp_terms && (rc = R(c->d_mp_terms, sizeof(double) * M_COUNT))) return rc;
-    SMD_HIP(c, hipMemset(c->d_mp_trq, 0, sizeof(double) * 15 * (size_t)c->n));
+    SMD_HIP(c, hipMemsetAsync(c->d_mp_trq, 0, sizeof(double) * 15 * (size_t)c->n, c->stream));
     SMD_HIP(c, hipMemcpy(ks.kvec, kv.data(), sizeof(double) * 3 * K, hipMemcpyHostToDevice));
     SMD_HIP(c, hipMemcpy(ks.kmod2, k2v.data(), sizeof(double) * K, hipMemcpyHostToDevice));
     SMD_HIP(c, hipMemcpy(ks.expk, ekv.data(), sizeof(double) * K, hipMemcpyHostToDevice));

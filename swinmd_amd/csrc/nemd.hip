@@ -1502,9 +1502,9 @@ extern "C" int smd_batch_create(smd_batch** out, const smd_batch_params* p, int 
                       dalloc(b, b->d_e1, n3) ? SMD_ENOMEM : SMD_OK;
     else rc = dalloc(b, b->d_kvec, kb) || dalloc(b, b->d_kf, kb) ? SMD_ENOMEM : SMD_OK;
     if (rc) return rc;
-    BHIP(b, hipMemset(b->d_err, 0, sizeof(unsigned)));
-    BHIP(b, hipMemset(b->d_out, 0, sizeof(smd_batch_report) * b->R));
-    BHIP(b, hipMemset(b->d_nb_cnt, 0, sizeof(int32_t) * a));
+    BHIP(b, hipMemsetAsync(b->d_err, 0, sizeof(unsigned), b->stream));
+    BHIP(b, hipMemsetAsync(b->d_out, 0, sizeof(smd_batch_report) * b->R, b->stream));
+    BHIP(b, hipMemsetAsync(b->d_nb_cnt, 0, sizeof(int32_t) * a, b->stream));
     return build_tables(b);
 }
 
@@ -1556,7 +1556,7 @@ extern "C" int smd_batch_set_state(smd_batch* b, const double* pos, const double
     BHIP(b, hipMemcpy(b->d_com, com.data(), sizeof(double) * com.size(), hipMemcpyHostToDevice));
     BHIP(b, hipMemcpy(b->d_mom, zero.data(), sizeof(double) * com.size(), hipMemcpyHostToDevice));
     BHIP(b, hipMemcpy(b->d_st, st.data(), sizeof(RepState) * b->R, hipMemcpyHostToDevice));
-    BHIP(b, hipMemset(b->d_err, 0, sizeof(unsigned)));
+    BHIP(b, hipMemsetAsync(b->d_err, 0, sizeof(unsigned), b->stream));
     b->have_state = true;
     b->started = false;
     return SMD_OK;

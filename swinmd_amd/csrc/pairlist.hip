@@ -679,7 +679,9 @@ int pairlist_build(Ctx* c, double cutoff, double cut_buff, int use_cells, bool o
             SMD_HIP(c, hipMalloc(&c->d_cell_cnt, sizeof(int32_t) * (nc + 1)));
             SMD_HIP(c, hipMalloc(&c->d_cell_start, sizeof(int32_t) * (nc + 1)));
             // k_list_hits clears the counts after each use; they start at zero
-            SMD_HIP(c, hipMemset(c->d_cell_cnt, 0, sizeof(int32_t) * (nc + 1)));
+            // (hipMemset returns before it is done, and this stream does not
+            // wait for the null stream)
+            SMD_HIP(c, hipMemsetAsync(c->d_cell_cnt, 0, sizeof(int32_t) * (nc + 1), c->stream));
             c->cell_alloc = nc + 1;
         }
         // hit bits for neighbour cells of up to twice the mean occupancy

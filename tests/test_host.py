@@ -39,6 +39,18 @@ def test_uniform_stream_is_the_reference_lcg():
     assert list(u) == [s1 / 1048576, s2 / 1048576, s3 / 1048576]
 
 
+def test_device_memory_is_cleared_on_the_stream_that_uses_it():
+    """hipMemset goes to the null stream and returns before it is done; the
+    library's streams are non-blocking and do not wait for it, so a kernel of
+    theirs could read or add to memory before it is cleared."""
+    src = os.path.join(ROOT, "swinmd_amd", "csrc")
+    for name in sorted(os.listdir(src)):
+        text = open(os.path.join(src, name)).read()
+        assert not re.search(r"\bhipMemset(D\d+|2D|3D)?\s*\(", text), name
+        for call in re.findall(r"\bhipMemset(?:D\d+|2D|3D)?Async\s*\([^;]*;", text):
+            assert re.search(r"stream2?\s*\)", call), (name, call)
+
+
 def _erfc_constants():
     src = open(os.path.join(ROOT, "swinmd_amd", "csrc", "smd_internal.h")).read()
     p = float(re.search(r"ERFC_P\s*=\s*([0-9.eE+-]+)f", src).group(1))

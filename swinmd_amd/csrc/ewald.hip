@@ -491,7 +491,7 @@ template <typename R, int NW>
 __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
     extern __shared__ double lds[];
     constexpr bool WALK = NW == 0, LUSTIG = NW != 1;
-    const int parts = (a.kr.n1 + a.nper - 1) / a.nper, row = blockIdx.x / parts, n0 = blockIdx.x % parts * a.nper;
+    const int row = blockIdx.y, n0 = blockIdx.x * a.nper, blocks = gridDim.x * gridDim.y;
     const int lane = threadIdx.x % WAVE, qt = threadIdx.x / WAVE;
     R* kf = static_cast<R*>(a.kf);
     if (n0 == 0) ks_coef_pad<R>(a.kr, kf, row, threadIdx.x, blockDim.x);
@@ -508,11 +508,12 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
                 const int n = n0 + v / (2 * WALK_SUMS), neg = v / WALK_SUMS & 1, k = zero + (neg ? -n : n);
                 return n <= m && k >= 0 ? (int64_t)(k0 + k) * WALK_SUMS + v % WALK_SUMS : -1;
             } else {
+                if (nn == a.kr.n1) return (int64_t)row * nv + v;
                 return ((int64_t)row * NW * 4 + v / nn) * a.kr.n1 + n0 + v % nn;
             }
         };
         // wave qt: share qt / vw of the chunks, values qt % vw of vw
-        const int nw = blockDim.x / WAVE, vw = min((nv + WAVE - 1) / WAVE, nw), nq = nw / vw, q = qt / vw;
+        const int nw = blockDim.x / WAVE, vw = NW == 1 ? 1 : min((nv + WAVE - 1) / WAVE, nw), nq = nw / vw, q = qt / vw;
         const int c0 = (a.chunks * q) / nq, c1 = (a.chunks * (q + 1)) / nq;
         const size_t stride = WALK ? (size_t)a.K * WALK_SUMS : (size_t)a.kr.nrows * NW * 4 * a.kr.n1;
         for (int v = (qt % vw) * WAVE + lane; v < nv && q < nq; v += vw * WAVE) {
@@ -609,8 +610,8 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
         o[3 + 7] = o[3 + 5];
     }
     // the sums are in the first wave; the rest of the block has none
-    if (threadIdx.x < WAVE && (int)gridDim.x <= a.red.cap) {
-        double* part = red_part(a.red, RS_RECIP) + blockIdx.x;
+    if (threadIdx.x < WAVE && blocks <= a.red.cap) {
+        double* part = red_part(a.red, RS_RECIP) + blockIdx.y * gridDim.x + blockIdx.x;
 #pragma unroll
         for (int k = 0; k < (LUSTIG ? 16 : 12); ++k) {
             const double t = wave_sum(o[k]);
@@ -621,12 +622,12 @@ __global__ __launch_bounds__(1024) void k_recip_reduce(RecipArgs a) {
 
 // Force on atom i, sum_k (b C q sin - b S q cos) k (:609-658).  FF: also the
 // block's sum of F . d (T_RC_FF).
-template <typename R, int KS, bool FF>
+template <typename R, int KS, bool FF, bool SPLIT>
 __global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<R>) void k_recip_force(RecipArgs a) {
     extern __shared__ double lds[];
     const int i0 = blockIdx.x * KS_TILE;
     const RecipPhases at{a.e1};
-    const double g = ks_force<R, KS, true>(a.kr, at, static_cast<const R*>(a.kf), i0, a.n, lds);
+    const double g = ks_force<R, KS, SPLIT>(a.kr, at, static_cast<const R*>(a.kf), i0, a.n, lds);
     const int i = i0 + (int)threadIdx.x / 3, d = threadIdx.x % 3;
     double ff[1] = {0.0};
     if (threadIdx.x < 3 * KS_TILE && i < a.n) {
@@ -641,27 +642,31 @@ __global__ __launch_bounds__(KS_THREADS, KS_FORCE_OCC<R>) void k_recip_force(Rec
     }
 }
 
-template <typename R, bool FF>
-static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
-    const dim3 g((a.n + KS_TILE - 1) / KS_TILE);
-    const int waves = ks_force_waves(a.kr, (int)g.x);
-    const dim3 b(waves * WAVE);
+template <typename R, bool FF, bool SPLIT>
+static void launch_recip_force(hipStream_t s, const RecipArgs& a, int waves) {
+    const dim3 g((a.n + KS_TILE - 1) / KS_TILE), b(waves * WAVE);
     const size_t lds = ks_force_lds<R>(a.kr, waves);
     switch (a.kr.steps()) {
-        case 1: hipLaunchKernelGGL((k_recip_force<R, 1, FF>), g, b, lds, s, a); break;
-        case 2: hipLaunchKernelGGL((k_recip_force<R, 2, FF>), g, b, lds, s, a); break;
-        case 3: hipLaunchKernelGGL((k_recip_force<R, 3, FF>), g, b, lds, s, a); break;
-        case 4: hipLaunchKernelGGL((k_recip_force<R, 4, FF>), g, b, lds, s, a); break;
-        case 5: hipLaunchKernelGGL((k_recip_force<R, 5, FF>), g, b, lds, s, a); break;
-        case 6: hipLaunchKernelGGL((k_recip_force<R, 6, FF>), g, b, lds, s, a); break;
-        case 7: hipLaunchKernelGGL((k_recip_force<R, 7, FF>), g, b, lds, s, a); break;
-        case 8: hipLaunchKernelGGL((k_recip_force<R, 8, FF>), g, b, lds, s, a); break;
-        default: hipLaunchKernelGGL((k_recip_force<R, 0, FF>), g, b, lds, s, a); break;
+        case 1: hipLaunchKernelGGL((k_recip_force<R, 1, FF, SPLIT>), g, b, lds, s, a); break;
+        case 2: hipLaunchKernelGGL((k_recip_force<R, 2, FF, SPLIT>), g, b, lds, s, a); break;
+        case 3: hipLaunchKernelGGL((k_recip_force<R, 3, FF, SPLIT>), g, b, lds, s, a); break;
+        case 4: hipLaunchKernelGGL((k_recip_force<R, 4, FF, SPLIT>), g, b, lds, s, a); break;
+        case 5: hipLaunchKernelGGL((k_recip_force<R, 5, FF, SPLIT>), g, b, lds, s, a); break;
+        case 6: hipLaunchKernelGGL((k_recip_force<R, 6, FF, SPLIT>), g, b, lds, s, a); break;
+        case 7: hipLaunchKernelGGL((k_recip_force<R, 7, FF, SPLIT>), g, b, lds, s, a); break;
+        case 8: hipLaunchKernelGGL((k_recip_force<R, 8, FF, SPLIT>), g, b, lds, s, a); break;
+        default: hipLaunchKernelGGL((k_recip_force<R, 0, FF, SPLIT>), g, b, lds, s, a); break;
     }
 }
+template <typename R, bool FF>
+static void launch_recip_force(hipStream_t s, const RecipArgs& a) {
+    const int waves = ks_force_waves(a.kr, (a.n + KS_TILE - 1) / KS_TILE, sizeof(R) == 4);
+    if (ks_force_split(a.kr.tiles(), waves) > 1) launch_recip_force<R, FF, true>(s, a, waves);
+    else launch_recip_force<R, FF, false>(s, a, waves);
+}
 
-static unsigned recip_reduce_blocks(const RecipArgs& a) {
-    return (unsigned)(a.kr.tiles() * KS_ROWS * ((a.kr.n1 + a.nper - 1) / a.nper));
+static dim3 recip_reduce_grid(const RecipArgs& a) {
+    return dim3((a.kr.n1 + a.nper - 1) / a.nper, a.kr.tiles() * KS_ROWS);
 }
 
 // NW 0: by k_recip_walk.
@@ -696,10 +701,10 @@ static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes
         // row's sums per share: the loads of one wave follow each other, the
         // epilogue waits for all
         const int nn = std::min(a.nper, a.kr.n1), nv = NW == 0 ? 2 * nn * WALK_SUMS : NW * 4 * nn;
-        const int vw = std::min(16, (nv + WAVE - 1) / WAVE);
+        const int vw = NW == 1 ? 1 : std::min(16, (nv + WAVE - 1) / WAVE);
         const int nq = std::max(1, std::min(16 / vw, (a.chunks + 11) / 12)), waves = std::max(4, vw * nq);
-        const size_t lds = sizeof(double) * std::max(waves * WAVE, nv);
-        hipLaunchKernelGGL((k_recip_reduce<R, NW>), dim3(recip_reduce_blocks(a)), dim3(waves * WAVE), lds, s, a);
+        const size_t lds = sizeof(double) * std::max(waves * std::max(WAVE, NW == 1 ? nv : 0), nv);
+        hipLaunchKernelGGL((k_recip_reduce<R, NW>), recip_reduce_grid(a), dim3(waves * WAVE), lds, s, a);
     }
 }
 
@@ -797,7 +802,8 @@ static int ewald_recip_with(Ctx* c, int prec, int lustig, unsigned passes, const
         }
         SMD_HIP(c, hipGetLastError());
         if (pass == RECIP_REDUCE) {
-            const int rc = red_finish(c, RS_RECIP, recip_reduce_blocks(a), lustig ? 16 : 12, c->d_terms + T_RC_E);
+            const dim3 g = recip_reduce_grid(a);
+            const int rc = red_finish(c, RS_RECIP, (int)(g.x * g.y), lustig ? 16 : 12, c->d_terms + T_RC_E);
             if (rc) return rc;
         }
     }

@@ -383,20 +383,24 @@ inline size_t ks_force_lds(const KsRows& kr, int waves) {
 
 // Waves of the force pass for so many blocks: the tiles in turn, or where
 // tiles and blocks are few, each tile's four groups of 16 atoms over two or
-// four waves (ks_force_split).
+// four waves (ks_force_split).  In FP64 over four only, up to a block for half
+// the CUs: beside the pair kernel its waves take what that kernel has (a step
+// of 4,096 waters with |n|^2 <= 27, three tiles over two waves 113 us, else
+// 104; 1,500, 90 and 86; mixed 86, 88).
 __host__ __device__ inline int ks_force_split(int tiles, int waves) {
     return 4 * tiles <= waves ? 4 : (2 * tiles <= waves ? 2 : 1);
 }
-inline int ks_force_waves(const KsRows& kr, int blocks) {
-    const int t = kr.tiles(), split = blocks > 256 ? 1 : ks_force_split(t, KS_MAXW);
+inline int ks_force_waves(const KsRows& kr, int blocks, bool mixed) {
+    const int t = kr.tiles(), most = ks_force_split(t, KS_MAXW);
+    const int split = (mixed ? blocks <= 256 : blocks <= 128 && most == 4) ? most : 1;
     return split == 1 ? ks_waves(t, 1, KS_MAXW, 3) : (split * t < 3 ? 3 : split * t);
 }
 
 // sum_k (bC sin(k.r) - bS cos(k.r)) (nx, ny, nz) of atoms [i0, i0 + 64), by
 // one block of three waves or more: thread t < 192 returns atom i0 + t / 3,
 // component t % 3.  A wave holds a tile's coefficients in registers, all KS
-// inner steps of them, or with KS = 0 (more than KS_MAXSTEP) KS_MAXSTEP (half
-// in FP64) at a time for two groups of atoms.  SPLIT: the launch may have split
+// inner steps of them, or with KS = 0 (more than KS_MAXSTEP) KS_MAXSTEP at a
+// time for two groups of atoms, in FP64 half of that for one.  SPLIT: the launch may have split
 // the tiles' atoms over waves.
 template <typename R, int KS, bool SPLIT, typename At>
 __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const R* __restrict__ coef, int i0, int i1,
@@ -416,7 +420,7 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
     const KsC<R>* tz = tab + (size_t)(kr.nx1 + kr.ny1) * kr.ts;
     const int steps = KS ? KS : kr.steps(), kp = 4 * steps;
     const int split = SPLIT ? ks_force_split(kr.tiles(), nw) : 1, tw = w / split, ntw = nw / split;
-    const int a0 = w % split * (4 / split), a1 = a0 + 4 / split;
+    const int a0 = SPLIT ? w % split * (4 / split) : 0, a1 = SPLIT ? a0 + 4 / split : 4;
     // functions 4 s + lane / 16: part (lane / 16) & 1 of power 2 s + lane / 32
     const R* tzp = reinterpret_cast<const R*>(tz) + ((lane / 16) & 1);
     double* part = reinterpret_cast<double*>(static_cast<char*>(lds) + ks_force_table<R>(kr)) + (size_t)w * KS_TILE * 3;
@@ -463,7 +467,7 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
             }
         };
         auto function = [&](int s, int a) {
-            return tzp[2 * ((size_t)min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + 16 * a + lane % 16)];
+            return tzp[2 * (min(2 * s + lane / 32, kr.n1 - 1) * kr.ts + 16 * a + lane % 16)];   // within KS_TABLE_LDS
         };
         if constexpr (KS > 0) {
             R A[4][KS];
@@ -486,12 +490,12 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
             else
                 for (int a = a0; a < a1; ++a) group(a);
         } else {
-            constexpr int HELD = sizeof(R) == 8 ? KS_MAXSTEP / 2 : KS_MAXSTEP;
-            // a group past the wave's last repeats it and is not added
-            for (int a = a0; a < a1; a += 2) {
-                const int b = min(a + 1, a1 - 1);
-                typename M::acc T[2][4] = {{{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
-                                           {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}}};
+            // FP64 holds half the steps for a group at a time, which leaves room
+            // for another wave (300 waters in a box of 1:1:12, 1:1:6 with 500:
+            // a step 93 -> 87 us, 85 -> 82)
+            constexpr int GROUPS = sizeof(R) == 8 ? 1 : 2, HELD = KS_MAXSTEP * GROUPS / 2;
+            for (int a = a0; a < a1; a += GROUPS) {
+                typename M::acc T[GROUPS][4] = {};
                 for (int s0 = 0; s0 < steps; s0 += HELD) {
                     R A[4][HELD];   // steps past the last: coefficients read again, times no function
 #pragma unroll
@@ -502,16 +506,19 @@ __device__ __forceinline__ double ks_force(const KsRows& kr, const At& at, const
 #pragma unroll
                     for (int s = 0; s < HELD; ++s) {
                         const bool in = s0 + s < steps;
-                        const R ba = in ? function(s0 + s, a) : R(0), bb = in ? function(s0 + s, b) : R(0);
+                        if (GROUPS == 1 && !in) break;
 #pragma unroll
-                        for (int o = 0; o < 4; ++o) {
-                            T[0][o] = M::mul(A[o][s], ba, T[0][o]);
-                            T[1][o] = M::mul(A[o][s], bb, T[1][o]);
+                        for (int u = 0; u < GROUPS; ++u) {
+                            // a group past the wave's last repeats it and is not added
+                            const R bz = in ? function(s0 + s, SPLIT ? min(a + u, a1 - 1) : a + u) : R(0);
+#pragma unroll
+                            for (int o = 0; o < 4; ++o) T[u][o] = M::mul(A[o][s], bz, T[u][o]);
                         }
                     }
                 }
-                add(a, T[0]);
-                if (b > a) add(b, T[1]);
+#pragma unroll
+                for (int u = 0; u < GROUPS; ++u)
+                    if (!SPLIT || a + u < a1) add(a + u, T[u]);
             }
         }
     }

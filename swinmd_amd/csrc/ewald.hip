@@ -48,7 +48,7 @@ static LustigPlan lustig_plan(const KsRows& kr, int n, int K, int runs, int most
     const int nt = (n + KS_TILE - 1) / KS_TILE;
     LustigPlan p;
     p.sets = ks_weight_sets(kr, nt);
-    p.walk = !mixed && p.sets.split == 2;
+    p.walk = !mixed && p.sets.split == 2 && (!kr.half() || kr.tiles() * nt > 3072);
     if (p.walk) {
         const int c = std::max(1, std::min(most, SF_CHUNKS / ((runs + WAVE - 1) / WAVE)));
         p.per = std::max(32, (n + c - 1) / c);
@@ -355,23 +355,26 @@ struct RecipPhases {
 // 3.8 (phases) + 23.0, 6.2 and 20.9.  3,063 atoms in FP64: 11, 7.3, 11.9
 // against 3.0 + 17.4, 6.0 and 23.7; 48,000 atoms beside the pair kernel: the
 // step 383 -> 316 us.
-template <typename R, int NW>
+template <typename R, int NW, bool HALF>
 __global__ __launch_bounds__(KS_THREADS) void k_recip_sfac(RecipArgs a) {
     extern __shared__ double lds[];
     const int i0 = blockIdx.x * a.per, i1 = min(a.n, i0 + a.per);
     const RecipAtoms at{a, blockIdx.y == 0};
     const int nt = ks_tables<R>(a.kr, NW, a.per / KS_TILE);
     double* part = a.part + (size_t)blockIdx.x * a.kr.nrows * NW * 4 * a.kr.n1;
-    if constexpr (NW > 1) ks_sfac_weights<R>(a.kr, at, i0, i1, blockIdx.y, a.sets.split, nt, lds, part);
+    if constexpr (NW > 1) ks_sfac_weights<R, HALF>(a.kr, at, i0, i1, blockIdx.y, a.sets.split, nt, lds, part);
     else ks_sfac<R>(a.kr, at, i0, i1, blockIdx.y, gridDim.y, a.vpw, nt, lds, part);
 }
 
 // FP64 with Lustig terms, many atoms: the matrix cores multiply FP64 at the
 // vector units' rate on this card, and five weights of 16-row tiles padded to
 // 16 functions are two to three times the arithmetic of a walk over the set
-// itself.  48,000 atoms: 725 k 45 us and the phases 5 (as products 65 to 77),
-// 1,535 k 93 + 6 (83 to 98); few atoms wait for latencies, which the products
-// spread over more blocks: 648 atoms, 1,535 k 13 + 2.5 us (10.5).
+// itself.  48,000 atoms, 1,535 k 93 us and the phases 6 (as products 83 to 98);
+// few atoms wait for latencies, which the products spread over more blocks:
+// 648 atoms, 1,535 k 13 + 2.5 us (10.5).  Where c_n and s_n share the columns
+// the padding is half, and the products hold longer (lustig_plan).  A call of
+// compute_long with |n|^2 <= 49 at 24,576, 48,000 and 96,000 atoms: walk 72, 95
+// and 141 us, products 70, 99 and 154; <= 27: 61, 71 and 94 against 58, 70, 97.
 __global__ __launch_bounds__(256) void k_recip_phase(RecipArgs a) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     const RecipAtoms at{a, true};
@@ -693,7 +696,9 @@ static void launch_recip_sums(hipStream_t s, const RecipArgs& a, unsigned passes
                 gy = (sets + (sets + gy - 1) / gy - 1) / ((sets + gy - 1) / gy);   // no block with one set more
             }
             const size_t lds = ks_table_bytes<R>(a.kr, NW) * ks_tables<R>(a.kr, NW, a.per / KS_TILE);
-            hipLaunchKernelGGL((k_recip_sfac<R, NW>), dim3(a.chunks, gy), dim3(waves * WAVE), lds, s, a);
+            const dim3 g(a.chunks, gy), b(waves * WAVE);
+            if (NW > 1 && a.kr.half()) hipLaunchKernelGGL((k_recip_sfac<R, NW, (NW > 1)>), g, b, lds, s, a);
+            else hipLaunchKernelGGL((k_recip_sfac<R, NW, false>), g, b, lds, s, a);
         }
     }
     if (passes & RECIP_REDUCE) {

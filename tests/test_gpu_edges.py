@@ -509,9 +509,11 @@ def test_cell_list_of_fewer_atoms_than_cells(n):
 
 # molecules, edges, k cut as a count of the longest edge's waves: many units of
 # rows and functions in several sets, functions past 16 with atoms enough for
-# the FP64 walk, five tiles, and one tile over several tables a chunk
+# the FP64 walk, five tiles, one tile over several tables a chunk, and eight and
+# nine functions, on both sides of the shared columns
 @pytest.mark.parametrize("n,edges,waves", [(1100, (3.2, 3.2, 3.2), 11.85), (1000, (1.5, 1.5, 18.0), 49.5),
-                                           (2200, (4.04, 4.04, 4.04), 7.04), (5600, (5.5, 5.5, 5.5), 2.1)])
+                                           (2200, (4.04, 4.04, 4.04), 7.04), (5600, (5.5, 5.5, 5.5), 2.1),
+                                           (700, (2.8, 2.8, 2.8), 7.9), (700, (2.8, 2.8, 2.8), 8.1)])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_lustig_sums_of_many_atoms_match_the_oracle(n, edges, waves, mixed):
     """Forces, energy, virial and volume derivatives of EwaldForce.compute_long,

@@ -371,7 +371,8 @@ __global__ __launch_bounds__(KS_THREADS) void k_recip_sfac(RecipArgs a) {
 // 16 functions are two to three times the arithmetic of a walk over the set
 // itself.  48,000 atoms, 1,535 k 93 us and the phases 6 (as products 83 to 98);
 // few atoms wait for latencies, which the products spread over more blocks:
-// 648 atoms, 1,535 k 13 + 2.5 us (10.5).  Where c_n and s_n share the columns
+// 648 atoms, 1,535 k 13 + 2.5 us (10.5).  Long axes pad most: 2,048 waters in a
+// 1:1:2 box, 78 us a call (86).  Where c_n and s_n share the columns
 // the padding is half, and the products hold longer (lustig_plan).  A call of
 // compute_long with |n|^2 <= 49 at 24,576, 48,000 and 96,000 atoms: walk 72, 95
 // and 141 us, products 70, 99 and 154; <= 27: 61, 71 and 94 against 58, 70, 97.
